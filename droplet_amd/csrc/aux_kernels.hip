@@ -2,6 +2,8 @@
 // field and diagnostics reductions (FP64).  None of these is on the per-step hot
 // path except the LES tau field, the eddy-viscosity part of the reference
 // `physics` (program/LES_drop.f90:598-693), computed after each step.
+#include <algorithm>
+
 #include "d3q15.h"
 #include "kernels.h"
 
@@ -217,14 +219,15 @@ constexpr int ZM_TX = 64, ZM_TY = 8, ZM_ZC = 16;
 constexpr int ZM_HX = ZM_TX + 2, ZM_HP = ZM_HX * (ZM_TY + 2), ZM_NT = ZM_TX * ZM_TY;
 constexpr int ZM_PER = (ZM_HP + ZM_NT - 1) / ZM_NT;  // plane nodes per thread
 
-template <typename T> struct ZmPlane {
-    T v[ZM_PER][3];
+// the plane nodes one thread moves, NC fields each (consecutive fields of `mac` from field F0)
+template <typename T, int NC> struct ZmPlane {
+    T v[ZM_PER][NC];
 };
 
-template <typename T>
-__device__ __forceinline__ ZmPlane<T> zm_fetch(const Grid& G, const T* __restrict__ mac, int64_t N, int x0, int y0,
-                                               int zg, bool small) {
-    ZmPlane<T> r;
+template <typename T, int NC, int F0>
+__device__ __forceinline__ ZmPlane<T, NC> zm_fetch(const Grid& G, const T* __restrict__ mac, int64_t N, int x0, int y0,
+                                                   int zg, bool small) {
+    ZmPlane<T, NC> r;
     const int64_t zoff = (int64_t)G.nx * G.ny * wrap_any(zg, G.nz, small);
 #pragma unroll
     for (int i = 0; i < ZM_PER; i++) {
@@ -233,18 +236,18 @@ __device__ __forceinline__ ZmPlane<T> zm_fetch(const Grid& G, const T* __restric
         const int64_t g = wrap_any(x0 + h % ZM_HX - 1, G.nx, small) +
                           (int64_t)G.nx * wrap_any(y0 + h / ZM_HX - 1, G.ny, small) + zoff;
 #pragma unroll
-        for (int k = 0; k < 3; k++) r.v[i][k] = mac[(2 + k) * N + g];
+        for (int k = 0; k < NC; k++) r.v[i][k] = mac[(F0 + k) * N + g];
     }
     return r;
 }
 
-template <typename T> __device__ __forceinline__ void zm_store(const ZmPlane<T>& r, T (*dst)[ZM_HP]) {
+template <typename T, int NC> __device__ __forceinline__ void zm_store(const ZmPlane<T, NC>& r, T (*dst)[ZM_HP]) {
 #pragma unroll
     for (int i = 0; i < ZM_PER; i++) {
         const int h = threadIdx.x + i * ZM_NT;
         if (h < ZM_HP)
 #pragma unroll
-            for (int k = 0; k < 3; k++) dst[k][h] = r.v[i][k];
+            for (int k = 0; k < NC; k++) dst[k][h] = r.v[i][k];
     }
 }
 
@@ -262,15 +265,15 @@ __global__ __launch_bounds__(ZM_NT) void les_tau_fp64_zm(Grid G, Phys P, const d
     const double rmax = from_ordered_bits(range[2 * slot]), rmin = from_ordered_bits(range[2 * slot + 1]);
     const double rg = rmax - rmin;
     // ring slot of plane z' is (z' - zs + 1) mod 3
-    zm_store(zm_fetch<double>(G, mac, N, x0, y0, zs - 1, small), su[0]);
-    zm_store(zm_fetch<double>(G, mac, N, x0, y0, zs, small), su[1]);
-    zm_store(zm_fetch<double>(G, mac, N, x0, y0, zs + 1, small), su[2]);
+    zm_store(zm_fetch<double, 3, 2>(G, mac, N, x0, y0, zs - 1, small), su[0]);
+    zm_store(zm_fetch<double, 3, 2>(G, mac, N, x0, y0, zs, small), su[1]);
+    zm_store(zm_fetch<double, 3, 2>(G, mac, N, x0, y0, zs + 1, small), su[2]);
     const int64_t col = (int64_t)(in ? x : 0) + (int64_t)G.nx * (in ? y : 0);
     double phi_next = mac[col + (int64_t)G.nx * G.ny * zs];
     for (int z = zs; z < ze; z++) {
         const bool more = z + 1 < ze;  // plane z+2 is needed by plane z+1
-        ZmPlane<double> next;
-        if (more) next = zm_fetch<double>(G, mac, N, x0, y0, z + 2, small);
+        ZmPlane<double, 3> next;
+        if (more) next = zm_fetch<double, 3, 2>(G, mac, N, x0, y0, z + 2, small);
         const double phi = phi_next;
         if (more) phi_next = mac[col + (int64_t)G.nx * G.ny * (z + 1)];
         __syncthreads();
@@ -309,57 +312,152 @@ __global__ __launch_bounds__(ZM_NT) void les_tau_fp64_zm(Grid G, Phys P, const d
     }
 }
 
-// Diagnostics: per-workgroup partial sums, reduced in fixed order on the host.
+// s + v with the rounding error collected in c (TwoSum, Knuth)
+__device__ __forceinline__ void add_comp(double& s, double& c, double v) {
+    const double t = s + v, b = t - s;
+    c += (s - (t - b)) + (v - b);
+    s = t;
+}
+
+// Diagnostics: per-workgroup partial sums.
 // [0] sum phi  [1] sum 0.5|u|^2  [2] sum (d_a u_b + d_b u_a)^2  [3] sum |grad phi|
 // [4] sum psi(phi)  [5] sum p  [6..8] sum u  [9] sum_ab d_a phi d_b phi S_ab
-__global__ void reduce_fp64(Grid G, Phys P, const double* __restrict__ mac, double* __restrict__ partial) {
-    __shared__ double sh[NPART][4];
-    const int64_t N = (int64_t)G.nx * G.ny * G.nz;
-    const int64_t s = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    double v[NPART] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-    if (s < N) {
-        const int x = s % G.nx, y = (s / G.nx) % G.ny, z = s / ((int64_t)G.nx * G.ny);
-        const double ph = mac[s], pr = mac[N + s];
-        const double u1 = mac[2 * N + s], u2 = mac[3 * N + s], u3 = mac[4 * N + s];
-        double lap, g0, g1, g2, gu[3][3];
-        phi_stencil(G, mac, x, y, z, lap, g0, g1, g2);
-        u_stencil(G, mac + 2 * N, mac + 3 * N, mac + 4 * N, x, y, z, gu);
-        double e = 0.0;
-        for (int b = 0; b < 3; b++)
-            for (int a = 0; a < 3; a++) {
-                const double sab = gu[a][b] + gu[b][a];
-                e += sab * sab;
+// The 40 B per node it must read take 0.11 ms at 256^3; gathering the 56
+// neighbour values of every node through L2 took 0.69 ms (this kernel 0.44, bound by
+// its 56 LDS reads and about 350 FP64 instructions per node), and 65536 records summed
+// on the host another 0.6 ms.  So the workgroups
+// march in z like les_tau_fp64_zm, with phi, u of three planes in an LDS ring and
+// the next plane's loads in flight, over columns of zc planes; at most
+// REDUCE_MAX_BLOCKS of them run, each over a fixed set of columns, and leave one
+// record each.  Per-thread sums are compensated, so the longer per-thread chain
+// costs no accuracy against the tree over single nodes.
+__global__ __launch_bounds__(ZM_NT) void reduce_fp64(Grid G, Phys P, const double* __restrict__ mac,
+                                                     double* __restrict__ partial, int tiles_x, int tiles_y, int zc,
+                                                     int64_t items) {
+    __shared__ double su[3][4][ZM_HP];  // [ring slot][phi, u1, u2, u3][plane node]
+    __shared__ double sh[NPART][ZM_NT / 64];
+    const int64_t N = (int64_t)G.nx * G.ny * G.nz, nxy = (int64_t)G.nx * G.ny;
+    const bool small = G.nx <= ZM_TX || G.ny <= ZM_TY || G.nz <= 2;
+    const int tx = threadIdx.x % ZM_TX, ty = threadIdx.x / ZM_TX;
+    double s[NPART] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0}, comp[NPART] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+    auto plane = [&](int x0, int y0, int zg) {
+        // phi is field 0, u fields 2..4: two fetches of consecutive fields
+        ZmPlane<double, 4> r;
+        const ZmPlane<double, 1> a = zm_fetch<double, 1, 0>(G, mac, N, x0, y0, zg, small);
+        const ZmPlane<double, 3> b = zm_fetch<double, 3, 2>(G, mac, N, x0, y0, zg, small);
+#pragma unroll
+        for (int i = 0; i < ZM_PER; i++) {
+            r.v[i][0] = a.v[i][0];
+#pragma unroll
+            for (int k = 0; k < 3; k++) r.v[i][1 + k] = b.v[i][k];
+        }
+        return r;
+    };
+    for (int64_t item = blockIdx.x; item < items; item += gridDim.x) {
+        const int x0 = (int)(item % tiles_x) * ZM_TX, y0 = (int)((item / tiles_x) % tiles_y) * ZM_TY;
+        const int zs = (int)(item / ((int64_t)tiles_x * tiles_y)) * zc, ze = min(zs + zc, G.nz);
+        const int x = x0 + tx, y = y0 + ty;
+        const bool in = x < G.nx && y < G.ny;
+        __syncthreads();  // the ring of the previous column is read no more
+        zm_store(plane(x0, y0, zs - 1), su[0]);
+        zm_store(plane(x0, y0, zs), su[1]);
+        zm_store(plane(x0, y0, zs + 1), su[2]);
+        const int64_t col = (int64_t)(in ? x : 0) + (int64_t)G.nx * (in ? y : 0);
+        double p_next = mac[N + col + nxy * zs];
+        int r0 = 0, r1 = 1, r2 = 2;  // ring slots of planes z-1, z, z+1
+        for (int z = zs; z < ze; z++) {
+            const bool more = z + 1 < ze;  // plane z+2 is needed by plane z+1
+            ZmPlane<double, 4> next;
+            if (more) next = plane(x0, y0, z + 2);
+            const double pr = p_next;
+            if (more) p_next = mac[N + col + nxy * (z + 1)];
+            __syncthreads();
+            if (in) {
+                const int rz[3] = {r0, r1, r2};
+                const int hc = (tx + 1) + ZM_HX * (ty + 1);
+                const double ph = su[r1][0][hc], u1 = su[r1][1][hc], u2 = su[r1][2][hc], u3 = su[r1][3][hc];
+                double gp[3] = {0.0, 0.0, 0.0}, gu[3][3];
+                for (int k = 0; k < 3; k++)
+                    for (int a = 0; a < 3; a++) gu[k][a] = 0.0;
+                sfor<1, 15>([&](auto qc) {
+                    constexpr int q = decltype(qc)::value;
+                    using D = Dir<q>;
+                    const int h = hc + D::cx + ZM_HX * D::cy;
+                    const double v = su[rz[1 + D::cz]][0][h];
+                    gp[0] = acc<D::cx>(gp[0], v);
+                    gp[1] = acc<D::cy>(gp[1], v);
+                    gp[2] = acc<D::cz>(gp[2], v);
+                    for (int k = 0; k < 3; k++) {
+                        const double w = su[rz[1 + D::cz]][1 + k][h];
+                        gu[k][0] = acc<D::cx>(gu[k][0], w);
+                        gu[k][1] = acc<D::cy>(gu[k][1], w);
+                        gu[k][2] = acc<D::cz>(gu[k][2], w);
+                    }
+                });
+                for (int a = 0; a < 3; a++) {
+                    gp[a] = div_const(gp[a], 10.0, 0.1);
+                    for (int k = 0; k < 3; k++) gu[k][a] = div_const(gu[k][a], 10.0, 0.1);
+                }
+                // interface-strain interaction, ref drop_analysis.f90 korteweg_cal /
+                // strain_cal / interaction_cal (:830-882): beta outer, alpha inner
+                double e = 0.0, it = 0.0;
+                for (int b = 0; b < 3; b++)
+                    for (int a = 0; a < 3; a++) {
+                        const double sab = gu[a][b] + gu[b][a];
+                        e += sab * sab;
+                        it = it + (gp[a] * gp[b]) * (0.5 * sab);
+                    }
+                add_comp(s[0], comp[0], ph);
+                add_comp(s[1], comp[1], 0.5 * (u1 * u1 + u2 * u2 + u3 * u3));
+                add_comp(s[2], comp[2], e);
+                add_comp(s[3], comp[3], sqrt(gp[0] * gp[0] + gp[1] * gp[1] + gp[2] * gp[2]));
+                add_comp(s[4], comp[4], ph * P.T * log(ph / (1.0 - P.b * ph)) - P.a * ph * ph);
+                add_comp(s[5], comp[5], pr);
+                add_comp(s[6], comp[6], u1);
+                add_comp(s[7], comp[7], u2);
+                add_comp(s[8], comp[8], u3);
+                add_comp(s[9], comp[9], it);
             }
-        v[0] = ph;
-        v[1] = 0.5 * (u1 * u1 + u2 * u2 + u3 * u3);
-        v[2] = e;
-        v[3] = sqrt(g0 * g0 + g1 * g1 + g2 * g2);
-        v[4] = ph * P.T * log(ph / (1.0 - P.b * ph)) - P.a * ph * ph;
-        v[5] = pr;
-        v[6] = u1;
-        v[7] = u2;
-        v[8] = u3;
-        // interface-strain interaction, ref drop_analysis.f90 korteweg_cal /
-        // strain_cal / interaction_cal (:830-882): beta outer, alpha inner
-        const double gp[3] = {g0, g1, g2};
-        double it = 0.0;
-        for (int b = 0; b < 3; b++)
-            for (int a = 0; a < 3; a++) it = it + (gp[a] * gp[b]) * (0.5 * (gu[a][b] + gu[b][a]));
-        v[9] = it;
-    }
-    for (int k = 0; k < NPART; k++) {
-        double t = v[k];
-        for (int off = 32; off > 0; off >>= 1) t += __shfl_xor(t, off, 64);
-        v[k] = t;
+            __syncthreads();
+            if (more) zm_store(next, su[r0]);  // the slot of plane z-1
+            const int t = r0;
+            r0 = r1;
+            r1 = r2;
+            r2 = t;
+        }
     }
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    if (lane == 0)
-        for (int k = 0; k < NPART; k++) sh[k][wave] = v[k];
+    for (int k = 0; k < NPART; k++) {
+        double t = s[k] + comp[k];
+        for (int off = 32; off > 0; off >>= 1) t += __shfl_xor(t, off, 64);
+        if (lane == 0) sh[k][wave] = t;
+    }
     __syncthreads();
     if (threadIdx.x < NPART) {
         const int k = threadIdx.x;
-        partial[blockIdx.x * NPART + k] = ((sh[k][0] + sh[k][1]) + sh[k][2]) + sh[k][3];
+        double t = sh[k][0];
+        for (int w = 1; w < ZM_NT / 64; w++) t += sh[k][w];
+        partial[(int64_t)blockIdx.x * NPART + k] = t;
     }
+}
+
+// Compensated sums of the workgroups' records (fixed order: lane l of wavefront k
+// takes records l, l + 64, ... of component k, then a tree over the lanes), and the
+// phi range slot next to them, so that one small copy returns everything.
+__global__ __launch_bounds__(64 * NPART) void reduce_final(const double* __restrict__ partial, int nblocks,
+                                                           const uint64_t* __restrict__ range_slot,
+                                                           double* __restrict__ out) {
+    const int lane = threadIdx.x & 63, k = threadIdx.x >> 6;
+    double s = 0.0, c = 0.0;
+#pragma unroll 4
+    for (int b = lane; b < nblocks; b += 64) add_comp(s, c, partial[(int64_t)b * NPART + k]);
+    for (int off = 32; off > 0; off >>= 1) {
+        const double so = __shfl_xor(s, off, 64), co = __shfl_xor(c, off, 64);
+        add_comp(s, c, so);
+        c += co;
+    }
+    if (lane == 0) out[k] = s + c;
+    if (threadIdx.x < 2) reinterpret_cast<uint64_t*>(out + NPART)[threadIdx.x] = range_slot[threadIdx.x];
 }
 
 __global__ void range_set(uint64_t* range, int slot, double vmax, double vmin) {
@@ -400,12 +498,21 @@ hipError_t launch_les_tau_fp64(int nx, int ny, int nz, const Phys& ph, const dou
     return hipGetLastError();
 }
 
-hipError_t launch_reduce_fp64(int nx, int ny, int nz, const Phys& ph, const double* mac, double* partial,
-                              int* nblocks, hipStream_t st) {
+hipError_t launch_reduce_fp64(int nx, int ny, int nz, const Phys& ph, const double* mac, const uint64_t* range_slot,
+                              double* work, hipStream_t st) {
     Grid G{nx, ny, nz};
-    const int64_t N = (int64_t)nx * ny * nz;
-    *nblocks = (int)nblk(N, 256);
-    hipLaunchKernelGGL(reduce_fp64, dim3(*nblocks), dim3(256), 0, st, G, ph, mac, partial);
+    const int mx = (nx + ZM_TX - 1) / ZM_TX, my = (ny + ZM_TY - 1) / ZM_TY;
+    // columns of up to 32 planes (the two halo planes cost 2 / zc), shorter where the
+    // lattice would leave less than four workgroups per CU
+    const int64_t planes = (int64_t)mx * my * nz;
+    const int zc = (int)std::min<int64_t>(std::min(32, nz), std::max<int64_t>(1, planes / 1024));
+    const int64_t items = (int64_t)mx * my * ((nz + zc - 1) / zc);
+    const int nblocks = (int)std::min<int64_t>(items, REDUCE_MAX_BLOCKS);
+    hipLaunchKernelGGL(reduce_fp64, dim3(nblocks), dim3(ZM_NT), 0, st, G, ph, mac, work, mx, my, zc, items);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(reduce_final, dim3(1), dim3(64 * NPART), 0, st, (const double*)work, nblocks, range_slot,
+                       work + REDUCE_OUT);
     return hipGetLastError();
 }
 

@@ -151,10 +151,14 @@ hipError_t launch_les_tau_fp64(int nx, int ny, int nz, const Phys& ph, const dou
 hipError_t launch_derived_fp64(int nx, int ny, int nz, const Phys& ph, const double* mac, int kind, double* out,
                                hipStream_t st);
 
-// diagnostics partial sums: NPART doubles per workgroup
+// diagnostics sums: NPART doubles per workgroup (at most REDUCE_MAX_BLOCKS), then at
+// work[REDUCE_OUT] the NPART total sums and the two words of the phi range slot
 constexpr int NPART = 10;
-hipError_t launch_reduce_fp64(int nx, int ny, int nz, const Phys& ph, const double* mac, double* partial,
-                              int* nblocks, hipStream_t st);
+constexpr int REDUCE_MAX_BLOCKS = 2048;
+constexpr int REDUCE_OUT = REDUCE_MAX_BLOCKS * NPART;
+constexpr int REDUCE_WORK_DOUBLES = REDUCE_OUT + 16;
+hipError_t launch_reduce_fp64(int nx, int ny, int nz, const Phys& ph, const double* mac, const uint64_t* range_slot,
+                              double* work, hipStream_t st);
 // fill a range slot with (max, min) = (vmax, vmin)
 hipError_t launch_range_set(uint64_t* range, int slot, double vmax, double vmin, hipStream_t st);
 

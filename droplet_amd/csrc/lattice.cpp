@@ -654,29 +654,14 @@ extern "C" int drp_reduce(drp_lattice* L, drp_stats* st) {
         int rc = fp32_macro_fp64_view(L, &mac);
         if (rc) return rc;
     }
-    const int64_t nb = (L->n + 255) / 256;
-    if (L->partial_cap < nb) {
-        if (L->partial) (void)hipFree(L->partial);
-        L->partial = nullptr;
-        HIP_TRY(hipMalloc((void**)&L->partial, nb * NPART * sizeof(double)));
-        L->partial_cap = nb;
-    }
-    int nblocks = 0;
-    HIP_TRY(launch_reduce_fp64(L->cfg.nx, L->cfg.ny, L->cfg.nz, L->phys, mac, L->partial, &nblocks, L->stream));
-    std::vector<double> part((size_t)nblocks * NPART);
-    uint64_t rg[2];
-    HIP_TRY(hipMemcpyAsync(part.data(), L->partial, part.size() * sizeof(double), hipMemcpyDeviceToHost, L->stream));
-    HIP_TRY(hipMemcpyAsync(rg, L->range + 2 * (L->step % 3), 2 * sizeof(uint64_t), hipMemcpyDeviceToHost, L->stream));
+    if (!L->partial) HIP_TRY(hipMalloc((void**)&L->partial, REDUCE_WORK_DOUBLES * sizeof(double)));
+    HIP_TRY(launch_reduce_fp64(L->cfg.nx, L->cfg.ny, L->cfg.nz, L->phys, mac, L->range + 2 * (L->step % 3), L->partial,
+                               L->stream));
+    double s[NPART + 2];
+    HIP_TRY(hipMemcpyAsync(s, L->partial + REDUCE_OUT, sizeof s, hipMemcpyDeviceToHost, L->stream));
     HIP_TRY(hipStreamSynchronize(L->stream));
-    // Neumaier-compensated sum of the workgroup partials (thousands of terms)
-    double s[NPART] = {0}, comp[NPART] = {0};
-    for (int b = 0; b < nblocks; b++)
-        for (int k = 0; k < NPART; k++) {
-            const double v = part[(size_t)b * NPART + k], t = s[k] + v;
-            comp[k] += (std::fabs(s[k]) >= std::fabs(v)) ? (s[k] - t) + v : (v - t) + s[k];
-            s[k] = t;
-        }
-    for (int k = 0; k < NPART; k++) s[k] += comp[k];
+    uint64_t rg[2];
+    std::memcpy(rg, s + NPART, sizeof rg);
     stats_from_sums(L, s, rg, st);
     return DRP_OK;
 }

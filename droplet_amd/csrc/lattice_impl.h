@@ -32,11 +32,10 @@ struct drp_lattice {
     drp::SpectralWork specw_adv{};
     double* uadv = nullptr;             // scale-separated advection: band-passed u1 | u2 | u3
     double* tg = nullptr;               // Taylor-Green sin/cos tables
-    double* partial = nullptr;          // diagnostics partial sums
-    int64_t partial_cap = 0;
+    double* partial = nullptr;          // diagnostics sums (REDUCE_WORK_DOUBLES)
     double* mac64 = nullptr;            // FP32 mode: FP64 copy of the macroscopic fields
     int* census = nullptr;              // droplet census work space (4 n + 4 ints, census.hip)
-    double* budget = nullptr;           // energy-budget work space (19 n doubles + partial sums, budget.hip)
+    double* budget = nullptr;           // energy-budget work space (7 n doubles + partial sums, budget.hip)
     void* fp32_state = nullptr;         // FP32 mode: shift constants etc.
 };
 

@@ -218,7 +218,7 @@ int drp_reduce(drp_lattice* lat, drp_stats* stats);
  * callers that cannot allocate device memory (code under HIP graph capture, tight
  * serving loops, harnesses that forbid hipMalloc).  The partial sums live in one
  * file-scope device array that each GPU holds until the process ends
- * (10 MiB + 128 B); lattices of more than DRP_REDUCE_NOALLOC_MAX_NODES nodes get
+ * (160 KiB + 128 B); lattices of more than DRP_REDUCE_NOALLOC_MAX_NODES nodes get
  * DRP_ERR_ARG, FP32 lattices DRP_ERR_UNSUPPORTED (their FP64 view allocates).
  * Returns the same statistics as drp_reduce.  Calls that overlap on one GPU share
  * the array and race: serialise them. */
