@@ -93,22 +93,23 @@ __device__ void stencils(const BGrid& G, const double* phi, const double* u1, co
 }
 
 __global__ __launch_bounds__(256) void derived_fp64(BGrid G, Phys P, const double* __restrict__ mac, int kind,
-                                                    double* __restrict__ out) {
+                                                    double* __restrict__ out, int64_t pitch) {
     const int64_t n = (int64_t)G.nx * G.ny * G.nz;
     const int64_t s = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     if (s >= n) return;
     const int x = (int)(s % G.nx), y = (int)((s / G.nx) % G.ny), z = (int)(s / ((int64_t)G.nx * G.ny));
+    double* const o = out + x + pitch * (y + (int64_t)G.ny * z);  // row pitch of the result
     const double ph = mac[s];
     if (kind == DRP_DERIVED_FREE_ENERGY) {
-        out[s] = ph * P.T * log(ph / (1.0 - P.b * ph)) - P.a * ph * ph;
+        *o = ph * P.T * log(ph / (1.0 - P.b * ph)) - P.a * ph * ph;
         return;
     }
     double lap, gp[3], gu[3][3];
     stencils(G, mac, nullptr, nullptr, nullptr, x, y, z, lap, gp, gu);
     if (kind == DRP_DERIVED_CHEMICAL_POTENTIAL) {
-        out[s] = P.T * log(ph / (1.0 - P.b * ph)) + P.T / (1.0 - P.b * ph) - 2.0 * P.a * ph - P.kg * lap;
+        *o = P.T * log(ph / (1.0 - P.b * ph)) + P.T / (1.0 - P.b * ph) - 2.0 * P.a * ph - P.kg * lap;
     } else {
-        out[s] = mac[2 * n + s] * gp[0] + mac[3 * n + s] * gp[1] + mac[4 * n + s] * gp[2];
+        *o = mac[2 * n + s] * gp[0] + mac[3 * n + s] * gp[1] + mac[4 * n + s] * gp[2];
     }
 }
 
@@ -440,10 +441,10 @@ __global__ __launch_bounds__(BT) void budget_pass2(BudgetArgs a) {
 }  // namespace
 
 hipError_t launch_derived_fp64(int nx, int ny, int nz, const Phys& ph, const double* mac, int kind, double* out,
-                               hipStream_t st) {
+                               int64_t pitch, hipStream_t st) {
     const int64_t n = (int64_t)nx * ny * nz;
     hipLaunchKernelGGL(derived_fp64, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, BGrid{nx, ny, nz}, ph, mac,
-                       kind, out);
+                       kind, out, pitch);
     return hipGetLastError();
 }
 
@@ -466,7 +467,7 @@ extern "C" int drp_get_derived(drp_lattice* L, int kind, double* host, size_t n_
     }
     double* out = nullptr;
     HIP_TRYB(hipMalloc((void**)&out, (size_t)L->n * sizeof(double)));
-    hipError_t e = launch_derived_fp64(L->cfg.nx, L->cfg.ny, L->cfg.nz, L->phys, mac, kind, out, L->stream);
+    hipError_t e = launch_derived_fp64(L->cfg.nx, L->cfg.ny, L->cfg.nz, L->phys, mac, kind, out, L->cfg.nx, L->stream);
     if (e == hipSuccess) e = hipMemcpyAsync(host, out, (size_t)L->n * sizeof(double), hipMemcpyDeviceToHost, L->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(L->stream);
     const hipError_t f = hipFree(out);

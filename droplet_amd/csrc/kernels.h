@@ -147,9 +147,10 @@ hipError_t launch_moments_fp64(int nx, int ny, int nz, const double* f, const do
 // blocks) and that step's phi range slot
 hipError_t launch_les_tau_fp64(int nx, int ny, int nz, const Phys& ph, const double* mac, const double* mac_old,
                                const LesBlocks& blk, const uint64_t* range, int slot, double* tau, hipStream_t st);
-// derived fields of the analysis programs (budget.hip): kind = DRP_DERIVED_*
+// derived fields of the analysis programs (budget.hip): kind = DRP_DERIVED_*; rows of
+// the result `pitch` doubles apart
 hipError_t launch_derived_fp64(int nx, int ny, int nz, const Phys& ph, const double* mac, int kind, double* out,
-                               hipStream_t st);
+                               int64_t pitch, hipStream_t st);
 
 // diagnostics sums: NPART doubles per workgroup (at most REDUCE_MAX_BLOCKS), then at
 // work[REDUCE_OUT] the NPART total sums and the two words of the phi range slot

@@ -296,6 +296,7 @@ void lattice_free(drp_lattice* L) {
     if (L->mac64) (void)hipFree(L->mac64);
     if (L->census) (void)hipFree(L->census);
     if (L->budget) (void)hipFree(L->budget);
+    diag_free(L);
     if (L->stream && L->owns_stream) (void)hipStreamDestroy(L->stream);
     L->stream = nullptr;
 }

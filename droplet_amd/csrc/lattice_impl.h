@@ -36,6 +36,7 @@ struct drp_lattice {
     double* mac64 = nullptr;            // FP32 mode: FP64 copy of the macroscopic fields
     int* census = nullptr;              // droplet census work space (4 n + 4 ints, census.hip)
     double* budget = nullptr;           // energy-budget work space (7 n doubles + partial sums, budget.hip)
+    struct drp_diag* diag = nullptr;    // plan and work space of the spectra (spectral_diag.hip)
     void* fp32_state = nullptr;         // FP32 mode: shift constants etc.
 };
 
@@ -56,6 +57,9 @@ void stats_from_sums(const drp_lattice* L, const double* sums, const uint64_t* r
 // LES tau for the next step: after a step (fresh = false, rank-block halos one
 // step old) or for a replaced state (fresh = true, all neighbours current)
 int les_update_tau(drp_lattice* L, bool fresh);
+
+// spectral_diag.hip
+void diag_free(drp_lattice* L);
 
 // deformation.cpp
 int deformation(drp_lattice* L, int mode, double* Lo, double* Bo, double* Do);

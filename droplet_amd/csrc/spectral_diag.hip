@@ -12,12 +12,20 @@
 //
 // The reference transforms with 2decomp/FFTW (r2c with the halved axis z,
 // u_hat = FFT(u) / (nx ny nz), signed wavenumber k = i - n for i >= n/2 + 1).
-// Here a complex 3-D FFT is done by one mixed-radix Stockham pass per axis
-// (radices 4, 2, 3, 5; every extent a product of those, at most 2048): each
-// workgroup loads G whole lines into LDS, runs the log_R(n) stages there with
-// twiddles from a table e^{-2 pi i t / n} evaluated on the host, and writes the
-// lines back in place.  Lines along y and z are taken G at a time with
-// consecutive x, so their loads and stores are coalesced.
+// Here a 3-D FFT is one mixed-radix Stockham pass per axis (radices 8, 4, 2, 3, 5;
+// every extent a product of those, at most 2048): each workgroup loads G whole
+// lines into LDS, runs the log_R(n) stages there with twiddles from a table
+// e^{-2 pi i t / n} evaluated on the host, and writes the lines back in place.
+// Lines along y and z are taken G at a time with consecutive x, so their loads and
+// stores are coalesced.
+//
+// The spectra transform real fields, so they keep the half spectrum kx = 0..nx/2:
+// the x pass packs two real rows into one complex line and separates their
+// transforms on the way out, the y pass works on nx/2 + 1 lines per plane, and the
+// z pass writes nothing back: its lines go from LDS straight into shell bins.  A
+// stored mode stands for itself and for its mirror image -k where that is not
+// stored too.  One field is transformed at a time, so its half spectrum (143 MB at
+// 256^3) passes from kernel to kernel through the 256 MB last-level cache.
 //
 // The per-scale interaction uses Parseval instead of one inverse transform per
 // shell: < u^(k) . w > = sum over the modes of shell k of Re(u_hat w_hat*), with
@@ -27,6 +35,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <new>
 #include <vector>
 
 #include "../../include/droplet.h"
@@ -46,9 +55,12 @@ namespace {
     } while (0)
 
 constexpr int FFT_MAX_STAGES = 12;
-constexpr int FFT_MAX_LINE = 2048;   // longest line (one line per workgroup: two 32 KiB buffers)
-constexpr int FFT_BLOCK_LINES = 1024;  // G * L complex numbers per buffer for shorter lines (2 x 16 KiB):
-                                       // four 256-point lines per workgroup ran 1.2x faster than eight
+constexpr int FFT_BLOCK = 256;       // threads per workgroup
+constexpr int FFT_MAX_LINE = 2048;   // longest line
+// complex numbers of one workgroup's G lines (32 KiB of LDS: five workgroups per CU).
+// Eight 256-point lines make the strided passes touch whole 128-byte lines of memory
+// (four lines, with a second LDS buffer for the stages, ran at 2.4 TB/s)
+constexpr int FFT_POINTS = 2048;
 
 struct FFTAxis {
     int L;                     // line length
@@ -59,6 +71,9 @@ struct FFTAxis {
     int G;                     // lines per workgroup
     int nst;                   // stages
     int rad[FFT_MAX_STAGES];   // radix of each stage
+    uint32_t mm[FFT_MAX_STAGES], mn[FFT_MAX_STAGES];  // 2^32 / M and 2^32 / Ns of each stage, rounded up
+                                                      // (0 for a divisor of 1): quotients by one multiply
+    uint32_t ml;               // the same for L
     const double2* tw;         // e^{-2 pi i t / L}, t = 0..L-1
 };
 
@@ -84,6 +99,21 @@ template <int R> __device__ __forceinline__ void small_dft(const double2 (&v)[R]
         o[1] = make_double2(b.x + wd.x, b.y + wd.y);
         o[2] = make_double2(a.x - c.x, a.y - c.y);
         o[3] = make_double2(b.x - wd.x, b.y - wd.y);
+    } else if constexpr (R == 8) {
+        // even and odd 4-point halves, W = (1 + s i) / sqrt 2
+        constexpr double H = 0.70710678118654752440;
+        const double2 ev[4] = {v[0], v[2], v[4], v[6]}, od[4] = {v[1], v[3], v[5], v[7]};
+        double2 e[4], d[4];
+        small_dft<4>(ev, e, sign);
+        small_dft<4>(od, d, sign);
+        const double2 w[4] = {d[0], make_double2(H * (d[1].x - s * d[1].y), H * (d[1].y + s * d[1].x)),
+                              make_double2(-s * d[2].y, s * d[2].x),
+                              make_double2(-H * (d[3].x + s * d[3].y), H * (s * d[3].x - d[3].y))};
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            o[q] = make_double2(e[q].x + w[q].x, e[q].y + w[q].y);
+            o[q + 4] = make_double2(e[q].x - w[q].x, e[q].y - w[q].y);
+        }
     } else {
         // R = 3, 5: cos and sin of 2 pi m / R
         constexpr double C3[3] = {1.0, -0.5, -0.5};
@@ -107,30 +137,62 @@ template <int R> __device__ __forceinline__ void small_dft(const double2 (&v)[R]
     }
 }
 
-// one Stockham stage of radix R over the ng lines of length L held in LDS
+// b / d for b < 2^16 from m = ceil(2^32 / d), d < 2^16 (m = 0: d = 1)
+__device__ __forceinline__ uint32_t quotient(uint32_t b, uint32_t m) { return m ? __umulhi(b, m) : b; }
+
+// one Stockham stage of radix R, in place, over the ng lines of length L held in
+// LDS: every thread reads its butterflies into registers before any is written
 template <int R>
-__device__ __forceinline__ void fft_stage(const double2* __restrict__ src, double2* __restrict__ dst, int L, int ng,
-                                          int Ns, const double2* __restrict__ tw, int sign) {
-    const int M = L / R, step = L / (Ns * R);
-    for (int b = threadIdx.x; b < ng * M; b += blockDim.x) {
-        const int g = b / M, j = b - g * M;
-        const int k = j % Ns;
-        const double2* sl = src + g * L;
-        double2 v[R], o[R];
+__device__ __forceinline__ void fft_stage(double2* buf, const FFTAxis& A, int st, int ng, int Ns, int sign) {
+    constexpr int NB = (FFT_POINTS / R + FFT_BLOCK - 1) / FFT_BLOCK;  // butterflies per thread
+    const int L = A.L, M = L / R, step = L / (Ns * R), nb = ng * M;
+    double2 o[NB][R];
+    int to[NB];
+#pragma unroll
+    for (int i = 0; i < NB; i++) {
+        const int b = threadIdx.x + i * FFT_BLOCK;
+        to[i] = -1;
+        if (b >= nb) continue;
+        const int g = (int)quotient(b, A.mm[st]), j = b - g * M;
+        const int k = j - (int)quotient(j, A.mn[st]) * Ns;
+        const double2* sl = buf + g * L;
+        double2 v[R];
 #pragma unroll
         for (int r = 0; r < R; r++) {
             double2 x = sl[j + r * M];
-            if (r > 0 && k > 0) {
-                double2 w = tw[k * r * step];  // k r step < L
+            if (r > 0 && Ns > 1) {
+                double2 w = A.tw[k * r * step];  // k r step < L
                 if (sign > 0) w.y = -w.y;
                 x = cmul(x, w);
             }
             v[r] = x;
         }
-        small_dft<R>(v, o, sign);
-        double2* dl = dst + g * L + (j - k) * R + k;
+        small_dft<R>(v, o[i], sign);
+        to[i] = g * L + (j - k) * R + k;
+    }
+    __syncthreads();
 #pragma unroll
-        for (int r = 0; r < R; r++) dl[r * Ns] = o[r];
+    for (int i = 0; i < NB; i++) {
+        if (to[i] < 0) continue;
+#pragma unroll
+        for (int r = 0; r < R; r++) buf[to[i] + r * Ns] = o[i][r];
+    }
+}
+
+// all stages over the ng lines a workgroup has written to `buf` (not yet
+// synchronised); the transforms are in `buf` afterwards, synchronised
+__device__ __forceinline__ void fft_stages(double2* buf, int ng, const FFTAxis& A, int sign) {
+    __syncthreads();
+    int Ns = 1;
+    for (int st = 0; st < A.nst; st++) {
+        const int R = A.rad[st];
+        if (R == 8) fft_stage<8>(buf, A, st, ng, Ns, sign);
+        else if (R == 4) fft_stage<4>(buf, A, st, ng, Ns, sign);
+        else if (R == 2) fft_stage<2>(buf, A, st, ng, Ns, sign);
+        else if (R == 3) fft_stage<3>(buf, A, st, ng, Ns, sign);
+        else fft_stage<5>(buf, A, st, ng, Ns, sign);
+        __syncthreads();
+        Ns *= R;
     }
 }
 
@@ -141,8 +203,7 @@ __device__ __forceinline__ void fft_stage(const double2* __restrict__ src, doubl
 __global__ __launch_bounds__(256) void fft_lines(double2* __restrict__ data, FFTAxis A, int sign) {
     extern __shared__ double2 lds[];
     const int L = A.L, G = A.G;
-    double2* buf0 = lds;
-    double2* buf1 = lds + (size_t)G * L;
+    double2* const buf = lds;
     const int64_t l0 = (int64_t)blockIdx.x * G;
     const int ng = (int)min<int64_t>(G, A.nlines - l0);
     const int tid = threadIdx.x, nth = blockDim.x;
@@ -150,42 +211,29 @@ __global__ __launch_bounds__(256) void fft_lines(double2* __restrict__ data, FFT
         for (int g = 0; g < ng; g++) {
             const int64_t l = l0 + g;
             const double2* line = data + (l % A.F) * A.sf + (l / A.F) * A.so;
-            for (int j = tid; j < L; j += nth) buf0[g * L + j] = line[j];
+            for (int j = tid; j < L; j += nth) buf[g * L + j] = line[j];
         }
     } else {
         const int g = tid % G, j0 = tid / G, js = nth / G;
         if (g < ng && j0 < js) {
             const int64_t l = l0 + g;
             const double2* line = data + (l % A.F) * A.sf + (l / A.F) * A.so;
-            for (int j = j0; j < L; j += js) buf0[g * L + j] = line[(int64_t)j * A.S];
+            for (int j = j0; j < L; j += js) buf[g * L + j] = line[(int64_t)j * A.S];
         }
     }
-    __syncthreads();
-    int Ns = 1;
-    for (int st = 0; st < A.nst; st++) {
-        const int R = A.rad[st];
-        if (R == 4) fft_stage<4>(buf0, buf1, L, ng, Ns, A.tw, sign);
-        else if (R == 2) fft_stage<2>(buf0, buf1, L, ng, Ns, A.tw, sign);
-        else if (R == 3) fft_stage<3>(buf0, buf1, L, ng, Ns, A.tw, sign);
-        else fft_stage<5>(buf0, buf1, L, ng, Ns, A.tw, sign);
-        __syncthreads();
-        double2* t = buf0;
-        buf0 = buf1;
-        buf1 = t;
-        Ns *= R;
-    }
+    fft_stages(buf, ng, A, sign);
     if (A.S == 1) {
         for (int g = 0; g < ng; g++) {
             const int64_t l = l0 + g;
             double2* line = data + (l % A.F) * A.sf + (l / A.F) * A.so;
-            for (int j = tid; j < L; j += nth) line[j] = buf0[g * L + j];
+            for (int j = tid; j < L; j += nth) line[j] = buf[g * L + j];
         }
     } else {
         const int g = tid % G, j0 = tid / G, js = nth / G;
         if (g < ng && j0 < js) {
             const int64_t l = l0 + g;
             double2* line = data + (l % A.F) * A.sf + (l / A.F) * A.so;
-            for (int j = j0; j < L; j += js) line[(int64_t)j * A.S] = buf0[g * L + j];
+            for (int j = j0; j < L; j += js) line[(int64_t)j * A.S] = buf[g * L + j];
         }
     }
 }
@@ -204,77 +252,131 @@ __device__ __forceinline__ int signed_k(int i, int n) { return i >= n / 2 + 1 ? 
 
 __device__ __forceinline__ int shell_of(int x, int y, int z, int nx, int ny, int nz) {
     const int k1 = signed_k(x, nx), k2 = signed_k(y, ny), k3 = signed_k(z, nz);
-    return (int)sqrt((double)(k1 * k1 + k2 * k2 + k3 * k3));
+    // |k|^2 <= 3 2^20 is exact in FP32, and below a square m^2 by at least 1, i.e. its
+    // root is below m by more than half an ulp: the correctly rounded root truncates right
+    return (int)sqrtf((float)(k1 * k1 + k2 * k2 + k3 * k3));
 }
 
-// spectrum over the reference's half space k3 = 0 .. nz/2 (index), weight 2 off the
-// k3 = 0 plane (the Nyquist plane included, as the reference counts it); shells
-// accumulated per workgroup in LDS, then one atomic per workgroup and shell
-__global__ __launch_bounds__(256) void shell_energy(int nx, int ny, int nz, const double2* __restrict__ u1,
-                                                    const double2* __restrict__ u2, const double2* __restrict__ u3,
-                                                    double inv, int nshells, double* __restrict__ E) {
-    extern __shared__ double bins[];
-    for (int s = threadIdx.x; s < nshells; s += blockDim.x) bins[s] = 0.0;
-    __syncthreads();
-    const int64_t half = (int64_t)nx * ny * (nz / 2 + 1);
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < half; i += (int64_t)gridDim.x * blockDim.x) {
-        const int x = (int)(i % nx), y = (int)((i / nx) % ny), z = (int)(i / ((int64_t)nx * ny));
-        const int s = shell_of(x, y, z, nx, ny, nz);
-        if (s >= nshells) continue;
-        const double2 a = u1[i], b = u2[i], c = u3[i];
-        const double e = ((a.x * a.x + a.y * a.y) + (b.x * b.x + b.y * b.y) + (c.x * c.x + c.y * c.y)) * inv * inv;
-        atomicAdd(&bins[s], 0.5 * e * (z == 0 ? 1.0 : 2.0));
+// x pass of a real field: G pairs of rows, row r at in + r in_pitch, into half
+// spectra of nx/2 + 1 modes, row r at out + r out_pitch.  Rows 2p and 2p + 1 form
+// one complex line Z = a + i b; with W = conj Z(-k), a_hat = (Z + W) / 2 and
+// b_hat = -i (Z - W) / 2.  in may be out (in_pitch = 2 out_pitch): a workgroup
+// reads its rows before it writes them.
+__global__ __launch_bounds__(256) void rfft_rows(const double* in, int64_t in_pitch, int64_t nrows, FFTAxis A,
+                                                 double2* out, int64_t out_pitch) {
+    extern __shared__ double2 lds[];
+    const int L = A.L, H = L / 2 + 1;
+    const int64_t pairs = (nrows + 1) / 2, p0 = (int64_t)blockIdx.x * A.G;
+    const int ng = (int)min<int64_t>(A.G, pairs - p0);
+    for (int g = 0; g < ng; g++) {
+        const int64_t r = 2 * (p0 + g);
+        const bool two = r + 1 < nrows;
+        for (int j = threadIdx.x; j < L; j += blockDim.x)
+            lds[g * L + j] = make_double2(in[r * in_pitch + j], two ? in[(r + 1) * in_pitch + j] : 0.0);
     }
-    __syncthreads();
-    for (int s = threadIdx.x; s < nshells; s += blockDim.x)
-        if (bins[s] != 0.0) atomicAdd(&E[s], bins[s]);
+    fft_stages(lds, ng, A, -1);
+    const double2* res = lds;
+    for (int g = 0; g < ng; g++) {
+        const int64_t r = 2 * (p0 + g);
+        const bool two = r + 1 < nrows;
+        for (int k = threadIdx.x; k < H; k += blockDim.x) {
+            const double2 Z = res[g * L + k], V = res[g * L + (k == 0 ? 0 : L - k)];
+            out[r * out_pitch + k] = make_double2(0.5 * (Z.x + V.x), 0.5 * (Z.y - V.y));
+            if (two) out[(r + 1) * out_pitch + k] = make_double2(0.5 * (Z.y + V.y), 0.5 * (V.x - Z.x));
+        }
+    }
 }
 
-// per-shell sum over the full spectrum of Re(u_hat . w_hat*), normalised
-__global__ __launch_bounds__(256) void shell_cross(int nx, int ny, int nz, const double2* __restrict__ u,
-                                                   const double2* __restrict__ w, double inv, int nshells,
-                                                   double* __restrict__ C) {
-    extern __shared__ double bins[];
-    for (int s = threadIdx.x; s < nshells; s += blockDim.x) bins[s] = 0.0;
-    __syncthreads();
-    const int64_t n = (int64_t)nx * ny * nz;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        const int x = (int)(i % nx), y = (int)((i / nx) % ny), z = (int)(i / ((int64_t)nx * ny));
-        const int s = shell_of(x, y, z, nx, ny, nz);
-        if (s >= nshells) continue;
-        for (int c = 0; c < 3; c++) {
-            const double2 a = u[c * n + i], b = w[c * n + i];
-            atomicAdd(&bins[s], (a.x * b.x + a.y * b.y) * inv * inv);
+// what the z pass adds to the shell of a mode
+enum { SHELL_ENERGY = 0,     // 0.5 |a|^2 on the half space k3 = 0..nz/2, weight 2 off k3 = 0 (the Nyquist plane
+                             // included, as enesupe_cal counts it)
+       SHELL_CROSS = 1,      // Re(a conj b) over all modes
+       SHELL_CROSS_HALF = 2  // Re(a conj b) and the weights themselves on that half space (contribution,
+                             // drop_analysis.f90:476-578); bins [sum | weight]
+};
+constexpr int SHELL_EL = FFT_POINTS / FFT_BLOCK;  // modes per thread of one workgroup's lines, at most
+
+// z pass of the half spectra a (and b): G lines (kx, y) per round, transformed in
+// LDS and added to the shells int|k| with the weight of the mode and its mirror
+// image; workgroups take groups of lines in turn and leave one record of bins each
+// (added to the one there if `more`), so that no bin is shared between workgroups.
+template <int MODE>
+__global__ __launch_bounds__(256) void zlines_shells(const double2* __restrict__ a, const double2* __restrict__ b,
+                                                     FFTAxis A, int nx, int ny, int nz, double inv, int nshells,
+                                                     int more, double* __restrict__ part) {
+    extern __shared__ double2 lds[];
+    const int L = A.L, G = A.G, tid = threadIdx.x, nbins = MODE == SHELL_CROSS_HALF ? 2 * nshells : nshells;
+    double* bins = reinterpret_cast<double*>(lds + (size_t)G * L);
+    double* rec = part + (int64_t)blockIdx.x * nbins;
+    for (int s = tid; s < nbins; s += blockDim.x) bins[s] = more ? rec[s] : 0.0;
+    const int64_t groups = (A.nlines + G - 1) / G;
+    for (int64_t grp = blockIdx.x; grp < groups; grp += gridDim.x) {
+        const int64_t l0 = grp * G;
+        const int ng = (int)min<int64_t>(G, A.nlines - l0);
+        auto transform = [&](const double2* __restrict__ src) {
+            __syncthreads();  // the previous transform in LDS is read no more
+            const int g = tid % G, j0 = tid / G, js = blockDim.x / G;
+            if (g < ng && j0 < js) {
+                const int64_t l = l0 + g;
+                const double2* line = src + (l % A.F) * A.sf + (l / A.F) * A.so;
+                for (int j = j0; j < L; j += js) lds[g * L + j] = line[(int64_t)j * A.S];
+            }
+            fft_stages(lds, ng, A, -1);
+        };
+        double2 va[SHELL_EL];
+        const double2* res = lds;
+        transform(a);
+        if constexpr (MODE != SHELL_ENERGY) {
+#pragma unroll
+            for (int i = 0; i < SHELL_EL; i++) {
+                const int m = tid + 256 * i;
+                va[i] = m < ng * L ? res[m] : make_double2(0.0, 0.0);
+            }
+            transform(b);
+        }
+#pragma unroll
+        for (int i = 0; i < SHELL_EL; i++) {
+            const int m = tid + 256 * i;
+            if (m >= ng * L) continue;
+            const int g = (int)quotient(m, A.ml), z = m - g * L;
+            const uint32_t l = (uint32_t)l0 + g;  // fewer than 2^22 lines
+            const int y = (int)(l / (uint32_t)A.F), x = (int)(l - (uint32_t)y * A.F);
+            const int s = shell_of(x, y, z, nx, ny, nz);
+            if (s >= nshells) continue;
+            const bool mirror = x != 0 && 2 * x != nx;  // -k is not among the stored modes
+            double w;
+            if constexpr (MODE == SHELL_CROSS) {
+                w = mirror ? 2.0 : 1.0;
+            } else {
+                const int zm = z == 0 ? 0 : nz - z;
+                w = (z <= nz / 2 ? (z == 0 ? 1.0 : 2.0) : 0.0) +
+                    (mirror && zm <= nz / 2 ? (zm == 0 ? 1.0 : 2.0) : 0.0);
+            }
+            if (w == 0.0) continue;
+            const double2 r = res[m];
+            if constexpr (MODE == SHELL_ENERGY) {
+                atomicAdd(&bins[s], 0.5 * ((r.x * r.x + r.y * r.y) * inv * inv) * w);
+            } else {
+                const double v = va[i].x * r.x + va[i].y * r.y;
+                atomicAdd(&bins[s], MODE == SHELL_CROSS ? w * (v * inv * inv) : w * v);
+                if constexpr (MODE == SHELL_CROSS_HALF) atomicAdd(&bins[nshells + s], w);
+            }
         }
     }
     __syncthreads();
-    for (int s = threadIdx.x; s < nshells; s += blockDim.x)
-        if (bins[s] != 0.0) atomicAdd(&C[s], bins[s]);
+    for (int s = tid; s < nbins; s += blockDim.x) rec[s] = bins[s];
 }
 
-// half-space cross spectrum of contribution (drop_analysis.f90:476-578): per shell the
-// sums of w Re(a conj(m)) and of w, w = 1 on the k3 = 0 plane and 2 elsewhere
-__global__ __launch_bounds__(256) void shell_cross_half(int nx, int ny, int nz, const double2* __restrict__ a,
-                                                        const double2* __restrict__ m, int nshells,
-                                                        double* __restrict__ C, double* __restrict__ W) {
-    extern __shared__ double bins[];  // [2][nshells]
-    for (int s = threadIdx.x; s < 2 * nshells; s += blockDim.x) bins[s] = 0.0;
+// out[s] = sum of the nrec workgroup records of bin s, fixed order, one workgroup per bin
+__global__ __launch_bounds__(256) void shells_final(const double* __restrict__ part, int nrec, int nbins,
+                                                    double* __restrict__ out) {
+    __shared__ double sh[4];
+    double v = 0.0;
+    for (int r = threadIdx.x; r < nrec; r += 256) v += part[(int64_t)r * nbins + blockIdx.x];
+    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
     __syncthreads();
-    const int64_t half = (int64_t)nx * ny * (nz / 2 + 1);
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < half; i += (int64_t)gridDim.x * blockDim.x) {
-        const int x = (int)(i % nx), y = (int)((i / nx) % ny), z = (int)(i / ((int64_t)nx * ny));
-        const int s = shell_of(x, y, z, nx, ny, nz);
-        if (s >= nshells) continue;
-        const double w = z == 0 ? 1.0 : 2.0;
-        const double2 av = a[i], mv = m[i];
-        atomicAdd(&bins[s], w * (av.x * mv.x + av.y * mv.y));
-        atomicAdd(&bins[nshells + s], w);
-    }
-    __syncthreads();
-    for (int s = threadIdx.x; s < nshells; s += blockDim.x) {
-        if (bins[s] != 0.0) atomicAdd(&C[s], bins[s]);
-        if (bins[nshells + s] != 0.0) atomicAdd(&W[s], bins[nshells + s]);
-    }
+    if (threadIdx.x == 0) out[blockIdx.x] = ((sh[0] + sh[1]) + sh[2]) + sh[3];
 }
 
 // keep the modes with lo <= int|k| < hi, zero the rest
@@ -287,48 +389,76 @@ __global__ void shell_mask(int nx, int ny, int nz, double2* __restrict__ a, int 
     if (s < lo || s >= hi) a[i] = make_double2(0.0, 0.0);
 }
 
-// grad phi by the D3Q15 stencil (grad_cal, drop_analysis.f90; sum of c phi(x + c) / 10)
-__global__ void grad_phi(int nx, int ny, int nz, const double* __restrict__ phi, double* __restrict__ g) {
-    const int64_t n = (int64_t)nx * ny * nz;
-    const int64_t s = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (s >= n) return;
-    const int x = (int)(s % nx), y = (int)((s / nx) % ny), z = (int)(s / ((int64_t)nx * ny));
-    double g0 = 0.0, g1 = 0.0, g2 = 0.0;
-    for (int q = 1; q < 15; q++) {
-        const int cx[15] = {0, 1, 0, 0, -1, 0, 0, 1, -1, 1, 1, -1, 1, -1, -1};
-        const int cy[15] = {0, 0, 1, 0, 0, -1, 0, 1, 1, -1, 1, -1, -1, 1, -1};
-        const int cz[15] = {0, 0, 0, 1, 0, 0, -1, 1, 1, 1, -1, -1, -1, -1, 1};
-        const int xx = (x + cx[q] + nx) % nx, yy = (y + cy[q] + ny) % ny, zz = (z + cz[q] + nz) % nz;
-        const double v = phi[xx + (int64_t)nx * (yy + (int64_t)ny * zz)];
-        g0 += cx[q] * v;
-        g1 += cy[q] * v;
-        g2 += cz[q] * v;
+// w_b = sum_a d_a (d_b phi d_a phi), b = 0..2, the stencil applied to the products
+// at the neighbours (grad_tensor, drop_analysis.f90:1121-1217) of grad phi = sum c
+// phi(x + c) / 10 (grad_cal); rows of w_b `pitch` apart, components `comp` apart.
+// A workgroup stages phi over its tile + 2 nodes and forms grad phi over the tile + 1
+// in LDS: two kernels gathering 14 neighbours through L2, with grad phi in memory
+// between them, took 0.67 + 0.25 ms at 256^3, this one takes 0.34 ms.
+constexpr int WTX = 32, WTY = 4, WTZ = 4, WNT = WTX * WTY * WTZ;
+template <int Q0, int Q1, typename Fn> __device__ __forceinline__ void sford(Fn&& fn) {
+    if constexpr (Q0 < Q1) {
+        fn(std::integral_constant<int, Q0>{});
+        sford<Q0 + 1, Q1>(fn);
     }
-    g[s] = g0 / 10.0;
-    g[n + s] = g1 / 10.0;
-    g[2 * n + s] = g2 / 10.0;
 }
-
-// w_b = sum_a d_a (d_b phi d_a phi), the stencil applied to the products at the
-// neighbours (grad_tensor, drop_analysis.f90:1121-1217), written as complex numbers
-__global__ void div_korteweg(int nx, int ny, int nz, const double* __restrict__ g, double2* __restrict__ w) {
-    const int64_t n = (int64_t)nx * ny * nz;
-    const int64_t s = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (s >= n) return;
-    const int x = (int)(s % nx), y = (int)((s / nx) % ny), z = (int)(s / ((int64_t)nx * ny));
-    double d[3] = {0.0, 0.0, 0.0};
-    for (int q = 1; q < 15; q++) {
-        const int cx[15] = {0, 1, 0, 0, -1, 0, 0, 1, -1, 1, 1, -1, 1, -1, -1};
-        const int cy[15] = {0, 0, 1, 0, 0, -1, 0, 1, 1, -1, 1, -1, -1, 1, -1};
-        const int cz[15] = {0, 0, 0, 1, 0, 0, -1, 1, 1, 1, -1, -1, -1, -1, 1};
-        const int xx = (x + cx[q] + nx) % nx, yy = (y + cy[q] + ny) % ny, zz = (z + cz[q] + nz) % nz;
-        const int64_t t = xx + (int64_t)nx * (yy + (int64_t)ny * zz);
-        const double ga[3] = {g[t], g[n + t], g[2 * n + t]};
-        const double c[3] = {(double)cx[q], (double)cy[q], (double)cz[q]};
-        for (int b = 0; b < 3; b++)
-            for (int a = 0; a < 3; a++) d[b] += c[a] * (ga[b] * ga[a]);
+__global__ __launch_bounds__(WNT) void div_korteweg(int nx, int ny, int nz, const double* __restrict__ phi,
+                                                    double* __restrict__ w, int64_t pitch, int64_t comp, int tiles_x,
+                                                    int tiles_y) {
+    constexpr int HX2 = WTX + 4, HY2 = WTY + 4, HZ2 = WTZ + 4, H2 = HX2 * HY2 * HZ2;
+    constexpr int HX1 = WTX + 2, HY1 = WTY + 2, HZ1 = WTZ + 2, H1 = HX1 * HY1 * HZ1;
+    __shared__ double sp[H2];
+    __shared__ double sg[3][H1];
+    const int tile = xcd_tile(blockIdx.x, gridDim.x);
+    const int x0 = (tile % tiles_x) * WTX, y0 = ((tile / tiles_x) % tiles_y) * WTY,
+              z0 = (tile / (tiles_x * tiles_y)) * WTZ;
+    const bool small = nx <= WTX || ny <= WTY || nz <= WTZ;  // a tile's halo may wrap more than once
+    auto wrap = [small](int v, int n) {
+        if (small) {
+            v %= n;
+            return v < 0 ? v + n : v;
+        }
+        return v < 0 ? v + n : (v >= n ? v - n : v);
+    };
+    for (int h = threadIdx.x; h < H2; h += WNT) {
+        const int gx = wrap(x0 - 2 + h % HX2, nx), gy = wrap(y0 - 2 + (h / HX2) % HY2, ny),
+                  gz = wrap(z0 - 2 + h / (HX2 * HY2), nz);
+        sp[h] = phi[gx + (int64_t)nx * (gy + (int64_t)ny * gz)];
     }
-    for (int b = 0; b < 3; b++) w[b * n + s] = make_double2(d[b] / 10.0, 0.0);
+    __syncthreads();
+    for (int h = threadIdx.x; h < H1; h += WNT) {
+        const int c = h % HX1 + HX2 * ((h / HX1) % HY1 + HY2 * (h / (HX1 * HY1)));
+        double g0 = 0.0, g1 = 0.0, g2 = 0.0;
+        sford<1, 15>([&](auto qc) {
+            constexpr int q = decltype(qc)::value;
+            using D = Dir<q>;
+            const double v = sp[c + (1 + D::cx) + HX2 * ((1 + D::cy) + HY2 * (1 + D::cz))];
+            g0 = acc<D::cx>(g0, v);
+            g1 = acc<D::cy>(g1, v);
+            g2 = acc<D::cz>(g2, v);
+        });
+        sg[0][h] = div_const(g0, 10.0, 0.1);
+        sg[1][h] = div_const(g1, 10.0, 0.1);
+        sg[2][h] = div_const(g2, 10.0, 0.1);
+    }
+    __syncthreads();
+    const int tx = threadIdx.x % WTX, ty = (threadIdx.x / WTX) % WTY, tz = threadIdx.x / (WTX * WTY);
+    const int x = x0 + tx, y = y0 + ty, z = z0 + tz;
+    if (x >= nx || y >= ny || z >= nz) return;
+    double d0 = 0.0, d1 = 0.0, d2 = 0.0;
+    sford<1, 15>([&](auto qc) {
+        constexpr int q = decltype(qc)::value;
+        using D = Dir<q>;
+        const int h = (tx + 1 + D::cx) + HX1 * ((ty + 1 + D::cy) + HY1 * (tz + 1 + D::cz));
+        const double g0 = sg[0][h], g1 = sg[1][h], g2 = sg[2][h], cg = cdot<q>(g0, g1, g2);
+        d0 += g0 * cg;
+        d1 += g1 * cg;
+        d2 += g2 * cg;
+    });
+    double* const o = w + x + pitch * (y + (int64_t)ny * z);
+    o[0] = div_const(d0, 10.0, 0.1);
+    o[comp] = div_const(d1, 10.0, 0.1);
+    o[2 * comp] = div_const(d2, 10.0, 0.1);
 }
 
 // ------------------------------------------------------------------ host side
@@ -345,8 +475,8 @@ struct FFTPlan {
 int factor(int L, int* rad, int* nst) {
     *nst = 0;
     int m = L;
-    for (const int R : {4, 2, 3, 5}) {
-        while (m % R == 0) {
+    for (const int R : {8, 4, 2, 3, 5}) {
+        while (m % R == 0 && !(R == 8 && m % 32 == 16)) {  // 16 = 4 x 4, not 8 x 2
             if (*nst >= FFT_MAX_STAGES) return -1;
             rad[(*nst)++] = R;
             m /= R;
@@ -379,7 +509,16 @@ int make_plan(int nx, int ny, int nz, FFTPlan& P) {
     P.ax[0].tw = P.tw;
     P.ax[1].tw = P.tw + nx;
     P.ax[2].tw = P.tw + nx + ny;
-    for (int a = 0; a < 3; a++) P.ax[a].G = std::max(1, std::min(16, FFT_BLOCK_LINES / P.ax[a].L));
+    auto magic = [](int d) { return d == 1 ? 0u : (uint32_t)((((uint64_t)1 << 32) + d - 1) / d); };
+    for (int a = 0; a < 3; a++) {
+        FFTAxis& A = P.ax[a];
+        A.G = std::max(1, std::min(16, FFT_POINTS / A.L));
+        A.ml = magic(A.L);
+        for (int st = 0, Ns = 1; st < A.nst; Ns *= A.rad[st++]) {
+            A.mm[st] = magic(A.L / A.rad[st]);
+            A.mn[st] = magic(Ns);
+        }
+    }
     return DRP_OK;
 }
 
@@ -387,7 +526,7 @@ hipError_t fft3d(const FFTPlan& P, double2* data, int sign, hipStream_t st) {
     for (int a = 0; a < 3; a++) {
         const FFTAxis& A = P.ax[a];
         const int64_t blocks = (A.nlines + A.G - 1) / A.G;
-        const size_t lds = 2 * (size_t)A.G * A.L * sizeof(double2);
+        const size_t lds = (size_t)A.G * A.L * sizeof(double2);
         hipLaunchKernelGGL(fft_lines, dim3((unsigned)blocks), dim3(256), lds, st, data, A, sign);
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
@@ -426,7 +565,145 @@ int transform_velocity(drp_lattice* L, const FFTPlan& P, double2* c) {
     return DRP_OK;
 }
 
-unsigned shell_blocks(int64_t n) { return (unsigned)std::min<int64_t>((n + 255) / 256, 2048); }
+}  // namespace
+
+// The spectra's plan, twiddles and work space of one lattice, kept from its first
+// spectrum until it is destroyed: one half spectrum (8.5 B per node) for the energy
+// spectrum, two for the cross spectrum, four for the interaction (34 B per node, 5 %
+// of an FP64 lattice's own memory), and the shell records.  Allocating and freeing the
+// work space per call (48 to 120 B per node of full complex transforms) took most of a
+// call: 10 ms for the analysis of a 256^3 state with an idle memory pool, up to 190 ms
+// when the freed blocks were still in use elsewhere.
+struct drp_diag {
+    FFTPlan P;
+    FFTAxis y, z;          // half-spectrum lines
+    int64_t pitch = 0;     // complex numbers per row: nx/2 + 1 rounded up to 128 bytes
+    int64_t rows = 0;      // ny nz
+    double2* half = nullptr;    // `spectra` half spectra
+    int spectra = 0;
+    double* part = nullptr;     // workgroup records, then the summed bins
+    size_t part_cap = 0;
+    ~drp_diag() {
+        if (half) (void)hipFree(half);
+        if (part) (void)hipFree(part);
+    }
+    double2* spectrum(int k) { return half + k * rows * pitch; }
+};
+
+void diag_free(drp_lattice* L) {
+    delete L->diag;
+    L->diag = nullptr;
+}
+
+namespace {
+
+constexpr int SHELL_WGS = 1280;  // five workgroups of the z pass per CU
+
+// L->diag with room for `spectra` half spectra
+int diag_get(drp_lattice* L, int spectra, drp_diag** out) {
+    if (!L->diag) {
+        drp_diag* D = new (std::nothrow) drp_diag();
+        if (!D) return drp_fail(DRP_ERR_ALLOC, "host allocation failed");
+        const drp_config& c = L->cfg;
+        int rc = make_plan(c.nx, c.ny, c.nz, D->P);
+        if (!rc) {
+            const int hx = c.nx / 2 + 1;
+            D->pitch = (hx + 7) / 8 * 8;
+            D->rows = (int64_t)c.ny * c.nz;
+            D->y = D->P.ax[1];
+            D->y.S = D->pitch;
+            D->y.nlines = (int64_t)hx * c.nz;
+            D->y.F = hx;
+            D->y.so = D->pitch * c.ny;
+            D->z = D->P.ax[2];
+            D->z.S = D->pitch * c.ny;
+            D->z.nlines = (int64_t)hx * c.ny;
+            D->z.F = hx;
+            D->z.so = D->pitch;
+        }
+        if (rc) {
+            delete D;
+            return rc;
+        }
+        L->diag = D;
+    }
+    drp_diag* D = L->diag;
+    if (D->spectra < spectra) {
+        if (D->half) (void)hipFree(D->half);
+        D->half = nullptr;
+        D->spectra = 0;
+        HIP_TRYS(hipMalloc((void**)&D->half, spectra * (size_t)(D->rows * D->pitch) * sizeof(double2)));
+        D->spectra = spectra;
+    }
+    *out = L->diag;
+    return DRP_OK;
+}
+
+// x and y passes of a real field with row pitch in_pitch into half spectrum k
+int half_transform(drp_diag* D, const double* in, int64_t in_pitch, int k, hipStream_t st) {
+    const FFTAxis& X = D->P.ax[0];
+    double2* out = D->spectrum(k);
+    const int64_t pairs = (D->rows + 1) / 2;
+    hipLaunchKernelGGL(rfft_rows, dim3((unsigned)((pairs + X.G - 1) / X.G)), dim3(256),
+                       (size_t)X.G * X.L * sizeof(double2), st, in, in_pitch, D->rows, X, out, D->pitch);
+    HIP_TRYS(hipGetLastError());
+    const FFTAxis& Y = D->y;
+    hipLaunchKernelGGL(fft_lines, dim3((unsigned)((Y.nlines + Y.G - 1) / Y.G)), dim3(256),
+                       (size_t)Y.G * Y.L * sizeof(double2), st, out, Y, -1);
+    HIP_TRYS(hipGetLastError());
+    return DRP_OK;
+}
+
+// the records of the z pass: their number for nbins bins, room for them and the sums
+int shell_records(drp_diag* D, int nbins, int* wgs) {
+    const int64_t groups = (D->z.nlines + D->z.G - 1) / D->z.G;
+    // a few thousand bins per workgroup would outgrow the transforms: fewer workgroups then
+    *wgs = (int)std::min<int64_t>(groups, std::max<int64_t>(256, std::min<int64_t>(SHELL_WGS, (int64_t)SHELL_WGS * 512 / nbins)));
+    const size_t need = ((size_t)*wgs + 1) * nbins;
+    if (D->part_cap < need) {
+        if (D->part) (void)hipFree(D->part);
+        D->part = nullptr;
+        D->part_cap = 0;
+        HIP_TRYS(hipMalloc((void**)&D->part, need * sizeof(double)));
+        D->part_cap = need;
+    }
+    return DRP_OK;
+}
+
+// z pass of half spectrum 0 (and `other`), added to the records
+template <int MODE>
+int shell_pass(drp_lattice* L, drp_diag* D, int other, double inv, int nshells, int nbins, int wgs, bool more) {
+    const FFTAxis& Z = D->z;
+    const size_t lds = (size_t)Z.G * Z.L * sizeof(double2) + nbins * sizeof(double);
+    // (thousands of shells need up to 96 KiB of the CU's 160)
+    if (lds > 64 * 1024)
+        HIP_TRYS(hipFuncSetAttribute(reinterpret_cast<const void*>(&zlines_shells<MODE>),
+                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    hipLaunchKernelGGL((zlines_shells<MODE>), dim3(wgs), dim3(256), lds, L->stream, D->spectrum(0), D->spectrum(other), Z,
+                       L->cfg.nx, L->cfg.ny, L->cfg.nz, inv, nshells, more ? 1 : 0, D->part);
+    HIP_TRYS(hipGetLastError());
+    return DRP_OK;
+}
+
+// the summed bins to the host
+int shell_sums(drp_lattice* L, drp_diag* D, int nbins, int wgs, double* host) {
+    double* out = D->part + (size_t)wgs * nbins;
+    hipLaunchKernelGGL(shells_final, dim3(nbins), dim3(256), 0, L->stream, D->part, wgs, nbins, out);
+    HIP_TRYS(hipGetLastError());
+    HIP_TRYS(hipMemcpyAsync(host, out, (size_t)nbins * sizeof(double), hipMemcpyDeviceToHost, L->stream));
+    HIP_TRYS(hipStreamSynchronize(L->stream));
+    return DRP_OK;
+}
+
+// w_b, b = 0..2, into the half spectra 1..3, in rows of 2 pitch doubles
+int korteweg_divergence(drp_lattice* L, drp_diag* D, const double* phi) {
+    const drp_config& c = L->cfg;
+    const int tx = (c.nx + WTX - 1) / WTX, ty = (c.ny + WTY - 1) / WTY, tz = (c.nz + WTZ - 1) / WTZ;
+    hipLaunchKernelGGL(div_korteweg, dim3((unsigned)(tx * ty * tz)), dim3(WNT), 0, L->stream, c.nx, c.ny, c.nz, phi,
+                       (double*)D->spectrum(1), 2 * D->pitch, 2 * D->pitch * D->rows, tx, ty);
+    HIP_TRYS(hipGetLastError());
+    return DRP_OK;
+}
 
 }  // namespace
 
@@ -451,24 +728,18 @@ constexpr int MAX_SHELLS = 8192;  // shell bins of one workgroup in LDS
 extern "C" int drp_energy_spectrum(drp_lattice* L, double* E, int nshells) {
     if (!L || !E || nshells < 1 || nshells > MAX_SHELLS) return drp_fail(DRP_ERR_ARG, "bad spectrum arguments");
     if (!L->initialized) return drp_fail(DRP_ERR_STATE, "lattice not initialised");
-    const drp_config& c = L->cfg;
-    FFTPlan P;
-    int rc = make_plan(c.nx, c.ny, c.nz, P);
+    drp_diag* D = nullptr;
+    int rc = diag_get(L, 1, &D);
     if (rc) return rc;
-    const int64_t n = L->n;
-    DevMem cu, dE;
-    HIP_TRYS(hipMalloc(&cu.p, 3 * (size_t)n * sizeof(double2)));
-    HIP_TRYS(hipMalloc(&dE.p, (size_t)nshells * sizeof(double)));
-    rc = transform_velocity(L, P, (double2*)cu.p);
-    if (rc) return rc;
-    HIP_TRYS(hipMemsetAsync(dE.p, 0, (size_t)nshells * sizeof(double), L->stream));
-    const double2* u = (const double2*)cu.p;
-    hipLaunchKernelGGL(shell_energy, dim3(shell_blocks(n)), dim3(256), (size_t)nshells * sizeof(double), L->stream,
-                       c.nx, c.ny, c.nz, u, u + n, u + 2 * n, 1.0 / (double)n, nshells, (double*)dE.p);
-    HIP_TRYS(hipGetLastError());
-    HIP_TRYS(hipMemcpyAsync(E, dE.p, (size_t)nshells * sizeof(double), hipMemcpyDeviceToHost, L->stream));
-    HIP_TRYS(hipStreamSynchronize(L->stream));
-    return DRP_OK;
+    const double* mac = nullptr;
+    int wgs = 0;
+    rc = velocity_view(L, &mac);
+    if (!rc) rc = shell_records(D, nshells, &wgs);
+    for (int k = 0; k < 3 && !rc; k++) {
+        rc = half_transform(D, mac + (2 + k) * L->n, L->cfg.nx, 0, L->stream);
+        if (!rc) rc = shell_pass<SHELL_ENERGY>(L, D, 0, 1.0 / (double)L->n, nshells, nshells, wgs, k > 0);
+    }
+    return rc ? rc : shell_sums(L, D, nshells, wgs, E);
 }
 
 extern "C" int drp_filter_velocity(drp_lattice* L, int kind, int k, double* u1, double* u2, double* u3, size_t n_) {
@@ -507,37 +778,23 @@ extern "C" int drp_filter_velocity(drp_lattice* L, int kind, int k, double* u1, 
 extern "C" int drp_scale_interaction(drp_lattice* L, double* C, int nshells) {
     if (!L || !C || nshells < 1 || nshells > MAX_SHELLS) return drp_fail(DRP_ERR_ARG, "bad interaction arguments");
     if (!L->initialized) return drp_fail(DRP_ERR_STATE, "lattice not initialised");
-    const drp_config& c = L->cfg;
-    FFTPlan P;
-    int rc = make_plan(c.nx, c.ny, c.nz, P);
-    if (rc) return rc;
-    const int64_t n = L->n;
-    DevMem cu, cw, gp, dC;
-    HIP_TRYS(hipMalloc(&cu.p, 3 * (size_t)n * sizeof(double2)));
-    HIP_TRYS(hipMalloc(&cw.p, 3 * (size_t)n * sizeof(double2)));
-    HIP_TRYS(hipMalloc(&gp.p, 3 * (size_t)n * sizeof(double)));
-    HIP_TRYS(hipMalloc(&dC.p, (size_t)nshells * sizeof(double)));
-    rc = transform_velocity(L, P, (double2*)cu.p);
+    drp_diag* D = nullptr;
+    int rc = diag_get(L, 4, &D);
     if (rc) return rc;
     const double* mac = nullptr;
+    int wgs = 0;
     rc = velocity_view(L, &mac);
-    if (rc) return rc;
-    const unsigned nb = (unsigned)((n + 255) / 256);
-    hipLaunchKernelGGL(grad_phi, dim3(nb), dim3(256), 0, L->stream, c.nx, c.ny, c.nz, mac, (double*)gp.p);
-    HIP_TRYS(hipGetLastError());
-    hipLaunchKernelGGL(div_korteweg, dim3(nb), dim3(256), 0, L->stream, c.nx, c.ny, c.nz, (const double*)gp.p,
-                       (double2*)cw.p);
-    HIP_TRYS(hipGetLastError());
-    for (int a = 0; a < 3; a++) HIP_TRYS(fft3d(P, (double2*)cw.p + a * n, -1, L->stream));
-    HIP_TRYS(hipMemsetAsync(dC.p, 0, (size_t)nshells * sizeof(double), L->stream));
-    hipLaunchKernelGGL(shell_cross, dim3(shell_blocks(n)), dim3(256), (size_t)nshells * sizeof(double), L->stream,
-                       c.nx, c.ny, c.nz, (const double2*)cu.p, (const double2*)cw.p, 1.0 / (double)n, nshells,
-                       (double*)dC.p);
-    HIP_TRYS(hipGetLastError());
+    if (!rc) rc = shell_records(D, nshells, &wgs);
+    if (!rc) rc = korteweg_divergence(L, D, mac);
+    for (int b = 0; b < 3 && !rc; b++) {
+        rc = half_transform(D, (const double*)D->spectrum(1 + b), 2 * D->pitch, 1 + b, L->stream);
+        if (!rc) rc = half_transform(D, mac + (2 + b) * L->n, L->cfg.nx, 0, L->stream);
+        if (!rc) rc = shell_pass<SHELL_CROSS>(L, D, 1 + b, 1.0 / (double)L->n, nshells, nshells, wgs, b > 0);
+    }
     std::vector<double> h(nshells);
-    HIP_TRYS(hipMemcpyAsync(h.data(), dC.p, (size_t)nshells * sizeof(double), hipMemcpyDeviceToHost, L->stream));
-    HIP_TRYS(hipStreamSynchronize(L->stream));
-    for (int s = 0; s < nshells; s++) C[s] = c.kappa_g * h[s];
+    if (!rc) rc = shell_sums(L, D, nshells, wgs, h.data());
+    if (rc) return rc;
+    for (int s = 0; s < nshells; s++) C[s] = L->cfg.kappa_g * h[s];
     return DRP_OK;
 }
 
@@ -547,36 +804,23 @@ extern "C" int drp_phi_contribution(drp_lattice* L, double* C, int nshells, doub
     const drp_config& c = L->cfg;
     const int nb = c.nx / 2 + 1;  // the reference's (xmax+1)/2 + 1 shells
     if (nshells < 1 || nshells > nb) return drp_fail(DRP_ERR_ARG, "nshells %d not in 1..%d", nshells, nb);
-    FFTPlan P;
-    int rc = make_plan(c.nx, c.ny, c.nz, P);
+    drp_diag* D = nullptr;
+    int rc = diag_get(L, 2, &D);
     if (rc) return rc;
     const double* mac = nullptr;
+    int wgs = 0;
     rc = velocity_view(L, &mac);
-    if (rc) return rc;
-    const int64_t n = L->n;
-    DevMem ca, tmp, dC;
-    HIP_TRYS(hipMalloc(&ca.p, 2 * (size_t)n * sizeof(double2)));
-    HIP_TRYS(hipMalloc(&tmp.p, (size_t)n * sizeof(double)));
-    HIP_TRYS(hipMalloc(&dC.p, 2 * (size_t)nb * sizeof(double)));
-    double2* adv = (double2*)ca.p;
-    double2* mu = adv + n;
-    const unsigned nblk = (unsigned)((n + 255) / 256);
+    if (!rc) rc = shell_records(D, 2 * nb, &wgs);
     const int kinds[2] = {DRP_DERIVED_ADVECTION, DRP_DERIVED_CHEMICAL_POTENTIAL};
-    double2* dst[2] = {adv, mu};
-    for (int k = 0; k < 2; k++) {
-        HIP_TRYS(launch_derived_fp64(c.nx, c.ny, c.nz, L->phys, mac, kinds[k], (double*)tmp.p, L->stream));
-        hipLaunchKernelGGL(to_complex, dim3(nblk), dim3(256), 0, L->stream, n, (const double*)tmp.p, dst[k]);
-        HIP_TRYS(hipGetLastError());
-        HIP_TRYS(fft3d(P, dst[k], -1, L->stream));
+    for (int k = 0; k < 2 && !rc; k++) {
+        double* field = (double*)D->spectrum(k);
+        HIP_TRYS(launch_derived_fp64(c.nx, c.ny, c.nz, L->phys, mac, kinds[k], field, 2 * D->pitch, L->stream));
+        rc = half_transform(D, field, 2 * D->pitch, k, L->stream);
     }
-    HIP_TRYS(hipMemsetAsync(dC.p, 0, 2 * (size_t)nb * sizeof(double), L->stream));
-    double* dsum = (double*)dC.p;
-    hipLaunchKernelGGL(shell_cross_half, dim3(shell_blocks(n)), dim3(256), 2 * (size_t)nb * sizeof(double), L->stream,
-                       c.nx, c.ny, c.nz, (const double2*)adv, (const double2*)mu, nb, dsum, dsum + nb);
-    HIP_TRYS(hipGetLastError());
+    if (!rc) rc = shell_pass<SHELL_CROSS_HALF>(L, D, 1, 1.0, nb, 2 * nb, wgs, false);
     std::vector<double> h(2 * (size_t)nb);
-    HIP_TRYS(hipMemcpyAsync(h.data(), dsum, h.size() * sizeof(double), hipMemcpyDeviceToHost, L->stream));
-    HIP_TRYS(hipStreamSynchronize(L->stream));
+    if (!rc) rc = shell_sums(L, D, 2 * nb, wgs, h.data());
+    if (rc) return rc;
     std::vector<double> res(nb);
     for (int s = 0; s < nb; s++) res[s] = h[nb + s] > 0.0 ? h[s] / h[nb + s] : 0.0;
     for (int s = 0; s < nshells; s++) C[s] = res[s];
