@@ -46,7 +46,7 @@ struct drp_tape {
     int64_t bytes = 0;
 };
 
-static size_t state_doubles(const drp_lattice* L) { return 35 * (size_t)L->n; }
+static size_t state_doubles(const drp_lattice* L) { return 35 * (size_t)L->ns; }
 
 static int tape_alloc(drp_tape* T, void** p, size_t bytes) {
     HIP_TRYA(hipMalloc(p, bytes));
@@ -56,7 +56,7 @@ static int tape_alloc(drp_tape* T, void** p, size_t bytes) {
 
 static int save_checkpoint(drp_tape* T) {
     drp_lattice* L = T->L;
-    const size_t n = (size_t)L->n;
+    const size_t n = (size_t)L->ns;
     double* c = nullptr;
     int rc = tape_alloc(T, (void**)&c, state_doubles(L) * sizeof(double));
     if (rc) return rc;
@@ -132,13 +132,13 @@ extern "C" int drp_tape_loss(drp_tape* T, const double w[2], double* loss, doubl
 
 static int ensure_work(drp_tape* T) {
     drp_lattice* L = T->L;
-    const size_t n = (size_t)L->n;
+    const size_t n = (size_t)L->ns;
     int rc = DRP_OK;
     if (!T->seg && T->K > 1) rc = tape_alloc(T, (void**)&T->seg, (size_t)(T->K - 1) * state_doubles(L) * sizeof(double));
     if (!rc && !T->adj) rc = tape_alloc(T, (void**)&T->adj, 2 * 30 * n * sizeof(double));
     if (!rc && !T->phin) rc = tape_alloc(T, (void**)&T->phin, 2 * n * sizeof(double));
     if (!rc && !T->work) rc = tape_alloc(T, (void**)&T->work, 4 * n * sizeof(double));
-    T->nblk = adj_block_count((int64_t)n);
+    T->nblk = adj_block_count(L->n);
     if (!rc && !T->acc) rc = tape_alloc(T, (void**)&T->acc, (size_t)T->nblk * 3 * sizeof(double));
     if (!rc && !T->plane) rc = tape_alloc(T, (void**)&T->plane, (size_t)L->cfg.nx * std::max(L->cfg.ny, L->cfg.nz) * sizeof(double));
     if (!rc && !T->range) {
@@ -162,7 +162,7 @@ extern "C" int drp_tape_backward(drp_tape* T, const double w[2], double* loss, d
     int rc = ensure_work(T);
     if (rc) return rc;
     const drp_config& c = L->cfg;
-    const int64_t n = L->n;
+    const int64_t n = L->ns;  // from one array of a state to the next
     hipStream_t st = L->stream;
 
     // ---- loss and its seed dJ/dphi at the final state
@@ -177,8 +177,8 @@ extern "C" int drp_tape_backward(drp_tape* T, const double w[2], double* loss, d
     double* gradA = T->work + n;
     HIP_TRYA(hipMemsetAsync(Fa[cur], 0, 30 * n * sizeof(double), st));
     HIP_TRYA(hipMemsetAsync(T->acc, 0, (size_t)T->nblk * 3 * sizeof(double), st));
-    HIP_TRYA(launch_adj_seed_area_fp64(c.nx, c.ny, c.nz, (const double*)L->mac[L->cur], w[1], lapA, gradA, st));
-    HIP_TRYA(launch_adj_stencil_fp64(c.nx, c.ny, c.nz, lapA, gradA, Pa[cur], st));
+    HIP_TRYA(launch_adj_seed_area_fp64(c.nx, c.ny, c.nz, n, (const double*)L->mac[L->cur], w[1], lapA, gradA, st));
+    HIP_TRYA(launch_adj_stencil_fp64(c.nx, c.ny, c.nz, n, lapA, gradA, Pa[cur], st));
     if (w[0] != 0.0) {
         double D;
         int n1 = 0, n2 = 0, third = 0;
@@ -223,7 +223,8 @@ extern "C" int drp_tape_backward(drp_tape* T, const double w[2], double* loss, d
             a.nx = c.nx;
             a.ny = c.ny;
             a.nz = c.nz;
-            a.n = n;
+            a.n = L->n;
+            a.ns = n;
             a.f = state;
             a.mac = state + 30 * n;
             a.Fin = Fa[cur];
@@ -251,7 +252,7 @@ extern "C" int drp_tape_backward(drp_tape* T, const double w[2], double* loss, d
             a.wall_active = (c.wall_axis != DRP_WALL_NONE && nstep >= c.wall_start) ? 1 : 0;
             a.first = (rel == 0 && T->start_eq) ? 1 : 0;
             HIP_TRYA(launch_adj_collide_fp64(a, st));
-            if (rel > 0) HIP_TRYA(launch_adj_stencil_fp64(c.nx, c.ny, c.nz, lapA, gradA, Pa[1 - cur], st));
+            if (rel > 0) HIP_TRYA(launch_adj_stencil_fp64(c.nx, c.ny, c.nz, n, lapA, gradA, Pa[1 - cur], st));
             cur = 1 - cur;
         }
     }

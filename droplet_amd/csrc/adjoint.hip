@@ -84,10 +84,10 @@ __device__ void block_accumulate(double v0, double v1, double v2, double* acc) {
 // five wavefronts per SIMD: 96 VGPRs hold the rolled direction loops without spilling
 __global__ __launch_bounds__(ADJ_BLOCK) __attribute__((amdgpu_waves_per_eu(5))) void adj_collide_fp64(AdjArgs a) {
     const int nx = a.nx, ny = a.ny, nz = a.nz;
-    const int64_t n = a.n;
+    const int64_t n = a.ns;  // from one array to the next
     const uint32_t s = blockIdx.x * (uint32_t)ADJ_BLOCK + threadIdx.x;
     double d_tauf = 0.0, d_kg = 0.0, d_u = 0.0;
-    if (s < (uint64_t)n) {
+    if (s < (uint64_t)a.n) {
         const Node c = coords(s, nx, ny);
         const double phi = a.mac[s];
         const double u[3] = {a.mac[2 * n + s], a.mac[3 * n + s], a.mac[4 * n + s]};
@@ -218,12 +218,11 @@ __global__ __launch_bounds__(ADJ_BLOCK) __attribute__((amdgpu_waves_per_eu(5))) 
 }
 
 // phih_st(x) = -14/5 laph(x) + sum_{q>=1} [laph(x - c_q)/5 + c_q . gradh(x - c_q)/10]
-__global__ __launch_bounds__(ADJ_BLOCK) void adj_stencil_fp64(int nx, int ny, int nz, const double* __restrict__ lapA,
+__global__ __launch_bounds__(ADJ_BLOCK) void adj_stencil_fp64(int nx, int ny, int nz, int64_t n, const double* __restrict__ lapA,
                                                               const double* __restrict__ gradA,
                                                               double* __restrict__ out) {
-    const int64_t n = (int64_t)nx * ny * nz;
     const uint32_t s = blockIdx.x * (uint32_t)ADJ_BLOCK + threadIdx.x;
-    if (s >= (uint64_t)n) return;
+    if (s >= (uint64_t)nx * ny * nz) return;
     const Node c = coords(s, nx, ny);
     double l = 0.0, g = 0.0;
 #pragma unroll
@@ -236,12 +235,11 @@ __global__ __launch_bounds__(ADJ_BLOCK) void adj_stencil_fp64(int nx, int ny, in
 }
 
 // seed of sum_x |grad phi(x)|: gradA = w grad phi / |grad phi| (0 where grad phi = 0), lapA = 0
-__global__ __launch_bounds__(ADJ_BLOCK) void adj_seed_area_fp64(int nx, int ny, int nz, const double* __restrict__ phi,
+__global__ __launch_bounds__(ADJ_BLOCK) void adj_seed_area_fp64(int nx, int ny, int nz, int64_t n, const double* __restrict__ phi,
                                                                 double w, double* __restrict__ lapA,
                                                                 double* __restrict__ gradA) {
-    const int64_t n = (int64_t)nx * ny * nz;
     const uint32_t s = blockIdx.x * (uint32_t)ADJ_BLOCK + threadIdx.x;
-    if (s >= (uint64_t)n) return;
+    if (s >= (uint64_t)nx * ny * nz) return;
     const Node c = coords(s, nx, ny);
     double gr[3] = {0.0, 0.0, 0.0};
 #pragma unroll
@@ -280,17 +278,17 @@ hipError_t launch_adj_collide_fp64(const AdjArgs& a, hipStream_t st) {
     return hipGetLastError();
 }
 
-hipError_t launch_adj_stencil_fp64(int nx, int ny, int nz, const double* lapA, const double* gradA, double* out,
+hipError_t launch_adj_stencil_fp64(int nx, int ny, int nz, int64_t ns, const double* lapA, const double* gradA, double* out,
                                    hipStream_t st) {
     hipLaunchKernelGGL(adj_stencil_fp64, dim3(nblocks((int64_t)nx * ny * nz)), dim3(ADJ_BLOCK), 0, st, nx, ny, nz,
-                       lapA, gradA, out);
+                       ns, lapA, gradA, out);
     return hipGetLastError();
 }
 
-hipError_t launch_adj_seed_area_fp64(int nx, int ny, int nz, const double* phi, double w, double* lapA,
+hipError_t launch_adj_seed_area_fp64(int nx, int ny, int nz, int64_t ns, const double* phi, double w, double* lapA,
                                      double* gradA, hipStream_t st) {
     hipLaunchKernelGGL(adj_seed_area_fp64, dim3(nblocks((int64_t)nx * ny * nz)), dim3(ADJ_BLOCK), 0, st, nx, ny,
-                       nz, phi, w, lapA, gradA);
+                       nz, ns, phi, w, lapA, gradA);
     return hipGetLastError();
 }
 

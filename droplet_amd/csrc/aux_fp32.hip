@@ -15,55 +15,55 @@ template <int Q0, int Q1, typename Fn> __device__ __forceinline__ void sforx(Fn&
 
 static inline dim3 grid_for(int64_t n) { return dim3((unsigned)((n + 255) / 256)); }
 
-__global__ void to_shifted(int64_t n, ShiftRef r, const double* __restrict__ pop64, const double* __restrict__ mac64,
+__global__ void to_shifted(int64_t n, int64_t ns, ShiftRef r, const double* __restrict__ pop64, const double* __restrict__ mac64,
                            float* __restrict__ pop32, float* __restrict__ mac32) {
     const int64_t s = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     if (s >= n) return;
     sforx<0, 15>([&](auto qc) {
         constexpr int q = decltype(qc)::value;
-        pop32[q * n + s] = (float)(pop64[q * n + s] - r.fr[q]);
-        pop32[(15 + q) * n + s] = (float)(pop64[(15 + q) * n + s] - weightE<q>());
+        pop32[q * ns + s] = (float)(pop64[q * ns + s] - r.fr[q]);
+        pop32[(15 + q) * ns + s] = (float)(pop64[(15 + q) * ns + s] - weightE<q>());
     });
     mac32[s] = (float)(mac64[s] - r.phi1);
-    mac32[n + s] = (float)(mac64[n + s] - 1.0 / 3.0);
-    mac32[2 * n + s] = (float)mac64[2 * n + s];
-    mac32[3 * n + s] = (float)mac64[3 * n + s];
-    mac32[4 * n + s] = (float)mac64[4 * n + s];
+    mac32[ns + s] = (float)(mac64[ns + s] - 1.0 / 3.0);
+    mac32[2 * ns + s] = (float)mac64[2 * ns + s];
+    mac32[3 * ns + s] = (float)mac64[3 * ns + s];
+    mac32[4 * ns + s] = (float)mac64[4 * ns + s];
 }
 
-__global__ void pops_from_shifted(int64_t n, ShiftRef r, const float* __restrict__ pop32, double* __restrict__ out,
+__global__ void pops_from_shifted(int64_t n, int64_t ns, ShiftRef r, const float* __restrict__ pop32, double* __restrict__ out,
                                   int set) {
     const int64_t s = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     if (s >= n) return;
     sforx<0, 15>([&](auto qc) {
         constexpr int q = decltype(qc)::value;
         const double ref = set == 0 ? r.fr[q] : weightE<q>();
-        out[q * n + s] = ref + (double)pop32[(set * 15 + q) * n + s];
+        out[q * n + s] = ref + (double)pop32[(set * 15 + q) * ns + s];
     });
 }
 
-__global__ void pops_to_shifted(int64_t n, ShiftRef r, const double* __restrict__ in, float* __restrict__ pop32,
+__global__ void pops_to_shifted(int64_t n, int64_t ns, ShiftRef r, const double* __restrict__ in, float* __restrict__ pop32,
                                 int set) {
     const int64_t s = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     if (s >= n) return;
     sforx<0, 15>([&](auto qc) {
         constexpr int q = decltype(qc)::value;
         const double ref = set == 0 ? r.fr[q] : weightE<q>();
-        pop32[(set * 15 + q) * n + s] = (float)(in[q * n + s] - ref);
+        pop32[(set * 15 + q) * ns + s] = (float)(in[q * n + s] - ref);
     });
 }
 
-__global__ void macro_from_shifted(int64_t n, double phi1, const float* __restrict__ m32, double* __restrict__ m64) {
+__global__ void macro_from_shifted(int64_t n, int64_t ns, double phi1, const float* __restrict__ m32, double* __restrict__ m64) {
     const int64_t s = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     if (s >= n) return;
     m64[s] = phi1 + (double)m32[s];
-    m64[n + s] = 1.0 / 3.0 + (double)m32[n + s];
-    m64[2 * n + s] = (double)m32[2 * n + s];
-    m64[3 * n + s] = (double)m32[3 * n + s];
-    m64[4 * n + s] = (double)m32[4 * n + s];
+    m64[ns + s] = 1.0 / 3.0 + (double)m32[ns + s];
+    m64[2 * ns + s] = (double)m32[2 * ns + s];
+    m64[3 * ns + s] = (double)m32[3 * ns + s];
+    m64[4 * ns + s] = (double)m32[4 * ns + s];
 }
 
-__global__ void moments_fp32(int64_t n, const float* __restrict__ f, const float* __restrict__ g,
+__global__ void moments_fp32(int64_t n, int64_t ns, const float* __restrict__ f, const float* __restrict__ g,
                              float* __restrict__ mac, int which) {
     const int64_t s = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     if (s >= n) return;
@@ -72,8 +72,8 @@ __global__ void moments_fp32(int64_t n, const float* __restrict__ f, const float
     sforx<0, 15>([&](auto qc) {
         constexpr int q = decltype(qc)::value;
         using D = Dir<q>;
-        const float gv = g[q * n + s];
-        ph += (double)f[q * n + s];
+        const float gv = g[q * ns + s];
+        ph += (double)f[q * ns + s];
         pr += gv;
         m1 = acc<D::cx>(m1, gv);
         m2 = acc<D::cy>(m2, gv);
@@ -81,10 +81,10 @@ __global__ void moments_fp32(int64_t n, const float* __restrict__ f, const float
     });
     if (which & 1) mac[s] = (float)ph;
     if (which & 2) {
-        mac[n + s] = pr * (1.0f / 3.0f);
-        mac[2 * n + s] = m1;
-        mac[3 * n + s] = m2;
-        mac[4 * n + s] = m3;
+        mac[ns + s] = pr * (1.0f / 3.0f);
+        mac[2 * ns + s] = m1;
+        mac[3 * ns + s] = m2;
+        mac[4 * ns + s] = m3;
     }
 }
 
@@ -92,7 +92,7 @@ __global__ void moments_fp32(int64_t n, const float* __restrict__ f, const float
 // the state a step left (mac) and the one it started from (mac_old), every
 // neighbour outside the node's rank block (B, periodic wraps included) from
 // mac_old (B.bx = 0: all from mac).
-__global__ void les_tau_fp32(int nx, int ny, int nz, Phys P, const float* __restrict__ mac,
+__global__ void les_tau_fp32(int nx, int ny, int nz, int64_t ns, Phys P, const float* __restrict__ mac,
                              const float* __restrict__ mac_old, LesBlocks B, const uint64_t* __restrict__ range,
                              int slot, float* __restrict__ tau) {
     const int64_t N = (int64_t)nx * ny * nz;
@@ -114,7 +114,7 @@ __global__ void les_tau_fp32(int nx, int ny, int nz, Phys P, const float* __rest
         zz = zz < 0 ? zz + nz : (zz >= nz ? zz - nz : zz);
         const int64_t t = xx + (int64_t)nx * (yy + (int64_t)ny * zz);
         for (int k = 0; k < 3; k++) {
-            const float v = u[(2 + k) * N + t];
+            const float v = u[(2 + k) * ns + t];
             gu[k][0] = acc<D::cx>(gu[k][0], v);
             gu[k][1] = acc<D::cy>(gu[k][1], v);
             gu[k][2] = acc<D::cz>(gu[k][2], v);
@@ -145,11 +145,10 @@ __device__ __forceinline__ int wrap_zm32(int v, int n, bool small) {
     if (small) return ((v % n) + n) % n;
     return v < 0 ? v + n : (v >= n ? v - n : v);
 }
-__global__ __launch_bounds__(ZM32_NT) void les_tau_fp32_zm(int nx, int ny, int nz, Phys P, const float* __restrict__ mac,
+__global__ __launch_bounds__(ZM32_NT) void les_tau_fp32_zm(int nx, int ny, int nz, int64_t N, Phys P, const float* __restrict__ mac,
                                                           const uint64_t* __restrict__ range, int slot,
                                                           float* __restrict__ tau, int tiles_x, int tiles_y) {
     __shared__ float su[3][3][ZM32_HP];  // [ring slot][component][plane node]
-    const int64_t N = (int64_t)nx * ny * nz;
     const int x0 = (blockIdx.x % tiles_x) * ZM32_TX, y0 = ((blockIdx.x / tiles_x) % tiles_y) * ZM32_TY;
     const int zs = (blockIdx.x / (tiles_x * tiles_y)) * ZM32_ZC, ze = min(zs + ZM32_ZC, nz);
     const bool small = nx <= ZM32_TX || ny <= ZM32_TY || nz <= 2;
@@ -222,38 +221,38 @@ __global__ __launch_bounds__(ZM32_NT) void les_tau_fp32_zm(int nx, int ny, int n
     }
 }
 
-hipError_t launch_to_shifted(int64_t n, const ShiftRef& r, const double* pop64, const double* mac64, float* pop32,
+hipError_t launch_to_shifted(int64_t n, int64_t ns, const ShiftRef& r, const double* pop64, const double* mac64, float* pop32,
                              float* mac32, hipStream_t st) {
-    hipLaunchKernelGGL(to_shifted, grid_for(n), dim3(256), 0, st, n, r, pop64, mac64, pop32, mac32);
+    hipLaunchKernelGGL(to_shifted, grid_for(n), dim3(256), 0, st, n, ns, r, pop64, mac64, pop32, mac32);
     return hipGetLastError();
 }
-hipError_t launch_pops_from_shifted(int64_t n, const ShiftRef& r, const float* pop32, double* pop64, int set,
+hipError_t launch_pops_from_shifted(int64_t n, int64_t ns, const ShiftRef& r, const float* pop32, double* pop64, int set,
                                     hipStream_t st) {
-    hipLaunchKernelGGL(pops_from_shifted, grid_for(n), dim3(256), 0, st, n, r, pop32, pop64, set);
+    hipLaunchKernelGGL(pops_from_shifted, grid_for(n), dim3(256), 0, st, n, ns, r, pop32, pop64, set);
     return hipGetLastError();
 }
-hipError_t launch_pops_to_shifted(int64_t n, const ShiftRef& r, const double* pop64, float* pop32, int set,
+hipError_t launch_pops_to_shifted(int64_t n, int64_t ns, const ShiftRef& r, const double* pop64, float* pop32, int set,
                                   hipStream_t st) {
-    hipLaunchKernelGGL(pops_to_shifted, grid_for(n), dim3(256), 0, st, n, r, pop64, pop32, set);
+    hipLaunchKernelGGL(pops_to_shifted, grid_for(n), dim3(256), 0, st, n, ns, r, pop64, pop32, set);
     return hipGetLastError();
 }
-hipError_t launch_macro_from_shifted(int64_t n, double phi1, const float* mac32, double* mac64, hipStream_t st) {
-    hipLaunchKernelGGL(macro_from_shifted, grid_for(n), dim3(256), 0, st, n, phi1, mac32, mac64);
+hipError_t launch_macro_from_shifted(int64_t n, int64_t ns, double phi1, const float* mac32, double* mac64, hipStream_t st) {
+    hipLaunchKernelGGL(macro_from_shifted, grid_for(n), dim3(256), 0, st, n, ns, phi1, mac32, mac64);
     return hipGetLastError();
 }
-hipError_t launch_moments_fp32(int64_t n, const float* f, const float* g, float* mac, int which, hipStream_t st) {
-    hipLaunchKernelGGL(moments_fp32, grid_for(n), dim3(256), 0, st, n, f, g, mac, which);
+hipError_t launch_moments_fp32(int64_t n, int64_t ns, const float* f, const float* g, float* mac, int which, hipStream_t st) {
+    hipLaunchKernelGGL(moments_fp32, grid_for(n), dim3(256), 0, st, n, ns, f, g, mac, which);
     return hipGetLastError();
 }
-hipError_t launch_les_tau_fp32(int nx, int ny, int nz, const Phys& ph, const float* mac, const float* mac_old,
+hipError_t launch_les_tau_fp32(int nx, int ny, int nz, int64_t ns, const Phys& ph, const float* mac, const float* mac_old,
                                const LesBlocks& blk, const uint64_t* range, int slot, float* tau, hipStream_t st) {
     const int64_t n = (int64_t)nx * ny * nz;
     if (blk.bx > 0 && mac_old != mac) {
-        hipLaunchKernelGGL(les_tau_fp32, grid_for(n), dim3(256), 0, st, nx, ny, nz, ph, mac, mac_old, blk, range, slot,
+        hipLaunchKernelGGL(les_tau_fp32, grid_for(n), dim3(256), 0, st, nx, ny, nz, ns, ph, mac, mac_old, blk, range, slot,
                            tau);
     } else {
         const int mx = (nx + ZM32_TX - 1) / ZM32_TX, my = (ny + ZM32_TY - 1) / ZM32_TY, mz = (nz + ZM32_ZC - 1) / ZM32_ZC;
-        hipLaunchKernelGGL(les_tau_fp32_zm, dim3((unsigned)(mx * my * mz)), dim3(ZM32_NT), 0, st, nx, ny, nz, ph, mac,
+        hipLaunchKernelGGL(les_tau_fp32_zm, dim3((unsigned)(mx * my * mz)), dim3(ZM32_NT), 0, st, nx, ny, nz, ns, ph, mac,
                            range, slot, tau, mx, my);
     }
     return hipGetLastError();

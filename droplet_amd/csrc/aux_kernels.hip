@@ -76,11 +76,10 @@ __device__ __forceinline__ bool les_halo(const LesBlocks& B, int x, int y, int z
     return xx < x0 || xx >= x0 + B.bx || yy < y0 || yy >= y0 + B.by || zz < z0 || zz >= z0 + B.bz;
 }
 
-__global__ void init_equilibrium_fp64(Grid G, Phys P, const double* __restrict__ mac, double* __restrict__ f,
+__global__ void init_equilibrium_fp64(Grid G, int64_t N, Phys P, const double* __restrict__ mac, double* __restrict__ f,
                                       double* __restrict__ g) {
-    const int64_t N = (int64_t)G.nx * G.ny * G.nz;
     const int64_t s = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (s >= N) return;
+    if (s >= (int64_t)G.nx * G.ny * G.nz) return;
     const int x = s % G.nx, y = (s / G.nx) % G.ny, z = s / ((int64_t)G.nx * G.ny);
     NodeEq<double> nd;
     nd.phi = mac[s];
@@ -103,10 +102,10 @@ __global__ void init_equilibrium_fp64(Grid G, Phys P, const double* __restrict__
     });
 }
 
-__global__ void moments_fp64(int64_t N, const double* __restrict__ f, const double* __restrict__ g,
+__global__ void moments_fp64(int64_t n, int64_t N, const double* __restrict__ f, const double* __restrict__ g,
                              double* __restrict__ mac, int which) {
     const int64_t s = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (s >= N) return;
+    if (s >= n) return;
     double ph = f[s], pr = g[s] / 3.0, m1 = 0.0, m2 = 0.0, m3 = 0.0;
     sfor<1, 15>([&](auto qc) {
         constexpr int q = decltype(qc)::value;
@@ -146,7 +145,7 @@ __device__ __forceinline__ int wrap_any(int v, int n, bool small) {
 // u (and, with rank blocks, the old u) of a tile and its 1-node halo are staged
 // in LDS once per workgroup.
 template <bool STALE>
-__global__ __launch_bounds__(LES_TX* LES_TY* LES_TZ) void les_tau_fp64(Grid G, Phys P, const double* __restrict__ mac,
+__global__ __launch_bounds__(LES_TX* LES_TY* LES_TZ) void les_tau_fp64(Grid G, int64_t N, Phys P, const double* __restrict__ mac,
                                                                        const double* __restrict__ mac_old, LesBlocks B,
                                                                        const uint64_t* __restrict__ range, int slot,
                                                                        double* __restrict__ tau, int tiles_x,
@@ -154,7 +153,6 @@ __global__ __launch_bounds__(LES_TX* LES_TY* LES_TZ) void les_tau_fp64(Grid G, P
     constexpr int HX = LES_TX + 2, HY = LES_TY + 2, HZ = LES_TZ + 2, H = HX * HY * HZ, NT = LES_TX * LES_TY * LES_TZ;
     __shared__ double su[3][H];
     __shared__ double so[STALE ? 3 : 1][STALE ? H : 1];
-    const int64_t N = (int64_t)G.nx * G.ny * G.nz;
     const int tile = blockIdx.x;
     const int x0 = (tile % tiles_x) * LES_TX, y0 = ((tile / tiles_x) % tiles_y) * LES_TY,
               z0 = (tile / (tiles_x * tiles_y)) * LES_TZ;
@@ -251,11 +249,10 @@ template <typename T, int NC> __device__ __forceinline__ void zm_store(const ZmP
     }
 }
 
-__global__ __launch_bounds__(ZM_NT) void les_tau_fp64_zm(Grid G, Phys P, const double* __restrict__ mac,
+__global__ __launch_bounds__(ZM_NT) void les_tau_fp64_zm(Grid G, int64_t N, Phys P, const double* __restrict__ mac,
                                                           const uint64_t* __restrict__ range, int slot,
                                                           double* __restrict__ tau, int tiles_x, int tiles_y) {
     __shared__ double su[3][3][ZM_HP];  // [ring slot][component][plane node]
-    const int64_t N = (int64_t)G.nx * G.ny * G.nz;
     const int x0 = (blockIdx.x % tiles_x) * ZM_TX, y0 = ((blockIdx.x / tiles_x) % tiles_y) * ZM_TY;
     const int zs = (blockIdx.x / (tiles_x * tiles_y)) * ZM_ZC, ze = min(zs + ZM_ZC, G.nz);
     const bool small = G.nx <= ZM_TX || G.ny <= ZM_TY || G.nz <= 2;
@@ -331,12 +328,12 @@ __device__ __forceinline__ void add_comp(double& s, double& c, double v) {
 // REDUCE_MAX_BLOCKS of them run, each over a fixed set of columns, and leave one
 // record each.  Per-thread sums are compensated, so the longer per-thread chain
 // costs no accuracy against the tree over single nodes.
-__global__ __launch_bounds__(ZM_NT) void reduce_fp64(Grid G, Phys P, const double* __restrict__ mac,
+__global__ __launch_bounds__(ZM_NT) void reduce_fp64(Grid G, int64_t N, Phys P, const double* __restrict__ mac,
                                                      double* __restrict__ partial, int tiles_x, int tiles_y, int zc,
                                                      int64_t items) {
     __shared__ double su[3][4][ZM_HP];  // [ring slot][phi, u1, u2, u3][plane node]
     __shared__ double sh[NPART][ZM_NT / 64];
-    const int64_t N = (int64_t)G.nx * G.ny * G.nz, nxy = (int64_t)G.nx * G.ny;
+    const int64_t nxy = (int64_t)G.nx * G.ny;
     const bool small = G.nx <= ZM_TX || G.ny <= ZM_TY || G.nz <= 2;
     const int tx = threadIdx.x % ZM_TX, ty = threadIdx.x / ZM_TX;
     double s[NPART] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0}, comp[NPART] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
@@ -468,37 +465,37 @@ __global__ void range_set(uint64_t* range, int slot, double vmax, double vmin) {
 // ------------------------------------------------------------------ launchers
 static inline int64_t nblk(int64_t n, int bs) { return (n + bs - 1) / bs; }
 
-hipError_t launch_init_equilibrium_fp64(int nx, int ny, int nz, const Phys& ph, const double* mac, double* f,
+hipError_t launch_init_equilibrium_fp64(int nx, int ny, int nz, int64_t ns, const Phys& ph, const double* mac, double* f,
                                         double* g, hipStream_t st) {
     Grid G{nx, ny, nz};
     const int64_t N = (int64_t)nx * ny * nz;
-    hipLaunchKernelGGL(init_equilibrium_fp64, dim3(nblk(N, 256)), dim3(256), 0, st, G, ph, mac, f, g);
+    hipLaunchKernelGGL(init_equilibrium_fp64, dim3(nblk(N, 256)), dim3(256), 0, st, G, ns, ph, mac, f, g);
     return hipGetLastError();
 }
 
-hipError_t launch_moments_fp64(int nx, int ny, int nz, const double* f, const double* g, double* mac, int which,
+hipError_t launch_moments_fp64(int nx, int ny, int nz, int64_t ns, const double* f, const double* g, double* mac, int which,
                                hipStream_t st) {
     const int64_t N = (int64_t)nx * ny * nz;
-    hipLaunchKernelGGL(moments_fp64, dim3(nblk(N, 256)), dim3(256), 0, st, N, f, g, mac, which);
+    hipLaunchKernelGGL(moments_fp64, dim3(nblk(N, 256)), dim3(256), 0, st, N, ns, f, g, mac, which);
     return hipGetLastError();
 }
 
-hipError_t launch_les_tau_fp64(int nx, int ny, int nz, const Phys& ph, const double* mac, const double* mac_old,
+hipError_t launch_les_tau_fp64(int nx, int ny, int nz, int64_t ns, const Phys& ph, const double* mac, const double* mac_old,
                                const LesBlocks& blk, const uint64_t* range, int slot, double* tau, hipStream_t st) {
     Grid G{nx, ny, nz};
     const int tx = (nx + LES_TX - 1) / LES_TX, ty = (ny + LES_TY - 1) / LES_TY, tz = (nz + LES_TZ - 1) / LES_TZ;
     const dim3 grid((unsigned)(tx * ty * tz)), block(LES_TX * LES_TY * LES_TZ);
     if (blk.bx > 0 && mac_old != mac) {
-        hipLaunchKernelGGL(les_tau_fp64<true>, grid, block, 0, st, G, ph, mac, mac_old, blk, range, slot, tau, tx, ty);
+        hipLaunchKernelGGL(les_tau_fp64<true>, grid, block, 0, st, G, ns, ph, mac, mac_old, blk, range, slot, tau, tx, ty);
     } else {
         const int mx = (nx + ZM_TX - 1) / ZM_TX, my = (ny + ZM_TY - 1) / ZM_TY, mz = (nz + ZM_ZC - 1) / ZM_ZC;
-        hipLaunchKernelGGL(les_tau_fp64_zm, dim3((unsigned)(mx * my * mz)), dim3(ZM_TX * ZM_TY), 0, st, G, ph, mac, range,
+        hipLaunchKernelGGL(les_tau_fp64_zm, dim3((unsigned)(mx * my * mz)), dim3(ZM_TX * ZM_TY), 0, st, G, ns, ph, mac, range,
                            slot, tau, mx, my);
     }
     return hipGetLastError();
 }
 
-hipError_t launch_reduce_fp64(int nx, int ny, int nz, const Phys& ph, const double* mac, const uint64_t* range_slot,
+hipError_t launch_reduce_fp64(int nx, int ny, int nz, int64_t ns, const Phys& ph, const double* mac, const uint64_t* range_slot,
                               double* work, hipStream_t st) {
     Grid G{nx, ny, nz};
     const int mx = (nx + ZM_TX - 1) / ZM_TX, my = (ny + ZM_TY - 1) / ZM_TY;
@@ -508,7 +505,7 @@ hipError_t launch_reduce_fp64(int nx, int ny, int nz, const Phys& ph, const doub
     const int zc = (int)std::min<int64_t>(std::min(32, nz), std::max<int64_t>(1, planes / 1024));
     const int64_t items = (int64_t)mx * my * ((nz + zc - 1) / zc);
     const int nblocks = (int)std::min<int64_t>(items, REDUCE_MAX_BLOCKS);
-    hipLaunchKernelGGL(reduce_fp64, dim3(nblocks), dim3(ZM_NT), 0, st, G, ph, mac, work, mx, my, zc, items);
+    hipLaunchKernelGGL(reduce_fp64, dim3(nblocks), dim3(ZM_NT), 0, st, G, ns, ph, mac, work, mx, my, zc, items);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(reduce_final, dim3(1), dim3(64 * NPART), 0, st, (const double*)work, nblocks, range_slot,

@@ -92,7 +92,7 @@ __device__ void stencils(const BGrid& G, const double* phi, const double* u1, co
     }
 }
 
-__global__ __launch_bounds__(256) void derived_fp64(BGrid G, Phys P, const double* __restrict__ mac, int kind,
+__global__ __launch_bounds__(256) void derived_fp64(BGrid G, int64_t ns, Phys P, const double* __restrict__ mac, int kind,
                                                     double* __restrict__ out, int64_t pitch) {
     const int64_t n = (int64_t)G.nx * G.ny * G.nz;
     const int64_t s = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
@@ -109,7 +109,7 @@ __global__ __launch_bounds__(256) void derived_fp64(BGrid G, Phys P, const doubl
     if (kind == DRP_DERIVED_CHEMICAL_POTENTIAL) {
         *o = P.T * log(ph / (1.0 - P.b * ph)) + P.T / (1.0 - P.b * ph) - 2.0 * P.a * ph - P.kg * lap;
     } else {
-        *o = mac[2 * n + s] * gp[0] + mac[3 * n + s] * gp[1] + mac[4 * n + s] * gp[2];
+        *o = mac[2 * ns + s] * gp[0] + mac[3 * ns + s] * gp[1] + mac[4 * ns + s] * gp[2];
     }
 }
 
@@ -140,6 +140,7 @@ struct BudgetArgs {
     const double *sinx, *cosx, *sinz, *cosz;   // Taylor-Green tables of the step, or null
     double tg_amp;
     double* work;     // [BWORK][ws]
+    int64_t ns;       // stride of the fields
     int64_t ws;       // stride of the work arrays (n)
     double* partial;  // [blocks][BPART]
 };
@@ -268,7 +269,7 @@ __device__ __forceinline__ void stencils_ring(const double* const (&sl)[3], doub
 __global__ __launch_bounds__(BT) __attribute__((amdgpu_waves_per_eu(4))) void budget_pass1(BudgetArgs a) {
     const BGrid& G = a.G;
     const Phys& P = a.P;
-    const int64_t n = (int64_t)G.nx * G.ny * G.nz;
+    const int64_t n = a.ns;
     const Brick b = brick(G);
     // ring of the old phi, u1, u2, u3
     constexpr int NA1 = 4;
@@ -343,7 +344,7 @@ enum { R_K = 0, R_V = 1, R_GP = 4, R_P = 7 };
 __global__ __launch_bounds__(BT) void budget_pass2(BudgetArgs a) {
     const BGrid& G = a.G;
     const Phys& P = a.P;
-    const int64_t n = (int64_t)G.nx * G.ny * G.nz;
+    const int64_t n = a.ns;
     const Brick b = brick(G);
     __shared__ double ring[3][NA2 * RN];
     const int lx = (int)threadIdx.x % BTX, ly = (int)threadIdx.x / BTX;
@@ -440,10 +441,10 @@ __global__ __launch_bounds__(BT) void budget_pass2(BudgetArgs a) {
 
 }  // namespace
 
-hipError_t launch_derived_fp64(int nx, int ny, int nz, const Phys& ph, const double* mac, int kind, double* out,
+hipError_t launch_derived_fp64(int nx, int ny, int nz, int64_t ns, const Phys& ph, const double* mac, int kind, double* out,
                                int64_t pitch, hipStream_t st) {
     const int64_t n = (int64_t)nx * ny * nz;
-    hipLaunchKernelGGL(derived_fp64, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, BGrid{nx, ny, nz}, ph, mac,
+    hipLaunchKernelGGL(derived_fp64, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, BGrid{nx, ny, nz}, ns, ph, mac,
                        kind, out, pitch);
     return hipGetLastError();
 }
@@ -467,7 +468,7 @@ extern "C" int drp_get_derived(drp_lattice* L, int kind, double* host, size_t n_
     }
     double* out = nullptr;
     HIP_TRYB(hipMalloc((void**)&out, (size_t)L->n * sizeof(double)));
-    hipError_t e = launch_derived_fp64(L->cfg.nx, L->cfg.ny, L->cfg.nz, L->phys, mac, kind, out, L->cfg.nx, L->stream);
+    hipError_t e = launch_derived_fp64(L->cfg.nx, L->cfg.ny, L->cfg.nz, L->ns, L->phys, mac, kind, out, L->cfg.nx, L->stream);
     if (e == hipSuccess) e = hipMemcpyAsync(host, out, (size_t)L->n * sizeof(double), hipMemcpyDeviceToHost, L->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(L->stream);
     const hipError_t f = hipFree(out);
@@ -509,6 +510,7 @@ extern "C" int drp_step_energy_budget(drp_lattice* L, double* terms) {
         a.tg_amp = sa.tg_amp;
     }
     a.work = L->budget;
+    a.ns = L->ns;
     a.ws = n;
     a.partial = L->budget + (size_t)BWORK * a.ws;
     hipLaunchKernelGGL(budget_pass1, dim3((unsigned)nb), dim3(BT), 0, L->stream, a);

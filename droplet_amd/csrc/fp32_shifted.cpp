@@ -39,16 +39,16 @@ struct DevBuf {
 };
 
 int fp32_init_from_host_fields(drp_lattice* L, const double* const* host) {
-    const int64_t n = L->n;
+    const int64_t n = L->n, ns = L->ns;
     DevBuf mac64, pop64;
-    HIP_TRY32(hipMalloc(&mac64.p, 5 * n * sizeof(double)));
-    HIP_TRY32(hipMalloc(&pop64.p, 30 * n * sizeof(double)));
+    HIP_TRY32(hipMalloc(&mac64.p, 5 * ns * sizeof(double)));
+    HIP_TRY32(hipMalloc(&pop64.p, 30 * ns * sizeof(double)));
     double* m = (double*)mac64.p;
     double* f = (double*)pop64.p;
     for (int k = 0; k < 5; k++)
-        HIP_TRY32(hipMemcpyAsync(m + k * n, host[k], n * sizeof(double), hipMemcpyHostToDevice, L->stream));
-    HIP_TRY32(launch_init_equilibrium_fp64(L->cfg.nx, L->cfg.ny, L->cfg.nz, L->phys, m, f, f + 15 * n, L->stream));
-    HIP_TRY32(launch_to_shifted(n, shift_ref(L->cfg), f, m, (float*)L->pop[L->cur], (float*)L->mac[L->cur],
+        HIP_TRY32(hipMemcpyAsync(m + k * ns, host[k], n * sizeof(double), hipMemcpyHostToDevice, L->stream));
+    HIP_TRY32(launch_init_equilibrium_fp64(L->cfg.nx, L->cfg.ny, L->cfg.nz, ns, L->phys, m, f, f + 15 * ns, L->stream));
+    HIP_TRY32(launch_to_shifted(n, ns, shift_ref(L->cfg), f, m, (float*)L->pop[L->cur], (float*)L->mac[L->cur],
                                 L->stream));
     int rc = reset_range(L);
     if (rc) return rc;
@@ -61,12 +61,13 @@ int fp32_init_from_host_fields(drp_lattice* L, const double* const* host) {
 StepArgs32 make_step_args32(drp_lattice* L, int64_t nstep) {
     const drp_config& c = L->cfg;
     const Phys& P = L->phys;
-    const int64_t n = L->n;
+    const int64_t n = L->ns;  // from one array to the next
     StepArgs32 a{};
     a.nx = c.nx;
     a.ny = c.ny;
     a.nz = c.nz;
-    a.n = n;
+    a.n = L->n;
+    a.ns = n;
     float* fi = (float*)L->pop[L->cur];
     float* fo = (float*)L->pop[1 - L->cur];
     a.f_in = fi;
@@ -129,8 +130,8 @@ int fp32_step(drp_lattice* L, int nsteps) {
 }
 
 int fp32_macro_fp64_view(drp_lattice* L, const double** mac) {
-    if (!L->mac64) HIP_TRY32(hipMalloc((void**)&L->mac64, 5 * L->n * sizeof(double)));
-    HIP_TRY32(launch_macro_from_shifted(L->n, L->cfg.phi1, (const float*)L->mac[L->cur], L->mac64, L->stream));
+    if (!L->mac64) HIP_TRY32(hipMalloc((void**)&L->mac64, 5 * L->ns * sizeof(double)));
+    HIP_TRY32(launch_macro_from_shifted(L->n, L->ns, L->cfg.phi1, (const float*)L->mac[L->cur], L->mac64, L->stream));
     *mac = L->mac64;
     return DRP_OK;
 }
@@ -139,7 +140,7 @@ int fp32_get_macro(drp_lattice* L, int field, double* host) {
     const double* m = nullptr;
     int rc = fp32_macro_fp64_view(L, &m);
     if (rc) return rc;
-    HIP_TRY32(hipMemcpyAsync(host, m + field * L->n, L->n * sizeof(double), hipMemcpyDeviceToHost, L->stream));
+    HIP_TRY32(hipMemcpyAsync(host, m + field * L->ns, L->n * sizeof(double), hipMemcpyDeviceToHost, L->stream));
     HIP_TRY32(hipStreamSynchronize(L->stream));
     return DRP_OK;
 }
@@ -147,7 +148,7 @@ int fp32_get_macro(drp_lattice* L, int field, double* host) {
 int fp32_get_populations(drp_lattice* L, int set, double* host) {
     DevBuf tmp;
     HIP_TRY32(hipMalloc(&tmp.p, 15 * L->n * sizeof(double)));
-    HIP_TRY32(launch_pops_from_shifted(L->n, shift_ref(L->cfg), (const float*)L->pop[L->cur], (double*)tmp.p, set,
+    HIP_TRY32(launch_pops_from_shifted(L->n, L->ns, shift_ref(L->cfg), (const float*)L->pop[L->cur], (double*)tmp.p, set,
                                        L->stream));
     HIP_TRY32(hipMemcpyAsync(host, tmp.p, 15 * L->n * sizeof(double), hipMemcpyDeviceToHost, L->stream));
     HIP_TRY32(hipStreamSynchronize(L->stream));
@@ -159,8 +160,8 @@ int fp32_set_populations(drp_lattice* L, int set, const double* host, int which)
     HIP_TRY32(hipMalloc(&tmp.p, 15 * L->n * sizeof(double)));
     HIP_TRY32(hipMemcpyAsync(tmp.p, host, 15 * L->n * sizeof(double), hipMemcpyHostToDevice, L->stream));
     float* pop = (float*)L->pop[L->cur];
-    HIP_TRY32(launch_pops_to_shifted(L->n, shift_ref(L->cfg), (const double*)tmp.p, pop, set, L->stream));
-    HIP_TRY32(launch_moments_fp32(L->n, pop, pop + 15 * L->n, (float*)L->mac[L->cur], which, L->stream));
+    HIP_TRY32(launch_pops_to_shifted(L->n, L->ns, shift_ref(L->cfg), (const double*)tmp.p, pop, set, L->stream));
+    HIP_TRY32(launch_moments_fp32(L->n, L->ns, pop, pop + 15 * L->ns, (float*)L->mac[L->cur], which, L->stream));
     HIP_TRY32(hipStreamSynchronize(L->stream));
     return DRP_OK;
 }

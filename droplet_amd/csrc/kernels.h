@@ -54,11 +54,12 @@ struct StepArgs {
     int nx, ny, nz;
     int tiles_x, tiles_y, tiles_z;
     int64_t n;
-    const double* f_in;   // [15][n] phi populations (reference f)
-    const double* g_in;   // [15][n] momentum populations (reference g)
+    int64_t ns;           // elements from one population, field or force array to the next
+    const double* f_in;   // [15][ns] phi populations (reference f)
+    const double* g_in;   // [15][ns] momentum populations (reference g)
     double* f_out;
     double* g_out;
-    const double* mac_in; // phi, p, u1, u2, u3 (5 x n)
+    const double* mac_in; // phi, p, u1, u2, u3 (5 x ns)
     double* mac_out;
     const double* tau_field;              // LES: tau_g per node, else nullptr
     const double *fx, *fy, *fz;           // FORCE_FIELD
@@ -86,12 +87,15 @@ struct StepArgs {
 
 hipError_t launch_step_fp64(const StepArgs& a, int shape, hipStream_t st, const BatchLaunch* batch = nullptr);
 
+// ns in the launchers below: elements from one population or field array to the next
+// (lattice_impl.h); arrays for the host are n apart
+
 // FP32 shifted storage (step_fp32.hip): populations and fields as FP32
 // deviations from the continuous phase at rest
 struct StepArgs32 {
     int nx, ny, nz;
     int tiles_x, tiles_y, tiles_z;
-    int64_t n;
+    int64_t n, ns;
     const float* f_in;
     const float* g_in;
     float* f_out;
@@ -125,31 +129,31 @@ struct ShiftRef {
     double fr[15];
     double phi1;
 };
-hipError_t launch_to_shifted(int64_t n, const ShiftRef& r, const double* pop64, const double* mac64, float* pop32,
+hipError_t launch_to_shifted(int64_t n, int64_t ns, const ShiftRef& r, const double* pop64, const double* mac64, float* pop32,
                              float* mac32, hipStream_t st);
-hipError_t launch_pops_from_shifted(int64_t n, const ShiftRef& r, const float* pop32, double* pop64, int set,
+hipError_t launch_pops_from_shifted(int64_t n, int64_t ns, const ShiftRef& r, const float* pop32, double* pop64, int set,
                                     hipStream_t st);
-hipError_t launch_pops_to_shifted(int64_t n, const ShiftRef& r, const double* pop64, float* pop32, int set,
+hipError_t launch_pops_to_shifted(int64_t n, int64_t ns, const ShiftRef& r, const double* pop64, float* pop32, int set,
                                   hipStream_t st);
-hipError_t launch_macro_from_shifted(int64_t n, double phi1, const float* mac32, double* mac64, hipStream_t st);
-hipError_t launch_moments_fp32(int64_t n, const float* f, const float* g, float* mac, int which, hipStream_t st);
-hipError_t launch_les_tau_fp32(int nx, int ny, int nz, const Phys& ph, const float* mac, const float* mac_old,
+hipError_t launch_macro_from_shifted(int64_t n, int64_t ns, double phi1, const float* mac32, double* mac64, hipStream_t st);
+hipError_t launch_moments_fp32(int64_t n, int64_t ns, const float* f, const float* g, float* mac, int which, hipStream_t st);
+hipError_t launch_les_tau_fp32(int nx, int ny, int nz, int64_t ns, const Phys& ph, const float* mac, const float* mac_old,
                                const LesBlocks& blk, const uint64_t* range, int slot, float* tau, hipStream_t st);
 
 // populations := equilibria of the macroscopic fields (ini, program/lbm_drop_xy.f90:244-251)
-hipError_t launch_init_equilibrium_fp64(int nx, int ny, int nz, const Phys& ph, const double* mac, double* f,
+hipError_t launch_init_equilibrium_fp64(int nx, int ny, int nz, int64_t ns, const Phys& ph, const double* mac, double* f,
                                         double* g, hipStream_t st);
 // recompute moments from populations: which & 1 -> phi from f, which & 2 -> p, u from g
-hipError_t launch_moments_fp64(int nx, int ny, int nz, const double* f, const double* g, double* mac, int which,
+hipError_t launch_moments_fp64(int nx, int ny, int nz, int64_t ns, const double* f, const double* g, double* mac, int which,
                                hipStream_t st);
 // Smagorinsky tau field for the next step (program/LES_drop.f90:598-693) from the
 // state a step left (mac), the one it started from (mac_old, read across rank
 // blocks) and that step's phi range slot
-hipError_t launch_les_tau_fp64(int nx, int ny, int nz, const Phys& ph, const double* mac, const double* mac_old,
+hipError_t launch_les_tau_fp64(int nx, int ny, int nz, int64_t ns, const Phys& ph, const double* mac, const double* mac_old,
                                const LesBlocks& blk, const uint64_t* range, int slot, double* tau, hipStream_t st);
 // derived fields of the analysis programs (budget.hip): kind = DRP_DERIVED_*; rows of
 // the result `pitch` doubles apart
-hipError_t launch_derived_fp64(int nx, int ny, int nz, const Phys& ph, const double* mac, int kind, double* out,
+hipError_t launch_derived_fp64(int nx, int ny, int nz, int64_t ns, const Phys& ph, const double* mac, int kind, double* out,
                                int64_t pitch, hipStream_t st);
 
 // diagnostics sums: NPART doubles per workgroup (at most REDUCE_MAX_BLOCKS), then at
@@ -158,7 +162,7 @@ constexpr int NPART = 10;
 constexpr int REDUCE_MAX_BLOCKS = 2048;
 constexpr int REDUCE_OUT = REDUCE_MAX_BLOCKS * NPART;
 constexpr int REDUCE_WORK_DOUBLES = REDUCE_OUT + 16;
-hipError_t launch_reduce_fp64(int nx, int ny, int nz, const Phys& ph, const double* mac, const uint64_t* range_slot,
+hipError_t launch_reduce_fp64(int nx, int ny, int nz, int64_t ns, const Phys& ph, const double* mac, const uint64_t* range_slot,
                               double* work, hipStream_t st);
 // fill a range slot with (max, min) = (vmax, vmin)
 hipError_t launch_range_set(uint64_t* range, int slot, double vmax, double vmin, hipStream_t st);
@@ -185,16 +189,16 @@ hipError_t launch_spectral_band(const SpectralWork& w, int nx, int ny, int nz, i
 // adjoint.hip: one reverse step of the FP64 step (equal viscosities, no LES)
 struct AdjArgs {
     int nx, ny, nz;
-    int64_t n;
-    const double* f;        // forward phi populations at step n (15n)
-    const double* mac;      // forward macroscopic fields at step n (5n)
-    const double* Fin;      // adjoint of f^{n+1} without its stencil part (15n)
+    int64_t n, ns;
+    const double* f;        // forward phi populations at step n (15 ns)
+    const double* mac;      // forward macroscopic fields at step n (5 ns)
+    const double* Fin;      // adjoint of f^{n+1} without its stencil part (15 ns)
     const double* phin_in;  // stencil part of the adjoint of phi^{n+1} (n), or nullptr
-    const double* Gin;      // adjoint of g^{n+1} (15n)
+    const double* Gin;      // adjoint of g^{n+1} (15 ns)
     double* Fout;           // adjoint of f^n without its stencil part
     double* Gout;           // adjoint of g^n
     double* lapA;           // adjoint of lap phi at step n (n)
-    double* gradA;          // adjoint of grad phi at step n (3n)
+    double* gradA;          // adjoint of grad phi at step n (3 ns)
     double* acc;            // [workgroups][3]: d/dtau_f, d/dkappa_g, d/dU_wall, accumulated
     double tau_f, tau_g, kf, kf6, kg, T, a, b;
     double rtau_f, rtau_g, rtau_f2;  // 1 / tau_f, 1 / tau_g, 1 / (tau_f tau_f)
@@ -205,9 +209,9 @@ struct AdjArgs {
 };
 int adj_block_count(int64_t n);
 hipError_t launch_adj_collide_fp64(const AdjArgs& a, hipStream_t st);
-hipError_t launch_adj_stencil_fp64(int nx, int ny, int nz, const double* lapA, const double* gradA, double* out,
+hipError_t launch_adj_stencil_fp64(int nx, int ny, int nz, int64_t ns, const double* lapA, const double* gradA, double* out,
                                    hipStream_t st);
-hipError_t launch_adj_seed_area_fp64(int nx, int ny, int nz, const double* phi, double w, double* lapA,
+hipError_t launch_adj_seed_area_fp64(int nx, int ny, int nz, int64_t ns, const double* phi, double w, double* lapA,
                                      double* gradA, hipStream_t st);
 hipError_t launch_adj_add_plane(int nx, int ny, int n1, int n2, int wall_y, int third, const double* vals,
                                 double* out, hipStream_t st);

@@ -86,6 +86,34 @@ Phys make_phys(const drp_config& c) {
     return p;
 }
 
+// Elements from one population (or field) array to the next.  A step reads and
+// writes 70 arrays of n at the same offset in each; where n times the element size
+// is a large power of two they meet in the same memory channels.  Arrays of 1 MiB
+// and more therefore start on 256-byte boundaries (whole lines also on odd grids)
+// and 8 KiB + 256 B further apart than their length.  MLUPS of the shear droplet,
+// arrays back to back -> apart: FP64 128^3 5040..6080 -> 8070, 192^3 7860 -> 8240,
+// 256^3 8130 -> 8350, 131 x 70 x 97 3790 -> 4120; FP32 128^3 14030 -> 15050,
+// 256^3 14730 -> 15850; 240^3 unchanged.  Of 0, 256, 512 .. 4096, 4352, 8448, 16640,
+// 64 KiB, 1 MiB and 2 MiB + 4352 B this is the best or within 2 % of it at all of
+// these.  Shorter arrays stay back to back: they live in the caches, and one copy
+// moves a whole population set to the host.
+static int64_t stream_stride(int64_t n, size_t esz) {
+    const int64_t bytes = n * (int64_t)esz;
+    if (bytes < ((int64_t)1 << 20)) return n;
+    return ((bytes + 255) / 256 * 256 + 8192 + 256) / (int64_t)esz;
+}
+
+// `count` arrays of n doubles, ds and ss doubles apart, in one copy where they are contiguous
+static hipError_t copy_streams(double* dst, int64_t ds, const double* src, int64_t ss, int count, int64_t n,
+                               hipMemcpyKind kind, hipStream_t st) {
+    if (ds == n && ss == n) return hipMemcpyAsync(dst, src, count * n * sizeof(double), kind, st);
+    for (int k = 0; k < count; k++) {
+        const hipError_t e = hipMemcpyAsync(dst + k * ds, src + k * ss, n * sizeof(double), kind, st);
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
+}
+
 static int validate(const drp_config* c) {
     if (!c) return drp_fail(DRP_ERR_ARG, "null config");
     if (c->nx < 3 || c->ny < 3 || c->nz < 3) return drp_fail(DRP_ERR_ARG, "grid must be at least 3^3");
@@ -184,6 +212,7 @@ int lattice_create(const drp_config* cfg, hipStream_t stream, drp_lattice** out)
     L->cfg = *cfg;
     L->phys = make_phys(*cfg);
     L->n = (int64_t)cfg->nx * cfg->ny * cfg->nz;
+    L->ns = stream_stride(L->n, cfg->precision == DRP_FP64 ? sizeof(double) : sizeof(float));
     L->shape = pick_shape(*cfg);
     L->stream = stream;
     (void)hipGetDevice(&L->dev);
@@ -204,7 +233,7 @@ extern "C" void drp_destroy(drp_lattice* L) {
 }
 
 int lattice_alloc(drp_lattice* L) {
-    const int64_t n = L->n;
+    const int64_t n = L->n, ns = L->ns;
     auto dalloc = [&](void** p, size_t bytes) -> int {
         if (hipMalloc(p, bytes) != hipSuccess) {
             *p = nullptr;
@@ -219,16 +248,16 @@ int lattice_alloc(drp_lattice* L) {
     int rc = 0;
     const size_t esz = (L->cfg.precision == DRP_FP64) ? sizeof(double) : sizeof(float);
     for (int k = 0; k < 2 && !rc; k++) {
-        rc |= dalloc(&L->pop[k], 2 * 15 * (size_t)n * esz);
-        rc |= dalloc((void**)&L->mac[k], 5 * (size_t)n * esz);
+        rc |= dalloc(&L->pop[k], 2 * 15 * (size_t)ns * esz);
+        rc |= dalloc((void**)&L->mac[k], 5 * (size_t)ns * esz);
     }
     if (!rc) rc = dalloc((void**)&L->range, 6 * sizeof(uint64_t));
     const bool noneq = L->phys.les && L->cfg.les_model == DRP_LES_NONEQ;
     if (!rc && L->phys.les && !noneq) rc = dalloc((void**)&L->tau, (size_t)n * sizeof(double));
     for (int k = 0; k < 2 && !rc && noneq; k++) rc = dalloc((void**)&L->qh[k], (size_t)n * sizeof(double));
     if (!rc && (L->cfg.force_kind == DRP_FORCE_FIELD || L->cfg.force_kind == DRP_FORCE_SPECTRAL)) {
-        rc = dalloc((void**)&L->force, 3 * (size_t)n * sizeof(double));
-        if (!rc) HIP_TRY(hipMemsetAsync(L->force, 0, 3 * (size_t)n * sizeof(double), L->stream));
+        rc = dalloc((void**)&L->force, 3 * (size_t)ns * sizeof(double));
+        if (!rc) HIP_TRY(hipMemsetAsync(L->force, 0, 3 * (size_t)ns * sizeof(double), L->stream));
     }
     // truncated-DFT work space for the modes |k_a| < kc: the spectral forcing
     // (kc = force_k) and the scale-separated advection (kc = advect_k_high)
@@ -254,7 +283,7 @@ int lattice_alloc(drp_lattice* L) {
     if (!rc && L->cfg.force_kind == DRP_FORCE_SPECTRAL) rc = spectral_alloc(&L->spec, L->specw, (int)L->cfg.force_k);
     if (!rc && L->cfg.advect_k_high != 0) {
         rc = spectral_alloc(&L->spec_adv, L->specw_adv, L->cfg.advect_k_high);
-        if (!rc) rc = dalloc((void**)&L->uadv, 3 * (size_t)n * sizeof(double));
+        if (!rc) rc = dalloc((void**)&L->uadv, 3 * (size_t)ns * sizeof(double));
     }
     if (!rc && L->cfg.force_kind == DRP_FORCE_TAYLOR_GREEN) {
         const int nx = L->cfg.nx, nz = L->cfg.nz;
@@ -334,10 +363,10 @@ int les_update_tau(drp_lattice* L, bool fresh) {
     const int slot = (int)(L->step % 3);
     const int old = fresh ? L->cur : 1 - L->cur;
     if (c.precision == DRP_FP64)
-        HIP_TRY(launch_les_tau_fp64(c.nx, c.ny, c.nz, L->phys, (const double*)L->mac[L->cur], (const double*)L->mac[old],
+        HIP_TRY(launch_les_tau_fp64(c.nx, c.ny, c.nz, L->ns, L->phys, (const double*)L->mac[L->cur], (const double*)L->mac[old],
                                     B, L->range, slot, L->tau, L->stream));
     else
-        HIP_TRY(launch_les_tau_fp32(c.nx, c.ny, c.nz, L->phys, (const float*)L->mac[L->cur], (const float*)L->mac[old],
+        HIP_TRY(launch_les_tau_fp32(c.nx, c.ny, c.nz, L->ns, L->phys, (const float*)L->mac[L->cur], (const float*)L->mac[old],
                                     B, L->range, slot, (float*)L->tau, L->stream));
     return DRP_OK;
 }
@@ -349,11 +378,11 @@ static int init_from_host_fields(drp_lattice* L, const double* const* host) {
         return rc ? rc : les_update_tau(L, true);
     }
     for (int k = 0; k < 5; k++)
-        HIP_TRY(hipMemcpyAsync((double*)L->mac[L->cur] + k * n, host[k], n * sizeof(double), hipMemcpyHostToDevice,
+        HIP_TRY(hipMemcpyAsync((double*)L->mac[L->cur] + k * L->ns, host[k], n * sizeof(double), hipMemcpyHostToDevice,
                                L->stream));
     double* f = (double*)L->pop[L->cur];
-    HIP_TRY(launch_init_equilibrium_fp64(L->cfg.nx, L->cfg.ny, L->cfg.nz, L->phys, (double*)L->mac[L->cur], f,
-                                         f + 15 * n, L->stream));
+    HIP_TRY(launch_init_equilibrium_fp64(L->cfg.nx, L->cfg.ny, L->cfg.nz, L->ns, L->phys, (double*)L->mac[L->cur],
+                                         f, f + 15 * L->ns, L->stream));
     int rc = reset_range(L);
     if (rc) return rc;
     HIP_TRY(hipStreamSynchronize(L->stream));
@@ -426,12 +455,13 @@ extern "C" int drp_init_fields(drp_lattice* L, const double* phi, const double* 
 StepArgs make_step_args(drp_lattice* L, int64_t nstep) {
     const drp_config& c = L->cfg;
     const Phys& P = L->phys;
-    const int64_t n = L->n;
+    const int64_t n = L->ns;  // from one array to the next
     StepArgs a{};
     a.nx = c.nx;
     a.ny = c.ny;
     a.nz = c.nz;
-    a.n = n;
+    a.n = L->n;
+    a.ns = n;
     double* fi = (double*)L->pop[L->cur];
     double* fo = (double*)L->pop[1 - L->cur];
     a.f_in = fi;
@@ -525,7 +555,7 @@ extern "C" int drp_step(drp_lattice* L, int nsteps) {
 int spectral_update(drp_lattice* L, int64_t nstep) {
     const drp_config& c = L->cfg;
     if (c.force_kind != DRP_FORCE_SPECTRAL || nstep < c.force_start) return DRP_OK;
-    const int64_t n = L->n;
+    const int64_t n = L->ns;
     double *fx = L->force, *fy = L->force + n, *fz = L->force + 2 * n;
     if (c.precision == DRP_FP64) {
         const double* m = (const double*)L->mac[L->cur];
@@ -546,7 +576,7 @@ int spectral_update(drp_lattice* L, int64_t nstep) {
 int advect_update(drp_lattice* L, int64_t nstep) {
     const drp_config& c = L->cfg;
     if (c.advect_k_high == 0 || nstep < c.advect_start) return DRP_OK;
-    const int64_t n = L->n;
+    const int64_t n = L->ns;
     const double* m = (const double*)L->mac[L->cur];
     HIP_TRY(launch_spectral_band(L->specw_adv, c.nx, c.ny, c.nz, c.advect_k_low, c.advect_k_high, m + 2 * n,
                                  m + 3 * n, m + 4 * n, L->uadv, L->uadv + n, L->uadv + 2 * n, L->stream));
@@ -569,7 +599,7 @@ extern "C" int drp_get_macro(drp_lattice* L, int field, double* host, size_t n) 
     if (n != (size_t)L->n) return drp_fail(DRP_ERR_ARG, "size %zu != %lld nodes", n, (long long)L->n);
     if (!L->initialized) return drp_fail(DRP_ERR_STATE, "lattice not initialised");
     if (L->cfg.precision != DRP_FP64) return fp32_get_macro(L, field, host);
-    HIP_TRY(hipMemcpyAsync(host, (const double*)L->mac[L->cur] + field * L->n, n * sizeof(double),
+    HIP_TRY(hipMemcpyAsync(host, (const double*)L->mac[L->cur] + field * L->ns, n * sizeof(double),
                            hipMemcpyDeviceToHost, L->stream));
     HIP_TRY(hipStreamSynchronize(L->stream));
     return DRP_OK;
@@ -583,8 +613,8 @@ extern "C" int drp_get_populations(drp_lattice* L, int set, double* host, size_t
     if (n != 15 * (size_t)L->n) return drp_fail(DRP_ERR_ARG, "size %zu != 15 x %lld", n, (long long)L->n);
     if (!L->initialized) return drp_fail(DRP_ERR_STATE, "lattice not initialised");
     if (L->cfg.precision != DRP_FP64) return fp32_get_populations(L, set, host);
-    const double* src = (const double*)L->pop[L->cur] + (set == DRP_POP_MOM ? 15 * L->n : 0);
-    HIP_TRY(hipMemcpyAsync(host, src, n * sizeof(double), hipMemcpyDeviceToHost, L->stream));
+    const double* src = (const double*)L->pop[L->cur] + (set == DRP_POP_MOM ? 15 * L->ns : 0);
+    HIP_TRY(copy_streams(host, L->n, src, L->ns, 15, L->n, hipMemcpyDeviceToHost, L->stream));
     HIP_TRY(hipStreamSynchronize(L->stream));
     return DRP_OK;
 }
@@ -604,10 +634,10 @@ static int set_pops(drp_lattice* L, int set, const double* host, size_t n, int w
         return rc || !replace ? rc : les_update_tau(L, true);
     }
     double* base = (double*)L->pop[L->cur];
-    double* dst = base + (set == DRP_POP_MOM ? 15 * L->n : 0);
+    double* dst = base + (set == DRP_POP_MOM ? 15 * L->ns : 0);
     L->eq_init = false;
-    HIP_TRY(hipMemcpyAsync(dst, host, n * sizeof(double), hipMemcpyHostToDevice, L->stream));
-    HIP_TRY(launch_moments_fp64(L->cfg.nx, L->cfg.ny, L->cfg.nz, base, base + 15 * L->n, (double*)L->mac[L->cur],
+    HIP_TRY(copy_streams(dst, L->ns, host, L->n, 15, L->n, hipMemcpyHostToDevice, L->stream));
+    HIP_TRY(launch_moments_fp64(L->cfg.nx, L->cfg.ny, L->cfg.nz, L->ns, base, base + 15 * L->ns, (double*)L->mac[L->cur],
                                 which, L->stream));
     HIP_TRY(hipStreamSynchronize(L->stream));
     return replace ? les_update_tau(L, true) : DRP_OK;
@@ -627,7 +657,7 @@ extern "C" int drp_set_force(drp_lattice* L, const double* fx, const double* fy,
     if (n != (size_t)L->n) return drp_fail(DRP_ERR_ARG, "size %zu != %lld nodes", n, (long long)L->n);
     const double* src[3] = {fx, fy, fz};
     for (int k = 0; k < 3; k++)
-        HIP_TRY(hipMemcpyAsync(L->force + k * L->n, src[k], n * sizeof(double), hipMemcpyHostToDevice, L->stream));
+        HIP_TRY(hipMemcpyAsync(L->force + k * L->ns, src[k], n * sizeof(double), hipMemcpyHostToDevice, L->stream));
     HIP_TRY(hipStreamSynchronize(L->stream));
     return DRP_OK;
 }
@@ -638,7 +668,7 @@ extern "C" int drp_get_force(drp_lattice* L, double* fx, double* fy, double* fz,
     if (n != (size_t)L->n) return drp_fail(DRP_ERR_ARG, "size %zu != %lld nodes", n, (long long)L->n);
     double* dst[3] = {fx, fy, fz};
     for (int k = 0; k < 3; k++)
-        HIP_TRY(hipMemcpyAsync(dst[k], L->force + k * L->n, n * sizeof(double), hipMemcpyDeviceToHost, L->stream));
+        HIP_TRY(hipMemcpyAsync(dst[k], L->force + k * L->ns, n * sizeof(double), hipMemcpyDeviceToHost, L->stream));
     HIP_TRY(hipStreamSynchronize(L->stream));
     return DRP_OK;
 }
@@ -656,7 +686,7 @@ extern "C" int drp_reduce(drp_lattice* L, drp_stats* st) {
         if (rc) return rc;
     }
     if (!L->partial) HIP_TRY(hipMalloc((void**)&L->partial, REDUCE_WORK_DOUBLES * sizeof(double)));
-    HIP_TRY(launch_reduce_fp64(L->cfg.nx, L->cfg.ny, L->cfg.nz, L->phys, mac, L->range + 2 * (L->step % 3), L->partial,
+    HIP_TRY(launch_reduce_fp64(L->cfg.nx, L->cfg.ny, L->cfg.nz, L->ns, L->phys, mac, L->range + 2 * (L->step % 3), L->partial,
                                L->stream));
     double s[NPART + 2];
     HIP_TRY(hipMemcpyAsync(s, L->partial + REDUCE_OUT, sizeof s, hipMemcpyDeviceToHost, L->stream));

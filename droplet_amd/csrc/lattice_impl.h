@@ -15,13 +15,14 @@ struct drp_lattice {
     hipStream_t stream = nullptr;
     bool owns_stream = false;   // false for members of a batch (shared stream)
     int64_t n = 0;
+    int64_t ns = 0;        // elements from one population, field or force array to the next (stream_stride)
     int64_t step = 0;      // reference loop counter of the last completed step
     bool initialized = false;
     bool eq_init = false;  // populations are the equilibria of fields set by drp_init_* (no step since)
     int shape = 0;         // tile shape of the step kernel
     int cur = 0;           // which ping-pong buffer holds the current state
-    void* pop[2] = {nullptr, nullptr};  // FP64: [f(15n) | g(15n)] doubles; FP32: floats
-    void* mac[2] = {nullptr, nullptr};  // phi, p, u1, u2, u3 (5n)
+    void* pop[2] = {nullptr, nullptr};  // FP64: [f (15 ns) | g (15 ns)] doubles; FP32: floats
+    void* mac[2] = {nullptr, nullptr};  // phi, p, u1, u2, u3 (5 ns)
     uint64_t* range = nullptr;          // 3 rotating (max, min) slots of the phi range
     double* tau = nullptr;              // LES relaxation-time field
     double* qh[2] = {nullptr, nullptr}; // non-equilibrium LES: sqrt(Pi:Pi) per node, with the populations' parity

@@ -558,7 +558,7 @@ int transform_velocity(drp_lattice* L, const FFTPlan& P, double2* c) {
     const int64_t n = L->n;
     const unsigned nb = (unsigned)((n + 255) / 256);
     for (int k = 0; k < 3; k++) {
-        hipLaunchKernelGGL(to_complex, dim3(nb), dim3(256), 0, L->stream, n, mac + (2 + k) * n, c + k * n);
+        hipLaunchKernelGGL(to_complex, dim3(nb), dim3(256), 0, L->stream, n, mac + (2 + k) * L->ns, c + k * n);
         HIP_TRYS(hipGetLastError());
         HIP_TRYS(fft3d(P, c + k * n, -1, L->stream));
     }
@@ -736,7 +736,7 @@ extern "C" int drp_energy_spectrum(drp_lattice* L, double* E, int nshells) {
     rc = velocity_view(L, &mac);
     if (!rc) rc = shell_records(D, nshells, &wgs);
     for (int k = 0; k < 3 && !rc; k++) {
-        rc = half_transform(D, mac + (2 + k) * L->n, L->cfg.nx, 0, L->stream);
+        rc = half_transform(D, mac + (2 + k) * L->ns, L->cfg.nx, 0, L->stream);
         if (!rc) rc = shell_pass<SHELL_ENERGY>(L, D, 0, 1.0 / (double)L->n, nshells, nshells, wgs, k > 0);
     }
     return rc ? rc : shell_sums(L, D, nshells, wgs, E);
@@ -788,7 +788,7 @@ extern "C" int drp_scale_interaction(drp_lattice* L, double* C, int nshells) {
     if (!rc) rc = korteweg_divergence(L, D, mac);
     for (int b = 0; b < 3 && !rc; b++) {
         rc = half_transform(D, (const double*)D->spectrum(1 + b), 2 * D->pitch, 1 + b, L->stream);
-        if (!rc) rc = half_transform(D, mac + (2 + b) * L->n, L->cfg.nx, 0, L->stream);
+        if (!rc) rc = half_transform(D, mac + (2 + b) * L->ns, L->cfg.nx, 0, L->stream);
         if (!rc) rc = shell_pass<SHELL_CROSS>(L, D, 1 + b, 1.0 / (double)L->n, nshells, nshells, wgs, b > 0);
     }
     std::vector<double> h(nshells);
@@ -814,7 +814,7 @@ extern "C" int drp_phi_contribution(drp_lattice* L, double* C, int nshells, doub
     const int kinds[2] = {DRP_DERIVED_ADVECTION, DRP_DERIVED_CHEMICAL_POTENTIAL};
     for (int k = 0; k < 2 && !rc; k++) {
         double* field = (double*)D->spectrum(k);
-        HIP_TRYS(launch_derived_fp64(c.nx, c.ny, c.nz, L->phys, mac, kinds[k], field, 2 * D->pitch, L->stream));
+        HIP_TRYS(launch_derived_fp64(c.nx, c.ny, c.nz, L->ns, L->phys, mac, kinds[k], field, 2 * D->pitch, L->stream));
         rc = half_transform(D, field, 2 * D->pitch, k, L->stream);
     }
     if (!rc) rc = shell_pass<SHELL_CROSS_HALF>(L, D, 1, 1.0, nb, 2 * nb, wgs, false);

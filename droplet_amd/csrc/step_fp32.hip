@@ -74,7 +74,7 @@ __device__ __forceinline__ void step_tile_fp32(const StepArgs32& a, int tile) {
     __shared__ double s_red[2][NT / 64];
 
     const int nx = a.nx, ny = a.ny, nz = a.nz;
-    const int64_t N = a.n;
+    const int64_t N = a.ns;  // from one population or field array to the next
     const int x0 = (tile % a.tiles_x) * TX;
     const int y0 = ((tile / a.tiles_x) % a.tiles_y) * TY;
     const int z0 = (tile / (a.tiles_x * a.tiles_y)) * TZ;

@@ -99,7 +99,7 @@ __device__ __forceinline__ void step_tile_fp64(const StepArgs& a, int tile) {
     __shared__ double s_red[2][NT / 64];
 
     const int nx = a.nx, ny = a.ny, nz = a.nz;
-    const int64_t N = a.n;
+    const int64_t N = a.ns;  // from one population or field array to the next
     // tiles run x fastest, then z, then y: the workgroups resident at one time
     // on an XCD (a contiguous range of tiles) cover consecutive z-layers of one
     // tile row, so the z halos (the deeper ones: TZ <= TY) are read from L2
