@@ -46,7 +46,7 @@ struct drp_tape {
     int64_t bytes = 0;
 };
 
-static size_t state_doubles(const drp_lattice* L) { return 35 * (size_t)L->ns; }
+static size_t state_doubles(const drp_lattice* L) { return 35 * (size_t)L->G.ns; }
 
 static int tape_alloc(drp_tape* T, void** p, size_t bytes) {
     HIP_TRYA(hipMalloc(p, bytes));
@@ -56,7 +56,7 @@ static int tape_alloc(drp_tape* T, void** p, size_t bytes) {
 
 static int save_checkpoint(drp_tape* T) {
     drp_lattice* L = T->L;
-    const size_t n = (size_t)L->ns;
+    const size_t n = (size_t)L->G.ns;
     double* c = nullptr;
     int rc = tape_alloc(T, (void**)&c, state_doubles(L) * sizeof(double));
     if (rc) return rc;
@@ -78,7 +78,7 @@ extern "C" int drp_tape_create(drp_lattice* L, int K, drp_tape** out) {
         return drp_fail(DRP_ERR_ARG, "the adjoint covers the free-energy model without scale-separated advection only");
     if (L->cfg.force_kind == DRP_FORCE_SPECTRAL)
         return drp_fail(DRP_ERR_ARG, "the adjoint does not cover the velocity-dependent spectral forcing");
-    if (L->n >= (int64_t)1 << 32) return drp_fail(DRP_ERR_ARG, "the adjoint supports grids of fewer than 2^32 nodes");
+    if (L->G.slots() >= (int64_t)1 << 32) return drp_fail(DRP_ERR_ARG, "the adjoint supports grids of fewer than 2^32 nodes");
     const int wn = L->cfg.wall_axis == DRP_WALL_Y ? L->cfg.ny : L->cfg.nz;
     if (L->cfg.wall_axis != DRP_WALL_NONE && wn < 3)
         return drp_fail(DRP_ERR_ARG, "the adjoint needs at least 3 layers between the walls");
@@ -132,13 +132,13 @@ extern "C" int drp_tape_loss(drp_tape* T, const double w[2], double* loss, doubl
 
 static int ensure_work(drp_tape* T) {
     drp_lattice* L = T->L;
-    const size_t n = (size_t)L->ns;
+    const size_t n = (size_t)L->G.ns;
     int rc = DRP_OK;
     if (!T->seg && T->K > 1) rc = tape_alloc(T, (void**)&T->seg, (size_t)(T->K - 1) * state_doubles(L) * sizeof(double));
     if (!rc && !T->adj) rc = tape_alloc(T, (void**)&T->adj, 2 * 30 * n * sizeof(double));
     if (!rc && !T->phin) rc = tape_alloc(T, (void**)&T->phin, 2 * n * sizeof(double));
     if (!rc && !T->work) rc = tape_alloc(T, (void**)&T->work, 4 * n * sizeof(double));
-    T->nblk = adj_block_count(L->n);
+    T->nblk = adj_block_count(L->G);
     if (!rc && !T->acc) rc = tape_alloc(T, (void**)&T->acc, (size_t)T->nblk * 3 * sizeof(double));
     if (!rc && !T->plane) rc = tape_alloc(T, (void**)&T->plane, (size_t)L->cfg.nx * std::max(L->cfg.ny, L->cfg.nz) * sizeof(double));
     if (!rc && !T->range) {
@@ -162,7 +162,7 @@ extern "C" int drp_tape_backward(drp_tape* T, const double w[2], double* loss, d
     int rc = ensure_work(T);
     if (rc) return rc;
     const drp_config& c = L->cfg;
-    const int64_t n = L->ns;  // from one array of a state to the next
+    const int64_t n = L->G.ns;  // from one array of a state to the next
     hipStream_t st = L->stream;
 
     // ---- loss and its seed dJ/dphi at the final state
@@ -177,8 +177,8 @@ extern "C" int drp_tape_backward(drp_tape* T, const double w[2], double* loss, d
     double* gradA = T->work + n;
     HIP_TRYA(hipMemsetAsync(Fa[cur], 0, 30 * n * sizeof(double), st));
     HIP_TRYA(hipMemsetAsync(T->acc, 0, (size_t)T->nblk * 3 * sizeof(double), st));
-    HIP_TRYA(launch_adj_seed_area_fp64(c.nx, c.ny, c.nz, n, (const double*)L->mac[L->cur], w[1], lapA, gradA, st));
-    HIP_TRYA(launch_adj_stencil_fp64(c.nx, c.ny, c.nz, n, lapA, gradA, Pa[cur], st));
+    HIP_TRYA(launch_adj_seed_area_fp64(L->G, (const double*)L->mac[L->cur], w[1], lapA, gradA, st));
+    HIP_TRYA(launch_adj_stencil_fp64(L->G, lapA, gradA, Pa[cur], st));
     if (w[0] != 0.0) {
         double D;
         int n1 = 0, n2 = 0, third = 0;
@@ -187,7 +187,7 @@ extern "C" int drp_tape_backward(drp_tape* T, const double w[2], double* loss, d
         if (rc) return rc;
         for (int k = 0; k < n1 * n2; k++) g[k] *= w[0];
         HIP_TRYA(hipMemcpyAsync(T->plane, g.data(), (size_t)n1 * n2 * sizeof(double), hipMemcpyHostToDevice, st));
-        HIP_TRYA(launch_adj_add_plane(c.nx, c.ny, n1, n2, c.wall_axis == DRP_WALL_Y, third, T->plane, Pa[cur], st));
+        HIP_TRYA(launch_adj_add_plane(L->G, n1, n2, c.wall_axis == DRP_WALL_Y, third, T->plane, Pa[cur], st));
         HIP_TRYA(hipStreamSynchronize(st));  // g is a host temporary
     }
 
@@ -220,11 +220,7 @@ extern "C" int drp_tape_backward(drp_tape* T, const double w[2], double* loss, d
             const int64_t nstep = T->start + rel + 1;       // forward step n -> n+1
             const double* state = seg_state(T, j, sgi);
             AdjArgs a{};
-            a.nx = c.nx;
-            a.ny = c.ny;
-            a.nz = c.nz;
-            a.n = L->n;
-            a.ns = n;
+            a.G = L->G;
             a.f = state;
             a.mac = state + 30 * n;
             a.Fin = Fa[cur];
@@ -252,7 +248,7 @@ extern "C" int drp_tape_backward(drp_tape* T, const double w[2], double* loss, d
             a.wall_active = (c.wall_axis != DRP_WALL_NONE && nstep >= c.wall_start) ? 1 : 0;
             a.first = (rel == 0 && T->start_eq) ? 1 : 0;
             HIP_TRYA(launch_adj_collide_fp64(a, st));
-            if (rel > 0) HIP_TRYA(launch_adj_stencil_fp64(c.nx, c.ny, c.nz, n, lapA, gradA, Pa[1 - cur], st));
+            if (rel > 0) HIP_TRYA(launch_adj_stencil_fp64(L->G, lapA, gradA, Pa[1 - cur], st));
             cur = 1 - cur;
         }
     }

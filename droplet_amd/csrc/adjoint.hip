@@ -44,21 +44,23 @@ constexpr int ADJ_BLOCK = 256;
 
 __device__ __forceinline__ int wrap1(int v, int n) { return v < 0 ? v + n : (v >= n ? v - n : v); }
 
-// node coordinates and indices in 32 bits: the tape admits fewer than 2^32 nodes
+// node coordinates and indices in 32 bits: the tape admits fewer than 2^32 nodes,
+// row padding included
 struct Node {
     int x, y, z;
 };
-__device__ __forceinline__ Node coords(uint32_t s, int nx, int ny) {
-    const uint32_t nxy = (uint32_t)nx * (uint32_t)ny;
+__device__ __forceinline__ Node coords(uint32_t s, const Grid& G) {
+    const uint32_t nxy = (uint32_t)G.px * (uint32_t)G.ny;
     Node c;
     c.z = (int)(s / nxy);
     const uint32_t r = s - (uint32_t)c.z * nxy;
-    c.y = (int)(r / (uint32_t)nx);
-    c.x = (int)(r - (uint32_t)c.y * (uint32_t)nx);
+    c.y = (int)(r / (uint32_t)G.px);
+    c.x = (int)(r - (uint32_t)c.y * (uint32_t)G.px);
     return c;
 }
-__device__ __forceinline__ uint32_t shifted(const Node& c, int dx, int dy, int dz, int nx, int ny, int nz) {
-    return (uint32_t)wrap1(c.x + dx, nx) + (uint32_t)nx * ((uint32_t)wrap1(c.y + dy, ny) + (uint32_t)ny * (uint32_t)wrap1(c.z + dz, nz));
+__device__ __forceinline__ uint32_t shifted(const Node& c, int dx, int dy, int dz, const Grid& G) {
+    return (uint32_t)wrap1(c.x + dx, G.nx) +
+           (uint32_t)G.px * ((uint32_t)wrap1(c.y + dy, G.ny) + (uint32_t)G.ny * (uint32_t)wrap1(c.z + dz, G.nz));
 }
 
 // workgroup sum of three partials, added into acc[blockIdx.x][0..2] (each
@@ -83,19 +85,20 @@ __device__ void block_accumulate(double v0, double v1, double v2, double* acc) {
 
 // five wavefronts per SIMD: 96 VGPRs hold the rolled direction loops without spilling
 __global__ __launch_bounds__(ADJ_BLOCK) __attribute__((amdgpu_waves_per_eu(5))) void adj_collide_fp64(AdjArgs a) {
-    const int nx = a.nx, ny = a.ny, nz = a.nz;
-    const int64_t n = a.ns;  // from one array to the next
+    const Grid& G = a.G;
+    const int ny = G.ny, nz = G.nz;
+    const int64_t n = G.ns;  // from one array to the next
     const uint32_t s = blockIdx.x * (uint32_t)ADJ_BLOCK + threadIdx.x;
     double d_tauf = 0.0, d_kg = 0.0, d_u = 0.0;
-    if (s < (uint64_t)a.n) {
-        const Node c = coords(s, nx, ny);
+    const Node c = coords(s, G);
+    if (c.x < G.nx && s < (uint64_t)G.slots()) {
         const double phi = a.mac[s];
         const double u[3] = {a.mac[2 * n + s], a.mac[3 * n + s], a.mac[4 * n + s]};
         // forward stencils at y (various_cal)
         double lap = -14.0 * phi, gr[3] = {0.0, 0.0, 0.0};
 #pragma unroll
         for (int q = 1; q < 15; q++) {
-            const double v = a.mac[shifted(c, CX[q], CY[q], CZ[q], nx, ny, nz)];
+            const double v = a.mac[shifted(c, CX[q], CY[q], CZ[q], G)];
             lap += v;
             gr[0] += CX[q] * v;
             gr[1] += CY[q] * v;
@@ -119,7 +122,7 @@ __global__ __launch_bounds__(ADJ_BLOCK) __attribute__((amdgpu_waves_per_eu(5))) 
         // adjoints, once for the outputs, the second time from L2) so that no
         // per-direction array stays in registers.
         auto adj_in = [&](int q, double& Fs, double& Gs) {
-            const uint32_t d = shifted(c, CX[q], CY[q], CZ[q], nx, ny, nz);
+            const uint32_t d = shifted(c, CX[q], CY[q], CZ[q], G);
             Fs = a.Fin[q * n + d];
             if (a.phin_in) Fs += a.phin_in[d];
             Gs = a.Gin[q * n + d];
@@ -218,16 +221,17 @@ __global__ __launch_bounds__(ADJ_BLOCK) __attribute__((amdgpu_waves_per_eu(5))) 
 }
 
 // phih_st(x) = -14/5 laph(x) + sum_{q>=1} [laph(x - c_q)/5 + c_q . gradh(x - c_q)/10]
-__global__ __launch_bounds__(ADJ_BLOCK) void adj_stencil_fp64(int nx, int ny, int nz, int64_t n, const double* __restrict__ lapA,
+__global__ __launch_bounds__(ADJ_BLOCK) void adj_stencil_fp64(Grid G, const double* __restrict__ lapA,
                                                               const double* __restrict__ gradA,
                                                               double* __restrict__ out) {
     const uint32_t s = blockIdx.x * (uint32_t)ADJ_BLOCK + threadIdx.x;
-    if (s >= (uint64_t)nx * ny * nz) return;
-    const Node c = coords(s, nx, ny);
+    const Node c = coords(s, G);
+    if (c.x >= G.nx || s >= (uint64_t)G.slots()) return;
+    const int64_t n = G.ns;
     double l = 0.0, g = 0.0;
 #pragma unroll
     for (int q = 1; q < 15; q++) {
-        const int64_t up = shifted(c, -CX[q], -CY[q], -CZ[q], nx, ny, nz);
+        const int64_t up = shifted(c, -CX[q], -CY[q], -CZ[q], G);
         l += lapA[up];
         g += CX[q] * gradA[up] + CY[q] * gradA[n + up] + CZ[q] * gradA[2 * n + up];
     }
@@ -235,16 +239,17 @@ __global__ __launch_bounds__(ADJ_BLOCK) void adj_stencil_fp64(int nx, int ny, in
 }
 
 // seed of sum_x |grad phi(x)|: gradA = w grad phi / |grad phi| (0 where grad phi = 0), lapA = 0
-__global__ __launch_bounds__(ADJ_BLOCK) void adj_seed_area_fp64(int nx, int ny, int nz, int64_t n, const double* __restrict__ phi,
+__global__ __launch_bounds__(ADJ_BLOCK) void adj_seed_area_fp64(Grid G, const double* __restrict__ phi,
                                                                 double w, double* __restrict__ lapA,
                                                                 double* __restrict__ gradA) {
     const uint32_t s = blockIdx.x * (uint32_t)ADJ_BLOCK + threadIdx.x;
-    if (s >= (uint64_t)nx * ny * nz) return;
-    const Node c = coords(s, nx, ny);
+    const Node c = coords(s, G);
+    if (c.x >= G.nx || s >= (uint64_t)G.slots()) return;
+    const int64_t n = G.ns;
     double gr[3] = {0.0, 0.0, 0.0};
 #pragma unroll
     for (int q = 1; q < 15; q++) {
-        const double v = phi[shifted(c, CX[q], CY[q], CZ[q], nx, ny, nz)];
+        const double v = phi[shifted(c, CX[q], CY[q], CZ[q], G)];
         gr[0] += CX[q] * v;
         gr[1] += CY[q] * v;
         gr[2] += CZ[q] * v;
@@ -259,42 +264,42 @@ __global__ __launch_bounds__(ADJ_BLOCK) void adj_seed_area_fp64(int nx, int ny, 
 
 // out[plane node (i, j)] += vals[j * n1 + i]; the plane is (x, y) at z = third
 // (wall_y) or (x, z) at y = third
-__global__ void adj_add_plane(int nx, int ny, int n1, int n2, int wall_y, int third, const double* __restrict__ vals,
+__global__ void adj_add_plane(Grid G, int n1, int n2, int wall_y, int third, const double* __restrict__ vals,
                               double* __restrict__ out) {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= n1 * n2) return;
     const int i = t % n1, j = t / n1;
-    const int64_t s = wall_y ? i + (int64_t)nx * (j + (int64_t)ny * third) : i + (int64_t)nx * (third + (int64_t)ny * j);
+    const int64_t s = wall_y ? G.node(i, j, third) : G.node(i, third, j);
     out[s] += vals[t];
 }
 
 // ------------------------------------------------------------------ launchers
 static inline int nblocks(int64_t n) { return (int)((n + ADJ_BLOCK - 1) / ADJ_BLOCK); }
 
-int adj_block_count(int64_t n) { return nblocks(n); }
+int adj_block_count(const Grid& G) { return nblocks(G.slots()); }
 
 hipError_t launch_adj_collide_fp64(const AdjArgs& a, hipStream_t st) {
-    hipLaunchKernelGGL(adj_collide_fp64, dim3(nblocks(a.n)), dim3(ADJ_BLOCK), 0, st, a);
+    hipLaunchKernelGGL(adj_collide_fp64, dim3(nblocks(a.G.slots())), dim3(ADJ_BLOCK), 0, st, a);
     return hipGetLastError();
 }
 
-hipError_t launch_adj_stencil_fp64(int nx, int ny, int nz, int64_t ns, const double* lapA, const double* gradA, double* out,
+hipError_t launch_adj_stencil_fp64(const Grid& G, const double* lapA, const double* gradA, double* out,
                                    hipStream_t st) {
-    hipLaunchKernelGGL(adj_stencil_fp64, dim3(nblocks((int64_t)nx * ny * nz)), dim3(ADJ_BLOCK), 0, st, nx, ny, nz,
-                       ns, lapA, gradA, out);
+    hipLaunchKernelGGL(adj_stencil_fp64, dim3(nblocks(G.slots())), dim3(ADJ_BLOCK), 0, st, G,
+                       lapA, gradA, out);
     return hipGetLastError();
 }
 
-hipError_t launch_adj_seed_area_fp64(int nx, int ny, int nz, int64_t ns, const double* phi, double w, double* lapA,
+hipError_t launch_adj_seed_area_fp64(const Grid& G, const double* phi, double w, double* lapA,
                                      double* gradA, hipStream_t st) {
-    hipLaunchKernelGGL(adj_seed_area_fp64, dim3(nblocks((int64_t)nx * ny * nz)), dim3(ADJ_BLOCK), 0, st, nx, ny,
-                       nz, ns, phi, w, lapA, gradA);
+    hipLaunchKernelGGL(adj_seed_area_fp64, dim3(nblocks(G.slots())), dim3(ADJ_BLOCK), 0, st, G,
+                       phi, w, lapA, gradA);
     return hipGetLastError();
 }
 
-hipError_t launch_adj_add_plane(int nx, int ny, int n1, int n2, int wall_y, int third, const double* vals,
+hipError_t launch_adj_add_plane(const Grid& G, int n1, int n2, int wall_y, int third, const double* vals,
                                 double* out, hipStream_t st) {
-    hipLaunchKernelGGL(adj_add_plane, dim3((n1 * n2 + 255) / 256), dim3(256), 0, st, nx, ny, n1, n2, wall_y, third,
+    hipLaunchKernelGGL(adj_add_plane, dim3((n1 * n2 + 255) / 256), dim3(256), 0, st, G, n1, n2, wall_y, third,
                        vals, out);
     return hipGetLastError();
 }

@@ -15,10 +15,10 @@ template <int Q0, int Q1, typename Fn> __device__ __forceinline__ void sforx(Fn&
 
 static inline dim3 grid_for(int64_t n) { return dim3((unsigned)((n + 255) / 256)); }
 
-__global__ void to_shifted(int64_t n, int64_t ns, ShiftRef r, const double* __restrict__ pop64, const double* __restrict__ mac64,
+__global__ void to_shifted(Grid G, ShiftRef r, const double* __restrict__ pop64, const double* __restrict__ mac64,
                            float* __restrict__ pop32, float* __restrict__ mac32) {
-    const int64_t s = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (s >= n) return;
+    const int64_t ns = G.ns, s = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if (s >= G.slots()) return;
     sforx<0, 15>([&](auto qc) {
         constexpr int q = decltype(qc)::value;
         pop32[q * ns + s] = (float)(pop64[q * ns + s] - r.fr[q]);
@@ -31,31 +31,31 @@ __global__ void to_shifted(int64_t n, int64_t ns, ShiftRef r, const double* __re
     mac32[4 * ns + s] = (float)mac64[4 * ns + s];
 }
 
-__global__ void pops_from_shifted(int64_t n, int64_t ns, ShiftRef r, const float* __restrict__ pop32, double* __restrict__ out,
+__global__ void pops_from_shifted(Grid G, ShiftRef r, const float* __restrict__ pop32, double* __restrict__ out,
                                   int set) {
-    const int64_t s = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (s >= n) return;
+    const int64_t ns = G.ns, s = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if (s >= G.slots()) return;
     sforx<0, 15>([&](auto qc) {
         constexpr int q = decltype(qc)::value;
         const double ref = set == 0 ? r.fr[q] : weightE<q>();
-        out[q * n + s] = ref + (double)pop32[(set * 15 + q) * ns + s];
+        out[q * ns + s] = ref + (double)pop32[(set * 15 + q) * ns + s];
     });
 }
 
-__global__ void pops_to_shifted(int64_t n, int64_t ns, ShiftRef r, const double* __restrict__ in, float* __restrict__ pop32,
+__global__ void pops_to_shifted(Grid G, ShiftRef r, const double* __restrict__ in, float* __restrict__ pop32,
                                 int set) {
-    const int64_t s = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (s >= n) return;
+    const int64_t ns = G.ns, s = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if (s >= G.slots()) return;
     sforx<0, 15>([&](auto qc) {
         constexpr int q = decltype(qc)::value;
         const double ref = set == 0 ? r.fr[q] : weightE<q>();
-        pop32[(set * 15 + q) * ns + s] = (float)(in[q * n + s] - ref);
+        pop32[(set * 15 + q) * ns + s] = (float)(in[q * ns + s] - ref);
     });
 }
 
-__global__ void macro_from_shifted(int64_t n, int64_t ns, double phi1, const float* __restrict__ m32, double* __restrict__ m64) {
-    const int64_t s = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (s >= n) return;
+__global__ void macro_from_shifted(Grid G, double phi1, const float* __restrict__ m32, double* __restrict__ m64) {
+    const int64_t ns = G.ns, s = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if (s >= G.slots()) return;
     m64[s] = phi1 + (double)m32[s];
     m64[ns + s] = 1.0 / 3.0 + (double)m32[ns + s];
     m64[2 * ns + s] = (double)m32[2 * ns + s];
@@ -63,10 +63,10 @@ __global__ void macro_from_shifted(int64_t n, int64_t ns, double phi1, const flo
     m64[4 * ns + s] = (double)m32[4 * ns + s];
 }
 
-__global__ void moments_fp32(int64_t n, int64_t ns, const float* __restrict__ f, const float* __restrict__ g,
+__global__ void moments_fp32(Grid G, const float* __restrict__ f, const float* __restrict__ g,
                              float* __restrict__ mac, int which) {
-    const int64_t s = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (s >= n) return;
+    const int64_t ns = G.ns, s = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if (s >= G.slots()) return;
     double ph = 0.0;
     float pr = 0.0f, m1 = 0.0f, m2 = 0.0f, m3 = 0.0f;
     sforx<0, 15>([&](auto qc) {
@@ -92,13 +92,13 @@ __global__ void moments_fp32(int64_t n, int64_t ns, const float* __restrict__ f,
 // the state a step left (mac) and the one it started from (mac_old), every
 // neighbour outside the node's rank block (B, periodic wraps included) from
 // mac_old (B.bx = 0: all from mac).
-__global__ void les_tau_fp32(int nx, int ny, int nz, int64_t ns, Phys P, const float* __restrict__ mac,
+__global__ void les_tau_fp32(Grid G, Phys P, const float* __restrict__ mac,
                              const float* __restrict__ mac_old, LesBlocks B, const uint64_t* __restrict__ range,
                              int slot, float* __restrict__ tau) {
-    const int64_t N = (int64_t)nx * ny * nz;
+    const int nx = G.nx, ny = G.ny, nz = G.nz;
     const int64_t s = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (s >= N) return;
-    const int x = s % nx, y = (s / nx) % ny, z = s / ((int64_t)nx * ny);
+    const int x = s % G.px, y = (s / G.px) % ny, z = s / ((int64_t)G.px * ny);
+    if (x >= nx || z >= nz) return;
     const int x0 = B.bx > 0 ? (x / B.bx) * B.bx : 0, y0 = B.bx > 0 ? (y / B.by) * B.by : 0,
               z0 = B.bx > 0 ? (z / B.bz) * B.bz : 0;
     float gu[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
@@ -112,9 +112,9 @@ __global__ void les_tau_fp32(int nx, int ny, int nz, int64_t ns, Phys P, const f
         xx = xx < 0 ? xx + nx : (xx >= nx ? xx - nx : xx);
         yy = yy < 0 ? yy + ny : (yy >= ny ? yy - ny : yy);
         zz = zz < 0 ? zz + nz : (zz >= nz ? zz - nz : zz);
-        const int64_t t = xx + (int64_t)nx * (yy + (int64_t)ny * zz);
+        const int64_t t = G.node(xx, yy, zz);
         for (int k = 0; k < 3; k++) {
-            const float v = u[(2 + k) * ns + t];
+            const float v = u[(2 + k) * G.ns + t];
             gu[k][0] = acc<D::cx>(gu[k][0], v);
             gu[k][1] = acc<D::cy>(gu[k][1], v);
             gu[k][2] = acc<D::cz>(gu[k][2], v);
@@ -145,10 +145,12 @@ __device__ __forceinline__ int wrap_zm32(int v, int n, bool small) {
     if (small) return ((v % n) + n) % n;
     return v < 0 ? v + n : (v >= n ? v - n : v);
 }
-__global__ __launch_bounds__(ZM32_NT) void les_tau_fp32_zm(int nx, int ny, int nz, int64_t N, Phys P, const float* __restrict__ mac,
+__global__ __launch_bounds__(ZM32_NT) void les_tau_fp32_zm(Grid G, Phys P, const float* __restrict__ mac,
                                                           const uint64_t* __restrict__ range, int slot,
                                                           float* __restrict__ tau, int tiles_x, int tiles_y) {
     __shared__ float su[3][3][ZM32_HP];  // [ring slot][component][plane node]
+    const int nx = G.nx, ny = G.ny, nz = G.nz;
+    const int64_t N = G.ns, nxy = (int64_t)G.px * ny;
     const int x0 = (blockIdx.x % tiles_x) * ZM32_TX, y0 = ((blockIdx.x / tiles_x) % tiles_y) * ZM32_TY;
     const int zs = (blockIdx.x / (tiles_x * tiles_y)) * ZM32_ZC, ze = min(zs + ZM32_ZC, nz);
     const bool small = nx <= ZM32_TX || ny <= ZM32_TY || nz <= 2;
@@ -158,12 +160,12 @@ __global__ __launch_bounds__(ZM32_NT) void les_tau_fp32_zm(int nx, int ny, int n
     const double rmax = from_ordered_bits(range[2 * slot]), rmin = from_ordered_bits(range[2 * slot + 1]);
     const double rg = rmax - rmin;
     auto fetch = [&](int zg, float (&r)[ZM32_PER][3]) {
-        const int64_t zoff = (int64_t)nx * ny * wrap_zm32(zg, nz, small);
+        const int64_t zoff = nxy * wrap_zm32(zg, nz, small);
 #pragma unroll
         for (int i = 0; i < ZM32_PER; i++) {
             const int h0 = threadIdx.x + i * ZM32_NT, h = h0 < ZM32_HP ? h0 : ZM32_HP - 1;
             const int64_t g = wrap_zm32(x0 + h % ZM32_HX - 1, nx, small) +
-                              (int64_t)nx * wrap_zm32(y0 + h / ZM32_HX - 1, ny, small) + zoff;
+                              (int64_t)G.px * wrap_zm32(y0 + h / ZM32_HX - 1, ny, small) + zoff;
 #pragma unroll
             for (int k = 0; k < 3; k++) r[i][k] = mac[(2 + k) * N + g];
         }
@@ -183,13 +185,13 @@ __global__ __launch_bounds__(ZM32_NT) void les_tau_fp32_zm(int nx, int ny, int n
         fetch(zs - 1 + p, next);
         store(next, su[p]);
     }
-    const int64_t col = (int64_t)(in ? x : 0) + (int64_t)nx * (in ? y : 0);
-    float phi_next = mac[col + (int64_t)nx * ny * zs];
+    const int64_t col = G.node(in ? x : 0, in ? y : 0, 0);
+    float phi_next = mac[col + nxy * zs];
     for (int z = zs; z < ze; z++) {
         const bool more = z + 1 < ze;  // plane z+2 is needed by plane z+1
         if (more) fetch(z + 2, next);
         const float phit = phi_next;
-        if (more) phi_next = mac[col + (int64_t)nx * ny * (z + 1)];
+        if (more) phi_next = mac[col + nxy * (z + 1)];
         __syncthreads();
         if (in) {
             const int rz[3] = {(z - zs) % 3, (z - zs + 1) % 3, (z - zs + 2) % 3};  // planes z-1, z, z+1
@@ -214,45 +216,44 @@ __global__ __launch_bounds__(ZM32_NT) void les_tau_fp32_zm(int nx, int ny, int n
             const double phi = P.phi1 + (double)phit;
             const double frac = rg == 0.0 ? 0.0 : (phi - rmin) / rg;
             const double nu = frac * P.dnu + P.nu1;
-            tau[col + (int64_t)nx * ny * z] = (float)(0.5 + 3.0 * (nu + P.les_c * sqrt(2.0 * (double)sum)));
+            tau[col + nxy * z] = (float)(0.5 + 3.0 * (nu + P.les_c * sqrt(2.0 * (double)sum)));
         }
         __syncthreads();
         if (more) store(next, su[(z - zs) % 3]);  // the slot of plane z-1
     }
 }
 
-hipError_t launch_to_shifted(int64_t n, int64_t ns, const ShiftRef& r, const double* pop64, const double* mac64, float* pop32,
+hipError_t launch_to_shifted(const Grid& G, const ShiftRef& r, const double* pop64, const double* mac64, float* pop32,
                              float* mac32, hipStream_t st) {
-    hipLaunchKernelGGL(to_shifted, grid_for(n), dim3(256), 0, st, n, ns, r, pop64, mac64, pop32, mac32);
+    hipLaunchKernelGGL(to_shifted, grid_for(G.slots()), dim3(256), 0, st, G, r, pop64, mac64, pop32, mac32);
     return hipGetLastError();
 }
-hipError_t launch_pops_from_shifted(int64_t n, int64_t ns, const ShiftRef& r, const float* pop32, double* pop64, int set,
+hipError_t launch_pops_from_shifted(const Grid& G, const ShiftRef& r, const float* pop32, double* pop64, int set,
                                     hipStream_t st) {
-    hipLaunchKernelGGL(pops_from_shifted, grid_for(n), dim3(256), 0, st, n, ns, r, pop32, pop64, set);
+    hipLaunchKernelGGL(pops_from_shifted, grid_for(G.slots()), dim3(256), 0, st, G, r, pop32, pop64, set);
     return hipGetLastError();
 }
-hipError_t launch_pops_to_shifted(int64_t n, int64_t ns, const ShiftRef& r, const double* pop64, float* pop32, int set,
+hipError_t launch_pops_to_shifted(const Grid& G, const ShiftRef& r, const double* pop64, float* pop32, int set,
                                   hipStream_t st) {
-    hipLaunchKernelGGL(pops_to_shifted, grid_for(n), dim3(256), 0, st, n, ns, r, pop64, pop32, set);
+    hipLaunchKernelGGL(pops_to_shifted, grid_for(G.slots()), dim3(256), 0, st, G, r, pop64, pop32, set);
     return hipGetLastError();
 }
-hipError_t launch_macro_from_shifted(int64_t n, int64_t ns, double phi1, const float* mac32, double* mac64, hipStream_t st) {
-    hipLaunchKernelGGL(macro_from_shifted, grid_for(n), dim3(256), 0, st, n, ns, phi1, mac32, mac64);
+hipError_t launch_macro_from_shifted(const Grid& G, double phi1, const float* mac32, double* mac64, hipStream_t st) {
+    hipLaunchKernelGGL(macro_from_shifted, grid_for(G.slots()), dim3(256), 0, st, G, phi1, mac32, mac64);
     return hipGetLastError();
 }
-hipError_t launch_moments_fp32(int64_t n, int64_t ns, const float* f, const float* g, float* mac, int which, hipStream_t st) {
-    hipLaunchKernelGGL(moments_fp32, grid_for(n), dim3(256), 0, st, n, ns, f, g, mac, which);
+hipError_t launch_moments_fp32(const Grid& G, const float* f, const float* g, float* mac, int which, hipStream_t st) {
+    hipLaunchKernelGGL(moments_fp32, grid_for(G.slots()), dim3(256), 0, st, G, f, g, mac, which);
     return hipGetLastError();
 }
-hipError_t launch_les_tau_fp32(int nx, int ny, int nz, int64_t ns, const Phys& ph, const float* mac, const float* mac_old,
+hipError_t launch_les_tau_fp32(const Grid& G, const Phys& ph, const float* mac, const float* mac_old,
                                const LesBlocks& blk, const uint64_t* range, int slot, float* tau, hipStream_t st) {
-    const int64_t n = (int64_t)nx * ny * nz;
     if (blk.bx > 0 && mac_old != mac) {
-        hipLaunchKernelGGL(les_tau_fp32, grid_for(n), dim3(256), 0, st, nx, ny, nz, ns, ph, mac, mac_old, blk, range, slot,
+        hipLaunchKernelGGL(les_tau_fp32, grid_for(G.slots()), dim3(256), 0, st, G, ph, mac, mac_old, blk, range, slot,
                            tau);
     } else {
-        const int mx = (nx + ZM32_TX - 1) / ZM32_TX, my = (ny + ZM32_TY - 1) / ZM32_TY, mz = (nz + ZM32_ZC - 1) / ZM32_ZC;
-        hipLaunchKernelGGL(les_tau_fp32_zm, dim3((unsigned)(mx * my * mz)), dim3(ZM32_NT), 0, st, nx, ny, nz, ns, ph, mac,
+        const int mx = (G.nx + ZM32_TX - 1) / ZM32_TX, my = (G.ny + ZM32_TY - 1) / ZM32_TY, mz = (G.nz + ZM32_ZC - 1) / ZM32_ZC;
+        hipLaunchKernelGGL(les_tau_fp32_zm, dim3((unsigned)(mx * my * mz)), dim3(ZM32_NT), 0, st, G, ph, mac,
                            range, slot, tau, mx, my);
     }
     return hipGetLastError();

@@ -16,16 +16,6 @@ template <int Q0, int Q1, typename Fn> __device__ __forceinline__ void sfor(Fn&&
     }
 }
 
-struct Grid {
-    int nx, ny, nz;
-    __device__ __forceinline__ int64_t at(int x, int y, int z) const {
-        x = x < 0 ? x + nx : (x >= nx ? x - nx : x);
-        y = y < 0 ? y + ny : (y >= ny ? y - ny : y);
-        z = z < 0 ? z + nz : (z >= nz ? z - nz : z);
-        return x + (int64_t)nx * (y + (int64_t)ny * z);
-    }
-};
-
 // lap phi and grad phi at (x,y,z) from global memory (various_cal :608-633)
 __device__ void phi_stencil(const Grid& G, const double* phi, int x, int y, int z, double& lap, double& g0,
                             double& g1, double& g2) {
@@ -76,11 +66,11 @@ __device__ __forceinline__ bool les_halo(const LesBlocks& B, int x, int y, int z
     return xx < x0 || xx >= x0 + B.bx || yy < y0 || yy >= y0 + B.by || zz < z0 || zz >= z0 + B.bz;
 }
 
-__global__ void init_equilibrium_fp64(Grid G, int64_t N, Phys P, const double* __restrict__ mac, double* __restrict__ f,
+__global__ void init_equilibrium_fp64(Grid G, Phys P, const double* __restrict__ mac, double* __restrict__ f,
                                       double* __restrict__ g) {
-    const int64_t s = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (s >= (int64_t)G.nx * G.ny * G.nz) return;
-    const int x = s % G.nx, y = (s / G.nx) % G.ny, z = s / ((int64_t)G.nx * G.ny);
+    const int64_t N = G.ns, s = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    const int x = s % G.px, y = (s / G.px) % G.ny, z = s / ((int64_t)G.px * G.ny);
+    if (x >= G.nx || z >= G.nz) return;
     NodeEq<double> nd;
     nd.phi = mac[s];
     nd.p = mac[N + s];
@@ -102,10 +92,10 @@ __global__ void init_equilibrium_fp64(Grid G, int64_t N, Phys P, const double* _
     });
 }
 
-__global__ void moments_fp64(int64_t n, int64_t N, const double* __restrict__ f, const double* __restrict__ g,
+__global__ void moments_fp64(Grid G, const double* __restrict__ f, const double* __restrict__ g,
                              double* __restrict__ mac, int which) {
-    const int64_t s = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (s >= n) return;
+    const int64_t N = G.ns, s = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if (s >= G.slots()) return;
     double ph = f[s], pr = g[s] / 3.0, m1 = 0.0, m2 = 0.0, m3 = 0.0;
     sfor<1, 15>([&](auto qc) {
         constexpr int q = decltype(qc)::value;
@@ -145,7 +135,7 @@ __device__ __forceinline__ int wrap_any(int v, int n, bool small) {
 // u (and, with rank blocks, the old u) of a tile and its 1-node halo are staged
 // in LDS once per workgroup.
 template <bool STALE>
-__global__ __launch_bounds__(LES_TX* LES_TY* LES_TZ) void les_tau_fp64(Grid G, int64_t N, Phys P, const double* __restrict__ mac,
+__global__ __launch_bounds__(LES_TX* LES_TY* LES_TZ) void les_tau_fp64(Grid G, Phys P, const double* __restrict__ mac,
                                                                        const double* __restrict__ mac_old, LesBlocks B,
                                                                        const uint64_t* __restrict__ range, int slot,
                                                                        double* __restrict__ tau, int tiles_x,
@@ -153,15 +143,15 @@ __global__ __launch_bounds__(LES_TX* LES_TY* LES_TZ) void les_tau_fp64(Grid G, i
     constexpr int HX = LES_TX + 2, HY = LES_TY + 2, HZ = LES_TZ + 2, H = HX * HY * HZ, NT = LES_TX * LES_TY * LES_TZ;
     __shared__ double su[3][H];
     __shared__ double so[STALE ? 3 : 1][STALE ? H : 1];
+    const int64_t N = G.ns;
     const int tile = blockIdx.x;
     const int x0 = (tile % tiles_x) * LES_TX, y0 = ((tile / tiles_x) % tiles_y) * LES_TY,
               z0 = (tile / (tiles_x * tiles_y)) * LES_TZ;
     const bool small = G.nx <= LES_TX || G.ny <= LES_TY || G.nz <= LES_TZ;
     for (int h = threadIdx.x; h < H; h += NT) {
         const int hx = h % HX, hy = (h / HX) % HY, hz = h / (HX * HY);
-        const int64_t g = wrap_any(x0 + hx - 1, G.nx, small) +
-                          (int64_t)G.nx * (wrap_any(y0 + hy - 1, G.ny, small) +
-                                           (int64_t)G.ny * wrap_any(z0 + hz - 1, G.nz, small));
+        const int64_t g = G.node(wrap_any(x0 + hx - 1, G.nx, small), wrap_any(y0 + hy - 1, G.ny, small),
+                                 wrap_any(z0 + hz - 1, G.nz, small));
         for (int k = 0; k < 3; k++) {
             su[k][h] = mac[(2 + k) * N + g];
             if constexpr (STALE) so[k][h] = mac_old[(2 + k) * N + g];
@@ -171,7 +161,7 @@ __global__ __launch_bounds__(LES_TX* LES_TY* LES_TZ) void les_tau_fp64(Grid G, i
     const int tx = threadIdx.x % LES_TX, ty = (threadIdx.x / LES_TX) % LES_TY, tz = threadIdx.x / (LES_TX * LES_TY);
     const int x = x0 + tx, y = y0 + ty, z = z0 + tz;
     if (x >= G.nx || y >= G.ny || z >= G.nz) return;
-    const int64_t s = x + (int64_t)G.nx * (y + (int64_t)G.ny * z);
+    const int64_t s = G.node(x, y, z);
     double gu[3][3];
     for (int k = 0; k < 3; k++)
         for (int a = 0; a < 3; a++) gu[k][a] = 0.0;
@@ -223,18 +213,18 @@ template <typename T, int NC> struct ZmPlane {
 };
 
 template <typename T, int NC, int F0>
-__device__ __forceinline__ ZmPlane<T, NC> zm_fetch(const Grid& G, const T* __restrict__ mac, int64_t N, int x0, int y0,
-                                                   int zg, bool small) {
+__device__ __forceinline__ ZmPlane<T, NC> zm_fetch(const Grid& G, const T* __restrict__ mac, int x0, int y0, int zg,
+                                                   bool small) {
     ZmPlane<T, NC> r;
-    const int64_t zoff = (int64_t)G.nx * G.ny * wrap_any(zg, G.nz, small);
+    const int64_t zoff = (int64_t)G.px * G.ny * wrap_any(zg, G.nz, small);
 #pragma unroll
     for (int i = 0; i < ZM_PER; i++) {
         // unconditional loads (index clamped into the plane) keep the wait a straight count
         const int h0 = threadIdx.x + i * ZM_NT, h = h0 < ZM_HP ? h0 : ZM_HP - 1;
         const int64_t g = wrap_any(x0 + h % ZM_HX - 1, G.nx, small) +
-                          (int64_t)G.nx * wrap_any(y0 + h / ZM_HX - 1, G.ny, small) + zoff;
+                          (int64_t)G.px * wrap_any(y0 + h / ZM_HX - 1, G.ny, small) + zoff;
 #pragma unroll
-        for (int k = 0; k < NC; k++) r.v[i][k] = mac[(F0 + k) * N + g];
+        for (int k = 0; k < NC; k++) r.v[i][k] = mac[(F0 + k) * G.ns + g];
     }
     return r;
 }
@@ -249,7 +239,7 @@ template <typename T, int NC> __device__ __forceinline__ void zm_store(const ZmP
     }
 }
 
-__global__ __launch_bounds__(ZM_NT) void les_tau_fp64_zm(Grid G, int64_t N, Phys P, const double* __restrict__ mac,
+__global__ __launch_bounds__(ZM_NT) void les_tau_fp64_zm(Grid G, Phys P, const double* __restrict__ mac,
                                                           const uint64_t* __restrict__ range, int slot,
                                                           double* __restrict__ tau, int tiles_x, int tiles_y) {
     __shared__ double su[3][3][ZM_HP];  // [ring slot][component][plane node]
@@ -262,17 +252,17 @@ __global__ __launch_bounds__(ZM_NT) void les_tau_fp64_zm(Grid G, int64_t N, Phys
     const double rmax = from_ordered_bits(range[2 * slot]), rmin = from_ordered_bits(range[2 * slot + 1]);
     const double rg = rmax - rmin;
     // ring slot of plane z' is (z' - zs + 1) mod 3
-    zm_store(zm_fetch<double, 3, 2>(G, mac, N, x0, y0, zs - 1, small), su[0]);
-    zm_store(zm_fetch<double, 3, 2>(G, mac, N, x0, y0, zs, small), su[1]);
-    zm_store(zm_fetch<double, 3, 2>(G, mac, N, x0, y0, zs + 1, small), su[2]);
-    const int64_t col = (int64_t)(in ? x : 0) + (int64_t)G.nx * (in ? y : 0);
-    double phi_next = mac[col + (int64_t)G.nx * G.ny * zs];
+    zm_store(zm_fetch<double, 3, 2>(G, mac, x0, y0, zs - 1, small), su[0]);
+    zm_store(zm_fetch<double, 3, 2>(G, mac, x0, y0, zs, small), su[1]);
+    zm_store(zm_fetch<double, 3, 2>(G, mac, x0, y0, zs + 1, small), su[2]);
+    const int64_t col = G.node(in ? x : 0, in ? y : 0, 0), nxy = (int64_t)G.px * G.ny;
+    double phi_next = mac[col + nxy * zs];
     for (int z = zs; z < ze; z++) {
         const bool more = z + 1 < ze;  // plane z+2 is needed by plane z+1
         ZmPlane<double, 3> next;
-        if (more) next = zm_fetch<double, 3, 2>(G, mac, N, x0, y0, z + 2, small);
+        if (more) next = zm_fetch<double, 3, 2>(G, mac, x0, y0, z + 2, small);
         const double phi = phi_next;
-        if (more) phi_next = mac[col + (int64_t)G.nx * G.ny * (z + 1)];
+        if (more) phi_next = mac[col + nxy * (z + 1)];
         __syncthreads();
         if (in) {
             const int rz[3] = {(z - zs) % 3, (z - zs + 1) % 3, (z - zs + 2) % 3};  // planes z-1, z, z+1
@@ -302,7 +292,7 @@ __global__ __launch_bounds__(ZM_NT) void les_tau_fp64_zm(Grid G, int64_t N, Phys
             double frac = (phi - rmin) / rg;
             if (rg == 0.0) frac = 0.0;
             const double nu = frac * P.dnu + P.nu1;
-            tau[col + (int64_t)G.nx * G.ny * z] = 0.5 + 3.0 * (nu + nue);
+            tau[col + nxy * z] = 0.5 + 3.0 * (nu + nue);
         }
         __syncthreads();
         if (more) zm_store(next, su[(z - zs) % 3]);  // the slot of plane z-1
@@ -328,20 +318,20 @@ __device__ __forceinline__ void add_comp(double& s, double& c, double v) {
 // REDUCE_MAX_BLOCKS of them run, each over a fixed set of columns, and leave one
 // record each.  Per-thread sums are compensated, so the longer per-thread chain
 // costs no accuracy against the tree over single nodes.
-__global__ __launch_bounds__(ZM_NT) void reduce_fp64(Grid G, int64_t N, Phys P, const double* __restrict__ mac,
+__global__ __launch_bounds__(ZM_NT) void reduce_fp64(Grid G, Phys P, const double* __restrict__ mac,
                                                      double* __restrict__ partial, int tiles_x, int tiles_y, int zc,
                                                      int64_t items) {
     __shared__ double su[3][4][ZM_HP];  // [ring slot][phi, u1, u2, u3][plane node]
     __shared__ double sh[NPART][ZM_NT / 64];
-    const int64_t nxy = (int64_t)G.nx * G.ny;
+    const int64_t N = G.ns, nxy = (int64_t)G.px * G.ny;
     const bool small = G.nx <= ZM_TX || G.ny <= ZM_TY || G.nz <= 2;
     const int tx = threadIdx.x % ZM_TX, ty = threadIdx.x / ZM_TX;
     double s[NPART] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0}, comp[NPART] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
     auto plane = [&](int x0, int y0, int zg) {
         // phi is field 0, u fields 2..4: two fetches of consecutive fields
         ZmPlane<double, 4> r;
-        const ZmPlane<double, 1> a = zm_fetch<double, 1, 0>(G, mac, N, x0, y0, zg, small);
-        const ZmPlane<double, 3> b = zm_fetch<double, 3, 2>(G, mac, N, x0, y0, zg, small);
+        const ZmPlane<double, 1> a = zm_fetch<double, 1, 0>(G, mac, x0, y0, zg, small);
+        const ZmPlane<double, 3> b = zm_fetch<double, 3, 2>(G, mac, x0, y0, zg, small);
 #pragma unroll
         for (int i = 0; i < ZM_PER; i++) {
             r.v[i][0] = a.v[i][0];
@@ -359,7 +349,7 @@ __global__ __launch_bounds__(ZM_NT) void reduce_fp64(Grid G, int64_t N, Phys P, 
         zm_store(plane(x0, y0, zs - 1), su[0]);
         zm_store(plane(x0, y0, zs), su[1]);
         zm_store(plane(x0, y0, zs + 1), su[2]);
-        const int64_t col = (int64_t)(in ? x : 0) + (int64_t)G.nx * (in ? y : 0);
+        const int64_t col = G.node(in ? x : 0, in ? y : 0, 0);
         double p_next = mac[N + col + nxy * zs];
         int r0 = 0, r1 = 1, r2 = 2;  // ring slots of planes z-1, z, z+1
         for (int z = zs; z < ze; z++) {
@@ -457,6 +447,18 @@ __global__ __launch_bounds__(64 * NPART) void reduce_final(const double* __restr
     if (threadIdx.x < 2) reinterpret_cast<uint64_t*>(out + NPART)[threadIdx.x] = range_slot[threadIdx.x];
 }
 
+// rows of nx doubles, `stride` apart in node arrays, to contiguous rows (or back);
+// one thread per value
+template <bool TO_NODES>
+__global__ __launch_bounds__(256) void pack_rows(int nx, int64_t rows, int64_t stride, double* nodes, double* packed) {
+    const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    const int64_t row = i / nx;
+    if (row >= rows) return;
+    const int64_t s = (i - row * nx) + stride * row;
+    if (TO_NODES) nodes[s] = packed[i];
+    else packed[i] = nodes[s];
+}
+
 __global__ void range_set(uint64_t* range, int slot, double vmax, double vmin) {
     range[2 * slot] = ordered_bits(vmax);
     range[2 * slot + 1] = ordered_bits(vmin);
@@ -465,51 +467,59 @@ __global__ void range_set(uint64_t* range, int slot, double vmax, double vmin) {
 // ------------------------------------------------------------------ launchers
 static inline int64_t nblk(int64_t n, int bs) { return (n + bs - 1) / bs; }
 
-hipError_t launch_init_equilibrium_fp64(int nx, int ny, int nz, int64_t ns, const Phys& ph, const double* mac, double* f,
+hipError_t launch_init_equilibrium_fp64(const Grid& G, const Phys& ph, const double* mac, double* f,
                                         double* g, hipStream_t st) {
-    Grid G{nx, ny, nz};
-    const int64_t N = (int64_t)nx * ny * nz;
-    hipLaunchKernelGGL(init_equilibrium_fp64, dim3(nblk(N, 256)), dim3(256), 0, st, G, ns, ph, mac, f, g);
+    hipLaunchKernelGGL(init_equilibrium_fp64, dim3(nblk(G.slots(), 256)), dim3(256), 0, st, G, ph, mac, f, g);
     return hipGetLastError();
 }
 
-hipError_t launch_moments_fp64(int nx, int ny, int nz, int64_t ns, const double* f, const double* g, double* mac, int which,
+hipError_t launch_moments_fp64(const Grid& G, const double* f, const double* g, double* mac, int which,
                                hipStream_t st) {
-    const int64_t N = (int64_t)nx * ny * nz;
-    hipLaunchKernelGGL(moments_fp64, dim3(nblk(N, 256)), dim3(256), 0, st, N, ns, f, g, mac, which);
+    hipLaunchKernelGGL(moments_fp64, dim3(nblk(G.slots(), 256)), dim3(256), 0, st, G, f, g, mac, which);
     return hipGetLastError();
 }
 
-hipError_t launch_les_tau_fp64(int nx, int ny, int nz, int64_t ns, const Phys& ph, const double* mac, const double* mac_old,
+hipError_t launch_les_tau_fp64(const Grid& G, const Phys& ph, const double* mac, const double* mac_old,
                                const LesBlocks& blk, const uint64_t* range, int slot, double* tau, hipStream_t st) {
-    Grid G{nx, ny, nz};
-    const int tx = (nx + LES_TX - 1) / LES_TX, ty = (ny + LES_TY - 1) / LES_TY, tz = (nz + LES_TZ - 1) / LES_TZ;
+    const int tx = (G.nx + LES_TX - 1) / LES_TX, ty = (G.ny + LES_TY - 1) / LES_TY, tz = (G.nz + LES_TZ - 1) / LES_TZ;
     const dim3 grid((unsigned)(tx * ty * tz)), block(LES_TX * LES_TY * LES_TZ);
     if (blk.bx > 0 && mac_old != mac) {
-        hipLaunchKernelGGL(les_tau_fp64<true>, grid, block, 0, st, G, ns, ph, mac, mac_old, blk, range, slot, tau, tx, ty);
+        hipLaunchKernelGGL(les_tau_fp64<true>, grid, block, 0, st, G, ph, mac, mac_old, blk, range, slot, tau, tx, ty);
     } else {
-        const int mx = (nx + ZM_TX - 1) / ZM_TX, my = (ny + ZM_TY - 1) / ZM_TY, mz = (nz + ZM_ZC - 1) / ZM_ZC;
-        hipLaunchKernelGGL(les_tau_fp64_zm, dim3((unsigned)(mx * my * mz)), dim3(ZM_TX * ZM_TY), 0, st, G, ns, ph, mac, range,
+        const int mx = (G.nx + ZM_TX - 1) / ZM_TX, my = (G.ny + ZM_TY - 1) / ZM_TY, mz = (G.nz + ZM_ZC - 1) / ZM_ZC;
+        hipLaunchKernelGGL(les_tau_fp64_zm, dim3((unsigned)(mx * my * mz)), dim3(ZM_TX * ZM_TY), 0, st, G, ph, mac, range,
                            slot, tau, mx, my);
     }
     return hipGetLastError();
 }
 
-hipError_t launch_reduce_fp64(int nx, int ny, int nz, int64_t ns, const Phys& ph, const double* mac, const uint64_t* range_slot,
+hipError_t launch_reduce_fp64(const Grid& G, const Phys& ph, const double* mac, const uint64_t* range_slot,
                               double* work, hipStream_t st) {
-    Grid G{nx, ny, nz};
-    const int mx = (nx + ZM_TX - 1) / ZM_TX, my = (ny + ZM_TY - 1) / ZM_TY;
+    const int mx = (G.nx + ZM_TX - 1) / ZM_TX, my = (G.ny + ZM_TY - 1) / ZM_TY;
     // columns of up to 32 planes (the two halo planes cost 2 / zc), shorter where the
     // lattice would leave less than four workgroups per CU
-    const int64_t planes = (int64_t)mx * my * nz;
-    const int zc = (int)std::min<int64_t>(std::min(32, nz), std::max<int64_t>(1, planes / 1024));
-    const int64_t items = (int64_t)mx * my * ((nz + zc - 1) / zc);
+    const int64_t planes = (int64_t)mx * my * G.nz;
+    const int zc = (int)std::min<int64_t>(std::min(32, G.nz), std::max<int64_t>(1, planes / 1024));
+    const int64_t items = (int64_t)mx * my * ((G.nz + zc - 1) / zc);
     const int nblocks = (int)std::min<int64_t>(items, REDUCE_MAX_BLOCKS);
-    hipLaunchKernelGGL(reduce_fp64, dim3(nblocks), dim3(ZM_NT), 0, st, G, ns, ph, mac, work, mx, my, zc, items);
+    hipLaunchKernelGGL(reduce_fp64, dim3(nblocks), dim3(ZM_NT), 0, st, G, ph, mac, work, mx, my, zc, items);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(reduce_final, dim3(1), dim3(64 * NPART), 0, st, (const double*)work, nblocks, range_slot,
                        work + REDUCE_OUT);
+    return hipGetLastError();
+}
+
+hipError_t launch_pack_rows(int nx, int64_t rows, int64_t stride, const double* nodes, double* packed, hipStream_t st) {
+    hipLaunchKernelGGL(pack_rows<false>, dim3(nblk(nx * rows, 256)), dim3(256), 0, st, nx, rows, stride,
+                       const_cast<double*>(nodes), packed);
+    return hipGetLastError();
+}
+
+hipError_t launch_unpack_rows(int nx, int64_t rows, int64_t stride, const double* packed, double* nodes,
+                              hipStream_t st) {
+    hipLaunchKernelGGL(pack_rows<true>, dim3(nblk(nx * rows, 256)), dim3(256), 0, st, nx, rows, stride, nodes,
+                       const_cast<double*>(packed));
     return hipGetLastError();
 }
 

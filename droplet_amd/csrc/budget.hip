@@ -46,21 +46,11 @@ template <int Q0, int Q1, typename Fn> __device__ __forceinline__ void sfor(Fn&&
     }
 }
 
-struct BGrid {
-    int nx, ny, nz;
-    __device__ __forceinline__ int64_t at(int x, int y, int z) const {
-        x = x < 0 ? x + nx : (x >= nx ? x - nx : x);
-        y = y < 0 ? y + ny : (y >= ny ? y - ny : y);
-        z = z < 0 ? z + nz : (z >= nz ? z - nz : z);
-        return x + (int64_t)nx * (y + (int64_t)ny * z);
-    }
-};
-
 // component A of direction Q
 template <int Q, int A> constexpr int cdir() { return A == 0 ? Dir<Q>::cx : (A == 1 ? Dir<Q>::cy : Dir<Q>::cz); }
 
 // lap_cal and grad_cal of phi, grad of u (gu[k][a] = d_a u_k) at one node
-__device__ void stencils(const BGrid& G, const double* phi, const double* u1, const double* u2, const double* u3,
+__device__ void stencils(const Grid& G, const double* phi, const double* u1, const double* u2, const double* u3,
                          int x, int y, int z, double& lap, double gp[3], double gu[3][3]) {
     lap = -14.0 * phi[G.at(x, y, z)];
     for (int a = 0; a < 3; a++) {
@@ -92,12 +82,11 @@ __device__ void stencils(const BGrid& G, const double* phi, const double* u1, co
     }
 }
 
-__global__ __launch_bounds__(256) void derived_fp64(BGrid G, int64_t ns, Phys P, const double* __restrict__ mac, int kind,
+__global__ __launch_bounds__(256) void derived_fp64(Grid G, Phys P, const double* __restrict__ mac, int kind,
                                                     double* __restrict__ out, int64_t pitch) {
-    const int64_t n = (int64_t)G.nx * G.ny * G.nz;
-    const int64_t s = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (s >= n) return;
-    const int x = (int)(s % G.nx), y = (int)((s / G.nx) % G.ny), z = (int)(s / ((int64_t)G.nx * G.ny));
+    const int64_t ns = G.ns, s = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    const int x = (int)(s % G.px), y = (int)((s / G.px) % G.ny), z = (int)(s / ((int64_t)G.px * G.ny));
+    if (x >= G.nx || z >= G.nz) return;
     double* const o = out + x + pitch * (y + (int64_t)G.ny * z);  // row pitch of the result
     const double ph = mac[s];
     if (kind == DRP_DERIVED_FREE_ENERGY) {
@@ -131,7 +120,7 @@ constexpr int BTX = 64, BTY = 4, BZC = 16;
 constexpr int BT = BTX * BTY, NW = BT / 64;  // threads and wavefronts per workgroup
 
 struct BudgetArgs {
-    BGrid G;
+    Grid G;
     Phys P;
     const double* old_mac;
     const double* new_mac;
@@ -140,8 +129,7 @@ struct BudgetArgs {
     const double *sinx, *cosx, *sinz, *cosz;   // Taylor-Green tables of the step, or null
     double tg_amp;
     double* work;     // [BWORK][ws]
-    int64_t ns;       // stride of the fields
-    int64_t ws;       // stride of the work arrays (n)
+    int64_t ws;       // stride of the work arrays (G.slots())
     double* partial;  // [blocks][BPART]
 };
 
@@ -181,7 +169,7 @@ struct Brick {
     int x, y, z0, z1;
     bool live;  // x < nx and y < ny
 };
-__device__ __forceinline__ Brick brick(const BGrid& G) {
+__device__ __forceinline__ Brick brick(const Grid& G) {
     const int bx = (G.nx + BTX - 1) / BTX, by = (G.ny + BTY - 1) / BTY;
     const int t = xcd_tile(blockIdx.x, gridDim.x);
     const int tx = t % bx, ty = (t / bx) % by, tz = t / (bx * by);
@@ -208,16 +196,16 @@ __device__ __forceinline__ int wrap_any(int v, int n) {  // v in [-1, n + BTX]
 // plane z of the NA arrays src(k) over the brick at (x0, y0) and its halo, into
 // registers (ring_per_thread<NA>() per thread)
 template <int NA, typename Src>
-__device__ __forceinline__ void ring_fetch(const BGrid& G, int x0, int y0, int z, Src&& src,
+__device__ __forceinline__ void ring_fetch(const Grid& G, int x0, int y0, int z, Src&& src,
                                            double (&r)[ring_per_thread<NA>()]) {
-    const int64_t zo = (int64_t)G.nx * G.ny * wrap_any(z, G.nz);
+    const int64_t zo = (int64_t)G.px * G.ny * wrap_any(z, G.nz);
 #pragma unroll
     for (int j = 0; j < ring_per_thread<NA>(); j++) {
         const int i = (int)threadIdx.x + BT * j;
         if (i < NA * RN) {
             const int k = i / RN, c = i - k * RN, ly = c / RX, lx = c - ly * RX;
             const int gx = wrap_any(x0 - 1 + lx, G.nx), gy = wrap_any(y0 - 1 + ly, G.ny);
-            r[j] = src(k)[zo + gx + (int64_t)G.nx * gy];
+            r[j] = src(k)[zo + gx + (int64_t)G.px * gy];
         }
     }
 }
@@ -267,9 +255,9 @@ __device__ __forceinline__ void stencils_ring(const double* const (&sl)[3], doub
 }
 
 __global__ __launch_bounds__(BT) __attribute__((amdgpu_waves_per_eu(4))) void budget_pass1(BudgetArgs a) {
-    const BGrid& G = a.G;
+    const Grid& G = a.G;
     const Phys& P = a.P;
-    const int64_t n = a.ns;
+    const int64_t n = G.ns;
     const Brick b = brick(G);
     // ring of the old phi, u1, u2, u3
     constexpr int NA1 = 4;
@@ -295,7 +283,7 @@ __global__ __launch_bounds__(BT) __attribute__((amdgpu_waves_per_eu(4))) void bu
         // branch would run twice in a wavefront whose lanes take both paths
         if (b.live) {
             const int x = b.x, y = b.y;
-            const int64_t s = x + (int64_t)G.nx * (y + (int64_t)G.ny * z);
+            const int64_t s = G.node(x, y, z);
             const double* nm = a.new_mac;
             const double* sl[3] = {ring[j % 3] + me, ring[(j + 1) % 3] + me, ring[(j + 2) % 3] + me};
             double lap, gp[3], gu[3][3];
@@ -342,9 +330,9 @@ constexpr int NA2 = 8;
 enum { R_K = 0, R_V = 1, R_GP = 4, R_P = 7 };
 
 __global__ __launch_bounds__(BT) void budget_pass2(BudgetArgs a) {
-    const BGrid& G = a.G;
+    const Grid& G = a.G;
     const Phys& P = a.P;
-    const int64_t n = a.ns;
+    const int64_t n = G.ns;
     const Brick b = brick(G);
     __shared__ double ring[3][NA2 * RN];
     const int lx = (int)threadIdx.x % BTX, ly = (int)threadIdx.x / BTX;
@@ -404,7 +392,7 @@ __global__ __launch_bounds__(BT) void budget_pass2(BudgetArgs a) {
                     asm volatile("" : "+v"(aG[0][A]), "+v"(aG[1][A]), "+v"(aG[2][A]));
                 }
             });
-            const int64_t s = b.x + (int64_t)G.nx * (b.y + (int64_t)G.ny * z);
+            const int64_t s = G.node(b.x, b.y, z);
             const double* nm = a.new_mac;
             const double u[3] = {nm[2 * n + s], nm[3 * n + s], nm[4 * n + s]};
             v[1] += u[0] * (aK[0] / 10.0) + u[1] * (aK[1] / 10.0) + u[2] * (aK[2] / 10.0);
@@ -441,10 +429,10 @@ __global__ __launch_bounds__(BT) void budget_pass2(BudgetArgs a) {
 
 }  // namespace
 
-hipError_t launch_derived_fp64(int nx, int ny, int nz, int64_t ns, const Phys& ph, const double* mac, int kind, double* out,
-                               int64_t pitch, hipStream_t st) {
-    const int64_t n = (int64_t)nx * ny * nz;
-    hipLaunchKernelGGL(derived_fp64, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, BGrid{nx, ny, nz}, ns, ph, mac,
+hipError_t launch_derived_fp64(const Grid& G, const Phys& ph, const double* mac, int kind, double* out, int64_t pitch,
+                               hipStream_t st) {
+    const int64_t n = G.slots();
+    hipLaunchKernelGGL(derived_fp64, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, G, ph, mac,
                        kind, out, pitch);
     return hipGetLastError();
 }
@@ -468,7 +456,7 @@ extern "C" int drp_get_derived(drp_lattice* L, int kind, double* host, size_t n_
     }
     double* out = nullptr;
     HIP_TRYB(hipMalloc((void**)&out, (size_t)L->n * sizeof(double)));
-    hipError_t e = launch_derived_fp64(L->cfg.nx, L->cfg.ny, L->cfg.nz, L->ns, L->phys, mac, kind, out, L->cfg.nx, L->stream);
+    hipError_t e = launch_derived_fp64(L->G, L->phys, mac, kind, out, L->cfg.nx, L->stream);
     if (e == hipSuccess) e = hipMemcpyAsync(host, out, (size_t)L->n * sizeof(double), hipMemcpyDeviceToHost, L->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(L->stream);
     const hipError_t f = hipFree(out);
@@ -483,17 +471,17 @@ extern "C" int drp_step_energy_budget(drp_lattice* L, double* terms) {
     const drp_config& c = L->cfg;
     if (c.precision != DRP_FP64) return drp_fail(DRP_ERR_UNSUPPORTED, "energy budget: FP64 lattices only");
     if (c.model != DRP_MODEL_FREE_ENERGY) return drp_fail(DRP_ERR_UNSUPPORTED, "energy budget: free-energy model only");
-    const int64_t n = L->n;
+    const int64_t ws = L->G.slots();
     const int64_t nb = budget_bricks(c.nx, c.ny, c.nz);
     if (!L->budget) {
-        HIP_TRYB(hipMalloc((void**)&L->budget, ((size_t)BWORK * n + (size_t)nb * BPART) * sizeof(double)));
+        HIP_TRYB(hipMalloc((void**)&L->budget, ((size_t)BWORK * ws + (size_t)nb * BPART) * sizeof(double)));
     }
     // the body force the step will use (its pointers do not depend on the ping-pong parity)
     const StepArgs sa = make_step_args(L, L->step + 1);
     int rc = drp_step(L, 1);
     if (rc) return rc;
     BudgetArgs a{};
-    a.G = BGrid{c.nx, c.ny, c.nz};
+    a.G = L->G;
     a.P = L->phys;
     a.old_mac = (const double*)L->mac[1 - L->cur];
     a.new_mac = (const double*)L->mac[L->cur];
@@ -510,8 +498,7 @@ extern "C" int drp_step_energy_budget(drp_lattice* L, double* terms) {
         a.tg_amp = sa.tg_amp;
     }
     a.work = L->budget;
-    a.ns = L->ns;
-    a.ws = n;
+    a.ws = ws;
     a.partial = L->budget + (size_t)BWORK * a.ws;
     hipLaunchKernelGGL(budget_pass1, dim3((unsigned)nb), dim3(BT), 0, L->stream, a);
     HIP_TRYB(hipGetLastError());

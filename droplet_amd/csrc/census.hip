@@ -65,11 +65,13 @@ __device__ void unite(int* lab, int a, int b) {
     }
 }
 
-__global__ __launch_bounds__(256) void cc_init(const double* __restrict__ phi, double thr, int n,
+__global__ __launch_bounds__(256) void cc_init(const double* __restrict__ phi, drp::Grid G, double thr, int n,
                                                int* __restrict__ lab, int* __restrict__ vol) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    lab[i] = phi[i] >= thr ? i : -1;
+    // labels are node numbers x + nx (y + ny z); phi lies in rows px apart
+    const int row = i / G.nx, x = i - row * G.nx;
+    lab[i] = phi[x + (int64_t)G.px * row] >= thr ? i : -1;
     vol[i] = 0;
 }
 
@@ -150,7 +152,7 @@ extern "C" int drp_droplet_census(drp_lattice* L, double threshold, int64_t* cou
     int* rec = vol + N;          // 2 (N / 2 + 1) ints
     int* counter = rec + 2 * (N / 2 + 1);
     const hipStream_t st = L->stream;
-    hipLaunchKernelGGL(cc_init, blocks(N), dim3(256), 0, st, phi, threshold, N, lab, vol);
+    hipLaunchKernelGGL(cc_init, blocks(N), dim3(256), 0, st, phi, L->G, threshold, N, lab, vol);
     hipLaunchKernelGGL(cc_union, blocks(N), dim3(256), 0, st, L->cfg.nx, L->cfg.ny, L->cfg.nz, lab);
     hipLaunchKernelGGL(cc_flatten, blocks(N), dim3(256), 0, st, N, lab, vol);
     hipLaunchKernelGGL(cc_zero, dim3(1), dim3(1), 0, st, counter);

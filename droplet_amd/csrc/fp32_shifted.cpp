@@ -39,18 +39,19 @@ struct DevBuf {
 };
 
 int fp32_init_from_host_fields(drp_lattice* L, const double* const* host) {
-    const int64_t n = L->n, ns = L->ns;
+    const int64_t ns = L->G.ns;
     DevBuf mac64, pop64;
     HIP_TRY32(hipMalloc(&mac64.p, 5 * ns * sizeof(double)));
     HIP_TRY32(hipMalloc(&pop64.p, 30 * ns * sizeof(double)));
     double* m = (double*)mac64.p;
     double* f = (double*)pop64.p;
-    for (int k = 0; k < 5; k++)
-        HIP_TRY32(hipMemcpyAsync(m + k * ns, host[k], n * sizeof(double), hipMemcpyHostToDevice, L->stream));
-    HIP_TRY32(launch_init_equilibrium_fp64(L->cfg.nx, L->cfg.ny, L->cfg.nz, ns, L->phys, m, f, f + 15 * ns, L->stream));
-    HIP_TRY32(launch_to_shifted(n, ns, shift_ref(L->cfg), f, m, (float*)L->pop[L->cur], (float*)L->mac[L->cur],
+    int rc = DRP_OK;
+    for (int k = 0; k < 5 && !rc; k++) rc = nodes_from_host(L, host[k], 1, m + k * ns);
+    if (rc) return rc;
+    HIP_TRY32(launch_init_equilibrium_fp64(L->G, L->phys, m, f, f + 15 * ns, L->stream));
+    HIP_TRY32(launch_to_shifted(L->G, shift_ref(L->cfg), f, m, (float*)L->pop[L->cur], (float*)L->mac[L->cur],
                                 L->stream));
-    int rc = reset_range(L);
+    rc = reset_range(L);
     if (rc) return rc;
     HIP_TRY32(hipStreamSynchronize(L->stream));
     L->step = 0;
@@ -61,12 +62,12 @@ int fp32_init_from_host_fields(drp_lattice* L, const double* const* host) {
 StepArgs32 make_step_args32(drp_lattice* L, int64_t nstep) {
     const drp_config& c = L->cfg;
     const Phys& P = L->phys;
-    const int64_t n = L->ns;  // from one array to the next
+    const int64_t n = L->G.ns;  // from one array to the next
     StepArgs32 a{};
     a.nx = c.nx;
     a.ny = c.ny;
     a.nz = c.nz;
-    a.n = L->n;
+    a.px = L->G.px;
     a.ns = n;
     float* fi = (float*)L->pop[L->cur];
     float* fo = (float*)L->pop[1 - L->cur];
@@ -130,8 +131,8 @@ int fp32_step(drp_lattice* L, int nsteps) {
 }
 
 int fp32_macro_fp64_view(drp_lattice* L, const double** mac) {
-    if (!L->mac64) HIP_TRY32(hipMalloc((void**)&L->mac64, 5 * L->ns * sizeof(double)));
-    HIP_TRY32(launch_macro_from_shifted(L->n, L->ns, L->cfg.phi1, (const float*)L->mac[L->cur], L->mac64, L->stream));
+    if (!L->mac64) HIP_TRY32(hipMalloc((void**)&L->mac64, 5 * L->G.ns * sizeof(double)));
+    HIP_TRY32(launch_macro_from_shifted(L->G, L->cfg.phi1, (const float*)L->mac[L->cur], L->mac64, L->stream));
     *mac = L->mac64;
     return DRP_OK;
 }
@@ -140,28 +141,25 @@ int fp32_get_macro(drp_lattice* L, int field, double* host) {
     const double* m = nullptr;
     int rc = fp32_macro_fp64_view(L, &m);
     if (rc) return rc;
-    HIP_TRY32(hipMemcpyAsync(host, m + field * L->ns, L->n * sizeof(double), hipMemcpyDeviceToHost, L->stream));
-    HIP_TRY32(hipStreamSynchronize(L->stream));
-    return DRP_OK;
+    return nodes_to_host(L, m + field * L->G.ns, 1, host);
 }
 
 int fp32_get_populations(drp_lattice* L, int set, double* host) {
     DevBuf tmp;
-    HIP_TRY32(hipMalloc(&tmp.p, 15 * L->n * sizeof(double)));
-    HIP_TRY32(launch_pops_from_shifted(L->n, L->ns, shift_ref(L->cfg), (const float*)L->pop[L->cur], (double*)tmp.p, set,
+    HIP_TRY32(hipMalloc(&tmp.p, 15 * L->G.ns * sizeof(double)));
+    HIP_TRY32(launch_pops_from_shifted(L->G, shift_ref(L->cfg), (const float*)L->pop[L->cur], (double*)tmp.p, set,
                                        L->stream));
-    HIP_TRY32(hipMemcpyAsync(host, tmp.p, 15 * L->n * sizeof(double), hipMemcpyDeviceToHost, L->stream));
-    HIP_TRY32(hipStreamSynchronize(L->stream));
-    return DRP_OK;
+    return nodes_to_host(L, (const double*)tmp.p, 15, host);
 }
 
 int fp32_set_populations(drp_lattice* L, int set, const double* host, int which) {
     DevBuf tmp;
-    HIP_TRY32(hipMalloc(&tmp.p, 15 * L->n * sizeof(double)));
-    HIP_TRY32(hipMemcpyAsync(tmp.p, host, 15 * L->n * sizeof(double), hipMemcpyHostToDevice, L->stream));
+    HIP_TRY32(hipMalloc(&tmp.p, 15 * L->G.ns * sizeof(double)));
+    const int rc = nodes_from_host(L, host, 15, (double*)tmp.p);
+    if (rc) return rc;
     float* pop = (float*)L->pop[L->cur];
-    HIP_TRY32(launch_pops_to_shifted(L->n, L->ns, shift_ref(L->cfg), (const double*)tmp.p, pop, set, L->stream));
-    HIP_TRY32(launch_moments_fp32(L->n, L->ns, pop, pop + 15 * L->ns, (float*)L->mac[L->cur], which, L->stream));
+    HIP_TRY32(launch_pops_to_shifted(L->G, shift_ref(L->cfg), (const double*)tmp.p, pop, set, L->stream));
+    HIP_TRY32(launch_moments_fp32(L->G, pop, pop + 15 * L->G.ns, (float*)L->mac[L->cur], which, L->stream));
     HIP_TRY32(hipStreamSynchronize(L->stream));
     return DRP_OK;
 }

@@ -15,6 +15,27 @@ __device__ __forceinline__ int xcd_tile(int b, int nb) {
     if ((nb & 7) != 0) return b;
     return (b & 7) * (nb >> 3) + (b >> 3);
 }
+// How the node arrays of a lattice lie in memory: rows of nx elements px apart
+// (px >= nx), arrays ns apart.  What lies between rows and arrays is never read as
+// a node.
+struct Grid {
+    int nx, ny, nz;
+    int px;      // elements from one x row to the next
+    int64_t ns;  // elements from one array to the next
+    // elements of one array, row padding included
+    __host__ __device__ __forceinline__ int64_t slots() const { return (int64_t)px * ny * nz; }
+    __host__ __device__ __forceinline__ int64_t node(int x, int y, int z) const {
+        return x + (int64_t)px * (y + (int64_t)ny * z);
+    }
+    // node of coordinates up to one period outside the lattice (periodic wrap)
+    __device__ __forceinline__ int64_t at(int x, int y, int z) const {
+        x = x < 0 ? x + nx : (x >= nx ? x - nx : x);
+        y = y < 0 ? y + ny : (y >= ny ? y - ny : y);
+        z = z < 0 ? z + nz : (z >= nz ? z - nz : z);
+        return node(x, y, z);
+    }
+};
+
 // batched launch: per-instance step arguments and first-tile offsets in device memory
 struct BatchLaunch {
     const void* args;      // StepArgs[ninst] or StepArgs32[ninst]
@@ -53,7 +74,7 @@ struct Phys {
 struct StepArgs {
     int nx, ny, nz;
     int tiles_x, tiles_y, tiles_z;
-    int64_t n;
+    int px;               // row pitch (Grid)
     int64_t ns;           // elements from one population, field or force array to the next
     const double* f_in;   // [15][ns] phi populations (reference f)
     const double* g_in;   // [15][ns] momentum populations (reference g)
@@ -87,15 +108,13 @@ struct StepArgs {
 
 hipError_t launch_step_fp64(const StepArgs& a, int shape, hipStream_t st, const BatchLaunch* batch = nullptr);
 
-// ns in the launchers below: elements from one population or field array to the next
-// (lattice_impl.h); arrays for the host are n apart
-
 // FP32 shifted storage (step_fp32.hip): populations and fields as FP32
 // deviations from the continuous phase at rest
 struct StepArgs32 {
     int nx, ny, nz;
     int tiles_x, tiles_y, tiles_z;
-    int64_t n, ns;
+    int px;
+    int64_t ns;
     const float* f_in;
     const float* g_in;
     float* f_out;
@@ -129,32 +148,31 @@ struct ShiftRef {
     double fr[15];
     double phi1;
 };
-hipError_t launch_to_shifted(int64_t n, int64_t ns, const ShiftRef& r, const double* pop64, const double* mac64, float* pop32,
+hipError_t launch_to_shifted(const Grid& G, const ShiftRef& r, const double* pop64, const double* mac64, float* pop32,
                              float* mac32, hipStream_t st);
-hipError_t launch_pops_from_shifted(int64_t n, int64_t ns, const ShiftRef& r, const float* pop32, double* pop64, int set,
+hipError_t launch_pops_from_shifted(const Grid& G, const ShiftRef& r, const float* pop32, double* pop64, int set,
                                     hipStream_t st);
-hipError_t launch_pops_to_shifted(int64_t n, int64_t ns, const ShiftRef& r, const double* pop64, float* pop32, int set,
+hipError_t launch_pops_to_shifted(const Grid& G, const ShiftRef& r, const double* pop64, float* pop32, int set,
                                   hipStream_t st);
-hipError_t launch_macro_from_shifted(int64_t n, int64_t ns, double phi1, const float* mac32, double* mac64, hipStream_t st);
-hipError_t launch_moments_fp32(int64_t n, int64_t ns, const float* f, const float* g, float* mac, int which, hipStream_t st);
-hipError_t launch_les_tau_fp32(int nx, int ny, int nz, int64_t ns, const Phys& ph, const float* mac, const float* mac_old,
+hipError_t launch_macro_from_shifted(const Grid& G, double phi1, const float* mac32, double* mac64, hipStream_t st);
+hipError_t launch_moments_fp32(const Grid& G, const float* f, const float* g, float* mac, int which, hipStream_t st);
+hipError_t launch_les_tau_fp32(const Grid& G, const Phys& ph, const float* mac, const float* mac_old,
                                const LesBlocks& blk, const uint64_t* range, int slot, float* tau, hipStream_t st);
 
 // populations := equilibria of the macroscopic fields (ini, program/lbm_drop_xy.f90:244-251)
-hipError_t launch_init_equilibrium_fp64(int nx, int ny, int nz, int64_t ns, const Phys& ph, const double* mac, double* f,
+hipError_t launch_init_equilibrium_fp64(const Grid& G, const Phys& ph, const double* mac, double* f,
                                         double* g, hipStream_t st);
 // recompute moments from populations: which & 1 -> phi from f, which & 2 -> p, u from g
-hipError_t launch_moments_fp64(int nx, int ny, int nz, int64_t ns, const double* f, const double* g, double* mac, int which,
+hipError_t launch_moments_fp64(const Grid& G, const double* f, const double* g, double* mac, int which,
                                hipStream_t st);
 // Smagorinsky tau field for the next step (program/LES_drop.f90:598-693) from the
 // state a step left (mac), the one it started from (mac_old, read across rank
 // blocks) and that step's phi range slot
-hipError_t launch_les_tau_fp64(int nx, int ny, int nz, int64_t ns, const Phys& ph, const double* mac, const double* mac_old,
+hipError_t launch_les_tau_fp64(const Grid& G, const Phys& ph, const double* mac, const double* mac_old,
                                const LesBlocks& blk, const uint64_t* range, int slot, double* tau, hipStream_t st);
 // derived fields of the analysis programs (budget.hip): kind = DRP_DERIVED_*; rows of
 // the result `pitch` doubles apart
-hipError_t launch_derived_fp64(int nx, int ny, int nz, int64_t ns, const Phys& ph, const double* mac, int kind, double* out,
-                               int64_t pitch, hipStream_t st);
+hipError_t launch_derived_fp64(const Grid& G, const Phys& ph, const double* mac, int kind, double* out, int64_t pitch, hipStream_t st);
 
 // diagnostics sums: NPART doubles per workgroup (at most REDUCE_MAX_BLOCKS), then at
 // work[REDUCE_OUT] the NPART total sums and the two words of the phi range slot
@@ -162,8 +180,12 @@ constexpr int NPART = 10;
 constexpr int REDUCE_MAX_BLOCKS = 2048;
 constexpr int REDUCE_OUT = REDUCE_MAX_BLOCKS * NPART;
 constexpr int REDUCE_WORK_DOUBLES = REDUCE_OUT + 16;
-hipError_t launch_reduce_fp64(int nx, int ny, int nz, int64_t ns, const Phys& ph, const double* mac, const uint64_t* range_slot,
+hipError_t launch_reduce_fp64(const Grid& G, const Phys& ph, const double* mac, const uint64_t* range_slot,
                               double* work, hipStream_t st);
+// rows of nx doubles, `stride` apart in node arrays, to contiguous rows, and back
+hipError_t launch_pack_rows(int nx, int64_t rows, int64_t stride, const double* nodes, double* packed, hipStream_t st);
+hipError_t launch_unpack_rows(int nx, int64_t rows, int64_t stride, const double* packed, double* nodes,
+                              hipStream_t st);
 // fill a range slot with (max, min) = (vmax, vmin)
 hipError_t launch_range_set(uint64_t* range, int slot, double vmax, double vmin, hipStream_t st);
 
@@ -175,21 +197,20 @@ struct SpectralWork {
 };
 size_t spectral_work_doubles(int nx, int ny, int nz, int kc);
 void spectral_work_layout(SpectralWork& w, double* base, int nx, int ny, int nz, int kc);
-hipError_t launch_spectral_force(const SpectralWork& w, int nx, int ny, int nz, int kc, double eps, const double* u1,
+hipError_t launch_spectral_force(const SpectralWork& w, const Grid& G, int kc, double eps, const double* u1,
                                  const double* u2, const double* u3, double* fx, double* fy, double* fz,
                                  hipStream_t st);
-hipError_t launch_spectral_force(const SpectralWork& w, int nx, int ny, int nz, int kc, double eps, const float* u1,
+hipError_t launch_spectral_force(const SpectralWork& w, const Grid& G, int kc, double eps, const float* u1,
                                  const float* u2, const float* u3, double* fx, double* fy, double* fz,
                                  hipStream_t st);
 // band-pass of u keeping the shells klo <= int|k| < khi (2 <= khi <= 5; work space of kc = khi)
-hipError_t launch_spectral_band(const SpectralWork& w, int nx, int ny, int nz, int klo, int khi, const double* u1,
+hipError_t launch_spectral_band(const SpectralWork& w, const Grid& G, int klo, int khi, const double* u1,
                                 const double* u2, const double* u3, double* o1, double* o2, double* o3,
                                 hipStream_t st);
 
 // adjoint.hip: one reverse step of the FP64 step (equal viscosities, no LES)
 struct AdjArgs {
-    int nx, ny, nz;
-    int64_t n, ns;
+    Grid G;
     const double* f;        // forward phi populations at step n (15 ns)
     const double* mac;      // forward macroscopic fields at step n (5 ns)
     const double* Fin;      // adjoint of f^{n+1} without its stencil part (15 ns)
@@ -207,13 +228,13 @@ struct AdjArgs {
     int wall_active;        // the walls move during step n -> n+1
     int first;              // step n is the initial equilibrium of constant fields
 };
-int adj_block_count(int64_t n);
+int adj_block_count(const Grid& G);
 hipError_t launch_adj_collide_fp64(const AdjArgs& a, hipStream_t st);
-hipError_t launch_adj_stencil_fp64(int nx, int ny, int nz, int64_t ns, const double* lapA, const double* gradA, double* out,
+hipError_t launch_adj_stencil_fp64(const Grid& G, const double* lapA, const double* gradA, double* out,
                                    hipStream_t st);
-hipError_t launch_adj_seed_area_fp64(int nx, int ny, int nz, int64_t ns, const double* phi, double w, double* lapA,
+hipError_t launch_adj_seed_area_fp64(const Grid& G, const double* phi, double w, double* lapA,
                                      double* gradA, hipStream_t st);
-hipError_t launch_adj_add_plane(int nx, int ny, int n1, int n2, int wall_y, int third, const double* vals,
+hipError_t launch_adj_add_plane(const Grid& G, int n1, int n2, int wall_y, int third, const double* vals,
                                 double* out, hipStream_t st);
 
 }  // namespace drp

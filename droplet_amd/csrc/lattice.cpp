@@ -86,32 +86,83 @@ Phys make_phys(const drp_config& c) {
     return p;
 }
 
+// Row pitch.  With rows that are no multiple of a 64-byte memory sector the step's
+// non-temporal stores leave partial sectors at both ends of every tile row: 190 x 121
+// x 150 took 732 us (FP64) and 493 us (FP32) where 192 x 121 x 150 takes 469 and 245,
+// 131 x 70 x 97 218 us where 136 x 70 x 97 takes 153; with ordinary loads and stores
+// 602 and 353 us.  Rows are padded to the next 64 bytes (200 x 121 x 150, such rows:
+// 6600 MLUPS in FP64, 128-byte rows 7400, 16-byte rows 4500), and to 128 bytes where
+// that costs at most 1/16; not at all where they would grow by more than a quarter,
+// nor where one tile spans the row (32 nodes) and writes it whole together with its
+// neighbours (28 x 100 x 100: 47 us as it is, 55 padded; 33 x 100 x 100: 87 and 82).
+static int row_pitch(int nx, int ny, size_t esz) {
+    auto up = [&](int bytes) { return (int64_t)((nx * (int64_t)esz + bytes - 1) / bytes * bytes / (int64_t)esz); };
+    int64_t px = up(128);
+    if (16 * px > 17 * (int64_t)nx) px = up(64);
+    if (nx <= 32 || 4 * px > 5 * (int64_t)nx || px * ny >= (int64_t)1 << 31) px = nx;
+    return (int)px;
+}
+
 // Elements from one population (or field) array to the next.  A step reads and
-// writes 70 arrays of n at the same offset in each; where n times the element size
-// is a large power of two they meet in the same memory channels.  Arrays of 1 MiB
-// and more therefore start on 256-byte boundaries (whole lines also on odd grids)
-// and 8 KiB + 256 B further apart than their length.  MLUPS of the shear droplet,
-// arrays back to back -> apart: FP64 128^3 5040..6080 -> 8070, 192^3 7860 -> 8240,
-// 256^3 8130 -> 8350, 131 x 70 x 97 3790 -> 4120; FP32 128^3 14030 -> 15050,
-// 256^3 14730 -> 15850; 240^3 unchanged.  Of 0, 256, 512 .. 4096, 4352, 8448, 16640,
-// 64 KiB, 1 MiB and 2 MiB + 4352 B this is the best or within 2 % of it at all of
-// these.  Shorter arrays stay back to back: they live in the caches, and one copy
-// moves a whole population set to the host.
-static int64_t stream_stride(int64_t n, size_t esz) {
-    const int64_t bytes = n * (int64_t)esz;
-    if (bytes < ((int64_t)1 << 20)) return n;
+// writes 70 arrays at the same offset in each; where their length is a large power
+// of two they meet in the same memory channels.  Arrays of 1 MiB and more therefore
+// start on 256-byte boundaries and 8 KiB + 256 B further apart than their length.
+// MLUPS of the shear droplet, arrays back to back -> apart: FP64 128^3 5040..6080 ->
+// 8070, 192^3 7860 -> 8240, 256^3 8130 -> 8350; FP32 128^3 14030 -> 15050, 256^3
+// 14730 -> 15850; 240^3 unchanged.  Of 0, 256, 512 .. 4096, 4352, 8448, 16640, 64 KiB,
+// 1 MiB and 2 MiB + 4352 B this is the best or within 2 % of it at all of these.
+// Shorter arrays stay back to back: they live in the caches, and one copy moves a
+// whole population set to the host.
+static int64_t stream_stride(int64_t slots, size_t esz) {
+    const int64_t bytes = slots * (int64_t)esz;
+    if (bytes < ((int64_t)1 << 20)) return slots;
     return ((bytes + 255) / 256 * 256 + 8192 + 256) / (int64_t)esz;
 }
 
-// `count` arrays of n doubles, ds and ss doubles apart, in one copy where they are contiguous
-static hipError_t copy_streams(double* dst, int64_t ds, const double* src, int64_t ss, int count, int64_t n,
-                               hipMemcpyKind kind, hipStream_t st) {
-    if (ds == n && ss == n) return hipMemcpyAsync(dst, src, count * n * sizeof(double), kind, st);
-    for (int k = 0; k < count; k++) {
-        const hipError_t e = hipMemcpyAsync(dst + k * ds, src + k * ss, n * sizeof(double), kind, st);
-        if (e != hipSuccess) return e;
+static Grid choose_layout(const drp_config& c, bool pad_rows) {
+    const size_t esz = c.precision == DRP_FP64 ? sizeof(double) : sizeof(float);
+    Grid G{c.nx, c.ny, c.nz, pad_rows ? row_pitch(c.nx, c.ny, esz) : c.nx, 0};
+    G.ns = stream_stride(G.slots(), esz);
+    return G;
+}
+
+// One array at a time through a buffer without row padding, or straight where the
+// rows have none; in one copy where the arrays are back to back too.
+int nodes_to_host(drp_lattice* L, const double* nodes, int count, double* host) {
+    const Grid& G = L->G;
+    const size_t n = (size_t)L->n;
+    if (G.px == G.nx && (G.ns == L->n || count == 1)) {
+        HIP_TRY(hipMemcpyAsync(host, nodes, count * n * sizeof(double), hipMemcpyDeviceToHost, L->stream));
+    } else {
+        if (G.px != G.nx && !L->pack) HIP_TRY(hipMalloc((void**)&L->pack, n * sizeof(double)));
+        for (int k = 0; k < count; k++) {
+            const double* src = nodes + k * G.ns;
+            if (G.px != G.nx) {
+                HIP_TRY(launch_pack_rows(G.nx, (int64_t)G.ny * G.nz, G.px, src, L->pack, L->stream));
+                src = L->pack;
+            }
+            HIP_TRY(hipMemcpyAsync(host + k * n, src, n * sizeof(double), hipMemcpyDeviceToHost, L->stream));
+        }
     }
-    return hipSuccess;
+    HIP_TRY(hipStreamSynchronize(L->stream));
+    return DRP_OK;
+}
+
+int nodes_from_host(drp_lattice* L, const double* host, int count, double* nodes) {
+    const Grid& G = L->G;
+    const size_t n = (size_t)L->n;
+    if (G.px == G.nx && (G.ns == L->n || count == 1)) {
+        HIP_TRY(hipMemcpyAsync(nodes, host, count * n * sizeof(double), hipMemcpyHostToDevice, L->stream));
+        return DRP_OK;
+    }
+    if (G.px != G.nx && !L->pack) HIP_TRY(hipMalloc((void**)&L->pack, n * sizeof(double)));
+    for (int k = 0; k < count; k++) {
+        double* dst = nodes + k * G.ns;
+        HIP_TRY(hipMemcpyAsync(G.px != G.nx ? L->pack : dst, host + k * n, n * sizeof(double), hipMemcpyHostToDevice,
+                               L->stream));
+        if (G.px != G.nx) HIP_TRY(launch_unpack_rows(G.nx, (int64_t)G.ny * G.nz, G.px, L->pack, dst, L->stream));
+    }
+    return DRP_OK;
 }
 
 static int validate(const drp_config* c) {
@@ -212,11 +263,25 @@ int lattice_create(const drp_config* cfg, hipStream_t stream, drp_lattice** out)
     L->cfg = *cfg;
     L->phys = make_phys(*cfg);
     L->n = (int64_t)cfg->nx * cfg->ny * cfg->nz;
-    L->ns = stream_stride(L->n, cfg->precision == DRP_FP64 ? sizeof(double) : sizeof(float));
+    L->G = choose_layout(*cfg, true);
     L->shape = pick_shape(*cfg);
     L->stream = stream;
     (void)hipGetDevice(&L->dev);
     rc = lattice_alloc(L);
+    if (rc == DRP_ERR_ALLOC && L->G.px != cfg->nx) {  // the row padding is a convenience: do without
+        lattice_free(L);
+        (void)hipGetLastError();  // the failed allocation is dealt with here
+        const int shape = L->shape, dev = L->dev;
+        *L = drp_lattice();
+        L->cfg = *cfg;
+        L->phys = make_phys(*cfg);
+        L->n = (int64_t)cfg->nx * cfg->ny * cfg->nz;
+        L->G = choose_layout(*cfg, false);
+        L->shape = shape;
+        L->stream = stream;
+        L->dev = dev;
+        rc = lattice_alloc(L);
+    }
     if (rc) {
         lattice_free(L);
         delete L;
@@ -233,7 +298,7 @@ extern "C" void drp_destroy(drp_lattice* L) {
 }
 
 int lattice_alloc(drp_lattice* L) {
-    const int64_t n = L->n, ns = L->ns;
+    const int64_t n = L->G.slots(), ns = L->G.ns;  // elements of one array, and from one to the next
     auto dalloc = [&](void** p, size_t bytes) -> int {
         if (hipMalloc(p, bytes) != hipSuccess) {
             *p = nullptr;
@@ -321,6 +386,7 @@ void lattice_free(drp_lattice* L) {
     if (L->spec_adv) (void)hipFree(L->spec_adv);
     if (L->uadv) (void)hipFree(L->uadv);
     if (L->tg) (void)hipFree(L->tg);
+    if (L->pack) (void)hipFree(L->pack);
     if (L->partial) (void)hipFree(L->partial);
     if (L->mac64) (void)hipFree(L->mac64);
     if (L->census) (void)hipFree(L->census);
@@ -355,7 +421,7 @@ int les_update_tau(drp_lattice* L, bool fresh) {
         // the step kernel keeps sqrt(Pi:Pi) itself; a state that replaced the
         // lattice's is an equilibrium or a restart: no non-equilibrium flux yet
         if (fresh)
-            for (int k = 0; k < 2; k++) HIP_TRY(hipMemsetAsync(L->qh[k], 0, (size_t)L->n * sizeof(double), L->stream));
+            for (int k = 0; k < 2; k++) HIP_TRY(hipMemsetAsync(L->qh[k], 0, (size_t)L->G.slots() * sizeof(double), L->stream));
         return DRP_OK;
     }
     LesBlocks B{0, 0, 0};
@@ -363,27 +429,26 @@ int les_update_tau(drp_lattice* L, bool fresh) {
     const int slot = (int)(L->step % 3);
     const int old = fresh ? L->cur : 1 - L->cur;
     if (c.precision == DRP_FP64)
-        HIP_TRY(launch_les_tau_fp64(c.nx, c.ny, c.nz, L->ns, L->phys, (const double*)L->mac[L->cur], (const double*)L->mac[old],
+        HIP_TRY(launch_les_tau_fp64(L->G, L->phys, (const double*)L->mac[L->cur], (const double*)L->mac[old],
                                     B, L->range, slot, L->tau, L->stream));
     else
-        HIP_TRY(launch_les_tau_fp32(c.nx, c.ny, c.nz, L->ns, L->phys, (const float*)L->mac[L->cur], (const float*)L->mac[old],
+        HIP_TRY(launch_les_tau_fp32(L->G, L->phys, (const float*)L->mac[L->cur], (const float*)L->mac[old],
                                     B, L->range, slot, (float*)L->tau, L->stream));
     return DRP_OK;
 }
 
 static int init_from_host_fields(drp_lattice* L, const double* const* host) {
-    const int64_t n = L->n;
     if (L->cfg.precision != DRP_FP64) {
         const int rc = fp32_init_from_host_fields(L, host);
         return rc ? rc : les_update_tau(L, true);
     }
-    for (int k = 0; k < 5; k++)
-        HIP_TRY(hipMemcpyAsync((double*)L->mac[L->cur] + k * L->ns, host[k], n * sizeof(double), hipMemcpyHostToDevice,
-                               L->stream));
+    const int64_t ns = L->G.ns;
+    int rc = DRP_OK;
+    for (int k = 0; k < 5 && !rc; k++) rc = nodes_from_host(L, host[k], 1, (double*)L->mac[L->cur] + k * ns);
+    if (rc) return rc;
     double* f = (double*)L->pop[L->cur];
-    HIP_TRY(launch_init_equilibrium_fp64(L->cfg.nx, L->cfg.ny, L->cfg.nz, L->ns, L->phys, (double*)L->mac[L->cur],
-                                         f, f + 15 * L->ns, L->stream));
-    int rc = reset_range(L);
+    HIP_TRY(launch_init_equilibrium_fp64(L->G, L->phys, (double*)L->mac[L->cur], f, f + 15 * ns, L->stream));
+    rc = reset_range(L);
     if (rc) return rc;
     HIP_TRY(hipStreamSynchronize(L->stream));
     L->step = 0;
@@ -455,12 +520,12 @@ extern "C" int drp_init_fields(drp_lattice* L, const double* phi, const double* 
 StepArgs make_step_args(drp_lattice* L, int64_t nstep) {
     const drp_config& c = L->cfg;
     const Phys& P = L->phys;
-    const int64_t n = L->ns;  // from one array to the next
+    const int64_t n = L->G.ns;  // from one array to the next
     StepArgs a{};
     a.nx = c.nx;
     a.ny = c.ny;
     a.nz = c.nz;
-    a.n = L->n;
+    a.px = L->G.px;
     a.ns = n;
     double* fi = (double*)L->pop[L->cur];
     double* fo = (double*)L->pop[1 - L->cur];
@@ -555,15 +620,15 @@ extern "C" int drp_step(drp_lattice* L, int nsteps) {
 int spectral_update(drp_lattice* L, int64_t nstep) {
     const drp_config& c = L->cfg;
     if (c.force_kind != DRP_FORCE_SPECTRAL || nstep < c.force_start) return DRP_OK;
-    const int64_t n = L->ns;
+    const int64_t n = L->G.ns;
     double *fx = L->force, *fy = L->force + n, *fz = L->force + 2 * n;
     if (c.precision == DRP_FP64) {
         const double* m = (const double*)L->mac[L->cur];
-        HIP_TRY(launch_spectral_force(L->specw, c.nx, c.ny, c.nz, (int)c.force_k, c.force_amp, m + 2 * n, m + 3 * n,
+        HIP_TRY(launch_spectral_force(L->specw, L->G, (int)c.force_k, c.force_amp, m + 2 * n, m + 3 * n,
                                       m + 4 * n, fx, fy, fz, L->stream));
     } else {
         const float* m = (const float*)L->mac[L->cur];
-        HIP_TRY(launch_spectral_force(L->specw, c.nx, c.ny, c.nz, (int)c.force_k, c.force_amp, m + 2 * n, m + 3 * n,
+        HIP_TRY(launch_spectral_force(L->specw, L->G, (int)c.force_k, c.force_amp, m + 2 * n, m + 3 * n,
                                       m + 4 * n, fx, fy, fz, L->stream));
     }
     return DRP_OK;
@@ -576,9 +641,9 @@ int spectral_update(drp_lattice* L, int64_t nstep) {
 int advect_update(drp_lattice* L, int64_t nstep) {
     const drp_config& c = L->cfg;
     if (c.advect_k_high == 0 || nstep < c.advect_start) return DRP_OK;
-    const int64_t n = L->ns;
+    const int64_t n = L->G.ns;
     const double* m = (const double*)L->mac[L->cur];
-    HIP_TRY(launch_spectral_band(L->specw_adv, c.nx, c.ny, c.nz, c.advect_k_low, c.advect_k_high, m + 2 * n,
+    HIP_TRY(launch_spectral_band(L->specw_adv, L->G, c.advect_k_low, c.advect_k_high, m + 2 * n,
                                  m + 3 * n, m + 4 * n, L->uadv, L->uadv + n, L->uadv + 2 * n, L->stream));
     return DRP_OK;
 }
@@ -599,10 +664,7 @@ extern "C" int drp_get_macro(drp_lattice* L, int field, double* host, size_t n) 
     if (n != (size_t)L->n) return drp_fail(DRP_ERR_ARG, "size %zu != %lld nodes", n, (long long)L->n);
     if (!L->initialized) return drp_fail(DRP_ERR_STATE, "lattice not initialised");
     if (L->cfg.precision != DRP_FP64) return fp32_get_macro(L, field, host);
-    HIP_TRY(hipMemcpyAsync(host, (const double*)L->mac[L->cur] + field * L->ns, n * sizeof(double),
-                           hipMemcpyDeviceToHost, L->stream));
-    HIP_TRY(hipStreamSynchronize(L->stream));
-    return DRP_OK;
+    return nodes_to_host(L, (const double*)L->mac[L->cur] + field * L->G.ns, 1, host);
 }
 
 extern "C" int drp_get_populations(drp_lattice* L, int set, double* host, size_t n) {
@@ -613,10 +675,7 @@ extern "C" int drp_get_populations(drp_lattice* L, int set, double* host, size_t
     if (n != 15 * (size_t)L->n) return drp_fail(DRP_ERR_ARG, "size %zu != 15 x %lld", n, (long long)L->n);
     if (!L->initialized) return drp_fail(DRP_ERR_STATE, "lattice not initialised");
     if (L->cfg.precision != DRP_FP64) return fp32_get_populations(L, set, host);
-    const double* src = (const double*)L->pop[L->cur] + (set == DRP_POP_MOM ? 15 * L->ns : 0);
-    HIP_TRY(copy_streams(host, L->n, src, L->ns, 15, L->n, hipMemcpyDeviceToHost, L->stream));
-    HIP_TRY(hipStreamSynchronize(L->stream));
-    return DRP_OK;
+    return nodes_to_host(L, (const double*)L->pop[L->cur] + (set == DRP_POP_MOM ? 15 * L->G.ns : 0), 15, host);
 }
 
 // Populations from the host, moments recomputed (which: 1 phi, 2 p and u).  A
@@ -634,11 +693,10 @@ static int set_pops(drp_lattice* L, int set, const double* host, size_t n, int w
         return rc || !replace ? rc : les_update_tau(L, true);
     }
     double* base = (double*)L->pop[L->cur];
-    double* dst = base + (set == DRP_POP_MOM ? 15 * L->ns : 0);
     L->eq_init = false;
-    HIP_TRY(copy_streams(dst, L->ns, host, L->n, 15, L->n, hipMemcpyHostToDevice, L->stream));
-    HIP_TRY(launch_moments_fp64(L->cfg.nx, L->cfg.ny, L->cfg.nz, L->ns, base, base + 15 * L->ns, (double*)L->mac[L->cur],
-                                which, L->stream));
+    const int rc = nodes_from_host(L, host, 15, base + (set == DRP_POP_MOM ? 15 * L->G.ns : 0));
+    if (rc) return rc;
+    HIP_TRY(launch_moments_fp64(L->G, base, base + 15 * L->G.ns, (double*)L->mac[L->cur], which, L->stream));
     HIP_TRY(hipStreamSynchronize(L->stream));
     return replace ? les_update_tau(L, true) : DRP_OK;
 }
@@ -656,8 +714,10 @@ extern "C" int drp_set_force(drp_lattice* L, const double* fx, const double* fy,
     if (L->cfg.force_kind != DRP_FORCE_FIELD) return drp_fail(DRP_ERR_STATE, "force_kind is not DRP_FORCE_FIELD");
     if (n != (size_t)L->n) return drp_fail(DRP_ERR_ARG, "size %zu != %lld nodes", n, (long long)L->n);
     const double* src[3] = {fx, fy, fz};
-    for (int k = 0; k < 3; k++)
-        HIP_TRY(hipMemcpyAsync(L->force + k * L->ns, src[k], n * sizeof(double), hipMemcpyHostToDevice, L->stream));
+    for (int k = 0; k < 3; k++) {
+        const int rc = nodes_from_host(L, src[k], 1, L->force + k * L->G.ns);
+        if (rc) return rc;
+    }
     HIP_TRY(hipStreamSynchronize(L->stream));
     return DRP_OK;
 }
@@ -667,9 +727,10 @@ extern "C" int drp_get_force(drp_lattice* L, double* fx, double* fy, double* fz,
     if (!L->force) return drp_fail(DRP_ERR_STATE, "no force field (force_kind is not FIELD or SPECTRAL)");
     if (n != (size_t)L->n) return drp_fail(DRP_ERR_ARG, "size %zu != %lld nodes", n, (long long)L->n);
     double* dst[3] = {fx, fy, fz};
-    for (int k = 0; k < 3; k++)
-        HIP_TRY(hipMemcpyAsync(dst[k], L->force + k * L->ns, n * sizeof(double), hipMemcpyDeviceToHost, L->stream));
-    HIP_TRY(hipStreamSynchronize(L->stream));
+    for (int k = 0; k < 3; k++) {
+        const int rc = nodes_to_host(L, L->force + k * L->G.ns, 1, dst[k]);
+        if (rc) return rc;
+    }
     return DRP_OK;
 }
 
@@ -686,7 +747,7 @@ extern "C" int drp_reduce(drp_lattice* L, drp_stats* st) {
         if (rc) return rc;
     }
     if (!L->partial) HIP_TRY(hipMalloc((void**)&L->partial, REDUCE_WORK_DOUBLES * sizeof(double)));
-    HIP_TRY(launch_reduce_fp64(L->cfg.nx, L->cfg.ny, L->cfg.nz, L->ns, L->phys, mac, L->range + 2 * (L->step % 3), L->partial,
+    HIP_TRY(launch_reduce_fp64(L->G, L->phys, mac, L->range + 2 * (L->step % 3), L->partial,
                                L->stream));
     double s[NPART + 2];
     HIP_TRY(hipMemcpyAsync(s, L->partial + REDUCE_OUT, sizeof s, hipMemcpyDeviceToHost, L->stream));

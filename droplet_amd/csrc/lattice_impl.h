@@ -14,15 +14,15 @@ struct drp_lattice {
     int dev = 0;
     hipStream_t stream = nullptr;
     bool owns_stream = false;   // false for members of a batch (shared stream)
-    int64_t n = 0;
-    int64_t ns = 0;        // elements from one population, field or force array to the next (stream_stride)
+    int64_t n = 0;         // nodes
+    drp::Grid G{};         // layout of the population, field, force and tau arrays (choose_layout)
     int64_t step = 0;      // reference loop counter of the last completed step
     bool initialized = false;
     bool eq_init = false;  // populations are the equilibria of fields set by drp_init_* (no step since)
     int shape = 0;         // tile shape of the step kernel
     int cur = 0;           // which ping-pong buffer holds the current state
-    void* pop[2] = {nullptr, nullptr};  // FP64: [f (15 ns) | g (15 ns)] doubles; FP32: floats
-    void* mac[2] = {nullptr, nullptr};  // phi, p, u1, u2, u3 (5 ns)
+    void* pop[2] = {nullptr, nullptr};  // FP64: [f (15 G.ns) | g (15 G.ns)] doubles; FP32: floats
+    void* mac[2] = {nullptr, nullptr};  // phi, p, u1, u2, u3 (5 G.ns)
     uint64_t* range = nullptr;          // 3 rotating (max, min) slots of the phi range
     double* tau = nullptr;              // LES relaxation-time field
     double* qh[2] = {nullptr, nullptr}; // non-equilibrium LES: sqrt(Pi:Pi) per node, with the populations' parity
@@ -32,6 +32,7 @@ struct drp_lattice {
     double* spec_adv = nullptr;         // scale-separated advection: transform work space
     drp::SpectralWork specw_adv{};
     double* uadv = nullptr;             // scale-separated advection: band-passed u1 | u2 | u3
+    double* pack = nullptr;             // one array without row padding, on its way to or from the host
     double* tg = nullptr;               // Taylor-Green sin/cos tables
     double* partial = nullptr;          // diagnostics sums (REDUCE_WORK_DOUBLES)
     double* mac64 = nullptr;            // FP32 mode: FP64 copy of the macroscopic fields
@@ -58,6 +59,11 @@ void stats_from_sums(const drp_lattice* L, const double* sums, const uint64_t* r
 // LES tau for the next step: after a step (fresh = false, rank-block halos one
 // step old) or for a replaced state (fresh = true, all neighbours current)
 int les_update_tau(drp_lattice* L, bool fresh);
+
+// `count` node arrays (G.ns apart) to contiguous host arrays of n doubles, and back;
+// to the host: returns when they are there
+int nodes_to_host(drp_lattice* L, const double* nodes, int count, double* host);
+int nodes_from_host(drp_lattice* L, const double* host, int count, double* nodes);
 
 // spectral_diag.hip
 void diag_free(drp_lattice* L);

@@ -74,7 +74,7 @@ template <int NV> __device__ __forceinline__ double wave_sums(double (&v)[32], i
 // pass 1: one wavefront per (y, z) row; the loads of four x-iterations are issued
 // together before their products are accumulated
 template <int K, typename T>
-__global__ __launch_bounds__(SF_BLOCK) void sf_rows_fwd(int nx, int ny, int nz, const T* __restrict__ u1,
+__global__ __launch_bounds__(SF_BLOCK) void sf_rows_fwd(int nx, int px, int ny, int nz, const T* __restrict__ u1,
                                                         const T* __restrict__ u2, const T* __restrict__ u3,
                                                         const double2* __restrict__ twx, double2* __restrict__ A) {
     constexpr int NV = 6 * (K + 1), CH = 4;
@@ -92,7 +92,7 @@ __global__ __launch_bounds__(SF_BLOCK) void sf_rows_fwd(int nx, int ny, int nz, 
         for (int j = 0; j < CH; j++) {
             const int x = x0 + 64 * j + lane;
             const bool ok = x < nx;
-            const long s = row * nx + (ok ? x : 0);
+            const long s = row * px + (ok ? x : 0);
 #pragma unroll
             for (int c = 0; c < 3; c++) v[j][c] = ok ? (double)u[c][s] : 0.0;
 #pragma unroll
@@ -236,7 +236,7 @@ __global__ __launch_bounds__(SF_BLOCK) void sf_rows_inv(int ny, int nz, const do
 // pass 6: the force field, one wavefront per (y, z) row: the row's coefficients are
 // the same for every lane (read once into scalar registers), the lanes run over x
 template <int K>
-__global__ __launch_bounds__(SF_BLOCK) void sf_force(int nx, int ny, int nz, const double2* __restrict__ H,
+__global__ __launch_bounds__(SF_BLOCK) void sf_force(int nx, int px, int ny, int nz, const double2* __restrict__ H,
                                                      const double2* __restrict__ twx, double* __restrict__ fx,
                                                      double* __restrict__ fy, double* __restrict__ fz) {
     const int lane = threadIdx.x & 63;
@@ -252,7 +252,7 @@ __global__ __launch_bounds__(SF_BLOCK) void sf_force(int nx, int ny, int nz, con
         double2 e[K + 1];
 #pragma unroll
         for (int k = 1; k <= K; k++) e[k] = twiddle(twx, k * x, nx, +1);
-        const long s = row * nx + x;
+        const long s = row * px + x;
 #pragma unroll
         for (int c = 0; c < 3; c++) {
             double v = h[c][0].x;
@@ -264,11 +264,12 @@ __global__ __launch_bounds__(SF_BLOCK) void sf_force(int nx, int ny, int nz, con
 }
 
 template <int K, typename T>
-hipError_t spectral_k(const SpectralWork& w, int nx, int ny, int nz, int k2lo, int k2hi, int band, double eps,
+hipError_t spectral_k(const SpectralWork& w, const Grid& G, int k2lo, int k2hi, int band, double eps,
                       const T* u1, const T* u2, const T* u3, double* fx, double* fy, double* fz, hipStream_t st) {
     constexpr int NK = 2 * K + 1, NB = 3 * (K + 1) * NK;
-    const long rows = (long)ny * nz, n = rows * nx;
-    hipLaunchKernelGGL((sf_rows_fwd<K, T>), dim3((rows + 3) / 4), dim3(SF_BLOCK), 0, st, nx, ny, nz, u1, u2, u3,
+    const int nx = G.nx, ny = G.ny, nz = G.nz;
+    const long rows = (long)ny * nz;
+    hipLaunchKernelGGL((sf_rows_fwd<K, T>), dim3((rows + 3) / 4), dim3(SF_BLOCK), 0, st, nx, G.px, ny, nz, u1, u2, u3,
                        w.twx, w.A);
     constexpr int NC = NB * NK, WPB = SF_BLOCK / 64;
     hipLaunchKernelGGL((sf_cols_fwd<K>), dim3((nz * NB + WPB - 1) / WPB), dim3(SF_BLOCK), 0, st, ny, nz, w.A, w.twy,
@@ -279,21 +280,21 @@ hipError_t spectral_k(const SpectralWork& w, int nx, int ny, int nz, int k2lo, i
                        w.twz, w.G);
     hipLaunchKernelGGL((sf_rows_inv<K>), dim3((rows * 3 * (K + 1) + SF_BLOCK - 1) / SF_BLOCK), dim3(SF_BLOCK), 0, st,
                        ny, nz, w.G, w.twy, w.A);  // H reuses A
-    hipLaunchKernelGGL((sf_force<K>), dim3((rows + 3) / 4), dim3(SF_BLOCK), 0, st, nx, ny, nz, w.A,
+    hipLaunchKernelGGL((sf_force<K>), dim3((rows + 3) / 4), dim3(SF_BLOCK), 0, st, nx, G.px, ny, nz, w.A,
                        w.twx, fx, fy, fz);
     return hipGetLastError();
 }
 
 // modes |k_a| <= kc - 1 transformed; kept: k2lo <= |k|^2 < k2hi
 template <typename T>
-hipError_t spectral_dispatch(const SpectralWork& w, int nx, int ny, int nz, int kc, int k2lo, int k2hi, int band,
+hipError_t spectral_dispatch(const SpectralWork& w, const Grid& G, int kc, int k2lo, int k2hi, int band,
                              double eps, const T* u1, const T* u2, const T* u3, double* fx, double* fy, double* fz,
                              hipStream_t st) {
     switch (kc - 1) {
-        case 1: return spectral_k<1, T>(w, nx, ny, nz, k2lo, k2hi, band, eps, u1, u2, u3, fx, fy, fz, st);
-        case 2: return spectral_k<2, T>(w, nx, ny, nz, k2lo, k2hi, band, eps, u1, u2, u3, fx, fy, fz, st);
-        case 3: return spectral_k<3, T>(w, nx, ny, nz, k2lo, k2hi, band, eps, u1, u2, u3, fx, fy, fz, st);
-        case 4: return spectral_k<4, T>(w, nx, ny, nz, k2lo, k2hi, band, eps, u1, u2, u3, fx, fy, fz, st);
+        case 1: return spectral_k<1, T>(w, G, k2lo, k2hi, band, eps, u1, u2, u3, fx, fy, fz, st);
+        case 2: return spectral_k<2, T>(w, G, k2lo, k2hi, band, eps, u1, u2, u3, fx, fy, fz, st);
+        case 3: return spectral_k<3, T>(w, G, k2lo, k2hi, band, eps, u1, u2, u3, fx, fy, fz, st);
+        case 4: return spectral_k<4, T>(w, G, k2lo, k2hi, band, eps, u1, u2, u3, fx, fy, fz, st);
         default: return hipErrorInvalidValue;
     }
 }
@@ -331,22 +332,22 @@ void spectral_work_layout(SpectralWork& w, double* base, int nx, int ny, int nz,
     w.elow = reinterpret_cast<double*>(p);
 }
 
-hipError_t launch_spectral_force(const SpectralWork& w, int nx, int ny, int nz, int kc, double eps, const double* u1,
+hipError_t launch_spectral_force(const SpectralWork& w, const Grid& G, int kc, double eps, const double* u1,
                                  const double* u2, const double* u3, double* fx, double* fy, double* fz,
                                  hipStream_t st) {
-    return spectral_dispatch<double>(w, nx, ny, nz, kc, 1, kc * kc, 0, eps, u1, u2, u3, fx, fy, fz, st);
+    return spectral_dispatch<double>(w, G, kc, 1, kc * kc, 0, eps, u1, u2, u3, fx, fy, fz, st);
 }
 
-hipError_t launch_spectral_force(const SpectralWork& w, int nx, int ny, int nz, int kc, double eps, const float* u1,
+hipError_t launch_spectral_force(const SpectralWork& w, const Grid& G, int kc, double eps, const float* u1,
                                  const float* u2, const float* u3, double* fx, double* fy, double* fz,
                                  hipStream_t st) {
-    return spectral_dispatch<float>(w, nx, ny, nz, kc, 1, kc * kc, 0, eps, u1, u2, u3, fx, fy, fz, st);
+    return spectral_dispatch<float>(w, G, kc, 1, kc * kc, 0, eps, u1, u2, u3, fx, fy, fz, st);
 }
 
-hipError_t launch_spectral_band(const SpectralWork& w, int nx, int ny, int nz, int klo, int khi, const double* u1,
+hipError_t launch_spectral_band(const SpectralWork& w, const Grid& G, int klo, int khi, const double* u1,
                                 const double* u2, const double* u3, double* o1, double* o2, double* o3,
                                 hipStream_t st) {
-    return spectral_dispatch<double>(w, nx, ny, nz, khi, klo * klo, khi * khi, 1, 0.0, u1, u2, u3, o1, o2, o3, st);
+    return spectral_dispatch<double>(w, G, khi, klo * klo, khi * khi, 1, 0.0, u1, u2, u3, o1, o2, o3, st);
 }
 
 }  // namespace drp

@@ -238,9 +238,12 @@ __global__ __launch_bounds__(256) void fft_lines(double2* __restrict__ data, FFT
     }
 }
 
-__global__ void to_complex(int64_t n, const double* __restrict__ a, double2* __restrict__ c) {
+// a node array as contiguous complex numbers
+__global__ void to_complex(Grid G, const double* __restrict__ a, double2* __restrict__ c) {
     const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (i < n) c[i] = make_double2(a[i], 0.0);
+    const int x = (int)(i % G.nx);
+    const int64_t row = i / G.nx;
+    if (row < (int64_t)G.ny * G.nz) c[i] = make_double2(a[x + G.px * row], 0.0);
 }
 
 __global__ void real_part_scaled(int64_t n, const double2* __restrict__ c, double s, double* __restrict__ a) {
@@ -402,13 +405,14 @@ template <int Q0, int Q1, typename Fn> __device__ __forceinline__ void sford(Fn&
         sford<Q0 + 1, Q1>(fn);
     }
 }
-__global__ __launch_bounds__(WNT) void div_korteweg(int nx, int ny, int nz, const double* __restrict__ phi,
+__global__ __launch_bounds__(WNT) void div_korteweg(Grid G, const double* __restrict__ phi,
                                                     double* __restrict__ w, int64_t pitch, int64_t comp, int tiles_x,
                                                     int tiles_y) {
     constexpr int HX2 = WTX + 4, HY2 = WTY + 4, HZ2 = WTZ + 4, H2 = HX2 * HY2 * HZ2;
     constexpr int HX1 = WTX + 2, HY1 = WTY + 2, HZ1 = WTZ + 2, H1 = HX1 * HY1 * HZ1;
     __shared__ double sp[H2];
     __shared__ double sg[3][H1];
+    const int nx = G.nx, ny = G.ny, nz = G.nz;
     const int tile = xcd_tile(blockIdx.x, gridDim.x);
     const int x0 = (tile % tiles_x) * WTX, y0 = ((tile / tiles_x) % tiles_y) * WTY,
               z0 = (tile / (tiles_x * tiles_y)) * WTZ;
@@ -423,7 +427,7 @@ __global__ __launch_bounds__(WNT) void div_korteweg(int nx, int ny, int nz, cons
     for (int h = threadIdx.x; h < H2; h += WNT) {
         const int gx = wrap(x0 - 2 + h % HX2, nx), gy = wrap(y0 - 2 + (h / HX2) % HY2, ny),
                   gz = wrap(z0 - 2 + h / (HX2 * HY2), nz);
-        sp[h] = phi[gx + (int64_t)nx * (gy + (int64_t)ny * gz)];
+        sp[h] = phi[G.node(gx, gy, gz)];
     }
     __syncthreads();
     for (int h = threadIdx.x; h < H1; h += WNT) {
@@ -558,7 +562,7 @@ int transform_velocity(drp_lattice* L, const FFTPlan& P, double2* c) {
     const int64_t n = L->n;
     const unsigned nb = (unsigned)((n + 255) / 256);
     for (int k = 0; k < 3; k++) {
-        hipLaunchKernelGGL(to_complex, dim3(nb), dim3(256), 0, L->stream, n, mac + (2 + k) * L->ns, c + k * n);
+        hipLaunchKernelGGL(to_complex, dim3(nb), dim3(256), 0, L->stream, L->G, mac + (2 + k) * L->G.ns, c + k * n);
         HIP_TRYS(hipGetLastError());
         HIP_TRYS(fft3d(P, c + k * n, -1, L->stream));
     }
@@ -697,9 +701,9 @@ int shell_sums(drp_lattice* L, drp_diag* D, int nbins, int wgs, double* host) {
 
 // w_b, b = 0..2, into the half spectra 1..3, in rows of 2 pitch doubles
 int korteweg_divergence(drp_lattice* L, drp_diag* D, const double* phi) {
-    const drp_config& c = L->cfg;
-    const int tx = (c.nx + WTX - 1) / WTX, ty = (c.ny + WTY - 1) / WTY, tz = (c.nz + WTZ - 1) / WTZ;
-    hipLaunchKernelGGL(div_korteweg, dim3((unsigned)(tx * ty * tz)), dim3(WNT), 0, L->stream, c.nx, c.ny, c.nz, phi,
+    const Grid& G = L->G;
+    const int tx = (G.nx + WTX - 1) / WTX, ty = (G.ny + WTY - 1) / WTY, tz = (G.nz + WTZ - 1) / WTZ;
+    hipLaunchKernelGGL(div_korteweg, dim3((unsigned)(tx * ty * tz)), dim3(WNT), 0, L->stream, G, phi,
                        (double*)D->spectrum(1), 2 * D->pitch, 2 * D->pitch * D->rows, tx, ty);
     HIP_TRYS(hipGetLastError());
     return DRP_OK;
@@ -736,7 +740,7 @@ extern "C" int drp_energy_spectrum(drp_lattice* L, double* E, int nshells) {
     rc = velocity_view(L, &mac);
     if (!rc) rc = shell_records(D, nshells, &wgs);
     for (int k = 0; k < 3 && !rc; k++) {
-        rc = half_transform(D, mac + (2 + k) * L->ns, L->cfg.nx, 0, L->stream);
+        rc = half_transform(D, mac + (2 + k) * L->G.ns, L->G.px, 0, L->stream);
         if (!rc) rc = shell_pass<SHELL_ENERGY>(L, D, 0, 1.0 / (double)L->n, nshells, nshells, wgs, k > 0);
     }
     return rc ? rc : shell_sums(L, D, nshells, wgs, E);
@@ -788,7 +792,7 @@ extern "C" int drp_scale_interaction(drp_lattice* L, double* C, int nshells) {
     if (!rc) rc = korteweg_divergence(L, D, mac);
     for (int b = 0; b < 3 && !rc; b++) {
         rc = half_transform(D, (const double*)D->spectrum(1 + b), 2 * D->pitch, 1 + b, L->stream);
-        if (!rc) rc = half_transform(D, mac + (2 + b) * L->ns, L->cfg.nx, 0, L->stream);
+        if (!rc) rc = half_transform(D, mac + (2 + b) * L->G.ns, L->G.px, 0, L->stream);
         if (!rc) rc = shell_pass<SHELL_CROSS>(L, D, 1 + b, 1.0 / (double)L->n, nshells, nshells, wgs, b > 0);
     }
     std::vector<double> h(nshells);
@@ -814,7 +818,7 @@ extern "C" int drp_phi_contribution(drp_lattice* L, double* C, int nshells, doub
     const int kinds[2] = {DRP_DERIVED_ADVECTION, DRP_DERIVED_CHEMICAL_POTENTIAL};
     for (int k = 0; k < 2 && !rc; k++) {
         double* field = (double*)D->spectrum(k);
-        HIP_TRYS(launch_derived_fp64(c.nx, c.ny, c.nz, L->ns, L->phys, mac, kinds[k], field, 2 * D->pitch, L->stream));
+        HIP_TRYS(launch_derived_fp64(L->G, L->phys, mac, kinds[k], field, 2 * D->pitch, L->stream));
         rc = half_transform(D, field, 2 * D->pitch, k, L->stream);
     }
     if (!rc) rc = shell_pass<SHELL_CROSS_HALF>(L, D, 1, 1.0, nb, 2 * nb, wgs, false);

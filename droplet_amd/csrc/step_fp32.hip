@@ -99,10 +99,11 @@ __device__ __forceinline__ void step_tile_fp32(const StepArgs32& a, int tile) {
     const int xc = inside ? x : 0, yc = inside ? y : 0, zc = inside ? z : 0;
     const int xs[3] = {xc + 1 == nx ? 0 : xc + 1, xc, xc == 0 ? nx - 1 : xc - 1};
     const int zs[3] = {zc + 1 == nz ? 0 : zc + 1, zc, zc == 0 ? nz - 1 : zc - 1};
-    // node indices as 32-bit factors (an x-y plane holds fewer than 2^31 nodes)
-    const uint32_t nxy32 = (uint32_t)nx * (uint32_t)ny;
-    const uint32_t yo[3] = {(uint32_t)(nx * (yc + 1 == ny ? 0 : yc + 1)), (uint32_t)(nx * yc),
-                            (uint32_t)(nx * (yc == 0 ? ny - 1 : yc - 1))};
+    // node indices as 32-bit factors (an x-y plane holds fewer than 2^31 elements)
+    const int px = a.px;
+    const uint32_t nxy32 = (uint32_t)px * (uint32_t)ny;
+    const uint32_t yo[3] = {(uint32_t)(px * (yc + 1 == ny ? 0 : yc + 1)), (uint32_t)(px * yc),
+                            (uint32_t)(px * (yc == 0 ? ny - 1 : yc - 1))};
     const uint64_t zo[3] = {(uint64_t)(uint32_t)zs[0] * nxy32, (uint64_t)(uint32_t)zs[1] * nxy32,
                             (uint64_t)(uint32_t)zs[2] * nxy32};
     // node index of the upstream node x - c of direction q
@@ -130,7 +131,7 @@ __device__ __forceinline__ void step_tile_fp32(const StepArgs32& a, int tile) {
             gy = wrap32(gy, ny, wm);
             gz = wrap32(gz, nz, wm);
         }
-        return (int64_t)((uint64_t)(uint32_t)gz * nxy32 + (uint32_t)(gy * nx));
+        return (int64_t)((uint64_t)(uint32_t)gz * nxy32 + (uint32_t)(gy * px));
     };
     const int c2 = tid % HX2, r2 = tid / HX2, c1 = tid % HX1, r1 = tid / HX1;
     const int gx2 = wrap32(x0 - 2 + c2, nx, wm), gx1 = wrap32(x0 - 1 + c1, nx, wm);
@@ -233,7 +234,7 @@ __device__ __forceinline__ void step_tile_fp32(const StepArgs32& a, int tile) {
     // phase 3: collide-stream
     double vmax = -__builtin_huge_val(), vmin = __builtin_huge_val();
     if (inside) {
-        const int64_t s = x + (int64_t)nx * (y + (int64_t)ny * z);
+        const int64_t s = x + (int64_t)px * (y + (int64_t)ny * z);
         const int hself = (tx + 1) + HX1 * ((ty + 1) + HY1 * (tz + 1));
         if (!mom) {
             double phs = 0.0;

@@ -130,16 +130,17 @@ __device__ __forceinline__ void step_tile_fp64(const StepArgs& a, int tile) {
     const int c2 = tid % HX2, r2 = tid / HX2;  // r2 < RP2: the thread stages phi rows
     const int c1 = tid % HX1, r1 = tid / HX1;  // r1 < RP1: the thread stages p, u rows
     const bool yz_in = !wm && y0 >= 2 && y0 + TY + 2 <= ny && z0 >= 2 && z0 + TZ + 2 <= nz;
-    // node index of (0, y, z): z nx ny in 64 bits from 32-bit factors (an x-y
-    // plane holds fewer than 2^31 nodes)
-    const uint32_t nxy32 = (uint32_t)nx * (uint32_t)ny;
+    // node index of (0, y, z): z px ny in 64 bits from 32-bit factors (an x-y
+    // plane holds fewer than 2^31 elements)
+    const int px = a.px;
+    const uint32_t nxy32 = (uint32_t)px * (uint32_t)ny;
     auto row_offset = [&](int hy, int hz, int halo) -> int64_t {
         int gy = y0 - halo + hy, gz = z0 - halo + hz;
         if (!yz_in) {
             gy = wrapi(gy, ny, wm);
             gz = wrapi(gz, nz, wm);
         }
-        return (int64_t)((uint64_t)(uint32_t)gz * nxy32 + (uint32_t)(gy * nx));
+        return (int64_t)((uint64_t)(uint32_t)gz * nxy32 + (uint32_t)(gy * px));
     };
     const int gx2 = wrapi(x0 - 2 + c2, nx, wm), gx1 = wrapi(x0 - 1 + c1, nx, wm);
     double vphi[IT2], vp[IT1], vu1[IT1], vu2[IT1], vu3[IT1], vtau[IT1];
@@ -179,8 +180,8 @@ __device__ __forceinline__ void step_tile_fp64(const StepArgs& a, int tile) {
     const int xc = inside ? x : 0, yc = inside ? y : 0, zc = inside ? z : 0;
     const int xs[3] = {xc + 1 == nx ? 0 : xc + 1, xc, xc == 0 ? nx - 1 : xc - 1};
     const int zs[3] = {zc + 1 == nz ? 0 : zc + 1, zc, zc == 0 ? nz - 1 : zc - 1};
-    const uint32_t yo[3] = {(uint32_t)(nx * (yc + 1 == ny ? 0 : yc + 1)), (uint32_t)(nx * yc),
-                            (uint32_t)(nx * (yc == 0 ? ny - 1 : yc - 1))};
+    const uint32_t yo[3] = {(uint32_t)(px * (yc + 1 == ny ? 0 : yc + 1)), (uint32_t)(px * yc),
+                            (uint32_t)(px * (yc == 0 ? ny - 1 : yc - 1))};
     const uint64_t zo[3] = {(uint64_t)(uint32_t)zs[0] * nxy32, (uint64_t)(uint32_t)zs[1] * nxy32,
                             (uint64_t)(uint32_t)zs[2] * nxy32};
     // node index of the upstream node x - c of direction q
@@ -288,7 +289,7 @@ __device__ __forceinline__ void step_tile_fp64(const StepArgs& a, int tile) {
     // ---------------- phase 3: collide-stream of this thread's population set
     double vmax = -__builtin_huge_val(), vmin = __builtin_huge_val();
     if (inside) {
-        const int64_t s = x + (int64_t)nx * (y + (int64_t)ny * z);
+        const int64_t s = x + (int64_t)px * (y + (int64_t)ny * z);
         if (!mom && MODEL == MODEL_AC) {
             // physics, dropac.f90:640-667: phi(x) <- sum_i [feq_i(x - c_i) + A E_i (phi(x) - phi(x - c_i))]
             // with feq_i = E_i phi (1 + 3 c.u) + 3 E_i M (1 - 4 phi^2) (c.n) / W (feq_cal :517-535),
@@ -469,7 +470,7 @@ __device__ __forceinline__ void step_tile_fp64(const StepArgs& a, int tile) {
                         using D = Dir<q>;
                         const int ux = wrapi(x - D::cx, nx, false), uy = wrapi(y - D::cy, ny, false),
                                   uz = wrapi(z - D::cz, nz, false);
-                        ps[q] = __builtin_nontemporal_load(&a.g_in[q * N + ux + (int64_t)nx * (uy + (int64_t)ny * uz)]);
+                        ps[q] = __builtin_nontemporal_load(&a.g_in[q * N + ux + (int64_t)px * (uy + (int64_t)ny * uz)]);
                     });
                     collide(std::true_type{});
                 }
