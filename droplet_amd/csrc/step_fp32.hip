@@ -47,6 +47,7 @@ __device__ __forceinline__ void step_tile_fp32(const StepArgs32& a, int tile) {
     constexpr int HX2 = TX + 4, HY2 = TY + 4, HZ2 = TZ + 4, H2 = HX2 * HY2 * HZ2;
     constexpr int HX1 = TX + 2, HY1 = TY + 2, HZ1 = TZ + 2, H1 = HX1 * HY1 * HZ1;
     static_assert(NN % 64 == 0, "a role must own whole wavefronts");
+    static_assert(HX1 + HZ1 <= NT, "one thread per staged table entry");
 
     // Per halo node the stencil phase leaves four float4 records, so that the
     // collision phase needs two 16-byte LDS reads and about ten FMAs per direction:
@@ -71,6 +72,10 @@ __device__ __forceinline__ void step_tile_fp32(const StepArgs32& a, int tile) {
     constexpr int RP1 = NT / HX1, R1 = HY1 * HZ1, IT1 = (R1 + RP1 - 1) / RP1;
     static_assert(RP2 >= 1 && RP1 >= 1, "a workgroup spans at least one halo row");
     float rt_reg[TAUMODE == 0 ? 1 : IT1];
+    // Taylor-Green: amp sin(kx), amp cos(kx) of the tile + 1 columns, sin(kz), cos(kz) of
+    // its + 1 layers.  Read from the tables in memory, each direction waited for two to
+    // four loads: 541 us a step at 192^3 with nu(phi), 480 from LDS (464 without force).
+    __shared__ double s_tg[FORCE == FORCE_TAYLOR_GREEN ? 2 * (HX1 + HZ1) : 1];
     __shared__ double s_red[2][NT / 64];
 
     const int nx = a.nx, ny = a.ny, nz = a.nz;
@@ -151,6 +156,17 @@ __device__ __forceinline__ void step_tile_fp32(const StepArgs32& a, int tile) {
             if constexpr (TAUMODE == 2) rt_reg[k] = 1.0f / a.tau_field[g];
         }
     });
+    if constexpr (FORCE == FORCE_TAYLOR_GREEN) {
+        if (tid < HX1) {
+            const int g = wrap32(x0 - 1 + tid, nx, wm);
+            s_tg[tid] = a.tg_amp * a.sinx[g];
+            s_tg[HX1 + tid] = a.tg_amp * a.cosx[g];
+        } else if (tid < HX1 + HZ1) {
+            const int i = tid - HX1, g = wrap32(z0 - 1 + i, nz, wm);
+            s_tg[2 * HX1 + i] = a.sinz[g];
+            s_tg[2 * HX1 + HZ1 + i] = a.cosz[g];
+        }
+    }
     __syncthreads();
 
     // phase 2: FP64-accumulated Laplacian and gradient, deviation F-bracket, the
@@ -281,9 +297,9 @@ __device__ __forceinline__ void step_tile_fp32(const StepArgs32& a, int tile) {
                 if constexpr (FORCE != FORCE_NONE && q != 0) {
                     float Fx = 0.0f, Fy = 0.0f, Fz = 0.0f;   // only the components that enter c . F
                     if constexpr (FORCE == FORCE_TAYLOR_GREEN) {
-                        const int xu = xs[1 + D::cx], zu = zs[1 + D::cz];
-                        if constexpr (D::cx != 0) Fx = (float)(a.tg_amp * a.sinx[xu] * a.cosz[zu]);
-                        if constexpr (D::cz != 0) Fz = (float)(-(a.tg_amp * a.cosx[xu] * a.sinz[zu]));
+                        const int xu = tx + 1 - D::cx, zu = 2 * HX1 + (tz + 1 - D::cz);
+                        if constexpr (D::cx != 0) Fx = (float)(s_tg[xu] * s_tg[zu + HZ1]);
+                        if constexpr (D::cz != 0) Fz = (float)(-(s_tg[HX1 + xu] * s_tg[zu]));
                     } else {
                         const int64_t src = upstream(qc);
                         if constexpr (D::cx != 0) Fx = (float)a.fx[src];

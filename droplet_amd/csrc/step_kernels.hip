@@ -89,7 +89,8 @@ __device__ __forceinline__ void step_tile_fp64(const StepArgs& a, int tile) {
     // Allen-Cahn: the unit normal n = grad phi / (|grad phi| + eps) per halo node
     // in s_A (n0), s_n1, s_n2 (the F-bracket has no role in that model)
     __shared__ double s_n1[MODEL == MODEL_AC ? H1 : 1], s_n2[MODEL == MODEL_AC ? H1 : 1];
-    constexpr int LDS_BASE = 8 * (H2 + 8 * H1 + (TAUMODE == TAU_CONST ? 1 : H1) + 2 * (NT / 64) +
+    constexpr int TG = FORCE == FORCE_TAYLOR_GREEN ? 2 * (HX1 + HZ1) : 0;
+    constexpr int LDS_BASE = 8 * (H2 + 8 * H1 + (TAUMODE == TAU_CONST ? 1 : H1) + 2 * (NT / 64) + TG +
                                   (MODEL == MODEL_AC ? 2 * H1 : 0));
     constexpr bool PRE_S = LDS_BASE + 8 * H1 <= 160 * 1024 && wg_per_cu_lds(LDS_BASE + 8 * H1) >= wg_per_cu_lds(LDS_BASE);
     constexpr bool PRE_U =
@@ -97,6 +98,11 @@ __device__ __forceinline__ void step_tile_fp64(const StepArgs& a, int tile) {
     __shared__ double s_s2h[PRE_S ? H1 : 1], s_usq15[PRE_U ? H1 : 1];  // 1.5 |grad phi|^2, 1.5 |u|^2
     __shared__ double s_tau[TAUMODE == TAU_CONST ? 1 : H1];
     __shared__ double s_red[2][NT / 64];
+    // Taylor-Green: amp sin(kx), amp cos(kx) of the tile + 1 columns, sin(kz), cos(kz) of
+    // its + 1 layers.  Read from the tables in memory, each direction waited for two to
+    // four loads: 966 us a step at 192^3 with nu(phi), 908 from LDS (862 without force).
+    __shared__ double s_tg[TG ? TG : 1];
+    static_assert(HX1 + HZ1 <= NT, "one thread per staged table entry");
 
     const int nx = a.nx, ny = a.ny, nz = a.nz;
     const int64_t N = a.ns;  // from one population or field array to the next
@@ -221,6 +227,17 @@ __device__ __forceinline__ void step_tile_fp64(const StepArgs& a, int tile) {
             if constexpr (TAUMODE == TAU_FIELD || TAUMODE == TAU_NONEQ) s_tau[h] = vtau[k];
         }
     });
+    if constexpr (FORCE == FORCE_TAYLOR_GREEN) {
+        if (tid < HX1) {
+            const int g = wrapi(x0 - 1 + tid, nx, wm);
+            s_tg[tid] = a.tg_amp * a.sinx[g];
+            s_tg[HX1 + tid] = a.tg_amp * a.cosx[g];
+        } else if (tid < HX1 + HZ1) {
+            const int i = tid - HX1, g = wrapi(z0 - 1 + i, nz, wm);
+            s_tg[2 * HX1 + i] = a.sinz[g];
+            s_tg[2 * HX1 + HZ1 + i] = a.cosz[g];
+        }
+    }
     __syncthreads();
 
     // ---------------- phase 2: stencils, F-bracket and tau at tile + 1 halo
@@ -442,9 +459,9 @@ __device__ __forceinline__ void step_tile_fp64(const StepArgs& a, int tile) {
                         // only the components that enter are loaded
                         double Fx = 0.0, Fy = 0.0, Fz = 0.0;
                         if constexpr (FORCE == FORCE_TAYLOR_GREEN) {
-                            const int xu = xs[1 + D::cx], zu = zs[1 + D::cz];
-                            if constexpr (D::cx != 0) Fx = a.tg_amp * a.sinx[xu] * a.cosz[zu];
-                            if constexpr (D::cz != 0) Fz = -(a.tg_amp * a.cosx[xu] * a.sinz[zu]);
+                            const int xu = tx + 1 - D::cx, zu = 2 * HX1 + (tz + 1 - D::cz);
+                            if constexpr (D::cx != 0) Fx = s_tg[xu] * s_tg[zu + HZ1];
+                            if constexpr (D::cz != 0) Fz = -(s_tg[HX1 + xu] * s_tg[zu]);
                         } else {  // field at the upstream node, loaded FPF directions ahead
                             const double* f = fring[q % FPF];
                             if constexpr (D::cx != 0) Fx = f[0];
