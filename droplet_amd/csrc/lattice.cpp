@@ -237,15 +237,11 @@ int default_shape(int precision) {
     }
     return precision == DRP_FP64 ? SHAPE_32x4x2 : SHAPE_32x4x4;
 }
-// per-variant defaults measured at 256^3 on MI355X (drp_autotune): the FP64 step
-// with a force field (the turbulent-droplet case) runs fastest on 32x4x4 tiles
-// (3.05 against 3.10 ms per step with LES and spectral forcing), the Allen-Cahn
+// per-variant default measured at 256^3 on MI355X (drp_autotune): the Allen-Cahn
 // step on 16x4x4 tiles (1.65 against 1.76 ms)
 static int pick_shape(const drp_config& c) {
     if (std::getenv("DROPLET_SHAPE")) return default_shape(c.precision);
     if (c.model == DRP_MODEL_ALLEN_CAHN) return SHAPE_16x4x4;
-    if (c.precision == DRP_FP64 && (c.force_kind == DRP_FORCE_FIELD || c.force_kind == DRP_FORCE_SPECTRAL))
-        return SHAPE_32x4x4;
     return default_shape(c.precision);
 }
 

@@ -75,9 +75,8 @@ __device__ __forceinline__ void step_tile_fp64(const StepArgs& a, int tile) {
     static_assert(NN % 64 == 0, "a role must own whole wavefronts");
     // relaxation by the shared-divisor division (d3q15.h) where it costs no
     // spilled registers: not in a role that carries a register ring (the
-    // band-passed velocity of the phi role, the force field of the momentum role)
+    // band-passed velocity of the phi role)
     constexpr bool FASTDIV_F = MODEL != MODEL_SCALE;
-    constexpr bool FASTDIV_G = FORCE != FORCE_FIELD;
 
     __shared__ double s_phi[H2];
     __shared__ double s_p3[H1], s_u1[H1], s_u2[H1], s_u3[H1];  // s_p3: 3 p
@@ -303,6 +302,25 @@ __device__ __forceinline__ void step_tile_fp64(const StepArgs& a, int tile) {
     });
     __syncthreads();
 
+    // the force field of the tile + 1 halo, in flight during the collisions
+    double vf[FORCE == FORCE_FIELD ? IT1 : 1][3];
+    if constexpr (FORCE == FORCE_FIELD)
+        static_for<0, IT1>([&](auto kc) {
+            constexpr int k = decltype(kc)::value;
+            const int r = r1 + k * RP1 < R1 ? r1 + k * RP1 : R1 - 1;
+            const int64_t g = gx1 + row_offset(r % HY1, r / HY1, 1);
+            vf[k][0] = a.fx[g];
+            vf[k][1] = a.fy[g];
+            vf[k][2] = a.fz[g];
+        });
+
+    // 3 E c . F with the zero-velocity terms dropped, as for c . u: the reference's
+    // (cx Fx + cy Fy) + cz Fz rounds identically
+    auto body_force = [&](auto qc, double Fx, double Fy, double Fz) -> double {
+        constexpr int q = decltype(qc)::value;
+        return 3.0 * weightE<q>() * cdot<q>(Fx, Fy, Fz);
+    };
+
     // ---------------- phase 3: collide-stream of this thread's population set
     double vmax = -__builtin_huge_val(), vmin = __builtin_huge_val();
     if (inside) {
@@ -409,27 +427,12 @@ __device__ __forceinline__ void step_tile_fp64(const StepArgs& a, int tile) {
             vmax = ph;
             vmin = ph;
         } else {
-            // force-field components of the upstream nodes, loaded FPF directions
-            // ahead of their use into a ring of FPF slots, so that the L2 latency
-            // of these loads overlaps the collisions in between
-            constexpr int FPF = 3;
-            double fring[FPF][3] = {};
-            auto load_force = [&](auto qc) {
-                constexpr int q = decltype(qc)::value;
-                using D = Dir<q>;
-                const int64_t src = upstream(qc);
-                double* f = fring[q % FPF];
-                if constexpr (D::cx != 0) f[0] = a.fx[src];
-                if constexpr (D::cy != 0) f[1] = a.fy[src];
-                if constexpr (D::cz != 0) f[2] = a.fz[src];
-            };
             // with a constant tau_g, relaxation as in the phi role (SharedDivisor, and
             // the collision again with full divisions for a node that needs them)
             const SharedDivisor dtau = shared_divisor(a.tau_const);
             bool redo = TAUMODE == TAU_CONST && !dtau.ok;
             auto collide = [&](auto full_c) {
                 constexpr bool FULL = decltype(full_c)::value;
-                if constexpr (FORCE == FORCE_FIELD) static_for<1, 1 + FPF>(load_force);
                 static_for<0, 15>([&](auto qc) {
                     constexpr int q = decltype(qc)::value;
                     using D = Dir<q>;
@@ -453,31 +456,19 @@ __device__ __forceinline__ void step_tile_fp64(const StepArgs& a, int tile) {
                         gv = ps[q] - div_shared_fast(dx, dtau);
                         redo |= !div_shared_exact(dx);
                     }
-                    if constexpr (FORCE != FORCE_NONE && q != 0) {
-                        // c . F with the zero-velocity terms dropped, as for c . u: the
-                        // reference's (cx Fx + cy Fy) + cz Fz rounds identically, and
-                        // only the components that enter are loaded
-                        double Fx = 0.0, Fy = 0.0, Fz = 0.0;
-                        if constexpr (FORCE == FORCE_TAYLOR_GREEN) {
-                            const int xu = tx + 1 - D::cx, zu = 2 * HX1 + (tz + 1 - D::cz);
-                            if constexpr (D::cx != 0) Fx = s_tg[xu] * s_tg[zu + HZ1];
-                            if constexpr (D::cz != 0) Fz = -(s_tg[HX1 + xu] * s_tg[zu]);
-                        } else {  // field at the upstream node, loaded FPF directions ahead
-                            const double* f = fring[q % FPF];
-                            if constexpr (D::cx != 0) Fx = f[0];
-                            if constexpr (D::cy != 0) Fy = f[1];
-                            if constexpr (D::cz != 0) Fz = f[2];
-                            if constexpr (q + FPF < 15) load_force(std::integral_constant<int, q + FPF>{});
-                        }
-                        const double dot = cdot<q>(Fx, Fy, Fz);
-                        gv = gv + 3.0 * weightE<q>() * dot;
+                    if constexpr (FORCE == FORCE_TAYLOR_GREEN && q != 0) {
+                        double Fx = 0.0, Fz = 0.0;
+                        const int xu = tx + 1 - D::cx, zu = 2 * HX1 + (tz + 1 - D::cz);
+                        if constexpr (D::cx != 0) Fx = s_tg[xu] * s_tg[zu + HZ1];
+                        if constexpr (D::cz != 0) Fz = -(s_tg[HX1 + xu] * s_tg[zu]);
+                        gv = gv + body_force(qc, Fx, 0.0, Fz);
                     }
                     ps[q] = gv;
                     __builtin_amdgcn_sched_barrier(0);  // keep each direction's LDS reads local
                 });
             };
-            collide(std::integral_constant<bool, !FASTDIV_G>{});
-            if constexpr (FASTDIV_G && TAUMODE == TAU_CONST) {
+            collide(std::false_type{});
+            if constexpr (TAUMODE == TAU_CONST) {
                 if (redo) {
                     // the populations this step started from, again, addressed from
                     // the node's coordinates (so that phase 1's upstream offsets
@@ -492,82 +483,109 @@ __device__ __forceinline__ void step_tile_fp64(const StepArgs& a, int tile) {
                     collide(std::true_type{});
                 }
             }
+        }
+    }
 
-            if constexpr (WALL) {
-                // bounce_back_LBM, dropch.f90:666-698: on the first/last fluid layer
-                // the populations entering the fluid are the reflected ones minus
-                // 6 E (U_wall . c_opp); bottom wall moves with -U, top with +U.
-                const int coord = (a.wall_axis == 2) ? y : z;
-                const int nax = (a.wall_axis == 2) ? ny : nz;
-                const bool bottom = coord == 0, top = coord == nax - 1;
-                if (bottom || top) {
-                    const double uw = bottom ? -a.wall_u_now : a.wall_u_now;
-                    const int want = bottom ? 1 : -1;
-                    static_for<1, 15>([&](auto qc) {
-                        constexpr int q = decltype(qc)::value;
-                        using D = Dir<q>;
-                        constexpr int o = D::opp;
-                        const int ca = (a.wall_axis == 2) ? D::cy : D::cz;
-                        if (ca == want) {
-                            const double dot = uw * (double)Dir<o>::cx;
-                            ps[q] = ps[o] - 6.0 * weightE<o>() * dot;
-                        }
-                    });
-                }
-            }
-
-            if constexpr (TAUMODE == TAU_NONEQ) {
-                // tensor_cal (LES_2.f90:530-551): Pi_ab = sum_i c_ia c_ib (g_i - geq_i) with
-                // this step's g and the equilibria of its start at this node; Q = Pi:Pi
-                // (beta outer, alpha inner); sqrt(Q) is kept for the next step's tau
-                const int hs = (tx + 1) + HX1 * ((ty + 1) + HY1 * (tz + 1));
-                const double p3 = s_p3[hs], u1 = s_u1[hs], u2 = s_u2[hs], u3 = s_u3[hs];
-                const double usq15 = PRE_U ? s_usq15[hs] : 1.5 * (u1 * u1 + u2 * u2 + u3 * u3);
-                const double g0 = s_g0[hs], g1 = s_g1[hs], g2 = s_g2[hs];
-                const double s2h = PRE_S ? s_s2h[hs] : 1.5 * (g0 * g0 + g1 * g1 + g2 * g2);
-                double t[3][3] = {{0.0, 0.0, 0.0}, {0.0, 0.0, 0.0}, {0.0, 0.0, 0.0}};
-                static_for<0, 15>([&](auto qc) {
-                    constexpr int q = decltype(qc)::value;
-                    using D = Dir<q>;
-                    constexpr int c[3] = {D::cx, D::cy, D::cz};
-                    const double d = ps[q] - geq_pre<q>(p3, u1, u2, u3, usq15, korteweg<q>(g0, g1, g2, s2h), a.ekg[wclass<q>()]);
+    if constexpr (FORCE == FORCE_FIELD) {
+        // the force at the upstream nodes, by way of LDS arrays that the collisions are
+        // done with (LDS of its own would leave one workgroup per CU; gathering the 30
+        // values per node through L2, three directions ahead of their use, took 2845 us a
+        // turbulent step at 256^3 on 32x4x4 tiles, this takes 2708 on 32x4x2)
+        double* const s_f[3] = {s_A, s_phi, TAUMODE == TAU_CONST ? s_p3 : s_tau};
+        __syncthreads();
+        static_for<0, IT1>([&](auto kc) {
+            constexpr int k = decltype(kc)::value;
+            const int r = r1 + k * RP1;
+            if (r1 < RP1 && r < R1)
 #pragma unroll
-                    for (int b = 0; b < 3; b++)
-#pragma unroll
-                        for (int al = 0; al < 3; al++) {
-                            const int cc = c[al] * c[b];
-                            if (cc == 1) t[al][b] = t[al][b] + d;
-                            else if (cc == -1) t[al][b] = t[al][b] - d;
-                        }
-                });
-                double Q = 0.0;
-#pragma unroll
-                for (int b = 0; b < 3; b++)
-#pragma unroll
-                    for (int al = 0; al < 3; al++) Q = Q + t[al][b] * t[al][b];
-                a.qh_out[s] = sqrt(Q);
-            }
-
-            // moments p = sum g/3, u = sum c g (physics :546-552), order i = 1..15
-            double pr = div_const(ps[0], 3.0, 1.0 / 3.0);
-            double m1 = 0.0, m2 = 0.0, m3 = 0.0;
+                for (int c = 0; c < 3; c++) s_f[c][c1 + HX1 * r] = vf[k][c];
+        });
+        __syncthreads();
+        if (inside && mom)
             static_for<1, 15>([&](auto qc) {
                 constexpr int q = decltype(qc)::value;
                 using D = Dir<q>;
-                pr = pr + div_const(ps[q], 3.0, 1.0 / 3.0);
-                m1 = acc<D::cx>(m1, ps[q]);
-                m2 = acc<D::cy>(m2, ps[q]);
-                m3 = acc<D::cz>(m3, ps[q]);
+                const int hu = hb1 + ((1 - D::cx) + HX1 * ((1 - D::cy) + HY1 * (1 - D::cz)));
+                ps[q] = ps[q] + body_force(qc, s_f[0][hu], s_f[1][hu], s_f[2][hu]);
             });
+    }
+
+    if (inside && mom) {
+        const int64_t s = x + (int64_t)px * (y + (int64_t)ny * z);
+        if constexpr (WALL) {
+            // bounce_back_LBM, dropch.f90:666-698: on the first/last fluid layer
+            // the populations entering the fluid are the reflected ones minus
+            // 6 E (U_wall . c_opp); bottom wall moves with -U, top with +U.
+            const int coord = (a.wall_axis == 2) ? y : z;
+            const int nax = (a.wall_axis == 2) ? ny : nz;
+            const bool bottom = coord == 0, top = coord == nax - 1;
+            if (bottom || top) {
+                const double uw = bottom ? -a.wall_u_now : a.wall_u_now;
+                const int want = bottom ? 1 : -1;
+                static_for<1, 15>([&](auto qc) {
+                    constexpr int q = decltype(qc)::value;
+                    using D = Dir<q>;
+                    constexpr int o = D::opp;
+                    const int ca = (a.wall_axis == 2) ? D::cy : D::cz;
+                    if (ca == want) {
+                        const double dot = uw * (double)Dir<o>::cx;
+                        ps[q] = ps[o] - 6.0 * weightE<o>() * dot;
+                    }
+                });
+            }
+        }
+
+        if constexpr (TAUMODE == TAU_NONEQ) {
+            // tensor_cal (LES_2.f90:530-551): Pi_ab = sum_i c_ia c_ib (g_i - geq_i) with
+            // this step's g and the equilibria of its start at this node; Q = Pi:Pi
+            // (beta outer, alpha inner); sqrt(Q) is kept for the next step's tau
+            const int hs = (tx + 1) + HX1 * ((ty + 1) + HY1 * (tz + 1));
+            const double p3 = s_p3[hs], u1 = s_u1[hs], u2 = s_u2[hs], u3 = s_u3[hs];
+            const double usq15 = PRE_U ? s_usq15[hs] : 1.5 * (u1 * u1 + u2 * u2 + u3 * u3);
+            const double g0 = s_g0[hs], g1 = s_g1[hs], g2 = s_g2[hs];
+            const double s2h = PRE_S ? s_s2h[hs] : 1.5 * (g0 * g0 + g1 * g1 + g2 * g2);
+            double t[3][3] = {{0.0, 0.0, 0.0}, {0.0, 0.0, 0.0}, {0.0, 0.0, 0.0}};
             static_for<0, 15>([&](auto qc) {
                 constexpr int q = decltype(qc)::value;
-                __builtin_nontemporal_store(ps[q], &a.g_out[q * N + s]);
+                using D = Dir<q>;
+                constexpr int c[3] = {D::cx, D::cy, D::cz};
+                const double d = ps[q] - geq_pre<q>(p3, u1, u2, u3, usq15, korteweg<q>(g0, g1, g2, s2h), a.ekg[wclass<q>()]);
+#pragma unroll
+                for (int b = 0; b < 3; b++)
+#pragma unroll
+                    for (int al = 0; al < 3; al++) {
+                        const int cc = c[al] * c[b];
+                        if (cc == 1) t[al][b] = t[al][b] + d;
+                        else if (cc == -1) t[al][b] = t[al][b] - d;
+                    }
             });
-            __builtin_nontemporal_store(pr, &a.mac_out[N + s]);
-            __builtin_nontemporal_store(m1, &a.mac_out[2 * N + s]);
-            __builtin_nontemporal_store(m2, &a.mac_out[3 * N + s]);
-            __builtin_nontemporal_store(m3, &a.mac_out[4 * N + s]);
+            double Q = 0.0;
+#pragma unroll
+            for (int b = 0; b < 3; b++)
+#pragma unroll
+                for (int al = 0; al < 3; al++) Q = Q + t[al][b] * t[al][b];
+            a.qh_out[s] = sqrt(Q);
         }
+
+        // moments p = sum g/3, u = sum c g (physics :546-552), order i = 1..15
+        double pr = div_const(ps[0], 3.0, 1.0 / 3.0);
+        double m1 = 0.0, m2 = 0.0, m3 = 0.0;
+        static_for<1, 15>([&](auto qc) {
+            constexpr int q = decltype(qc)::value;
+            using D = Dir<q>;
+            pr = pr + div_const(ps[q], 3.0, 1.0 / 3.0);
+            m1 = acc<D::cx>(m1, ps[q]);
+            m2 = acc<D::cy>(m2, ps[q]);
+            m3 = acc<D::cz>(m3, ps[q]);
+        });
+        static_for<0, 15>([&](auto qc) {
+            constexpr int q = decltype(qc)::value;
+            __builtin_nontemporal_store(ps[q], &a.g_out[q * N + s]);
+        });
+        __builtin_nontemporal_store(pr, &a.mac_out[N + s]);
+        __builtin_nontemporal_store(m1, &a.mac_out[2 * N + s]);
+        __builtin_nontemporal_store(m2, &a.mac_out[3 * N + s]);
+        __builtin_nontemporal_store(m3, &a.mac_out[4 * N + s]);
     }
 
     // ---------------- global phi range for the next step's nu(phi)
