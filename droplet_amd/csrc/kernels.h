@@ -191,7 +191,7 @@ hipError_t launch_range_set(uint64_t* range, int slot, double vmax, double vmin,
 
 // spectral.hip: linear forcing of the shells 1 <= |k| < kc from the velocity field
 struct SpectralWork {
-    double2 *A, *B, *C, *G;   // transform stages (A also holds the inverse row stage)
+    double2 *A, *B, *C;       // forward transform stages
     double2 *twx, *twy, *twz; // e^{2 pi i j / n} tables
     double* elow;             // energy of the forced shells (last call)
 };

@@ -13,14 +13,16 @@
 //                                                               -kx is conj(kx))
 //   cols_fwd  B(kx, ky, z)  = sum_y A e^{-2 pi i ky y/ny}        ky = -K..K
 //   zsum      u_hat(k)      = sum_z B e^{-2 pi i kz z/nz} / N^3
-//   coef      E_low and the coefficients C(k) = eps / (2 E_low) u_hat(k) on S
-//   cols_inv  G(kx, ky, z)  = sum_kz C e^{+2 pi i kz z/nz}
-//   rows_inv  H(kx, y, z)   = sum_ky G e^{+2 pi i ky y/ny}
-//   force     F(x, y, z)    = Re H(0) + 2 sum_{kx>0} Re(H(kx) e^{+2 pi i kx x/nx})
+//   force     E_low and the coefficients C(k) = eps / (2 E_low) u_hat(k) on S,
+//             G(kx, ky)     = sum_kz C e^{+2 pi i kz z/nz}       for its plane z,
+//             H(kx, y)      = sum_ky G e^{+2 pi i ky y/ny}       for its rows,
+//             F(x, y, z)    = Re H(0) + 2 sum_{kx>0} Re(H(kx) e^{+2 pi i kx x/nx})
 // The first and last passes touch every node once (read u, write F); the others
 // work on N^2 rows or less, one wavefront per output with the lanes over the
-// summed axis.  E_low = 0 gives F = 0 (the reference would divide
-// by zero).
+// summed axis.  The coefficients are few (225 for kc = 3), so every workgroup of the
+// last pass forms what it needs of C, G and H by itself: as passes of their own these
+// took three launches and 19 us a step at 192^3 and below.  E_low = 0 gives F = 0 (the
+// reference would divide by zero).
 //
 // The same passes with unit coefficients on the shells klo <= int|k| < khi give
 // the band-pass of u that advects phi in the scale-separated model
@@ -47,12 +49,12 @@ __device__ __forceinline__ double2 twiddle(const double2* tw, int m, int n, int 
     return make_double2(t.x, s * t.y);
 }
 
-// Sum of NV per-lane values over the 64 lanes of a wavefront with NV - 1 + 1
-// shuffles instead of 6 NV: at each offset o = 32 .. 2 a lane keeps one half of
-// its values (the upper one when lane & o) and adds the partner's copy of that
-// half; after the last halving lane l holds value l >> 1 (summed over its pair's
-// 32 lanes) and one exchange with lane l ^ 1 completes it.  NV <= 32.
-template <int O, int HALF> __device__ __forceinline__ void halve(double (&v)[32], int lane) {
+// Sum of NV per-lane values over the 64 lanes of a wavefront with about 2 SL shuffles
+// (SL = NV rounded up to 16 or 32) instead of 6 NV: at each offset 32, 16, .. a lane
+// keeps one half of its values (the upper one when lane & offset) and adds the
+// partner's copy of that half; when one value is left, lane l holds value
+// l / (64 / SL), and the remaining offsets complete it.
+template <int O, int HALF, int SL> __device__ __forceinline__ void halve(double (&v)[SL], int lane) {
     const bool up = (lane & O) != 0;
 #pragma unroll
     for (int i = 0; i < HALF; i++) {
@@ -60,60 +62,77 @@ template <int O, int HALF> __device__ __forceinline__ void halve(double (&v)[32]
         const double give = up ? v[i] : v[i + HALF];
         v[i] = keep + __shfl_xor(give, O, 64);
     }
-    if constexpr (O > 2) halve<O / 2, HALF / 2>(v, lane);
+    if constexpr (HALF > 1) halve<O / 2, HALF / 2>(v, lane);
 }
 
-template <int NV> __device__ __forceinline__ double wave_sums(double (&v)[32], int lane) {
-    static_assert(NV <= 32, "at most 32 values");
+template <int SL> __device__ __forceinline__ double wave_sums(double (&v)[SL], int lane) {
+    static_assert(SL == 16 || SL == 32, "16 or 32 values");
+    halve<32, SL / 2>(v, lane);
 #pragma unroll
-    for (int i = NV; i < 32; i++) v[i] = 0.0;
-    halve<32, 16>(v, lane);
-    return v[0] + __shfl_xor(v[0], 1, 64);
+    for (int o = 32 / SL; o > 0; o /= 2) v[0] += __shfl_xor(v[0], o, 64);
+    return v[0];
 }
 
-// pass 1: one wavefront per (y, z) row; the loads of four x-iterations are issued
-// together before their products are accumulated
+// pass 1: a wavefront takes RF_ROWS (y, z) rows in turn; the loads of CH x-iterations
+// are issued together before their products are accumulated, and rows of up to 64 CH
+// nodes keep their twiddles in registers.  Measured at 256^3, FP64 / FP32: one row per
+// wavefront with kx = 0 multiplied like the others 97 / 131 us (128^3 FP32: 28), this 85 us (128^3 FP32: 19); with the
+// next row's loads in flight during the sums 121 us (fewer wavefronts fit).
+constexpr int RF_ROWS = 4;
 template <int K, typename T>
 __global__ __launch_bounds__(SF_BLOCK) void sf_rows_fwd(int nx, int px, int ny, int nz, const T* __restrict__ u1,
                                                         const T* __restrict__ u2, const T* __restrict__ u3,
                                                         const double2* __restrict__ twx, double2* __restrict__ A) {
-    constexpr int NV = 6 * (K + 1), CH = 4;
+    constexpr int PC = 2 * K + 1, NV = 3 * PC, SL = NV <= 16 ? 16 : 32, CH = 4;  // per component: re 0, (re, im) 1..K
     const int lane = threadIdx.x & 63;
-    const long row = (long)blockIdx.x * (SF_BLOCK / 64) + (threadIdx.x >> 6);
-    if (row >= (long)ny * nz) return;  // uniform per wavefront
+    const long rows = (long)ny * nz;
+    const long row0 = ((long)blockIdx.x * (SF_BLOCK / 64) + (threadIdx.x >> 6)) * RF_ROWS;
     const T* u[3] = {u1, u2, u3};
-    double acc[32];  // [c][k][re, im]
-#pragma unroll
-    for (int i = 0; i < NV; i++) acc[i] = 0.0;
-    for (int x0 = 0; x0 < nx; x0 += 64 * CH) {
-        double v[CH][3];
-        double2 e[CH][K + 1];
+    double2 e[CH][K];
+    auto twiddles = [&](int x0) {
 #pragma unroll
         for (int j = 0; j < CH; j++) {
             const int x = x0 + 64 * j + lane;
-            const bool ok = x < nx;
-            const long s = row * px + (ok ? x : 0);
 #pragma unroll
-            for (int c = 0; c < 3; c++) v[j][c] = ok ? (double)u[c][s] : 0.0;
-#pragma unroll
-            for (int k = 0; k <= K; k++) e[j][k] = twiddle(twx, k * (ok ? x : 0), nx, -1);
+            for (int k = 1; k <= K; k++) e[j][k - 1] = twiddle(twx, k * (x < nx ? x : 0), nx, -1);
         }
+    };
+    twiddles(0);
+    for (long row = row0; row < min(row0 + RF_ROWS, rows); row++) {  // uniform per wavefront
+        double acc[SL];
 #pragma unroll
-        for (int j = 0; j < CH; j++)
+        for (int i = 0; i < SL; i++) acc[i] = 0.0;
+        for (int x0 = 0; x0 < nx; x0 += 64 * CH) {
+            if (nx > 64 * CH) twiddles(x0);
+            double v[CH][3];
 #pragma unroll
-            for (int k = 0; k <= K; k++)
+            for (int j = 0; j < CH; j++) {
+                const int x = x0 + 64 * j + lane;
+                const bool ok = x < nx;
+                const long s = row * px + (ok ? x : 0);
+#pragma unroll
+                for (int c = 0; c < 3; c++) v[j][c] = ok ? (double)u[c][s] : 0.0;
+            }
+#pragma unroll
+            for (int j = 0; j < CH; j++)
 #pragma unroll
                 for (int c = 0; c < 3; c++) {
-                    acc[(c * (K + 1) + k) * 2 + 0] += v[j][c] * e[j][k].x;
-                    acc[(c * (K + 1) + k) * 2 + 1] += v[j][c] * e[j][k].y;
+                    acc[c * PC] += v[j][c];
+#pragma unroll
+                    for (int k = 1; k <= K; k++) {
+                        acc[c * PC + 2 * k - 1] += v[j][c] * e[j][k - 1].x;
+                        acc[c * PC + 2 * k] += v[j][c] * e[j][k - 1].y;
+                    }
                 }
-    }
-    const double t = wave_sums<NV>(acc, lane);
-    const int idx = lane >> 1;
-    if ((lane & 1) == 0 && idx < NV) {
-        // idx = (c (K+1) + k) 2 + part
-        double* out = reinterpret_cast<double*>(A + (row * 3) * (K + 1));
-        out[idx] = t;
+        }
+        const double t = wave_sums<SL>(acc, lane);
+        const int idx = lane / (64 / SL);
+        if (lane % (64 / SL) == 0 && idx < NV) {
+            const int c = idx / PC, i = idx - c * PC;  // i = 0: re of kx = 0, whose im is 0
+            double* out = reinterpret_cast<double*>(A + (row * 3 + c) * (K + 1));
+            out[i == 0 ? 0 : i + 1] = t;
+            if (i == 0) out[1] = 0.0;
+        }
     }
 }
 
@@ -163,102 +182,83 @@ __global__ __launch_bounds__(SF_BLOCK) void sf_zsum(int nx, int ny, int nz, cons
     if (lane == 0) U[t] = make_double2(sr * inv, si * inv);
 }
 
-// pass 3b: one workgroup; the coefficients of the kept modes k2lo <= |k|^2 < k2hi,
-// in place, the others zeroed.  Forcing (band = 0): scaled by eps / (2 E_low) with
-// E_low the energy of the kept modes; band-pass (band = 1): unscaled.
+// pass 4: SF_ROWS rows of one z plane per workgroup.  The coefficients of the kept
+// modes k2lo <= |k|^2 < k2hi, the others zeroed: forcing (band = 0) scaled by eps /
+// (2 E_low) with E_low the energy of the kept modes, band-pass (band = 1) unscaled;
+// then the inverse transform along z for the plane, along y for the rows, and along
+// x with the lanes over x and the rows of a wavefront sharing the twiddles.
+constexpr int SF_ROWS = 16;
 template <int K>
-__global__ __launch_bounds__(SF_BLOCK) void sf_coef(int k2lo, int k2hi, int band, double eps,
-                                                    double2* __restrict__ C, double* __restrict__ elow_out) {
-    constexpr int NK = 2 * K + 1, NB = 3 * (K + 1) * NK, NC = NB * NK;
-    __shared__ double2 s_u[NC];
-    __shared__ double s_e[SF_BLOCK / 64];
-    double e = 0.0;
-    for (int t = threadIdx.x; t < NC; t += SF_BLOCK) {
-        const double2 s = C[t];
-        s_u[t] = s;
+__global__ __launch_bounds__(SF_BLOCK) void sf_force(int nx, int px, int ny, int nz, int k2lo, int k2hi, int band,
+                                                     double eps, const double2* __restrict__ U,
+                                                     const double2* __restrict__ twx, const double2* __restrict__ twy,
+                                                     const double2* __restrict__ twz, double* __restrict__ elow_out,
+                                                     double* __restrict__ fx, double* __restrict__ fy,
+                                                     double* __restrict__ fz) {
+    constexpr int NK = 2 * K + 1, NH = 3 * (K + 1), NB = NH * NK, NC = NB * NK, W = SF_BLOCK / 64;
+    __shared__ double2 s_u[NC], s_g[NB], s_h[SF_ROWS][NH];
+    __shared__ double s_e[W];
+    const int chunks = (ny + SF_ROWS - 1) / SF_ROWS;
+    const int z = blockIdx.x / chunks, y0 = (blockIdx.x - z * chunks) * SF_ROWS, nr = min(SF_ROWS, ny - y0);
+    auto k_squared = [](int t) {
         const int kz = t % NK - K, b = t / NK;
         const int ky = b % NK - K, kx = (b / NK) % (K + 1);
-        const int k2 = kx * kx + ky * ky + kz * kz;
-        if (k2 >= k2lo && k2 < k2hi) e += (kx == 0 ? 0.5 : 1.0) * (s.x * s.x + s.y * s.y);
+        return kx * kx + ky * ky + kz * kz;
+    };
+    double e = 0.0;
+    for (int t = threadIdx.x; t < NC; t += SF_BLOCK) {
+        const double2 s = U[t];
+        const int k2 = k_squared(t);
+        const bool in = k2 >= k2lo && k2 < k2hi;
+        s_u[t] = in ? s : make_double2(0.0, 0.0);
+        if (in) e += ((t / NK / NK) % (K + 1) == 0 ? 0.5 : 1.0) * (s.x * s.x + s.y * s.y);
     }
     for (int off = 32; off > 0; off >>= 1) e += __shfl_xor(e, off, 64);
     if ((threadIdx.x & 63) == 0) s_e[threadIdx.x >> 6] = e;
     __syncthreads();
     double elow = 0.0;
-    for (int w = 0; w < SF_BLOCK / 64; w++) elow += s_e[w];
+    for (int w = 0; w < W; w++) elow += s_e[w];
     const double alpha = band ? 1.0 : (elow > 0.0 ? 0.5 * eps / elow : 0.0);
-    for (int t = threadIdx.x; t < NC; t += SF_BLOCK) {
-        const int kz = t % NK - K, b = t / NK;
-        const int ky = b % NK - K, kx = (b / NK) % (K + 1);
-        const int k2 = kx * kx + ky * ky + kz * kz;
-        const bool in = k2 >= k2lo && k2 < k2hi;
-        C[t] = in ? make_double2(alpha * s_u[t].x, alpha * s_u[t].y) : make_double2(0.0, 0.0);
+    if (blockIdx.x == 0 && threadIdx.x == 0) *elow_out = elow;
+    for (int t = threadIdx.x; t < NB; t += SF_BLOCK) {  // [c][kx][ky]
+        double2 s = make_double2(0.0, 0.0);
+        for (int kz = -K; kz <= K; kz++) {
+            const double2 c = s_u[t * NK + (kz + K)];
+            const double2 p = cmul(make_double2(alpha * c.x, alpha * c.y), twiddle(twz, kz * z, nz, +1));
+            s.x += p.x;
+            s.y += p.y;
+        }
+        s_g[t] = s;
     }
-    if (threadIdx.x == 0) *elow_out = elow;
-}
-
-// pass 4: G(c, kx, ky, z); one thread per output
-template <int K>
-__global__ __launch_bounds__(SF_BLOCK) void sf_cols_inv(int nz, const double2* __restrict__ C,
-                                                        const double2* __restrict__ twz, double2* __restrict__ G) {
-    constexpr int NK = 2 * K + 1, NB = 3 * (K + 1) * NK;
-    const long t = blockIdx.x * (long)SF_BLOCK + threadIdx.x;
-    if (t >= (long)nz * NB) return;
-    const int b = (int)(t % NB), z = (int)(t / NB);
-    double2 s = make_double2(0.0, 0.0);
-    for (int kz = -K; kz <= K; kz++) {
-        const double2 p = cmul(C[b * NK + (kz + K)], twiddle(twz, kz * z, nz, +1));
-        s.x += p.x;
-        s.y += p.y;
+    __syncthreads();
+    for (int t = threadIdx.x; t < nr * NH; t += SF_BLOCK) {
+        const int r = t / NH, ck = t - r * NH, y = y0 + r;  // ck = c (K + 1) + kx
+        double2 s = make_double2(0.0, 0.0);
+        for (int ky = -K; ky <= K; ky++) {
+            const double2 p = cmul(s_g[ck * NK + (ky + K)], twiddle(twy, ky * y, ny, +1));
+            s.x += p.x;
+            s.y += p.y;
+        }
+        s_h[r][ck] = s;
     }
-    G[t] = s;  // [z][c][kx][ky]
-}
-
-// pass 5: H(c, kx, y, z); one thread per output
-template <int K>
-__global__ __launch_bounds__(SF_BLOCK) void sf_rows_inv(int ny, int nz, const double2* __restrict__ G,
-                                                        const double2* __restrict__ twy, double2* __restrict__ H) {
-    constexpr int NK = 2 * K + 1, NB = 3 * (K + 1) * NK, NH = 3 * (K + 1);
-    const long t = blockIdx.x * (long)SF_BLOCK + threadIdx.x;
-    if (t >= (long)ny * nz * NH) return;
-    const int ck = (int)(t % NH);                  // c * (K+1) + kx
-    const long row = t / NH;
-    const int y = (int)(row % ny), z = (int)(row / ny);
-    double2 s = make_double2(0.0, 0.0);
-    for (int ky = -K; ky <= K; ky++) {
-        const double2 p = cmul(G[(long)z * NB + ck * NK + (ky + K)], twiddle(twy, ky * y, ny, +1));
-        s.x += p.x;
-        s.y += p.y;
-    }
-    H[t] = s;  // [row][c][kx]
-}
-
-// pass 6: the force field, one wavefront per (y, z) row: the row's coefficients are
-// the same for every lane (read once into scalar registers), the lanes run over x
-template <int K>
-__global__ __launch_bounds__(SF_BLOCK) void sf_force(int nx, int px, int ny, int nz, const double2* __restrict__ H,
-                                                     const double2* __restrict__ twx, double* __restrict__ fx,
-                                                     double* __restrict__ fy, double* __restrict__ fz) {
-    const int lane = threadIdx.x & 63;
-    const long row = (long)blockIdx.x * (SF_BLOCK / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    if (row >= (long)ny * nz) return;  // uniform per wavefront
-    double2 h[3][K + 1];
-#pragma unroll
-    for (int c = 0; c < 3; c++)
-#pragma unroll
-        for (int k = 0; k <= K; k++) h[c][k] = H[(row * 3 + c) * (K + 1) + k];
+    __syncthreads();
     double* const f[3] = {fx, fy, fz};
-    for (int x = lane; x < nx; x += 64) {
-        double2 e[K + 1];
+    for (int x = threadIdx.x & 63; x < nx; x += 64) {
+        double2 w[K + 1];
 #pragma unroll
-        for (int k = 1; k <= K; k++) e[k] = twiddle(twx, k * x, nx, +1);
-        const long s = row * px + x;
+        for (int k = 1; k <= K; k++) w[k] = twiddle(twx, k * x, nx, +1);
+        for (int r = threadIdx.x >> 6; r < nr; r += W) {
+            const long s = ((long)z * ny + y0 + r) * px + x;
 #pragma unroll
-        for (int c = 0; c < 3; c++) {
-            double v = h[c][0].x;
+            for (int c = 0; c < 3; c++) {
+                double v = s_h[r][c * (K + 1)].x;
 #pragma unroll
-            for (int k = 1; k <= K; k++) v += 2.0 * (h[c][k].x * e[k].x - h[c][k].y * e[k].y);
-            f[c][s] = v;
+                for (int k = 1; k <= K; k++) {
+                    const double2 h = s_h[r][c * (K + 1) + k];
+                    v += 2.0 * (h.x * w[k].x - h.y * w[k].y);
+                }
+                f[c][s] = v;
+            }
         }
     }
 }
@@ -269,19 +269,16 @@ hipError_t spectral_k(const SpectralWork& w, const Grid& G, int k2lo, int k2hi, 
     constexpr int NK = 2 * K + 1, NB = 3 * (K + 1) * NK;
     const int nx = G.nx, ny = G.ny, nz = G.nz;
     const long rows = (long)ny * nz;
-    hipLaunchKernelGGL((sf_rows_fwd<K, T>), dim3((rows + 3) / 4), dim3(SF_BLOCK), 0, st, nx, G.px, ny, nz, u1, u2, u3,
-                       w.twx, w.A);
+    constexpr int RPB = SF_BLOCK / 64 * RF_ROWS;
+    hipLaunchKernelGGL((sf_rows_fwd<K, T>), dim3((rows + RPB - 1) / RPB), dim3(SF_BLOCK), 0, st, nx, G.px, ny, nz, u1,
+                       u2, u3, w.twx, w.A);
     constexpr int NC = NB * NK, WPB = SF_BLOCK / 64;
     hipLaunchKernelGGL((sf_cols_fwd<K>), dim3((nz * NB + WPB - 1) / WPB), dim3(SF_BLOCK), 0, st, ny, nz, w.A, w.twy,
                        w.B);
     hipLaunchKernelGGL((sf_zsum<K>), dim3((NC + WPB - 1) / WPB), dim3(SF_BLOCK), 0, st, nx, ny, nz, w.B, w.twz, w.C);
-    hipLaunchKernelGGL((sf_coef<K>), dim3(1), dim3(SF_BLOCK), 0, st, k2lo, k2hi, band, eps, w.C, w.elow);
-    hipLaunchKernelGGL((sf_cols_inv<K>), dim3((nz * NB + SF_BLOCK - 1) / SF_BLOCK), dim3(SF_BLOCK), 0, st, nz, w.C,
-                       w.twz, w.G);
-    hipLaunchKernelGGL((sf_rows_inv<K>), dim3((rows * 3 * (K + 1) + SF_BLOCK - 1) / SF_BLOCK), dim3(SF_BLOCK), 0, st,
-                       ny, nz, w.G, w.twy, w.A);  // H reuses A
-    hipLaunchKernelGGL((sf_force<K>), dim3((rows + 3) / 4), dim3(SF_BLOCK), 0, st, nx, G.px, ny, nz, w.A,
-                       w.twx, fx, fy, fz);
+    const int chunks = (ny + SF_ROWS - 1) / SF_ROWS;
+    hipLaunchKernelGGL((sf_force<K>), dim3((unsigned)chunks * nz), dim3(SF_BLOCK), 0, st, nx, G.px, ny, nz, k2lo, k2hi,
+                       band, eps, w.C, w.twx, w.twy, w.twz, w.elow, fx, fy, fz);
     return hipGetLastError();
 }
 
@@ -304,10 +301,9 @@ hipError_t spectral_dispatch(const SpectralWork& w, const Grid& G, int kc, int k
 size_t spectral_work_doubles(int nx, int ny, int nz, int kc) {
     const size_t K = (size_t)(kc - 1), NK = 2 * K + 1, NB = 3 * (K + 1) * NK;
     const size_t rows = (size_t)ny * nz;
-    const size_t cplx = rows * 3 * (K + 1)      // A / H
+    const size_t cplx = rows * 3 * (K + 1)      // A
                         + (size_t)nz * NB        // B
                         + NB * NK                // C
-                        + (size_t)nz * NB        // G
                         + (size_t)nx + ny + nz;  // twiddle tables
     return 2 * cplx + 1;                         // + E_low
 }
@@ -321,8 +317,6 @@ void spectral_work_layout(SpectralWork& w, double* base, int nx, int ny, int nz,
     p += (size_t)nz * NB;
     w.C = p;
     p += NB * NK;
-    w.G = p;
-    p += (size_t)nz * NB;
     w.twx = p;
     p += nx;
     w.twy = p;
