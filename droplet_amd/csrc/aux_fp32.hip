@@ -31,17 +31,6 @@ __global__ void to_shifted(Grid G, ShiftRef r, const double* __restrict__ pop64,
     mac32[4 * ns + s] = (float)mac64[4 * ns + s];
 }
 
-__global__ void pops_from_shifted(Grid G, ShiftRef r, const float* __restrict__ pop32, double* __restrict__ out,
-                                  int set) {
-    const int64_t ns = G.ns, s = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (s >= G.slots()) return;
-    sforx<0, 15>([&](auto qc) {
-        constexpr int q = decltype(qc)::value;
-        const double ref = set == 0 ? r.fr[q] : weightE<q>();
-        out[q * ns + s] = ref + (double)pop32[(set * 15 + q) * ns + s];
-    });
-}
-
 __global__ void pops_to_shifted(Grid G, ShiftRef r, const double* __restrict__ in, float* __restrict__ pop32,
                                 int set) {
     const int64_t ns = G.ns, s = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
@@ -226,11 +215,6 @@ __global__ __launch_bounds__(ZM32_NT) void les_tau_fp32_zm(Grid G, Phys P, const
 hipError_t launch_to_shifted(const Grid& G, const ShiftRef& r, const double* pop64, const double* mac64, float* pop32,
                              float* mac32, hipStream_t st) {
     hipLaunchKernelGGL(to_shifted, grid_for(G.slots()), dim3(256), 0, st, G, r, pop64, mac64, pop32, mac32);
-    return hipGetLastError();
-}
-hipError_t launch_pops_from_shifted(const Grid& G, const ShiftRef& r, const float* pop32, double* pop64, int set,
-                                    hipStream_t st) {
-    hipLaunchKernelGGL(pops_from_shifted, grid_for(G.slots()), dim3(256), 0, st, G, r, pop32, pop64, set);
     return hipGetLastError();
 }
 hipError_t launch_pops_to_shifted(const Grid& G, const ShiftRef& r, const double* pop64, float* pop32, int set,

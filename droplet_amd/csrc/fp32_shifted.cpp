@@ -22,6 +22,10 @@ static const double kF[15] = {-7.0 / 3.0, 1.0 / 3.0, 1.0 / 3.0, 1.0 / 3.0, 1.0 /
                               1.0 / 24.0, 1.0 / 24.0, 1.0 / 24.0, 1.0 / 24.0, 1.0 / 24.0, 1.0 / 24.0, 1.0 / 24.0,
                               1.0 / 24.0};
 
+static const double kE[15] = {2.0 / 9.0, 1.0 / 9.0, 1.0 / 9.0, 1.0 / 9.0, 1.0 / 9.0, 1.0 / 9.0, 1.0 / 9.0,
+                              1.0 / 72.0, 1.0 / 72.0, 1.0 / 72.0, 1.0 / 72.0, 1.0 / 72.0, 1.0 / 72.0, 1.0 / 72.0,
+                              1.0 / 72.0};
+
 // reference phi populations of the continuous phase at rest: H phi1 + F p0(phi1)
 static ShiftRef shift_ref(const drp_config& c) {
     ShiftRef r;
@@ -138,18 +142,16 @@ int fp32_macro_fp64_view(drp_lattice* L, const double** mac) {
 }
 
 int fp32_get_macro(drp_lattice* L, int field, double* host) {
-    const double* m = nullptr;
-    int rc = fp32_macro_fp64_view(L, &m);
-    if (rc) return rc;
-    return nodes_to_host(L, m + field * L->G.ns, 1, host);
+    HostRef ref;
+    ref.r[0] = field == DRP_FIELD_PHI ? L->cfg.phi1 : (field == DRP_FIELD_P ? 1.0 / 3.0 : 0.0);
+    return nodes_to_host(L, (const float*)L->mac[L->cur] + field * L->G.ns, 1, ref, host);
 }
 
 int fp32_get_populations(drp_lattice* L, int set, double* host) {
-    DevBuf tmp;
-    HIP_TRY32(hipMalloc(&tmp.p, 15 * L->G.ns * sizeof(double)));
-    HIP_TRY32(launch_pops_from_shifted(L->G, shift_ref(L->cfg), (const float*)L->pop[L->cur], (double*)tmp.p, set,
-                                       L->stream));
-    return nodes_to_host(L, (const double*)tmp.p, 15, host);
+    const ShiftRef s = shift_ref(L->cfg);
+    HostRef ref;
+    for (int q = 0; q < 15; q++) ref.r[q] = set == DRP_POP_PHI ? s.fr[q] : kE[q];
+    return nodes_to_host(L, (const float*)L->pop[L->cur] + set * 15 * L->G.ns, 15, ref, host);
 }
 
 int fp32_set_populations(drp_lattice* L, int set, const double* host, int which) {

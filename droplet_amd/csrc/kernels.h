@@ -150,8 +150,6 @@ struct ShiftRef {
 };
 hipError_t launch_to_shifted(const Grid& G, const ShiftRef& r, const double* pop64, const double* mac64, float* pop32,
                              float* mac32, hipStream_t st);
-hipError_t launch_pops_from_shifted(const Grid& G, const ShiftRef& r, const float* pop32, double* pop64, int set,
-                                    hipStream_t st);
 hipError_t launch_pops_to_shifted(const Grid& G, const ShiftRef& r, const double* pop64, float* pop32, int set,
                                   hipStream_t st);
 hipError_t launch_macro_from_shifted(const Grid& G, double phi1, const float* mac32, double* mac64, hipStream_t st);

@@ -128,26 +128,6 @@ static Grid choose_layout(const drp_config& c, bool pad_rows) {
 
 // One array at a time through a buffer without row padding, or straight where the
 // rows have none; in one copy where the arrays are back to back too.
-int nodes_to_host(drp_lattice* L, const double* nodes, int count, double* host) {
-    const Grid& G = L->G;
-    const size_t n = (size_t)L->n;
-    if (G.px == G.nx && (G.ns == L->n || count == 1)) {
-        HIP_TRY(hipMemcpyAsync(host, nodes, count * n * sizeof(double), hipMemcpyDeviceToHost, L->stream));
-    } else {
-        if (G.px != G.nx && !L->pack) HIP_TRY(hipMalloc((void**)&L->pack, n * sizeof(double)));
-        for (int k = 0; k < count; k++) {
-            const double* src = nodes + k * G.ns;
-            if (G.px != G.nx) {
-                HIP_TRY(launch_pack_rows(G.nx, (int64_t)G.ny * G.nz, G.px, src, L->pack, L->stream));
-                src = L->pack;
-            }
-            HIP_TRY(hipMemcpyAsync(host + k * n, src, n * sizeof(double), hipMemcpyDeviceToHost, L->stream));
-        }
-    }
-    HIP_TRY(hipStreamSynchronize(L->stream));
-    return DRP_OK;
-}
-
 int nodes_from_host(drp_lattice* L, const double* host, int count, double* nodes) {
     const Grid& G = L->G;
     const size_t n = (size_t)L->n;
@@ -302,6 +282,8 @@ int lattice_alloc(drp_lattice* L) {
         }
         return DRP_OK;
     };
+    host_io_retain();
+    L->host_io = true;
     if (!L->stream) {
         HIP_TRY(hipStreamCreateWithFlags(&L->stream, hipStreamNonBlocking));
         L->owns_stream = true;
@@ -369,6 +351,8 @@ int lattice_alloc(drp_lattice* L) {
 
 void lattice_free(drp_lattice* L) {
     if (L->stream) (void)hipStreamSynchronize(L->stream);
+    if (L->host_io) host_io_release();
+    L->host_io = false;
     for (int k = 0; k < 2; k++) {
         if (L->pop[k]) (void)hipFree(L->pop[k]);
         if (L->mac[k]) (void)hipFree(L->mac[k]);

@@ -14,6 +14,7 @@ struct drp_lattice {
     int dev = 0;
     hipStream_t stream = nullptr;
     bool owns_stream = false;   // false for members of a batch (shared stream)
+    bool host_io = false;       // counted by host_io_retain
     int64_t n = 0;         // nodes
     drp::Grid G{};         // layout of the population, field, force and tau arrays (choose_layout)
     int64_t step = 0;      // reference loop counter of the last completed step
@@ -60,9 +61,17 @@ void stats_from_sums(const drp_lattice* L, const double* sums, const uint64_t* r
 // step old) or for a replaced state (fresh = true, all neighbours current)
 int les_update_tau(drp_lattice* L, bool fresh);
 
-// `count` node arrays (G.ns apart) to contiguous host arrays of n doubles, and back;
-// to the host: returns when they are there
+// host_io.hip: `count` node arrays (G.ns apart) to contiguous host arrays of n doubles;
+// returns when they are there.  FP32 arrays hold deviations from ref.r[array].
+struct HostRef {
+    double r[15] = {};
+};
 int nodes_to_host(drp_lattice* L, const double* nodes, int count, double* host);
+int nodes_to_host(drp_lattice* L, const float* nodes, int count, const HostRef& ref, double* host);
+// a lattice that uses it exists, or no longer does
+void host_io_retain();
+void host_io_release();
+// and contiguous host arrays to node arrays (lattice.cpp)
 int nodes_from_host(drp_lattice* L, const double* host, int count, double* nodes);
 
 // spectral_diag.hip
