@@ -5,8 +5,8 @@
 // faults, at 8..10 GB/s (66 ms for the five fields of a 256^3 lattice, as long as 30 of
 // its steps).  Here a kernel drops the row padding (and widens FP32 deviations)
 // straight into pinned host memory, chunk by chunk, and several host threads copy the
-// chunks out, so that the link, the copies and the page faults overlap: 19 ms
-// (64^3: 0.63 -> 0.52, 16^3: 0.12 -> 0.09; both populations of 64^3 6.5 -> 2.4).
+// chunks out (one thread, for short arrays), so that the link, the copies and the page
+// faults overlap: 19 ms.
 //
 // The pinned chunks belong to the process: at most MAX_SLOTS of CHUNK_BYTES, made on
 // demand, shared by all lattices and threads (a transfer takes what is free, at least
@@ -33,7 +33,13 @@ namespace {
 constexpr size_t CHUNK_BYTES = (size_t)4 << 20;
 constexpr int64_t CHUNK = (int64_t)(CHUNK_BYTES / sizeof(double));
 constexpr int MAX_SLOTS = 8;
-constexpr int64_t PER_THREAD = (int64_t)1 << 17;  // doubles (1 MiB) that are worth a thread of their own (25 us to start)
+// Doubles (16 MiB) that are worth a host thread.  Shorter transfers use the caller's
+// thread alone, two chunks deep: in a program whose other threads are busy (spinning
+// OpenMP workers on every core) eight threads took 38 ms for the 60 fields of twelve
+// FP32 members of 48..128^3, one thread 18 ms; the fields of 256^3 take 86 ms with
+// one and 35 ms with eight threads there, 63 and 17 ms on idle cores.
+constexpr int64_t PER_THREAD = (int64_t)1 << 21;
+constexpr int64_t SHORT_CHUNK = (int64_t)1 << 17;  // doubles (1 MiB): smallest chunk of a transfer in parts
 
 // values [first, first + len) of the contiguous sequence of node arrays (nx ny nz
 // each), G.ns apart in memory, FP32 ones added to ref[array]
@@ -122,30 +128,42 @@ int to_host(drp_lattice* L, const Grid& G, const T* nodes, int count, const Host
     const int want = (int)std::max<int64_t>(1, std::min<int64_t>({MAX_SLOTS, cores, total / PER_THREAD}));
     std::vector<void*> slot;
     try {
-        slot = slots().take(want);
+        slot = slots().take(want == 1 && total > SHORT_CHUNK ? 2 : want);
     } catch (...) {
         return drp_fail(DRP_ERR_ALLOC, "host allocation failed");
     }
     if (slot.empty()) return drp_fail(DRP_ERR_ALLOC, "no pinned host memory");
-    const int nt = (int)slot.size();
-    const int64_t chunk = std::min(CHUNK, (total + nt - 1) / nt), chunks = (total + chunk - 1) / chunk;
+    const int nt = std::min<int>(want, (int)slot.size()), deep = want == 1 ? (int)slot.size() : 1;
+    const int64_t chunk = std::min(CHUNK, nt > 1 ? (total + nt - 1) / nt : std::max(SHORT_CHUNK, (total + 3) / 4));
+    const int64_t chunks = (total + chunk - 1) / chunk;
     int dev = 0;
     (void)hipGetDevice(&dev);
     std::atomic<int64_t> next{0};
     std::atomic<int> failed{(int)hipSuccess};
-    // each thread takes the next chunk, waits for its own slot to be filled and empties it
+    // each thread takes the next chunk, has its slot filled (with two slots the other one
+    // meanwhile), waits for it and empties it
     auto work = [&](int t, bool own_thread) {
         hipError_t e = own_thread ? hipSetDevice(dev) : hipSuccess;
-        hipEvent_t ev = nullptr;
-        if (e == hipSuccess && nt > 1) e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
-        for (int64_t c; e == hipSuccess && failed.load() == (int)hipSuccess && (c = next.fetch_add(1)) < chunks;) {
-            const int64_t first = c * chunk, len = std::min(chunk, total - first);
-            e = launch_pack(G, nodes, ref, first, len, (double*)slot[t], L->stream);
-            if (e == hipSuccess && ev) e = hipEventRecord(ev, L->stream);
-            if (e == hipSuccess) e = ev ? hipEventSynchronize(ev) : hipStreamSynchronize(L->stream);
-            if (e == hipSuccess) std::memcpy(host + first, slot[t], (size_t)len * sizeof(double));
+        hipEvent_t ev[2] = {nullptr, nullptr};
+        int64_t chunk_of[2] = {chunks, chunks};
+        for (int k = 0; k < deep && e == hipSuccess && chunks > 1; k++)
+            e = hipEventCreateWithFlags(&ev[k], hipEventDisableTiming);
+        auto fill = [&](int k) {
+            const int64_t c = chunk_of[k] = next.fetch_add(1);
+            if (c >= chunks || e != hipSuccess) return;
+            e = launch_pack(G, nodes, ref, c * chunk, std::min(chunk, total - c * chunk), (double*)slot[t + k], L->stream);
+            if (e == hipSuccess && ev[k]) e = hipEventRecord(ev[k], L->stream);
+        };
+        for (int k = 0; k < deep; k++) fill(k);
+        for (int k = 0; e == hipSuccess && chunk_of[k] < chunks && failed.load() == (int)hipSuccess; k = (k + 1) % deep) {
+            e = ev[k] ? hipEventSynchronize(ev[k]) : hipStreamSynchronize(L->stream);
+            if (e != hipSuccess) break;
+            const int64_t first = chunk_of[k] * chunk;
+            std::memcpy(host + first, slot[t + k], (size_t)std::min(chunk, total - first) * sizeof(double));
+            fill(k);
         }
-        if (ev) (void)hipEventDestroy(ev);
+        for (int k = 0; k < 2; k++)
+            if (ev[k]) (void)hipEventDestroy(ev[k]);
         if (e != hipSuccess) failed.store((int)e);
     };
     std::thread threads[MAX_SLOTS];
