@@ -142,7 +142,7 @@ static int ensure_work(drp_tape* T) {
     if (!rc && !T->acc) rc = tape_alloc(T, (void**)&T->acc, (size_t)T->nblk * 3 * sizeof(double));
     if (!rc && !T->plane) rc = tape_alloc(T, (void**)&T->plane, (size_t)L->cfg.nx * std::max(L->cfg.ny, L->cfg.nz) * sizeof(double));
     if (!rc && !T->range) {
-        rc = tape_alloc(T, (void**)&T->range, 6 * sizeof(uint64_t));
+        rc = tape_alloc(T, (void**)&T->range, RANGE_WORDS * sizeof(uint64_t));
         for (int k = 0; k < 3 && !rc; k++)
             if (launch_range_set(T->range, k, L->cfg.phi1, L->cfg.phi2, L->stream) != hipSuccess)
                 rc = drp_fail(DRP_ERR_HIP, "range initialisation failed");

@@ -115,7 +115,9 @@ __global__ void les_tau_fp32(Grid G, Phys P, const float* __restrict__ mac,
             const float sab = 0.05f * (gu[a][b] + gu[b][a]);  // 0.5 (d_b u_a + d_a u_b), gradients / 10
             sum += sab * sab;
         }
-    const double rmax = from_ordered_bits(range[2 * slot]), rmin = from_ordered_bits(range[2 * slot + 1]);
+    uint64_t mx_bits, mn_bits;
+    range_words(range, slot, mx_bits, mn_bits);
+    const double rmax = from_ordered_bits(mx_bits), rmin = from_ordered_bits(mn_bits);
     const double rg = rmax - rmin;
     const double phi = P.phi1 + (double)mac[s];
     const double frac = rg == 0.0 ? 0.0 : (phi - rmin) / rg;
@@ -146,7 +148,9 @@ __global__ __launch_bounds__(ZM32_NT) void les_tau_fp32_zm(Grid G, Phys P, const
     const int tx = threadIdx.x % ZM32_TX, ty = threadIdx.x / ZM32_TX;
     const int x = x0 + tx, y = y0 + ty;
     const bool in = x < nx && y < ny;
-    const double rmax = from_ordered_bits(range[2 * slot]), rmin = from_ordered_bits(range[2 * slot + 1]);
+    uint64_t mx_bits, mn_bits;
+    range_words(range, slot, mx_bits, mn_bits);
+    const double rmax = from_ordered_bits(mx_bits), rmin = from_ordered_bits(mn_bits);
     const double rg = rmax - rmin;
     auto fetch = [&](int zg, float (&r)[ZM32_PER][3]) {
         const int64_t zoff = nxy * wrap_zm32(zg, nz, small);

@@ -187,7 +187,9 @@ __global__ __launch_bounds__(LES_TX* LES_TY* LES_TZ) void les_tau_fp64(Grid G, P
             sum = sum + sab * sab;
         }
     const double nue = P.les_c * sqrt(2.0 * sum);
-    const double rmax = from_ordered_bits(range[2 * slot]), rmin = from_ordered_bits(range[2 * slot + 1]);
+    uint64_t mx_bits, mn_bits;
+    range_words(range, slot, mx_bits, mn_bits);
+    const double rmax = from_ordered_bits(mx_bits), rmin = from_ordered_bits(mn_bits);
     const double rg = rmax - rmin;
     double frac = (mac[s] - rmin) / rg;
     if (rg == 0.0) frac = 0.0;
@@ -249,7 +251,9 @@ __global__ __launch_bounds__(ZM_NT) void les_tau_fp64_zm(Grid G, Phys P, const d
     const int tx = threadIdx.x % ZM_TX, ty = threadIdx.x / ZM_TX;
     const int x = x0 + tx, y = y0 + ty;
     const bool in = x < G.nx && y < G.ny;
-    const double rmax = from_ordered_bits(range[2 * slot]), rmin = from_ordered_bits(range[2 * slot + 1]);
+    uint64_t mx_bits, mn_bits;
+    range_words(range, slot, mx_bits, mn_bits);
+    const double rmax = from_ordered_bits(mx_bits), rmin = from_ordered_bits(mn_bits);
     const double rg = rmax - rmin;
     // ring slot of plane z' is (z' - zs + 1) mod 3
     zm_store(zm_fetch<double, 3, 2>(G, mac, x0, y0, zs - 1, small), su[0]);
@@ -430,9 +434,9 @@ __global__ __launch_bounds__(ZM_NT) void reduce_fp64(Grid G, Phys P, const doubl
 
 // Compensated sums of the workgroups' records (fixed order: lane l of wavefront k
 // takes records l, l + 64, ... of component k, then a tree over the lanes), and the
-// phi range slot next to them, so that one small copy returns everything.
+// phi range next to them, so that one small copy returns everything.
 __global__ __launch_bounds__(64 * NPART) void reduce_final(const double* __restrict__ partial, int nblocks,
-                                                           const uint64_t* __restrict__ range_slot,
+                                                           const uint64_t* __restrict__ range, int slot,
                                                            double* __restrict__ out) {
     const int lane = threadIdx.x & 63, k = threadIdx.x >> 6;
     double s = 0.0, c = 0.0;
@@ -444,7 +448,10 @@ __global__ __launch_bounds__(64 * NPART) void reduce_final(const double* __restr
         c += co;
     }
     if (lane == 0) out[k] = s + c;
-    if (threadIdx.x < 2) reinterpret_cast<uint64_t*>(out + NPART)[threadIdx.x] = range_slot[threadIdx.x];
+    if (threadIdx.x == 0) {
+        uint64_t* const words = reinterpret_cast<uint64_t*>(out + NPART);
+        range_words(range, slot, words[0], words[1]);
+    }
 }
 
 // rows of nx doubles, `stride` apart in node arrays, to contiguous rows (or back);
@@ -460,8 +467,7 @@ __global__ __launch_bounds__(256) void pack_rows(int nx, int64_t rows, int64_t s
 }
 
 __global__ void range_set(uint64_t* range, int slot, double vmax, double vmin) {
-    range[2 * slot] = ordered_bits(vmax);
-    range[2 * slot + 1] = ordered_bits(vmin);
+    range_set_part(range, slot, threadIdx.x, ordered_bits(vmax), ordered_bits(vmin));
 }
 
 // ------------------------------------------------------------------ launchers
@@ -493,7 +499,7 @@ hipError_t launch_les_tau_fp64(const Grid& G, const Phys& ph, const double* mac,
     return hipGetLastError();
 }
 
-hipError_t launch_reduce_fp64(const Grid& G, const Phys& ph, const double* mac, const uint64_t* range_slot,
+hipError_t launch_reduce_fp64(const Grid& G, const Phys& ph, const double* mac, const uint64_t* range, int slot,
                               double* work, hipStream_t st) {
     const int mx = (G.nx + ZM_TX - 1) / ZM_TX, my = (G.ny + ZM_TY - 1) / ZM_TY;
     // columns of up to 32 planes (the two halo planes cost 2 / zc), shorter where the
@@ -505,7 +511,7 @@ hipError_t launch_reduce_fp64(const Grid& G, const Phys& ph, const double* mac, 
     hipLaunchKernelGGL(reduce_fp64, dim3(nblocks), dim3(ZM_NT), 0, st, G, ph, mac, work, mx, my, zc, items);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(reduce_final, dim3(1), dim3(64 * NPART), 0, st, (const double*)work, nblocks, range_slot,
+    hipLaunchKernelGGL(reduce_final, dim3(1), dim3(64 * NPART), 0, st, (const double*)work, nblocks, range, slot,
                        work + REDUCE_OUT);
     return hipGetLastError();
 }
@@ -524,7 +530,7 @@ hipError_t launch_unpack_rows(int nx, int64_t rows, int64_t stride, const double
 }
 
 hipError_t launch_range_set(uint64_t* range, int slot, double vmax, double vmin, hipStream_t st) {
-    hipLaunchKernelGGL(range_set, dim3(1), dim3(1), 0, st, range, slot, vmax, vmin);
+    hipLaunchKernelGGL(range_set, dim3(1), dim3(RANGE_PARTS), 0, st, range, slot, vmax, vmin);
     return hipGetLastError();
 }
 

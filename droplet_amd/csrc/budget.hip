@@ -124,7 +124,8 @@ struct BudgetArgs {
     Phys P;
     const double* old_mac;
     const double* new_mac;
-    const uint64_t* range;  // the slot of the new phi range
+    const uint64_t* range;
+    int slot;               // of the new phi range
     const double *fx, *fy, *fz;                // body force field of the step, or null
     const double *sinx, *cosx, *sinz, *cosz;   // Taylor-Green tables of the step, or null
     double tg_amp;
@@ -133,12 +134,20 @@ struct BudgetArgs {
     double* partial;  // [blocks][BPART]
 };
 
-__device__ __forceinline__ double nu_new(const BudgetArgs& a, double phn) {
-    const double rmax = from_ordered_bits(a.range[0]), rmin = from_ordered_bits(a.range[1]);
-    const double rg = rmax - rmin;
-    const double frac = rg == 0.0 ? 0.0 : (phn - rmin) / rg;
-    return frac * a.P.dnu + a.P.nu1;
-}
+// nu(phi) with the new phi range, which a kernel reads once
+struct NewNu {
+    double rmin, rg;
+    __device__ __forceinline__ explicit NewNu(const BudgetArgs& a) {
+        uint64_t mx, mn;
+        range_words(a.range, a.slot, mx, mn);
+        rmin = from_ordered_bits(mn);
+        rg = from_ordered_bits(mx) - rmin;
+    }
+    __device__ __forceinline__ double operator()(const BudgetArgs& a, double phn) const {
+        const double frac = rg == 0.0 ? 0.0 : (phn - rmin) / rg;
+        return frac * a.P.dnu + a.P.nu1;
+    }
+};
 
 // workgroup partial sums of v[k] for the columns in [k0, k1)
 template <int K0, int K1> __device__ __forceinline__ void block_partials(double (&v)[BPART], double* partial) {
@@ -258,6 +267,7 @@ __global__ __launch_bounds__(BT) __attribute__((amdgpu_waves_per_eu(4))) void bu
     const Grid& G = a.G;
     const Phys& P = a.P;
     const int64_t n = G.ns;
+    const NewNu nu_new(a);
     const Brick b = brick(G);
     // ring of the old phi, u1, u2, u3
     constexpr int NA1 = 4;
@@ -333,6 +343,7 @@ __global__ __launch_bounds__(BT) void budget_pass2(BudgetArgs a) {
     const Grid& G = a.G;
     const Phys& P = a.P;
     const int64_t n = G.ns;
+    const NewNu nu_new(a);
     const Brick b = brick(G);
     __shared__ double ring[3][NA2 * RN];
     const int lx = (int)threadIdx.x % BTX, ly = (int)threadIdx.x / BTX;
@@ -485,7 +496,8 @@ extern "C" int drp_step_energy_budget(drp_lattice* L, double* terms) {
     a.P = L->phys;
     a.old_mac = (const double*)L->mac[1 - L->cur];
     a.new_mac = (const double*)L->mac[L->cur];
-    a.range = L->range + 2 * (L->step % 3);
+    a.range = L->range;
+    a.slot = (int)(L->step % 3);
     if (sa.force_kind == FORCE_FIELD) {
         a.fx = sa.fx;
         a.fy = sa.fy;

@@ -36,6 +36,62 @@ struct Grid {
     }
 };
 
+// The global phi range of a step lives in one of three rotating slots, as
+// order-preserving integers (d3q15.h).  A slot is kept in parts, 256 bytes apart,
+// each folded into by every eighth workgroup with atomics: on one pair of addresses
+// the workgroups of a small lattice, which end together, queue.  Step with one and with
+// eight parts: 15.2 and 13.3 us at 32^3, 42.4 and 39.8 at 64^3, 25.0 and 18.5 at 64^3 in
+// FP32.  Above RANGE_PARTS_MAX_NODES the workgroups end at different times, eight parts
+// bring nothing (119 and 119 us at 96^3), and a step that reads the range pays for eight
+// loads in each workgroup (viscosity of phi, 256^3: 1984 and 2023 us, FP32 1061 and 1095):
+// there, and below RANGE_PARTS_MIN_NODES, where at most 32 workgroups fold (viscosity of
+// phi, 16^3: 11.6 and 12.1 us), only part 0 takes the folds of a step and only it is read
+// by one.  The parts that take none hold the limits that a slot is reset to, or a range
+// set on all parts, so that the fold over all of them is the range at every size.
+constexpr int RANGE_PARTS = 8, RANGE_PART_WORDS = 32;
+constexpr int RANGE_SLOT_WORDS = RANGE_PARTS * RANGE_PART_WORDS;
+constexpr int RANGE_WORDS = 3 * RANGE_SLOT_WORDS;
+constexpr int64_t RANGE_PARTS_MIN_NODES = 1 << 13, RANGE_PARTS_MAX_NODES = 1 << 19;
+// a step's mask of parts: RANGE_PARTS - 1 or 0
+inline int range_mask(int64_t nodes) {
+    return nodes >= RANGE_PARTS_MIN_NODES && nodes <= RANGE_PARTS_MAX_NODES ? RANGE_PARTS - 1 : 0;
+}
+// (max, min) of a slot; a step passes its mask
+__device__ __forceinline__ void range_words(const uint64_t* __restrict__ range, int slot, uint64_t& mx, uint64_t& mn,
+                                            int mask = RANGE_PARTS - 1) {
+    const uint64_t* r = range + slot * RANGE_SLOT_WORDS;
+    if (mask == 0) {
+        mx = r[0];
+        mn = r[1];
+        return;
+    }
+    // part 0 is read with the others: read before the branch, they would wait for it
+    uint64_t a[RANGE_PARTS], b[RANGE_PARTS];
+#pragma unroll
+    for (int p = 0; p < RANGE_PARTS; p++) {
+        a[p] = r[p * RANGE_PART_WORDS];
+        b[p] = r[p * RANGE_PART_WORDS + 1];
+    }
+    mx = a[0];
+    mn = b[0];
+#pragma unroll
+    for (int p = 1; p < RANGE_PARTS; p++) {
+        mx = a[p] > mx ? a[p] : mx;
+        mn = b[p] < mn ? b[p] : mn;
+    }
+}
+// set part p of a slot
+__device__ __forceinline__ void range_set_part(uint64_t* range, int slot, int p, uint64_t mx, uint64_t mn) {
+    range[slot * RANGE_SLOT_WORDS + p * RANGE_PART_WORDS] = mx;
+    range[slot * RANGE_SLOT_WORDS + p * RANGE_PART_WORDS + 1] = mn;
+}
+// fold a workgroup's (max, min) into its part of a slot
+__device__ __forceinline__ void range_fold(uint64_t* range, int slot, int mask, uint64_t mx, uint64_t mn) {
+    uint64_t* r = range + slot * RANGE_SLOT_WORDS + (blockIdx.x & mask) * RANGE_PART_WORDS;
+    atomicMax(reinterpret_cast<unsigned long long*>(r), (unsigned long long)mx);
+    atomicMin(reinterpret_cast<unsigned long long*>(r + 1), (unsigned long long)mn);
+}
+
 // batched launch: per-instance step arguments and first-tile offsets in device memory
 struct BatchLaunch {
     const void* args;      // StepArgs[ninst] or StepArgs32[ninst]
@@ -91,8 +147,9 @@ struct StepArgs {
     double wall_u_now;
     int wall_axis;        // 0, 2 (y) or 3 (z)
     int force_kind;
-    uint64_t* range;      // 3 slots x (max, min) as order-preserving bits
+    uint64_t* range;      // RANGE_WORDS
     int slot_read, slot_write, slot_reset;
+    int range_mask;       // parts of a slot that a step uses
     int wrap_mod;         // set by the launcher: a grid extent does not exceed the tile extent
     int model;            // 0 free energy (phi populations), 1 Allen-Cahn (phi stencil update)
     double ac_a, ac_m, ac_w;  // Allen-Cahn A, mobility M = (1 - A)/6, interface width W
@@ -131,6 +188,7 @@ struct StepArgs32 {
     int wall_axis, force_kind;
     uint64_t* range;
     int slot_read, slot_write, slot_reset;
+    int range_mask;       // parts of a slot that a step uses
     int wrap_mod;
 };
 hipError_t launch_step_fp32(const StepArgs32& a, int shape, hipStream_t st, const BatchLaunch* batch = nullptr);
@@ -178,7 +236,7 @@ constexpr int NPART = 10;
 constexpr int REDUCE_MAX_BLOCKS = 2048;
 constexpr int REDUCE_OUT = REDUCE_MAX_BLOCKS * NPART;
 constexpr int REDUCE_WORK_DOUBLES = REDUCE_OUT + 16;
-hipError_t launch_reduce_fp64(const Grid& G, const Phys& ph, const double* mac, const uint64_t* range_slot,
+hipError_t launch_reduce_fp64(const Grid& G, const Phys& ph, const double* mac, const uint64_t* range, int slot,
                               double* work, hipStream_t st);
 // rows of nx doubles, `stride` apart in node arrays, to contiguous rows, and back
 hipError_t launch_pack_rows(int nx, int64_t rows, int64_t stride, const double* nodes, double* packed, hipStream_t st);

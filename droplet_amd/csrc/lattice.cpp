@@ -294,7 +294,7 @@ int lattice_alloc(drp_lattice* L) {
         rc |= dalloc(&L->pop[k], 2 * 15 * (size_t)ns * esz);
         rc |= dalloc((void**)&L->mac[k], 5 * (size_t)ns * esz);
     }
-    if (!rc) rc = dalloc((void**)&L->range, 6 * sizeof(uint64_t));
+    if (!rc) rc = dalloc((void**)&L->range, RANGE_WORDS * sizeof(uint64_t));
     const bool noneq = L->phys.les && L->cfg.les_model == DRP_LES_NONEQ;
     if (!rc && L->phys.les && !noneq) rc = dalloc((void**)&L->tau, (size_t)n * sizeof(double));
     for (int k = 0; k < 2 && !rc && noneq; k++) rc = dalloc((void**)&L->qh[k], (size_t)n * sizeof(double));
@@ -567,6 +567,7 @@ StepArgs make_step_args(drp_lattice* L, int64_t nstep) {
     a.slot_read = (int)((nstep - 1) % 3);
     a.slot_write = (int)(nstep % 3);
     a.slot_reset = (int)((nstep + 1) % 3);
+    a.range_mask = range_mask((int64_t)c.nx * c.ny * c.nz);
     return a;
 }
 
@@ -727,7 +728,7 @@ extern "C" int drp_reduce(drp_lattice* L, drp_stats* st) {
         if (rc) return rc;
     }
     if (!L->partial) HIP_TRY(hipMalloc((void**)&L->partial, REDUCE_WORK_DOUBLES * sizeof(double)));
-    HIP_TRY(launch_reduce_fp64(L->G, L->phys, mac, L->range + 2 * (L->step % 3), L->partial,
+    HIP_TRY(launch_reduce_fp64(L->G, L->phys, mac, L->range, (int)(L->step % 3), L->partial,
                                L->stream));
     double s[NPART + 2];
     HIP_TRY(hipMemcpyAsync(s, L->partial + REDUCE_OUT, sizeof s, hipMemcpyDeviceToHost, L->stream));

@@ -24,7 +24,7 @@ struct drp_lattice {
     int cur = 0;           // which ping-pong buffer holds the current state
     void* pop[2] = {nullptr, nullptr};  // FP64: [f (15 G.ns) | g (15 G.ns)] doubles; FP32: floats
     void* mac[2] = {nullptr, nullptr};  // phi, p, u1, u2, u3 (5 G.ns)
-    uint64_t* range = nullptr;          // 3 rotating (max, min) slots of the phi range
+    uint64_t* range = nullptr;          // 3 rotating slots of the phi range (RANGE_WORDS)
     double* tau = nullptr;              // LES relaxation-time field
     double* qh[2] = {nullptr, nullptr}; // non-equilibrium LES: sqrt(Pi:Pi) per node, with the populations' parity
     double* force = nullptr;            // FORCE_FIELD / SPECTRAL: fx | fy | fz

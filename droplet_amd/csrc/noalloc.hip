@@ -63,7 +63,7 @@ extern "C" int drp_reduce_noalloc(drp_lattice* L, drp_stats* st) {
     int rc = scratch_for(L->dev, &ptr);
     if (rc) return rc;
     hipError_t e = launch_reduce_fp64(L->G, L->phys, (const double*)L->mac[L->cur],
-                                      L->range + 2 * (L->step % 3), ptr, L->stream);
+                                      L->range, (int)(L->step % 3), ptr, L->stream);
     if (e != hipSuccess) return drp_fail(DRP_ERR_HIP, "reduce launch failed: %s", hipGetErrorString(e));
     double host[NPART + 2];
     if ((e = hipMemcpyAsync(host, ptr + REDUCE_OUT, sizeof host, hipMemcpyDeviceToHost, L->stream)) != hipSuccess ||

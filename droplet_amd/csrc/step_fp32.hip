@@ -88,6 +88,16 @@ __device__ __forceinline__ void step_tile_fp32(const StepArgs32& a, int tile) {
     const int nid = mom ? tid - NN : tid;
     __builtin_assume(nid >= 0 && nid < NN);
 
+    // the phi range of the last step, first, so that it is there when phase 2 starts
+    float range = 0.0f, rminf = 0.0f;
+    if constexpr (TAUMODE == 1) {
+        uint64_t mx, mn;
+        range_words(a.range, a.slot_read, mx, mn, a.range_mask);
+        const double rmin = from_ordered_bits(mn);
+        range = (float)(from_ordered_bits(mx) - rmin);
+        rminf = (float)(rmin - a.phi1);
+    }
+
     const float* __restrict__ phi_in = a.mac_in;
     const float* __restrict__ p_in = a.mac_in + N;
     const float* __restrict__ u1_in = a.mac_in + 2 * N;
@@ -171,9 +181,6 @@ __device__ __forceinline__ void step_tile_fp32(const StepArgs32& a, int tile) {
 
     // phase 2: FP64-accumulated Laplacian and gradient, deviation F-bracket, the
     // equilibrium records, 1/tau
-    const double rmax = from_ordered_bits(a.range[2 * a.slot_read + 0]);
-    const double rmin = from_ordered_bits(a.range[2 * a.slot_read + 1]);
-    const float range = (float)(rmax - rmin), rminf = (float)(rmin - a.phi1);
     sfor32<0, IT1>([&](auto kc) {
         constexpr int k = decltype(kc)::value;
         const int r = r1 + k * RP1;
@@ -394,15 +401,10 @@ __device__ __forceinline__ void step_tile_fp32(const StepArgs32& a, int tile) {
             mx = fmax(mx, s_red[0][w]);
             mn = fmin(mn, s_red[1][w]);
         }
-        atomicMax(reinterpret_cast<unsigned long long*>(&a.range[2 * a.slot_write + 0]),
-                  (unsigned long long)ordered_bits(mx));
-        atomicMin(reinterpret_cast<unsigned long long*>(&a.range[2 * a.slot_write + 1]),
-                  (unsigned long long)ordered_bits(mn));
-        if (tile == 0) {
-            a.range[2 * a.slot_reset + 0] = ordered_bits(a.phi1);
-            a.range[2 * a.slot_reset + 1] = ordered_bits(a.phi2);
-        }
+        range_fold(a.range, a.slot_write, a.range_mask, ordered_bits(mx), ordered_bits(mn));
     }
+    if (tile == 0 && tid < RANGE_PARTS)
+        range_set_part(a.range, a.slot_reset, tid, ordered_bits(a.phi1), ordered_bits(a.phi2));
 }
 
 // Resident wavefronts per SIMD the register allocation targets: two workgroups

@@ -117,6 +117,15 @@ __device__ __forceinline__ void step_tile_fp64(const StepArgs& a, int tile) {
     const int nid = mom ? tid - NN : tid;
     __builtin_assume(nid >= 0 && nid < NN);
 
+    // the phi range of the last step, first, so that it is there when phase 2 starts
+    double rmin = 0.0, range = 0.0;
+    if constexpr (TAUMODE == TAU_PHI || TAUMODE == TAU_NONEQ) {
+        uint64_t mx, mn;
+        range_words(a.range, a.slot_read, mx, mn, a.range_mask);
+        rmin = from_ordered_bits(mn);
+        range = from_ordered_bits(mx) - rmin;
+    }
+
     const double* __restrict__ phi_in = a.mac_in;
     const double* __restrict__ p_in = a.mac_in + N;
     const double* __restrict__ u1_in = a.mac_in + 2 * N;
@@ -240,9 +249,6 @@ __device__ __forceinline__ void step_tile_fp64(const StepArgs& a, int tile) {
     __syncthreads();
 
     // ---------------- phase 2: stencils, F-bracket and tau at tile + 1 halo
-    const double rmax = from_ordered_bits(a.range[2 * a.slot_read + 0]);
-    const double rmin = from_ordered_bits(a.range[2 * a.slot_read + 1]);
-    const double range = rmax - rmin;
     static_for<0, IT1>([&](auto kc) {
         constexpr int k = decltype(kc)::value;
         const int r = r1 + k * RP1;
@@ -606,15 +612,10 @@ __device__ __forceinline__ void step_tile_fp64(const StepArgs& a, int tile) {
             mx = fmax(mx, s_red[0][w]);
             mn = fmin(mn, s_red[1][w]);
         }
-        atomicMax(reinterpret_cast<unsigned long long*>(&a.range[2 * a.slot_write + 0]),
-                  (unsigned long long)ordered_bits(mx));
-        atomicMin(reinterpret_cast<unsigned long long*>(&a.range[2 * a.slot_write + 1]),
-                  (unsigned long long)ordered_bits(mn));
-        if (tile == 0) {
-            a.range[2 * a.slot_reset + 0] = ordered_bits(a.phi1);
-            a.range[2 * a.slot_reset + 1] = ordered_bits(a.phi2);
-        }
+        range_fold(a.range, a.slot_write, a.range_mask, ordered_bits(mx), ordered_bits(mn));
     }
+    if (tile == 0 && tid < RANGE_PARTS)
+        range_set_part(a.range, a.slot_reset, tid, ordered_bits(a.phi1), ordered_bits(a.phi2));
 }
 
 // one lattice: workgroup id -> tile (XCD-contiguous)
