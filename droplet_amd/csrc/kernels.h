@@ -270,13 +270,13 @@ struct AdjArgs {
     const double* f;        // forward phi populations at step n (15 ns)
     const double* mac;      // forward macroscopic fields at step n (5 ns)
     const double* Fin;      // adjoint of f^{n+1} without its stencil part (15 ns)
-    const double* phin_in;  // stencil part of the adjoint of phi^{n+1} (n), or nullptr
+    const double* phin_in;  // stencil part of the adjoint of phi^{n+1} (n)
     const double* Gin;      // adjoint of g^{n+1} (15 ns)
     double* Fout;           // adjoint of f^n without its stencil part
     double* Gout;           // adjoint of g^n
     double* lapA;           // adjoint of lap phi at step n (n)
     double* gradA;          // adjoint of grad phi at step n (3 ns)
-    double* acc;            // [workgroups][3]: d/dtau_f, d/dkappa_g, d/dU_wall, accumulated
+    double* acc;            // [tiles][3]: d/dtau_f, d/dkappa_g, d/dU_wall, accumulated
     double tau_f, tau_g, kf, kf6, kg, T, a, b;
     double rtau_f, rtau_g, rtau_f2;  // 1 / tau_f, 1 / tau_g, 1 / (tau_f tau_f)
     double om_f, om_g;               // 1 - 1 / tau_f, 1 - 1 / tau_g
