@@ -129,7 +129,7 @@ __global__ void les_tau_fp32(Grid G, Phys P, const float* __restrict__ mac,
 // of nodes with the planes z-1, z, z+1 of u (one-node x-y halo) in a ring of
 // three LDS planes; the loads of plane z+2 are in flight into registers while
 // plane z is computed.  The arithmetic and its order are those of les_tau_fp32.
-constexpr int ZM32_TX = 64, ZM32_TY = 8, ZM32_ZC = 16;
+constexpr int ZM32_TX = 64, ZM32_TY = 8;
 constexpr int ZM32_HX = ZM32_TX + 2, ZM32_HP = ZM32_HX * (ZM32_TY + 2), ZM32_NT = ZM32_TX * ZM32_TY;
 constexpr int ZM32_PER = (ZM32_HP + ZM32_NT - 1) / ZM32_NT;
 __device__ __forceinline__ int wrap_zm32(int v, int n, bool small) {
@@ -138,12 +138,12 @@ __device__ __forceinline__ int wrap_zm32(int v, int n, bool small) {
 }
 __global__ __launch_bounds__(ZM32_NT) void les_tau_fp32_zm(Grid G, Phys P, const float* __restrict__ mac,
                                                           const uint64_t* __restrict__ range, int slot,
-                                                          float* __restrict__ tau, int tiles_x, int tiles_y) {
+                                                          float* __restrict__ tau, int tiles_x, int tiles_y, int zc) {
     __shared__ float su[3][3][ZM32_HP];  // [ring slot][component][plane node]
     const int nx = G.nx, ny = G.ny, nz = G.nz;
     const int64_t N = G.ns, nxy = (int64_t)G.px * ny;
     const int x0 = (blockIdx.x % tiles_x) * ZM32_TX, y0 = ((blockIdx.x / tiles_x) % tiles_y) * ZM32_TY;
-    const int zs = (blockIdx.x / (tiles_x * tiles_y)) * ZM32_ZC, ze = min(zs + ZM32_ZC, nz);
+    const int zs = (blockIdx.x / (tiles_x * tiles_y)) * zc, ze = min(zs + zc, nz);
     const bool small = nx <= ZM32_TX || ny <= ZM32_TY || nz <= 2;
     const int tx = threadIdx.x % ZM32_TX, ty = threadIdx.x / ZM32_TX;
     const int x = x0 + tx, y = y0 + ty;
@@ -172,12 +172,14 @@ __global__ __launch_bounds__(ZM32_NT) void les_tau_fp32_zm(Grid G, Phys P, const
                 for (int k = 0; k < 3; k++) dst[k][h] = r[i][k];
         }
     };
-    float next[ZM32_PER][3];
+    float next[ZM32_PER][3], first[2][ZM32_PER][3];
     // ring slot of plane z' is (z' - zs + 1) mod 3
-    for (int p = 0; p < 3; p++) {
-        fetch(zs - 1 + p, next);
-        store(next, su[p]);
-    }
+    fetch(zs - 1, first[0]);
+    fetch(zs, first[1]);
+    fetch(zs + 1, next);
+    store(first[0], su[0]);
+    store(first[1], su[1]);
+    store(next, su[2]);
     const int64_t col = G.node(in ? x : 0, in ? y : 0, 0);
     float phi_next = mac[col + nxy * zs];
     for (int z = zs; z < ze; z++) {
@@ -240,9 +242,10 @@ hipError_t launch_les_tau_fp32(const Grid& G, const Phys& ph, const float* mac, 
         hipLaunchKernelGGL(les_tau_fp32, grid_for(G.slots()), dim3(256), 0, st, G, ph, mac, mac_old, blk, range, slot,
                            tau);
     } else {
-        const int mx = (G.nx + ZM32_TX - 1) / ZM32_TX, my = (G.ny + ZM32_TY - 1) / ZM32_TY, mz = (G.nz + ZM32_ZC - 1) / ZM32_ZC;
+        const int mx = (G.nx + ZM32_TX - 1) / ZM32_TX, my = (G.ny + ZM32_TY - 1) / ZM32_TY;
+        const int zc = les_planes(mx * my, G.nz), mz = (G.nz + zc - 1) / zc;
         hipLaunchKernelGGL(les_tau_fp32_zm, dim3((unsigned)(mx * my * mz)), dim3(ZM32_NT), 0, st, G, ph, mac,
-                           range, slot, tau, mx, my);
+                           range, slot, tau, mx, my, zc);
     }
     return hipGetLastError();
 }

@@ -198,14 +198,14 @@ __global__ __launch_bounds__(LES_TX* LES_TY* LES_TZ) void les_tau_fp64(Grid G, P
 }
 
 // The same tau with every neighbour current (no rank blocks), marching in z: a
-// workgroup owns a ZM_TX x ZM_TY column of nodes over ZM_ZC planes and keeps the
+// workgroup owns a ZM_TX x ZM_TY column of nodes over zc planes and keeps the
 // planes z-1, z, z+1 of u (with a one-node x-y halo) in a ring of three LDS
 // planes.  While plane z is computed, the loads of plane z+2 are already in
 // flight into registers (stored into the ring slot of plane z-1 afterwards), so
 // their latency overlaps the stencil work.  u is read from L2 / HBM about
-// (66 x 10)/(64 x 8) (ZM_ZC + 2)/ZM_ZC times.  Sums are formed in the order of
+// (66 x 10)/(64 x 8) (zc + 2)/zc times.  Sums are formed in the order of
 // les_tau_fp64 (the divisions by 10 correctly rounded), so both give identical tau.
-constexpr int ZM_TX = 64, ZM_TY = 8, ZM_ZC = 16;
+constexpr int ZM_TX = 64, ZM_TY = 8;
 constexpr int ZM_HX = ZM_TX + 2, ZM_HP = ZM_HX * (ZM_TY + 2), ZM_NT = ZM_TX * ZM_TY;
 constexpr int ZM_PER = (ZM_HP + ZM_NT - 1) / ZM_NT;  // plane nodes per thread
 
@@ -243,10 +243,10 @@ template <typename T, int NC> __device__ __forceinline__ void zm_store(const ZmP
 
 __global__ __launch_bounds__(ZM_NT) void les_tau_fp64_zm(Grid G, Phys P, const double* __restrict__ mac,
                                                           const uint64_t* __restrict__ range, int slot,
-                                                          double* __restrict__ tau, int tiles_x, int tiles_y) {
+                                                          double* __restrict__ tau, int tiles_x, int tiles_y, int zc) {
     __shared__ double su[3][3][ZM_HP];  // [ring slot][component][plane node]
     const int x0 = (blockIdx.x % tiles_x) * ZM_TX, y0 = ((blockIdx.x / tiles_x) % tiles_y) * ZM_TY;
-    const int zs = (blockIdx.x / (tiles_x * tiles_y)) * ZM_ZC, ze = min(zs + ZM_ZC, G.nz);
+    const int zs = (blockIdx.x / (tiles_x * tiles_y)) * zc, ze = min(zs + zc, G.nz);
     const bool small = G.nx <= ZM_TX || G.ny <= ZM_TY || G.nz <= 2;
     const int tx = threadIdx.x % ZM_TX, ty = threadIdx.x / ZM_TX;
     const int x = x0 + tx, y = y0 + ty;
@@ -256,9 +256,12 @@ __global__ __launch_bounds__(ZM_NT) void les_tau_fp64_zm(Grid G, Phys P, const d
     const double rmax = from_ordered_bits(mx_bits), rmin = from_ordered_bits(mn_bits);
     const double rg = rmax - rmin;
     // ring slot of plane z' is (z' - zs + 1) mod 3
-    zm_store(zm_fetch<double, 3, 2>(G, mac, x0, y0, zs - 1, small), su[0]);
-    zm_store(zm_fetch<double, 3, 2>(G, mac, x0, y0, zs, small), su[1]);
-    zm_store(zm_fetch<double, 3, 2>(G, mac, x0, y0, zs + 1, small), su[2]);
+    const auto p0 = zm_fetch<double, 3, 2>(G, mac, x0, y0, zs - 1, small);
+    const auto p1 = zm_fetch<double, 3, 2>(G, mac, x0, y0, zs, small);
+    const auto p2 = zm_fetch<double, 3, 2>(G, mac, x0, y0, zs + 1, small);
+    zm_store(p0, su[0]);
+    zm_store(p1, su[1]);
+    zm_store(p2, su[2]);
     const int64_t col = G.node(in ? x : 0, in ? y : 0, 0), nxy = (int64_t)G.px * G.ny;
     double phi_next = mac[col + nxy * zs];
     for (int z = zs; z < ze; z++) {
@@ -492,9 +495,10 @@ hipError_t launch_les_tau_fp64(const Grid& G, const Phys& ph, const double* mac,
     if (blk.bx > 0 && mac_old != mac) {
         hipLaunchKernelGGL(les_tau_fp64<true>, grid, block, 0, st, G, ph, mac, mac_old, blk, range, slot, tau, tx, ty);
     } else {
-        const int mx = (G.nx + ZM_TX - 1) / ZM_TX, my = (G.ny + ZM_TY - 1) / ZM_TY, mz = (G.nz + ZM_ZC - 1) / ZM_ZC;
+        const int mx = (G.nx + ZM_TX - 1) / ZM_TX, my = (G.ny + ZM_TY - 1) / ZM_TY;
+        const int zc = les_planes(mx * my, G.nz), mz = (G.nz + zc - 1) / zc;
         hipLaunchKernelGGL(les_tau_fp64_zm, dim3((unsigned)(mx * my * mz)), dim3(ZM_TX * ZM_TY), 0, st, G, ph, mac, range,
-                           slot, tau, mx, my);
+                           slot, tau, mx, my, zc);
     }
     return hipGetLastError();
 }

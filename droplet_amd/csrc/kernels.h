@@ -212,6 +212,17 @@ hipError_t launch_pops_to_shifted(const Grid& G, const ShiftRef& r, const double
                                   hipStream_t st);
 hipError_t launch_macro_from_shifted(const Grid& G, double phi1, const float* mac32, double* mac64, hipStream_t st);
 hipError_t launch_moments_fp32(const Grid& G, const float* f, const float* g, float* mac, int which, hipStream_t st);
+// Planes a workgroup of the LES kernels marches over: 16 where that leaves four
+// workgroups per CU, else fewer, down to 2.  A short march reads its two halo planes more
+// often, from L2, but a small lattice leaves most CUs idle with a long one.  Spectral-forced
+// step with 16 and with this: FP64 92 and 71 us at 64^3, 186 and 180 at 96^3, 351 and 346 at
+// 128^3; FP32 67 and 52, 225 and 222 at 64^3 and 128^3; the same from 192^3 on.
+constexpr int LES_ZC_MIN = 2, LES_BLOCKS = 1024;
+inline int les_planes(int columns, int nz) {
+    int zc = 16;
+    while (zc > LES_ZC_MIN && (int64_t)columns * ((nz + zc - 1) / zc) < LES_BLOCKS) zc /= 2;
+    return zc;
+}
 hipError_t launch_les_tau_fp32(const Grid& G, const Phys& ph, const float* mac, const float* mac_old,
                                const LesBlocks& blk, const uint64_t* range, int slot, float* tau, hipStream_t st);
 
