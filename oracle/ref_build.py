@@ -85,7 +85,9 @@ def build(rel_source: str, exe_name: str, params: dict[str, str]) -> str:
 
 
 def available() -> bool:
-    return os.path.isdir(REF_ROOT) and os.path.exists(FC) and os.path.exists(os.path.join(MPI_PREFIX, "bin", "mpiexec"))
+    # the sources themselves: the folder may be there and empty
+    return (all(os.path.exists(os.path.join(REF_ROOT, src)) for src, _ in STANDARD.values()) and os.path.exists(FC)
+            and os.path.exists(os.path.join(MPI_PREFIX, "bin", "mpiexec")))
 
 
 
