@@ -378,7 +378,9 @@ int drp_droplet_census(drp_lattice* lat, double threshold, int64_t* count, int64
  * 0.5 (|u1_hat|^2 + |u2_hat|^2 + |u3_hat|^2), weighted 2 off the k3 = 0 plane
  * (the Nyquist plane k3 = nz/2 included, as the reference counts it), for
  * s = 0 .. nshells-1 (the reference's enesupe(s+1), an array of nx/2 + 1;
- * modes of higher shells, which it writes past that array, are dropped here). */
+ * modes of higher shells, which it writes past that array, are dropped here).
+ * The transforms' work space stays with the lattice from the first of these calls
+ * on and is freed by drp_destroy. */
 int drp_energy_spectrum(drp_lattice* lat, double* E, int nshells);
 
 /* Spectral filters of the velocity (results to host, x fastest):
