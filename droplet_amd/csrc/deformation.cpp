@@ -42,6 +42,7 @@ struct Plane {
 }  // namespace
 
 int copy_phi_plane(drp_lattice* L, int third, double* host, int* n1, int* n2) {
+    const OnDevice on(L->dev);
     const drp_config& c = L->cfg;
     const bool wall_y = c.wall_axis == DRP_WALL_Y;
     *n1 = c.nx;

@@ -123,6 +123,7 @@ hipError_t launch_pack(const Grid& G, const T* nodes, const HostRef& ref, int64_
 
 template <typename T>
 int to_host(drp_lattice* L, const Grid& G, const T* nodes, int count, const HostRef& ref, double* host) {
+    const OnDevice on(L->dev);
     const int64_t total = (int64_t)G.nx * G.ny * G.nz * count;
     const int cores = std::max(1, (int)std::thread::hardware_concurrency());
     const int want = (int)std::max<int64_t>(1, std::min<int64_t>({MAX_SLOTS, cores, total / PER_THREAD}));
@@ -136,14 +137,12 @@ int to_host(drp_lattice* L, const Grid& G, const T* nodes, int count, const Host
     const int nt = std::min<int>(want, (int)slot.size()), deep = want == 1 ? (int)slot.size() : 1;
     const int64_t chunk = std::min(CHUNK, nt > 1 ? (total + nt - 1) / nt : std::max(SHORT_CHUNK, (total + 3) / 4));
     const int64_t chunks = (total + chunk - 1) / chunk;
-    int dev = 0;
-    (void)hipGetDevice(&dev);
     std::atomic<int64_t> next{0};
     std::atomic<int> failed{(int)hipSuccess};
     // each thread takes the next chunk, has its slot filled (with two slots the other one
     // meanwhile), waits for it and empties it
     auto work = [&](int t, bool own_thread) {
-        hipError_t e = own_thread ? hipSetDevice(dev) : hipSuccess;
+        hipError_t e = own_thread ? hipSetDevice(L->dev) : hipSuccess;
         hipEvent_t ev[2] = {nullptr, nullptr};
         int64_t chunk_of[2] = {chunks, chunks};
         for (int k = 0; k < deep && e == hipSuccess && chunks > 1; k++)

@@ -129,6 +129,7 @@ static Grid choose_layout(const drp_config& c, bool pad_rows) {
 // One array at a time through a buffer without row padding, or straight where the
 // rows have none; in one copy where the arrays are back to back too.
 int nodes_from_host(drp_lattice* L, const double* host, int count, double* nodes) {
+    const OnDevice on(L->dev);
     const Grid& G = L->G;
     const size_t n = (size_t)L->n;
     if (G.px == G.nx && (G.ns == L->n || count == 1)) {

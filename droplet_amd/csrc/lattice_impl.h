@@ -43,6 +43,25 @@ struct drp_lattice {
     void* fp32_state = nullptr;         // FP32 mode: shift constants etc.
 };
 
+// The lattice's device, current for as long as one of these lives: copies between node
+// arrays and the host are called from any thread, whose current device may be another,
+// and launch kernels, record events and allocate.
+class OnDevice {
+  public:
+    explicit OnDevice(int dev) {
+        if (hipGetDevice(&prev_) == hipSuccess && prev_ != dev) other_ = hipSetDevice(dev) == hipSuccess;
+    }
+    ~OnDevice() {
+        if (other_) (void)hipSetDevice(prev_);
+    }
+    OnDevice(const OnDevice&) = delete;
+    OnDevice& operator=(const OnDevice&) = delete;
+
+  private:
+    int prev_ = 0;
+    bool other_ = false;
+};
+
 int drp_fail(int code, const char* fmt, ...);
 drp::Phys make_phys(const drp_config& c);
 int lattice_alloc(drp_lattice* L);

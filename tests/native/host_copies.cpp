@@ -1,0 +1,171 @@
+// Copies between node arrays and host memory on the HIP double: one check per run, named
+// by the first argument.  Exit status 0: it holds.
+#include <hip/hip_runtime.h>
+
+#include <cstdio>
+#include <map>
+#include <random>
+#include <thread>
+
+#include "../../droplet_amd/csrc/lattice_impl.h"
+
+int copy_phi_plane(drp_lattice* L, int third, double* host, int* n1, int* n2);
+void diag_free(drp_lattice*) {}  // the spectra's work space: not part of this program
+
+using hip_double::rt;
+
+namespace {
+
+int failures = 0;
+void check(bool ok, const char* what, const std::string& where) {
+    if (!ok) {
+        std::printf("%s: %s\n", where.c_str(), what);
+        failures++;
+    }
+}
+
+void done(int rc, const std::string& where) { check(rc == DRP_OK, drp_last_error(), where); }
+
+drp_config config(int nx, int ny, int nz, int precision, int force = DRP_FORCE_NONE) {
+    drp_config c;
+    drp_config_default(&c);
+    c.nx = nx;
+    c.ny = ny;
+    c.nz = nz;
+    c.precision = precision;
+    c.force_kind = force;
+    return c;
+}
+
+std::vector<double> values(size_t n, unsigned seed, double lo, double hi) {
+    std::mt19937 gen(seed);
+    std::uniform_real_distribution<double> d(lo, hi);
+    std::vector<double> v(n);
+    for (double& x : v) x = d(gen);
+    return v;
+}
+
+std::string where(const drp_lattice* L) {
+    return std::to_string(L->cfg.nx) + "x" + std::to_string(L->cfg.ny) + "x" + std::to_string(L->cfg.nz) +
+           (L->cfg.precision == DRP_FP64 ? " FP64" : " FP32");
+}
+
+// the lattice with random fields and populations, and a copy of every node value as the
+// entry points must give it
+struct State {
+    drp_lattice* L = nullptr;
+    std::vector<double> macro[5], pop[2], force[3];
+    explicit State(const drp_config& c, unsigned seed = 1) {
+        if (drp_create(&c, &L) != DRP_OK) {
+            std::printf("create failed: %s\n", drp_last_error());
+            std::exit(2);
+        }
+        const size_t n = (size_t)L->n;
+        L->initialized = true;
+        const bool f64 = c.precision == DRP_FP64;
+        // a value of the arrays: a random number, for FP32 as the deviation from its reference
+        auto fill = [&](void* base, int count, const double* ref, std::vector<double>* all, int first, unsigned s) {
+            for (int a = 0; a < count; a++) {
+                std::vector<double> v = values(n, s + a, 0.1, 1.0);
+                for (size_t i = 0; i < n; i++) {
+                    const size_t row = i / c.nx, at = (first + a) * L->G.ns + row * L->G.px + i % c.nx;
+                    if (f64) {
+                        ((double*)base)[at] = v[i];
+                    } else {
+                        ((float*)base)[at] = (float)v[i];
+                        v[i] = ref[a] != 0.0 ? ref[a] + (double)(float)v[i] : (double)(float)v[i];
+                    }
+                }
+                all->insert(all->end(), v.begin(), v.end());
+            }
+        };
+        const double mref[5] = {c.phi1, 1.0 / 3.0, 0.0, 0.0, 0.0};
+        for (int k = 0; k < 5; k++) fill(L->mac[L->cur], 1, &mref[k], &macro[k], k, seed * 100 + k);
+        const double E[3] = {2.0 / 9.0, 1.0 / 9.0, 1.0 / 72.0}, F[3] = {-7.0 / 3.0, 1.0 / 3.0, 1.0 / 24.0};
+        const double p0 = c.phi1 * c.T / (1.0 - c.b * c.phi1) - c.a * c.phi1 * c.phi1;
+        double ref[2][15];
+        for (int q = 0; q < 15; q++) {
+            const int w = q == 0 ? 0 : (q <= 6 ? 1 : 2);
+            ref[0][q] = (q == 0 ? c.phi1 : 0.0) + F[w] * p0;
+            ref[1][q] = E[w];
+        }
+        for (int s = 0; s < 2; s++) fill(L->pop[L->cur], 15, ref[s], &pop[s], 15 * s, seed * 100 + 10 + 20 * s);
+        if (L->force)
+            for (int k = 0; k < 3; k++) force[k] = values(n, seed * 100 + 60 + k, -1.0, 1.0);
+    }
+    State(const State&) = delete;
+    ~State() { drp_destroy(L); }
+
+    // every output call gives the values (FP32 populations: the references' own rounding)
+    void read(const char* what) const {
+        const size_t n = (size_t)L->n;
+        std::vector<double> out(15 * n);
+        for (int k = 0; k < 5; k++) {
+            done(drp_get_macro(L, k, out.data(), n), where(L));
+            check(std::memcmp(out.data(), macro[k].data(), n * sizeof(double)) == 0, what, where(L) + " field");
+        }
+        for (int s = 0; s < 2; s++) {
+            done(drp_get_populations(L, s, out.data(), 15 * n), where(L));
+            double err = 0.0;
+            for (size_t i = 0; i < 15 * n; i++) err = std::fmax(err, std::fabs(out[i] - pop[s][i]));
+            check(err <= (L->cfg.precision == DRP_FP64 ? 0.0 : 1e-15), what, where(L) + " populations");
+        }
+        if (L->force) {
+            done(drp_set_force(L, force[0].data(), force[1].data(), force[2].data(), n), where(L));
+            std::vector<double> f[3];
+            for (auto& v : f) v.resize(n);
+            done(drp_get_force(L, f[0].data(), f[1].data(), f[2].data(), n), where(L));
+            for (int k = 0; k < 3; k++) check(f[k] == force[k], what, where(L) + " force");
+        }
+    }
+
+    // the deformation's plane (x, z) at y = 2
+    void plane() const {
+        const size_t nx = L->cfg.nx, ny = L->cfg.ny, nz = L->cfg.nz;
+        std::vector<double> out(nx * nz);
+        int n1 = 0, n2 = 0;
+        done(copy_phi_plane(L, 2, out.data(), &n1, &n2), where(L));
+        bool same = (size_t)n1 == nx && (size_t)n2 == nz;
+        for (size_t z = 0; z < nz && same; z++)
+            same = std::memcmp(&out[z * nx], &macro[0][nx * (2 + ny * z)], nx * sizeof(double)) == 0;
+        check(same, "plane differs", where(L));
+    }
+};
+
+// rows without and with padding; less and more than one thread's worth of populations
+const int GRIDS[][3] = {{16, 7, 5}, {45, 22, 26}, {131, 70, 33}, {64, 96, 50}};
+
+// A lattice of device 1 while the caller's current device is 0: everything that touches
+// a stream or allocates has to run on the lattice's device, and the caller's stays.
+void devices() {
+    for (const auto& g : GRIDS)
+        for (int precision : {DRP_FP64, DRP_FP32_SHIFTED}) {
+            hipSetDevice(1);
+            State s(config(g[0], g[1], g[2], precision, DRP_FORCE_FIELD));
+            hipSetDevice(0);
+            s.read("values differ");
+            s.plane();
+            check(hip_double::current == 0, "the caller's current device changed", where(s.L));
+            for (auto& m : rt.live) check(m.second.host || m.second.dev == 1, "memory on another device", where(s.L));
+        }
+}
+
+const struct {
+    const char* name;
+    void (*run)();
+} CHECKS[] = {{"devices", devices}};
+
+}  // namespace
+
+int main(int argc, char** argv) {
+    for (const auto& c : CHECKS)
+        if (argc == 2 && std::string(argv[1]) == c.name) {
+            c.run();
+            std::map<std::string, int> kinds;
+            for (const auto& v : rt.violations) kinds[v]++;
+            for (const auto& v : kinds) check(false, (v.first + ", times " + std::to_string(v.second)).c_str(), c.name);
+            for (const auto& m : rt.live) check(false, m.second.host ? "pinned memory left" : "device memory left", c.name);
+            return failures ? 1 : 0;
+        }
+    return 3;
+}
