@@ -82,7 +82,9 @@ class Slots {
             }
             while ((int)got.size() < want && made_ < MAX_SLOTS) {
                 void* p = nullptr;
-                if (hipHostMalloc(&p, CHUNK_BYTES, hipHostMallocPortable | hipHostMallocMapped) != hipSuccess) {
+                // coherent, whatever the environment's default: an event's wait makes only such memory visible
+                if (hipHostMalloc(&p, CHUNK_BYTES, hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent) !=
+                    hipSuccess) {
                     (void)hipGetLastError();
                     break;
                 }

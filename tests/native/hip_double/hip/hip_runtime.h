@@ -205,6 +205,14 @@ inline hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) {
 }
 inline hipError_t hipEventSynchronize(hipEvent_t e) {
     if (e->stream) e->stream->wait();
+    // an event without a system-scope release makes coherent host memory visible, no other
+    bool coherent = true;
+    {
+        std::lock_guard<std::mutex> lock(hip_double::rt.m);
+        for (auto& b : hip_double::rt.live) coherent &= !b.second.host || (b.second.flags & hipHostMallocCoherent);
+    }
+    if (!coherent && !(e->flags & hipEventReleaseToSystem))
+        hip_double::rt.violation("event of device scope waited for before reading non-coherent host memory");
     return hipSuccess;
 }
 inline hipError_t hipEventElapsedTime(float* ms, hipEvent_t, hipEvent_t) { return *ms = 0.0f, hipSuccess; }

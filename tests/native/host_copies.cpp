@@ -150,10 +150,19 @@ void devices() {
         }
 }
 
+// What a kernel wrote to pinned memory is read after a wait that makes it visible.
+void visibility() {
+    for (const auto& g : GRIDS)
+        for (int precision : {DRP_FP64, DRP_FP32_SHIFTED}) {
+            State s(config(g[0], g[1], g[2], precision));
+            s.read("values differ");
+        }
+}
+
 const struct {
     const char* name;
     void (*run)();
-} CHECKS[] = {{"devices", devices}};
+} CHECKS[] = {{"devices", devices}, {"visibility", visibility}};
 
 }  // namespace
 

@@ -12,6 +12,7 @@ CSRC = os.path.join(os.path.dirname(HERE), "droplet_amd", "csrc")
 SOURCES = ["host_io.hip", "lattice.cpp", "fp32_shifted.cpp", "deformation.cpp", "aux_kernels.hip", "aux_fp32.hip"]
 CHECKS = {
     "devices": "a lattice's copies run on its own device whatever the caller's current one is",
+    "visibility": "what a kernel wrote to pinned memory is visible to the thread that reads it",
 }
 
 
