@@ -123,6 +123,35 @@ hipError_t launch_pack(const Grid& G, const T* nodes, const HostRef& ref, int64_
     return hipGetLastError();
 }
 
+// One array after the other by the runtime's own copies, for a process that can have no
+// pinned memory: packed on the device, or row by row where that has no memory either.
+template <typename T>
+int to_host_unpinned(drp_lattice* L, const Grid& G, const T* nodes, int count, const HostRef& ref, double* host) {
+    const bool doubles = sizeof(T) == sizeof(double);
+    const int64_t n = (int64_t)G.nx * G.ny * G.nz;
+    const size_t row = G.nx * sizeof(double);
+    double* const pack = doubles && G.px == G.nx ? nullptr : pack_buffer(L);
+    if (!doubles && !pack) return drp_fail(DRP_ERR_ALLOC, "no device memory to widen an array");
+    hipError_t e = hipSuccess;
+    for (int a = 0; a < count && e == hipSuccess; a++) {
+        const T* src = nodes + a * G.ns;
+        double* const dst = host + a * n;
+        if (pack) {
+            e = launch_pack(G, nodes, ref, a * n, n, pack, L->stream);
+            if (e == hipSuccess) e = hipMemcpyAsync(dst, pack, n * sizeof(double), hipMemcpyDeviceToHost, L->stream);
+        } else if (G.px == G.nx) {
+            e = hipMemcpyAsync(dst, src, n * sizeof(double), hipMemcpyDeviceToHost, L->stream);
+        } else {
+            e = hipMemcpy2DAsync(dst, row, src, G.px * sizeof(double), row, (size_t)G.ny * G.nz, hipMemcpyDeviceToHost,
+                                 L->stream);
+        }
+    }
+    const hipError_t s = hipStreamSynchronize(L->stream);
+    if (e == hipSuccess) e = s;
+    if (e != hipSuccess) return drp_fail(DRP_ERR_HIP, "copy to the host failed: %s", hipGetErrorString(e));
+    return DRP_OK;
+}
+
 template <typename T>
 int to_host(drp_lattice* L, const Grid& G, const T* nodes, int count, const HostRef& ref, double* host) {
     const OnDevice on(L->dev);
@@ -135,7 +164,7 @@ int to_host(drp_lattice* L, const Grid& G, const T* nodes, int count, const Host
     } catch (...) {
         return drp_fail(DRP_ERR_ALLOC, "host allocation failed");
     }
-    if (slot.empty()) return drp_fail(DRP_ERR_ALLOC, "no pinned host memory");
+    if (slot.empty()) return to_host_unpinned(L, G, nodes, count, ref, host);
     const int nt = std::min<int>(want, (int)slot.size()), deep = want == 1 ? (int)slot.size() : 1;
     const int64_t chunk = std::min(CHUNK, nt > 1 ? (total + nt - 1) / nt : std::max(SHORT_CHUNK, (total + 3) / 4));
     const int64_t chunks = (total + chunk - 1) / chunk;

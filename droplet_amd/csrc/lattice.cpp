@@ -126,6 +126,14 @@ static Grid choose_layout(const drp_config& c, bool pad_rows) {
     return G;
 }
 
+double* pack_buffer(drp_lattice* L) {
+    if (!L->pack && hipMalloc((void**)&L->pack, (size_t)L->n * sizeof(double)) != hipSuccess) {
+        (void)hipGetLastError();  // the caller does without
+        L->pack = nullptr;
+    }
+    return L->pack;
+}
+
 // One array at a time through a buffer without row padding, or straight where the
 // rows have none; in one copy where the arrays are back to back too.
 int nodes_from_host(drp_lattice* L, const double* host, int count, double* nodes) {

@@ -90,8 +90,10 @@ int nodes_to_host(drp_lattice* L, const float* nodes, int count, const HostRef& 
 // a lattice that uses it exists, or no longer does
 void host_io_retain();
 void host_io_release();
-// and contiguous host arrays to node arrays (lattice.cpp)
+// lattice.cpp: contiguous host arrays to node arrays
 int nodes_from_host(drp_lattice* L, const double* host, int count, double* nodes);
+// L->pack, n doubles, made on first use; null where there is no memory for it
+double* pack_buffer(drp_lattice* L);
 
 // spectral_diag.hip
 void diag_free(drp_lattice* L);

@@ -159,10 +159,27 @@ void visibility() {
         }
 }
 
+// No pinned memory at all: the values come by the runtime's own copies.
+void no_pinned_memory() {
+    rt.pinned_limit = 0;
+    for (const auto& g : GRIDS)
+        for (int precision : {DRP_FP64, DRP_FP32_SHIFTED}) {
+            State s(config(g[0], g[1], g[2], precision, DRP_FORCE_FIELD));
+            s.read("values differ");
+            // FP64 values need no memory of the device on their way either
+            if (precision == DRP_FP64) {
+                State t(config(g[0], g[1], g[2], precision, DRP_FORCE_NONE));
+                rt.device_limit = rt.device_bytes;
+                t.read("values differ without device memory");
+                rt.device_limit = SIZE_MAX;
+            }
+        }
+}
+
 const struct {
     const char* name;
     void (*run)();
-} CHECKS[] = {{"devices", devices}, {"visibility", visibility}};
+} CHECKS[] = {{"devices", devices}, {"visibility", visibility}, {"no pinned memory", no_pinned_memory}};
 
 }  // namespace
 

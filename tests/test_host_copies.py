@@ -13,6 +13,7 @@ SOURCES = ["host_io.hip", "lattice.cpp", "fp32_shifted.cpp", "deformation.cpp", 
 CHECKS = {
     "devices": "a lattice's copies run on its own device whatever the caller's current one is",
     "visibility": "what a kernel wrote to pinned memory is visible to the thread that reads it",
+    "no pinned memory": "output calls do without pinned memory",
 }
 
 
