@@ -55,17 +55,20 @@ int copy_phi_plane(drp_lattice* L, int third, double* host, int* n1, int* n2) {
         if (rc) return rc;
     }
     // the plane's rows (y or z) packed on the device: a strided copy to pageable
-    // memory goes row by row (35 us each)
-    const size_t px = L->G.px, plane = (size_t)*n1 * *n2;
+    // memory goes row by row (35 us each), and is left for where the buffer has no memory
+    const size_t px = L->G.px, row = c.nx * sizeof(double);
     const double* src = phi + third * px * (wall_y ? c.ny : 1);
     const int64_t stride = wall_y ? (int64_t)px : (int64_t)px * c.ny;
+    double* const pack = stride != c.nx ? pack_buffer(L) : nullptr;
     hipError_t e = hipSuccess;
-    if (stride != c.nx) {
-        if (!L->pack) e = hipMalloc((void**)&L->pack, (size_t)L->n * sizeof(double));
-        if (e == hipSuccess) e = drp::launch_pack_rows(c.nx, *n2, stride, src, L->pack, L->stream);
-        src = L->pack;
+    if (pack) {
+        e = drp::launch_pack_rows(c.nx, *n2, stride, src, pack, L->stream);
+        if (e == hipSuccess) e = hipMemcpyAsync(host, pack, *n2 * row, hipMemcpyDeviceToHost, L->stream);
+    } else if (stride == c.nx) {
+        e = hipMemcpyAsync(host, src, *n2 * row, hipMemcpyDeviceToHost, L->stream);
+    } else {
+        e = hipMemcpy2DAsync(host, row, src, stride * sizeof(double), row, *n2, hipMemcpyDeviceToHost, L->stream);
     }
-    if (e == hipSuccess) e = hipMemcpyAsync(host, src, plane * sizeof(double), hipMemcpyDeviceToHost, L->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(L->stream);
     if (e != hipSuccess) return drp_fail(DRP_ERR_HIP, "plane copy failed: %s", hipGetErrorString(e));
     return DRP_OK;

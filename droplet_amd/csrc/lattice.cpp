@@ -135,21 +135,29 @@ double* pack_buffer(drp_lattice* L) {
 }
 
 // One array at a time through a buffer without row padding, or straight where the
-// rows have none; in one copy where the arrays are back to back too.
+// rows have none; in one copy where the arrays are back to back too.  Without memory
+// for the buffer the runtime copies padded rows one by one.
 int nodes_from_host(drp_lattice* L, const double* host, int count, double* nodes) {
     const OnDevice on(L->dev);
     const Grid& G = L->G;
-    const size_t n = (size_t)L->n;
+    const size_t n = (size_t)L->n, row = G.nx * sizeof(double);
     if (G.px == G.nx && (G.ns == L->n || count == 1)) {
         HIP_TRY(hipMemcpyAsync(nodes, host, count * n * sizeof(double), hipMemcpyHostToDevice, L->stream));
         return DRP_OK;
     }
-    if (G.px != G.nx && !L->pack) HIP_TRY(hipMalloc((void**)&L->pack, n * sizeof(double)));
+    double* const pack = G.px != G.nx ? pack_buffer(L) : nullptr;
     for (int k = 0; k < count; k++) {
+        const double* src = host + k * n;
         double* dst = nodes + k * G.ns;
-        HIP_TRY(hipMemcpyAsync(G.px != G.nx ? L->pack : dst, host + k * n, n * sizeof(double), hipMemcpyHostToDevice,
-                               L->stream));
-        if (G.px != G.nx) HIP_TRY(launch_unpack_rows(G.nx, (int64_t)G.ny * G.nz, G.px, L->pack, dst, L->stream));
+        if (pack) {
+            HIP_TRY(hipMemcpyAsync(pack, src, n * sizeof(double), hipMemcpyHostToDevice, L->stream));
+            HIP_TRY(launch_unpack_rows(G.nx, (int64_t)G.ny * G.nz, G.px, pack, dst, L->stream));
+        } else if (G.px == G.nx) {
+            HIP_TRY(hipMemcpyAsync(dst, src, n * sizeof(double), hipMemcpyHostToDevice, L->stream));
+        } else {
+            HIP_TRY(hipMemcpy2DAsync(dst, G.px * sizeof(double), src, row, row, (size_t)G.ny * G.nz,
+                                     hipMemcpyHostToDevice, L->stream));
+        }
     }
     return DRP_OK;
 }

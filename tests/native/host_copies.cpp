@@ -119,6 +119,28 @@ struct State {
         }
     }
 
+    // new fields and populations from the host
+    void write(unsigned seed) {
+        const size_t n = (size_t)L->n;
+        for (int k = 0; k < 5; k++) macro[k] = values(n, seed + k, 0.1, 1.0);
+        done(drp_init_fields(L, macro[0].data(), macro[1].data(), macro[2].data(), macro[3].data(), macro[4].data()), where(L));
+        std::vector<double> out(n);
+        for (int k = 0; k < 5; k++) {
+            done(drp_get_macro(L, k, out.data(), n), where(L));
+            check(out == macro[k], "fields set differ", where(L));
+        }
+        plane();
+        for (int s = 0; s < 2; s++) {
+            pop[s] = values(15 * n, seed + 10 + s, 0.1, 1.0);
+            done(drp_set_populations(L, s, pop[s].data(), 15 * n), where(L));
+        }
+        for (int s = 0; s < 2; s++) {
+            out.resize(15 * n);
+            done(drp_get_populations(L, s, out.data(), 15 * n), where(L));
+            check(out == pop[s], "populations set differ", where(L));
+        }
+    }
+
     // the deformation's plane (x, z) at y = 2
     void plane() const {
         const size_t nx = L->cfg.nx, ny = L->cfg.ny, nz = L->cfg.nz;
@@ -176,10 +198,25 @@ void no_pinned_memory() {
         }
 }
 
+// No device memory beyond the lattice's own: an FP64 lattice takes and gives everything.
+void no_device_memory() {
+    for (const auto& g : GRIDS) {
+        State s(config(g[0], g[1], g[2], DRP_FP64, DRP_FORCE_FIELD));
+        rt.device_limit = rt.device_bytes;
+        s.read("values differ");
+        s.plane();
+        s.write(7);
+        rt.device_limit = SIZE_MAX;
+        check(hipGetLastError() == hipSuccess, "an error was left behind", where(s.L));
+        s.write(8);
+    }
+}
+
 const struct {
     const char* name;
     void (*run)();
-} CHECKS[] = {{"devices", devices}, {"visibility", visibility}, {"no pinned memory", no_pinned_memory}};
+} CHECKS[] = {{"devices", devices}, {"visibility", visibility}, {"no pinned memory", no_pinned_memory},
+              {"no device memory", no_device_memory}};
 
 }  // namespace
 

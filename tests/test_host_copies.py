@@ -14,6 +14,7 @@ CHECKS = {
     "devices": "a lattice's copies run on its own device whatever the caller's current one is",
     "visibility": "what a kernel wrote to pinned memory is visible to the thread that reads it",
     "no pinned memory": "output calls do without pinned memory",
+    "no device memory": "host arrays go in and out without device memory beyond the lattice's own",
 }
 
 
