@@ -45,10 +45,12 @@ struct drp_lattice {
 
 // The lattice's device, current for as long as one of these lives: copies between node
 // arrays and the host are called from any thread, whose current device may be another,
-// and launch kernels, record events and allocate.
+// and launch kernels, record events and allocate.  A launch reports through the thread's
+// last error, so one that an earlier call left there is cleared first: it is not the copy's.
 class OnDevice {
   public:
     explicit OnDevice(int dev) {
+        (void)hipGetLastError();
         if (hipGetDevice(&prev_) == hipSuccess && prev_ != dev) other_ = hipSetDevice(dev) == hipSuccess;
     }
     ~OnDevice() {

@@ -212,11 +212,31 @@ void no_device_memory() {
     }
 }
 
+// An error that an earlier HIP call of the caller's thread left behind is not a copy's.
+void earlier_error() {
+    for (const auto& g : GRIDS) {
+        State s(config(g[0], g[1], g[2], DRP_FP64, DRP_FORCE_FIELD));
+        const size_t n = (size_t)s.L->n;
+        std::vector<double> out(15 * n);
+        auto leave = [] { hip_double::last = hipErrorOutOfMemory; };
+        leave();
+        done(drp_get_macro(s.L, 0, out.data(), n), where(s.L));
+        leave();
+        done(drp_get_populations(s.L, 0, out.data(), 15 * n), where(s.L));
+        leave();
+        done(drp_set_force(s.L, s.force[0].data(), s.force[1].data(), s.force[2].data(), n), where(s.L));
+        leave();
+        done(drp_get_force(s.L, out.data(), out.data() + n, out.data() + 2 * n, n), where(s.L));
+        leave();
+        s.plane();
+    }
+}
+
 const struct {
     const char* name;
     void (*run)();
 } CHECKS[] = {{"devices", devices}, {"visibility", visibility}, {"no pinned memory", no_pinned_memory},
-              {"no device memory", no_device_memory}};
+              {"no device memory", no_device_memory}, {"earlier error", earlier_error}};
 
 }  // namespace
 

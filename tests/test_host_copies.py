@@ -15,6 +15,7 @@ CHECKS = {
     "visibility": "what a kernel wrote to pinned memory is visible to the thread that reads it",
     "no pinned memory": "output calls do without pinned memory",
     "no device memory": "host arrays go in and out without device memory beyond the lattice's own",
+    "earlier error": "an error that an earlier call left behind does not fail a copy",
 }
 
 
