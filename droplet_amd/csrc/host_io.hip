@@ -8,14 +8,14 @@
 // chunks out (one thread, for short arrays), so that the link, the copies and the page
 // faults overlap: 19 ms.
 //
-// The pinned chunks belong to the process: at most MAX_SLOTS of CHUNK_BYTES, made on
-// demand, shared by all lattices and threads (a transfer takes what is free, at least
-// one), and freed with the last lattice.
+// The pinned chunks belong to the process: at most POOL_SLOTS of CHUNK_BYTES (64 MiB),
+// made on demand, shared by all lattices and threads, and freed with the last lattice.  A
+// transfer takes what is free and never waits for another one, whose stream may stand
+// still for as long as its owner likes: one that finds none goes by the runtime's copies.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <atomic>
-#include <condition_variable>
 #include <cstring>
 #include <mutex>
 #include <system_error>
@@ -32,7 +32,8 @@ namespace {
 
 constexpr size_t CHUNK_BYTES = (size_t)4 << 20;
 constexpr int64_t CHUNK = (int64_t)(CHUNK_BYTES / sizeof(double));
-constexpr int MAX_SLOTS = 8;
+constexpr int MAX_SLOTS = 8;               // chunks of one transfer
+constexpr int POOL_SLOTS = 2 * MAX_SLOTS;  // chunks of the process
 // Doubles (16 MiB) that are worth a host thread.  Shorter transfers use the caller's
 // thread alone, two chunks deep: in a program whose other threads are busy (spinning
 // OpenMP workers on every core) eight threads took 38 ms for the 60 fields of twelve
@@ -69,43 +70,43 @@ class Slots {
         made_ -= (int)free_.size();
         free_.clear();
     }
-    // up to `want` chunks, at least one unless pinned memory cannot be had at all
+    // up to `want` chunks: fewer, or none, where other transfers hold them or pinned
+    // memory cannot be had
     std::vector<void*> take(int want) {
-        std::unique_lock<std::mutex> lock(mu_);
-        free_.reserve(MAX_SLOTS);  // so that giving back cannot fail
         std::vector<void*> got;
         got.reserve(want);
-        for (;;) {
+        int make = 0;
+        {
+            std::lock_guard<std::mutex> lock(mu_);
+            free_.reserve(POOL_SLOTS);  // so that giving back cannot fail
             while ((int)got.size() < want && !free_.empty()) {
                 got.push_back(free_.back());
                 free_.pop_back();
             }
-            while ((int)got.size() < want && made_ < MAX_SLOTS) {
-                void* p = nullptr;
-                // coherent, whatever the environment's default: an event's wait makes only such memory visible
-                if (hipHostMalloc(&p, CHUNK_BYTES, hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent) !=
-                    hipSuccess) {
-                    (void)hipGetLastError();
-                    break;
-                }
-                made_++;
-                got.push_back(p);
-            }
-            if (!got.empty() || made_ == 0) return got;
-            cv_.wait(lock);  // other transfers hold them all
+            make = std::min(want - (int)got.size(), POOL_SLOTS - made_);
+            made_ += make;
         }
+        for (; make > 0; make--) {
+            void* p = nullptr;
+            // coherent, whatever the environment's default: an event's wait makes only such memory visible
+            if (hipHostMalloc(&p, CHUNK_BYTES, hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent) !=
+                hipSuccess) {
+                (void)hipGetLastError();
+                std::lock_guard<std::mutex> lock(mu_);
+                made_ -= make;
+                break;
+            }
+            got.push_back(p);
+        }
+        return got;
     }
     void give(const std::vector<void*>& v) {
-        {
-            std::lock_guard<std::mutex> lock(mu_);
-            free_.insert(free_.end(), v.begin(), v.end());
-        }
-        cv_.notify_all();
+        std::lock_guard<std::mutex> lock(mu_);
+        free_.insert(free_.end(), v.begin(), v.end());
     }
 
   private:
     std::mutex mu_;
-    std::condition_variable cv_;
     std::vector<void*> free_;
     int made_ = 0, users_ = 0;
 };
@@ -123,8 +124,8 @@ hipError_t launch_pack(const Grid& G, const T* nodes, const HostRef& ref, int64_
     return hipGetLastError();
 }
 
-// One array after the other by the runtime's own copies, for a process that can have no
-// pinned memory: packed on the device, or row by row where that has no memory either.
+// One array after the other by the runtime's own copies, for a transfer that gets no
+// pinned chunk: packed on the device, or row by row where that has no memory for it.
 template <typename T>
 int to_host_unpinned(drp_lattice* L, const Grid& G, const T* nodes, int count, const HostRef& ref, double* host) {
     const bool doubles = sizeof(T) == sizeof(double);

@@ -2,8 +2,12 @@
 // by the first argument.  Exit status 0: it holds.
 #include <hip/hip_runtime.h>
 
+#include <atomic>
+#include <chrono>
 #include <cstdio>
+#include <future>
 #include <map>
+#include <memory>
 #include <random>
 #include <thread>
 
@@ -16,7 +20,7 @@ using hip_double::rt;
 
 namespace {
 
-int failures = 0;
+std::atomic<int> failures{0};
 void check(bool ok, const char* what, const std::string& where) {
     if (!ok) {
         std::printf("%s: %s\n", where.c_str(), what);
@@ -232,11 +236,45 @@ void earlier_error() {
     }
 }
 
+// Transfers whose streams do not end hold as many chunks as they can get; one of another
+// lattice ends all the same.
+void independence() {
+    const drp_config c = config(104, 104, 104, DRP_FP32_SHIFTED);  // 17 million values: eight threads
+    std::vector<std::unique_ptr<State>> busy;
+    std::vector<std::thread> threads;
+    for (int k = 0; k < 3; k++) {
+        busy.emplace_back(new State(c, 2 + k));
+        busy.back()->L->stream->stall(true);
+    }
+    for (auto& b : busy) {
+        drp_lattice* L = b->L;
+        threads.emplace_back([L] {
+            std::vector<double> out(15 * (size_t)L->n);
+            done(drp_get_populations(L, 0, out.data(), out.size()), where(L));
+        });
+    }
+    std::this_thread::sleep_for(std::chrono::seconds(1));
+    State s(config(45, 22, 26, DRP_FP64));
+    std::promise<void> ended;
+    std::thread reader([&] {
+        s.read("values differ");
+        ended.set_value();
+    });
+    check(ended.get_future().wait_for(std::chrono::seconds(10)) == std::future_status::ready,
+          "a transfer waited for other lattices' transfers", "independence");
+    check(rt.pinned_blocks() <= 16, "more pinned memory than the pool's", "independence");
+    for (auto& b : busy) b->L->stream->stall(false);
+    for (auto& t : threads) t.join();
+    reader.join();
+    for (auto& b : busy) b->read("values differ");
+}
+
 const struct {
     const char* name;
     void (*run)();
 } CHECKS[] = {{"devices", devices}, {"visibility", visibility}, {"no pinned memory", no_pinned_memory},
-              {"no device memory", no_device_memory}, {"earlier error", earlier_error}};
+              {"no device memory", no_device_memory}, {"earlier error", earlier_error},
+              {"independence", independence}};
 
 }  // namespace
 
