@@ -59,7 +59,7 @@ int copy_phi_plane(drp_lattice* L, int third, double* host, int* n1, int* n2) {
     const size_t px = L->G.px, row = c.nx * sizeof(double);
     const double* src = phi + third * px * (wall_y ? c.ny : 1);
     const int64_t stride = wall_y ? (int64_t)px : (int64_t)px * c.ny;
-    double* const pack = stride != c.nx ? pack_buffer(L) : nullptr;
+    double* const pack = stride != c.nx ? pack_buffer(L, (size_t)*n1 * *n2) : nullptr;
     hipError_t e = hipSuccess;
     if (pack) {
         e = drp::launch_pack_rows(c.nx, *n2, stride, src, pack, L->stream);

@@ -131,7 +131,7 @@ int to_host_unpinned(drp_lattice* L, const Grid& G, const T* nodes, int count, c
     const bool doubles = sizeof(T) == sizeof(double);
     const int64_t n = (int64_t)G.nx * G.ny * G.nz;
     const size_t row = G.nx * sizeof(double);
-    double* const pack = doubles && G.px == G.nx ? nullptr : pack_buffer(L);
+    double* const pack = doubles && G.px == G.nx ? nullptr : pack_buffer(L, n);
     if (!doubles && !pack) return drp_fail(DRP_ERR_ALLOC, "no device memory to widen an array");
     hipError_t e = hipSuccess;
     for (int a = 0; a < count && e == hipSuccess; a++) {

@@ -126,10 +126,17 @@ static Grid choose_layout(const drp_config& c, bool pad_rows) {
     return G;
 }
 
-double* pack_buffer(drp_lattice* L) {
-    if (!L->pack && hipMalloc((void**)&L->pack, (size_t)L->n * sizeof(double)) != hipSuccess) {
-        (void)hipGetLastError();  // the caller does without
+double* pack_buffer(drp_lattice* L, size_t doubles) {
+    if (L->pack_cap < doubles) {
+        if (L->pack) (void)hipFree(L->pack);
         L->pack = nullptr;
+        L->pack_cap = 0;
+        if (hipMalloc((void**)&L->pack, doubles * sizeof(double)) == hipSuccess) {
+            L->pack_cap = doubles;
+        } else {
+            (void)hipGetLastError();  // the caller does without
+            L->pack = nullptr;
+        }
     }
     return L->pack;
 }
@@ -145,7 +152,7 @@ int nodes_from_host(drp_lattice* L, const double* host, int count, double* nodes
         HIP_TRY(hipMemcpyAsync(nodes, host, count * n * sizeof(double), hipMemcpyHostToDevice, L->stream));
         return DRP_OK;
     }
-    double* const pack = G.px != G.nx ? pack_buffer(L) : nullptr;
+    double* const pack = G.px != G.nx ? pack_buffer(L, n) : nullptr;
     for (int k = 0; k < count; k++) {
         const double* src = host + k * n;
         double* dst = nodes + k * G.ns;

@@ -33,7 +33,8 @@ struct drp_lattice {
     double* spec_adv = nullptr;         // scale-separated advection: transform work space
     drp::SpectralWork specw_adv{};
     double* uadv = nullptr;             // scale-separated advection: band-passed u1 | u2 | u3
-    double* pack = nullptr;             // one array without row padding, on its way to or from the host
+    double* pack = nullptr;             // one array (or plane) without row padding, on its way to or from the host
+    size_t pack_cap = 0;                // its doubles
     double* tg = nullptr;               // Taylor-Green sin/cos tables
     double* partial = nullptr;          // diagnostics sums (REDUCE_WORK_DOUBLES)
     double* mac64 = nullptr;            // FP32 mode: FP64 copy of the macroscopic fields
@@ -94,8 +95,8 @@ void host_io_retain();
 void host_io_release();
 // lattice.cpp: contiguous host arrays to node arrays
 int nodes_from_host(drp_lattice* L, const double* host, int count, double* nodes);
-// L->pack, n doubles, made on first use; null where there is no memory for it
-double* pack_buffer(drp_lattice* L);
+// L->pack with room for that many doubles; null where there is no memory for it
+double* pack_buffer(drp_lattice* L, size_t doubles);
 
 // spectral_diag.hip
 void diag_free(drp_lattice* L);

@@ -269,12 +269,25 @@ void independence() {
     for (auto& b : busy) b->read("values differ");
 }
 
+// A deformation plane takes a plane's worth of device memory, not a lattice's; what needs
+// more afterwards gets it.
+void plane_memory() {
+    for (const auto& g : GRIDS) {
+        State s(config(g[0], g[1], g[2], DRP_FP64, DRP_FORCE_FIELD));
+        rt.largest = 0;
+        s.plane();
+        check(rt.largest <= (size_t)g[0] * g[2] * sizeof(double), "more device memory than the plane", where(s.L));
+        s.read("values differ");
+        s.write(9);
+    }
+}
+
 const struct {
     const char* name;
     void (*run)();
 } CHECKS[] = {{"devices", devices}, {"visibility", visibility}, {"no pinned memory", no_pinned_memory},
               {"no device memory", no_device_memory}, {"earlier error", earlier_error},
-              {"independence", independence}};
+              {"independence", independence}, {"plane memory", plane_memory}};
 
 }  // namespace
 

@@ -17,6 +17,7 @@ CHECKS = {
     "no device memory": "host arrays go in and out without device memory beyond the lattice's own",
     "earlier error": "an error that an earlier call left behind does not fail a copy",
     "independence": "a copy does not wait for those of other lattices",
+    "plane memory": "a deformation plane takes a plane's worth of device memory",
 }
 
 
