@@ -119,10 +119,10 @@ static int64_t stream_stride(int64_t slots, size_t esz) {
     return ((bytes + 255) / 256 * 256 + 8192 + 256) / (int64_t)esz;
 }
 
-static Grid choose_layout(const drp_config& c, bool pad_rows) {
+static Grid choose_layout(const drp_config& c, bool apart) {
     const size_t esz = c.precision == DRP_FP64 ? sizeof(double) : sizeof(float);
-    Grid G{c.nx, c.ny, c.nz, pad_rows ? row_pitch(c.nx, c.ny, esz) : c.nx, 0};
-    G.ns = stream_stride(G.slots(), esz);
+    Grid G{c.nx, c.ny, c.nz, apart ? row_pitch(c.nx, c.ny, esz) : c.nx, 0};
+    G.ns = apart ? stream_stride(G.slots(), esz) : G.slots();
     return G;
 }
 
@@ -274,7 +274,8 @@ int lattice_create(const drp_config* cfg, hipStream_t stream, drp_lattice** out)
     L->stream = stream;
     (void)hipGetDevice(&L->dev);
     rc = lattice_alloc(L);
-    if (rc == DRP_ERR_ALLOC && L->G.px != cfg->nx) {  // the row padding is a convenience: do without
+    // rows and arrays lie apart for speed only: back to back where there is no memory for that
+    if (rc == DRP_ERR_ALLOC && L->G.ns != L->n) {
         lattice_free(L);
         (void)hipGetLastError();  // the failed allocation is dealt with here
         const int shape = L->shape, dev = L->dev;

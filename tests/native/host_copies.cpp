@@ -282,12 +282,32 @@ void plane_memory() {
     }
 }
 
+// A lattice whose arrays back to back just fit the device is made, without row padding
+// and distances between arrays, and works.
+void tight_lattice() {
+    for (const auto& g : GRIDS)
+        for (int precision : {DRP_FP64, DRP_FP32_SHIFTED}) {
+            const size_t n = (size_t)g[0] * g[1] * g[2], value = precision == DRP_FP64 ? sizeof(double) : sizeof(float);
+            rt.device_limit = 70 * n * value + drp::RANGE_WORDS * sizeof(uint64_t);
+            {
+                State s(config(g[0], g[1], g[2], precision));
+                s.read("values differ");
+            }
+            rt.device_limit -= 1;
+            const drp_config c = config(g[0], g[1], g[2], precision);
+            drp_lattice* L = nullptr;
+            check(drp_create(&c, &L) == DRP_ERR_ALLOC && !L, "a lattice that cannot fit was made", "tight lattice");
+            rt.device_limit = SIZE_MAX;
+        }
+}
+
 const struct {
     const char* name;
     void (*run)();
 } CHECKS[] = {{"devices", devices}, {"visibility", visibility}, {"no pinned memory", no_pinned_memory},
               {"no device memory", no_device_memory}, {"earlier error", earlier_error},
-              {"independence", independence}, {"plane memory", plane_memory}};
+              {"independence", independence}, {"plane memory", plane_memory},
+              {"tight lattice", tight_lattice}};
 
 }  // namespace
 

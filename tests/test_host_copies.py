@@ -18,6 +18,7 @@ CHECKS = {
     "earlier error": "an error that an earlier call left behind does not fail a copy",
     "independence": "a copy does not wait for those of other lattices",
     "plane memory": "a deformation plane takes a plane's worth of device memory",
+    "tight lattice": "a lattice that fits the device without padding is made without it",
 }
 
 
