@@ -55,3 +55,25 @@ def test_range_fp32(dims):
         out.append(lat.fields())
     for k in ("u1", "u2", "u3"):
         assert np.abs(out[0][k] - out[1][k]).max() < 2e-6
+
+
+@pytest.mark.parametrize("dims", GRIDS)
+def test_range_of_a_reduction(dims):
+    """What a reduction folds from all parts of a slot, whichever of them the step used:
+    the restatement's range at the start and after 1, 2, 3 and 7 steps, so in each of the
+    three slots, and the extremes of the field.  (The fields pass the two values at both
+    ends.)"""
+    from droplet_amd.lattice import Lattice
+    cfg = make_config(*dims, kappa_g=0.004, nu1=0.05, nu2=0.2, wall_axis=DRP_WALL_Z, wall_u=0.01)
+    f = _state(dims, cfg.phi1, cfg.phi2)
+    lat, ora = Lattice(cfg), OracleLattice(cfg, threads=4)
+    for o in (lat, ora):
+        o.init_fields(*f)
+    for n in (0, 1, 1, 1, 4):
+        for o in (lat, ora):
+            o.step(n)
+        a, b = lat.reduce(), ora.reduce()
+        assert (a["phi_min"], a["phi_max"]) == (b["phi_min"], b["phi_max"])
+        if n > 0:
+            phi = lat.fields()["phi"]
+            assert a["phi_min"] == min(phi.min(), cfg.phi2) and a["phi_max"] == max(phi.max(), cfg.phi1)
