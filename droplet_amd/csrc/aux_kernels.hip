@@ -36,26 +36,6 @@ __device__ void phi_stencil(const Grid& G, const double* phi, int x, int y, int 
     g2 = g2 / 10.0;
 }
 
-// grad u (gu[k][a] = d_a u_k) at (x,y,z) (various_cal :616-633)
-__device__ void u_stencil(const Grid& G, const double* u1, const double* u2, const double* u3, int x, int y, int z,
-                          double gu[3][3]) {
-    for (int k = 0; k < 3; k++)
-        for (int a = 0; a < 3; a++) gu[k][a] = 0.0;
-    sfor<1, 15>([&](auto qc) {
-        constexpr int q = decltype(qc)::value;
-        using D = Dir<q>;
-        const int64_t t = G.at(x + D::cx, y + D::cy, z + D::cz);
-        const double v[3] = {u1[t], u2[t], u3[t]};
-        for (int k = 0; k < 3; k++) {
-            gu[k][0] = acc<D::cx>(gu[k][0], v[k]);
-            gu[k][1] = acc<D::cy>(gu[k][1], v[k]);
-            gu[k][2] = acc<D::cz>(gu[k][2], v[k]);
-        }
-    });
-    for (int k = 0; k < 3; k++)
-        for (int a = 0; a < 3; a++) gu[k][a] = gu[k][a] / 10.0;
-}
-
 // True when the neighbour (xx, yy, zz) (not wrapped) of node (x, y, z) lies
 // outside the node's rank block: program/LES_drop.f90 (:153-157) and
 // LES_drop_xy.f90 (:150-153) take every such neighbour from the halo exchanged
