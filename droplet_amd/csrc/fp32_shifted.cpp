@@ -116,7 +116,7 @@ StepArgs32 make_step_args32(drp_lattice* L, int64_t nstep) {
     a.slot_read = (int)((nstep - 1) % 3);
     a.slot_write = (int)(nstep % 3);
     a.slot_reset = (int)((nstep + 1) % 3);
-    a.range_mask = range_mask((int64_t)c.nx * c.ny * c.nz);
+    a.range_mask = L->range_mask;
     return a;
 }
 

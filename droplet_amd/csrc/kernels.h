@@ -40,21 +40,25 @@ struct Grid {
 // order-preserving integers (d3q15.h).  A slot is kept in parts, 256 bytes apart,
 // each folded into by every eighth workgroup with atomics: on one pair of addresses
 // the workgroups of a small lattice, which end together, queue.  Step with one and with
-// eight parts: 15.2 and 13.3 us at 32^3, 42.4 and 39.8 at 64^3, 25.0 and 18.5 at 64^3 in
-// FP32.  Above RANGE_PARTS_MAX_NODES the workgroups end at different times, eight parts
-// bring nothing (119 and 119 us at 96^3), and a step that reads the range pays for eight
-// loads in each workgroup (viscosity of phi, 256^3: 1984 and 2023 us, FP32 1061 and 1095):
-// there, and below RANGE_PARTS_MIN_NODES, where at most 32 workgroups fold (viscosity of
-// phi, 16^3: 11.6 and 12.1 us), only part 0 takes the folds of a step and only it is read
+// eight parts, us: FP64 98 tiles (28^3) 12.2 and 11.2, 128 (32^3) 12.8 and 10.8, 1024
+// (64^3) 40.5 and 37.7; FP32 64 tiles (32^3) 11.0 and 10.2, 512 (64^3) 23.6 and 18.1,
+// 1728 (96^3) 65.3 and 62.9.  With many more tiles than fit the card at once their
+// workgroups end at different times, eight parts bring nothing, and a step that reads the
+// range pays for eight loads in each workgroup: with the viscosity of phi FP64 2904 tiles
+// (88^3) 101.1 and 102.4, FP32 2704 (104^3) 103.4 and 105.6; 256^3 1984 and 2023.  With
+// few tiles it pays without a queue: FP32 36 tiles (24^3) 11.1 and 11.5, FP64 50 (20^3)
+// 11.6 and 12.1.  On both sides only part 0 takes the folds of a step and only it is read
 // by one.  The parts that take none hold the limits that a slot is reset to, or a range
 // set on all parts, so that the fold over all of them is the range at every size.
 constexpr int RANGE_PARTS = 8, RANGE_PART_WORDS = 32;
 constexpr int RANGE_SLOT_WORDS = RANGE_PARTS * RANGE_PART_WORDS;
 constexpr int RANGE_WORDS = 3 * RANGE_SLOT_WORDS;
-constexpr int64_t RANGE_PARTS_MIN_NODES = 1 << 13, RANGE_PARTS_MAX_NODES = 1 << 19;
-// a step's mask of parts: RANGE_PARTS - 1 or 0
-inline int range_mask(int64_t nodes) {
-    return nodes >= RANGE_PARTS_MIN_NODES && nodes <= RANGE_PARTS_MAX_NODES ? RANGE_PARTS - 1 : 0;
+constexpr int64_t RANGE_PARTS_MIN_TILES = 64, RANGE_PARTS_MAX_TILES = 2048;
+// a lattice's mask of parts, RANGE_PARTS - 1 or 0, from the tiles of its default shape: a
+// step reads the parts that the step before it folded into, so it does not follow a later
+// change of the shape
+inline int range_mask(int64_t tiles) {
+    return tiles >= RANGE_PARTS_MIN_TILES && tiles <= RANGE_PARTS_MAX_TILES ? RANGE_PARTS - 1 : 0;
 }
 // (max, min) of a slot; a step passes its mask
 __device__ __forceinline__ void range_words(const uint64_t* __restrict__ range, int slot, uint64_t& mx, uint64_t& mn,

@@ -241,6 +241,10 @@ int default_shape(int precision) {
     }
     return precision == DRP_FP64 ? SHAPE_32x4x2 : SHAPE_32x4x4;
 }
+static int64_t tile_count(const drp_config& c, int shape) {
+    const int* d = SHAPE_DIMS[shape];
+    return (int64_t)((c.nx + d[0] - 1) / d[0]) * ((c.ny + d[1] - 1) / d[1]) * ((c.nz + d[2] - 1) / d[2]);
+}
 // per-variant default measured at 256^3 on MI355X (drp_autotune): the Allen-Cahn
 // step on 16x4x4 tiles (1.65 against 1.76 ms)
 static int pick_shape(const drp_config& c) {
@@ -266,27 +270,24 @@ int lattice_create(const drp_config* cfg, hipStream_t stream, drp_lattice** out)
     if (hipGetDeviceCount(&ndev) != hipSuccess || ndev == 0) return drp_fail(DRP_ERR_HIP, "no HIP device");
     drp_lattice* L = new (std::nothrow) drp_lattice();
     if (!L) return drp_fail(DRP_ERR_ALLOC, "host allocation failed");
-    L->cfg = *cfg;
-    L->phys = make_phys(*cfg);
-    L->n = (int64_t)cfg->nx * cfg->ny * cfg->nz;
-    L->G = choose_layout(*cfg, true);
-    L->shape = pick_shape(*cfg);
-    L->stream = stream;
-    (void)hipGetDevice(&L->dev);
+    auto describe = [&](bool apart) {
+        *L = drp_lattice();
+        L->cfg = *cfg;
+        L->phys = make_phys(*cfg);
+        L->n = (int64_t)cfg->nx * cfg->ny * cfg->nz;
+        L->G = choose_layout(*cfg, apart);
+        L->shape = pick_shape(*cfg);
+        L->range_mask = range_mask(tile_count(*cfg, L->shape));
+        L->stream = stream;
+        (void)hipGetDevice(&L->dev);
+    };
+    describe(true);
     rc = lattice_alloc(L);
     // rows and arrays lie apart for speed only: back to back where there is no memory for that
     if (rc == DRP_ERR_ALLOC && L->G.ns != L->n) {
         lattice_free(L);
         (void)hipGetLastError();  // the failed allocation is dealt with here
-        const int shape = L->shape, dev = L->dev;
-        *L = drp_lattice();
-        L->cfg = *cfg;
-        L->phys = make_phys(*cfg);
-        L->n = (int64_t)cfg->nx * cfg->ny * cfg->nz;
-        L->G = choose_layout(*cfg, false);
-        L->shape = shape;
-        L->stream = stream;
-        L->dev = dev;
+        describe(false);
         rc = lattice_alloc(L);
     }
     if (rc) {
@@ -598,7 +599,7 @@ StepArgs make_step_args(drp_lattice* L, int64_t nstep) {
     a.slot_read = (int)((nstep - 1) % 3);
     a.slot_write = (int)(nstep % 3);
     a.slot_reset = (int)((nstep + 1) % 3);
-    a.range_mask = range_mask((int64_t)c.nx * c.ny * c.nz);
+    a.range_mask = L->range_mask;
     return a;
 }
 

@@ -21,6 +21,7 @@ struct drp_lattice {
     bool initialized = false;
     bool eq_init = false;  // populations are the equilibria of fields set by drp_init_* (no step since)
     int shape = 0;         // tile shape of the step kernel
+    int range_mask = 0;    // parts of a phi-range slot that its steps use
     int cur = 0;           // which ping-pong buffer holds the current state
     void* pop[2] = {nullptr, nullptr};  // FP64: [f (15 G.ns) | g (15 G.ns)] doubles; FP32: floats
     void* mac[2] = {nullptr, nullptr};  // phi, p, u1, u2, u3 (5 G.ns)

@@ -301,13 +301,36 @@ void tight_lattice() {
         }
 }
 
+// The parts of a phi-range slot that a step uses follow the tiles of the default shape,
+// also on thin lattices, and stay with the lattice: a step reads what the last one folded.
+void range_parts() {
+    const struct {
+        int nx, ny, nz, precision, parts;
+    } cases[] = {{16, 16, 16, DRP_FP64, 1},  {32, 32, 14, DRP_FP64, 1},          {32, 32, 16, DRP_FP64, 8},
+                 {3, 3, 900, DRP_FP64, 8},   {17, 17, 28, DRP_FP64, 8},          {128, 64, 64, DRP_FP64, 8},
+                 {130, 64, 64, DRP_FP64, 1}, {24, 24, 24, DRP_FP32_SHIFTED, 1},  {32, 32, 32, DRP_FP32_SHIFTED, 8},
+                 {3, 3, 900, DRP_FP32_SHIFTED, 8}, {128, 128, 64, DRP_FP32_SHIFTED, 8}, {130, 128, 64, DRP_FP32_SHIFTED, 1}};
+    for (const auto& k : cases) {
+        const drp_config c = config(k.nx, k.ny, k.nz, k.precision);
+        drp_lattice* L = nullptr;
+        done(drp_create(&c, &L), "range parts");
+        if (!L) continue;
+        for (int shape = -1; shape < drp_tile_shape_count(); shape++) {
+            if (shape >= 0) drp_set_tile_shape(L, shape);
+            const int mask = k.precision == DRP_FP64 ? make_step_args(L, 1).range_mask : make_step_args32(L, 1).range_mask;
+            check(mask == k.parts - 1, "wrong parts", where(L) + " shape " + std::to_string(shape));
+        }
+        drp_destroy(L);
+    }
+}
+
 const struct {
     const char* name;
     void (*run)();
 } CHECKS[] = {{"devices", devices}, {"visibility", visibility}, {"no pinned memory", no_pinned_memory},
               {"no device memory", no_device_memory}, {"earlier error", earlier_error},
               {"independence", independence}, {"plane memory", plane_memory},
-              {"tight lattice", tight_lattice}};
+              {"tight lattice", tight_lattice}, {"range parts", range_parts}};
 
 }  // namespace
 

@@ -77,3 +77,34 @@ def test_range_of_a_reduction(dims):
         if n > 0:
             phi = lat.fields()["phi"]
             assert a["phi_min"] == min(phi.min(), cfg.phi2) and a["phi_max"] == max(phi.max(), cfg.phi1)
+
+
+# Tiles of the default shape: 225, 56, 64 and 2560 in both.
+# From 64 to 2048 of them a step folds into eight parts.
+@pytest.mark.parametrize("dims", [(3, 3, 900), (32, 32, 14), (32, 32, 16), (130, 62, 64)])
+def test_range_tile_counts_fp64(dims):
+    test_range_fp64(dims)
+    test_range_of_a_reduction(dims)
+
+
+@pytest.mark.parametrize("dims", [(3, 3, 900), (32, 32, 28), (32, 32, 32), (130, 128, 64)])
+def test_range_tile_counts_fp32(dims):
+    test_range_fp32(dims)
+
+
+def test_range_keeps_its_parts_when_the_tile_shape_changes():
+    """Tiles of another shape from step to step: bit-identical to the restatement, whose
+    viscosity hangs on the range at every node."""
+    from droplet_amd.lattice import Lattice
+    dims = (32, 32, 16)
+    cfg = make_config(*dims, kappa_g=0.004, nu1=0.05, nu2=0.2, wall_axis=DRP_WALL_Z, wall_u=0.01)
+    lat, ora = Lattice(cfg), OracleLattice(cfg, threads=4)
+    for o in (lat, ora):
+        o.init_fields(*_state(dims, cfg.phi1, cfg.phi2))
+    for shape in (0, 6, 1, 2, 4, 3):
+        lat.tile_shape = shape
+        for o in (lat, ora):
+            o.step(1)
+        a, b = lat.fields(), ora.fields()
+        for k in ("phi", "p", "u1", "u2", "u3"):
+            np.testing.assert_array_equal(a[k], b[k])

@@ -19,6 +19,7 @@ CHECKS = {
     "independence": "a copy does not wait for those of other lattices",
     "plane memory": "a deformation plane takes a plane's worth of device memory",
     "tight lattice": "a lattice that fits the device without padding is made without it",
+    "range parts": "the parts of a phi-range slot follow the default shape's tiles and stay with the lattice",
 }
 
 
