@@ -245,6 +245,7 @@ static int64_t tile_count(const drp_config& c, int shape) {
     const int* d = SHAPE_DIMS[shape];
     return (int64_t)((c.nx + d[0] - 1) / d[0]) * ((c.ny + d[1] - 1) / d[1]) * ((c.nz + d[2] - 1) / d[2]);
 }
+constexpr int CUS = 256;  // of an MI355X
 // per-variant default measured at 256^3 on MI355X (drp_autotune): the Allen-Cahn
 // step on 16x4x4 tiles (1.65 against 1.76 ms)
 static int pick_shape(const drp_config& c) {
@@ -256,7 +257,19 @@ static int pick_shape(const drp_config& c) {
     // and 24, 22 and 14; with forces, LES and nu(phi) alike.  Longer rows have no such line
     // (48^3 23.7 and 20.0, 40^3 15.8 and 22.4, 64^3 39.9 and 41.3)
     if (c.nx <= SHAPE_DIMS[SHAPE_16x4x4][0]) return SHAPE_16x4x4;
-    return default_shape(c.precision);
+    const int usual = default_shape(c.precision);
+    // A force field takes two barriers and a pass through LDS more in each workgroup: where
+    // few of them run, a smaller one is done sooner.  FP64 where 16x4x4 tiles leave one
+    // workgroup to a CU and the usual ones two (us a step with forces gathered through L2,
+    // on the usual tiles and on these: 33^3 18.4, 20.1, 14.0; 36^3 19.4, 21.9, 14.8; 100 x 20
+    // x 28 19.5, 22.6, 14.9; with one workgroup on either 64 x 32 x 32 18.5, 13.5, 13.5, with
+    // two 60 x 20 x 64 19.7, 20.7, 22.0); FP32 up to half the CUs (20^3 12.0, 12.3, 10.0;
+    // 28^3 12.7, 13.1, 12.0; 32^3 13.0, 13.1, 10.2; beyond, 48 x 48 x 28 14.5, 12.3, 12.8)
+    if (c.force_kind == DRP_FORCE_FIELD || c.force_kind == DRP_FORCE_SPECTRAL) {
+        const int64_t small = tile_count(c, SHAPE_16x4x4);
+        if (c.precision == DRP_FP64 ? small <= CUS && tile_count(c, usual) > CUS : small <= CUS / 2) return SHAPE_16x4x4;
+    }
+    return usual;
 }
 
 extern "C" int drp_create(const drp_config* cfg, drp_lattice** out) { return lattice_create(cfg, nullptr, out); }

@@ -324,13 +324,33 @@ void range_parts() {
     }
 }
 
+// Default tiles of a lattice with a force field, on both sides of the rule's lines.
+void forced_tiles() {
+    const struct {
+        int nx, ny, nz, precision, shape;
+    } cases[] = {{32, 32, 32, DRP_FP64, drp::SHAPE_32x4x2},         {33, 33, 33, DRP_FP64, drp::SHAPE_16x4x4},
+                 {64, 32, 32, DRP_FP64, drp::SHAPE_32x4x2},         {100, 20, 28, DRP_FP64, drp::SHAPE_16x4x4},
+                 {60, 20, 64, DRP_FP64, drp::SHAPE_32x4x2},         {256, 64, 64, DRP_FP64, drp::SHAPE_32x4x2},
+                 {32, 32, 32, DRP_FP32_SHIFTED, drp::SHAPE_16x4x4}, {32, 32, 33, DRP_FP32_SHIFTED, drp::SHAPE_32x4x4}};
+    for (const auto& k : cases)
+        for (int force : {DRP_FORCE_FIELD, DRP_FORCE_NONE}) {
+            const drp_config c = config(k.nx, k.ny, k.nz, k.precision, force);
+            drp_lattice* L = nullptr;
+            done(drp_create(&c, &L), "forced tiles");
+            if (!L) continue;
+            check(L->shape == (force == DRP_FORCE_FIELD ? k.shape : default_shape(k.precision)), "wrong tiles", where(L));
+            drp_destroy(L);
+        }
+}
+
 const struct {
     const char* name;
     void (*run)();
 } CHECKS[] = {{"devices", devices}, {"visibility", visibility}, {"no pinned memory", no_pinned_memory},
               {"no device memory", no_device_memory}, {"earlier error", earlier_error},
               {"independence", independence}, {"plane memory", plane_memory},
-              {"tight lattice", tight_lattice}, {"range parts", range_parts}};
+              {"tight lattice", tight_lattice}, {"range parts", range_parts},
+              {"forced tiles", forced_tiles}};
 
 }  // namespace
 

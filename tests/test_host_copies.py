@@ -20,6 +20,7 @@ CHECKS = {
     "plane memory": "a deformation plane takes a plane's worth of device memory",
     "tight lattice": "a lattice that fits the device without padding is made without it",
     "range parts": "the parts of a phi-range slot follow the default shape's tiles and stay with the lattice",
+    "forced tiles": "default tiles of lattices with a force field",
 }
 
 
