@@ -49,8 +49,7 @@ int fp32_init_from_host_fields(drp_lattice* L, const double* const* host) {
     HIP_TRY32(hipMalloc(&pop64.p, 30 * ns * sizeof(double)));
     double* m = (double*)mac64.p;
     double* f = (double*)pop64.p;
-    int rc = DRP_OK;
-    for (int k = 0; k < 5 && !rc; k++) rc = nodes_from_host(L, host[k], 1, m + k * ns);
+    int rc = nodes_from_host(L, host, 5, m);
     if (rc) return rc;
     HIP_TRY32(launch_init_equilibrium_fp64(L->G, L->phys, m, f, f + 15 * ns, L->stream));
     HIP_TRY32(launch_to_shifted(L->G, shift_ref(L->cfg), f, m, (float*)L->pop[L->cur], (float*)L->mac[L->cur],

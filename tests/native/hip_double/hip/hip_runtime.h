@@ -6,6 +6,7 @@
 // in `violations` when it is not met.
 #pragma once
 
+#include <atomic>
 #include <cmath>
 #include <condition_variable>
 #include <cstddef>
@@ -83,6 +84,7 @@ struct Runtime {
     std::map<void*, Block> live;
     size_t device_limit = SIZE_MAX, device_bytes = 0;  // hipMalloc fails beyond the limit
     size_t largest = 0;                                // largest device allocation asked for since it was cleared
+    std::atomic<int> copies{0}, launches{0};           // asked for since they were cleared
     int pinned_limit = 1 << 30;                        // blocks of pinned memory that can be had
     std::vector<std::string> violations;
     void violation(const std::string& s) {
@@ -108,6 +110,7 @@ void launch(void (*kernel)(P...), dim3 grid, dim3 block, Stream* s, A&&... args)
         fail(hipErrorInvalidHandle);
         return;
     }
+    rt.launches++;
     grid_dim = grid;
     block_dim = block;
     for (block_idx.x = 0; block_idx.x < grid.x; block_idx.x++)
@@ -218,10 +221,12 @@ inline hipError_t hipEventSynchronize(hipEvent_t e) {
 inline hipError_t hipEventElapsedTime(float* ms, hipEvent_t, hipEvent_t) { return *ms = 0.0f, hipSuccess; }
 inline hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind) { return std::memcpy(d, s, n), hipSuccess; }
 inline hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t) {
+    hip_double::rt.copies++;
     return std::memcpy(d, s, n), hipSuccess;
 }
 inline hipError_t hipMemcpy2DAsync(void* d, size_t dpitch, const void* s, size_t spitch, size_t width, size_t height,
                                    hipMemcpyKind, hipStream_t) {
+    hip_double::rt.copies++;
     for (size_t r = 0; r < height; r++) std::memcpy((char*)d + r * dpitch, (const char*)s + r * spitch, width);
     return hipSuccess;
 }

@@ -343,6 +343,38 @@ void forced_tiles() {
         }
 }
 
+// Arrays with padded rows: one copy where they lie behind each other on the host, and one
+// launch for all.
+void few_copies() {
+    State s(config(45, 22, 26, DRP_FP64, DRP_FORCE_FIELD));
+    auto asked = [&](int copies, int launches, const char* what) {
+        check(rt.copies == copies && rt.launches == launches,
+              (std::to_string(rt.copies) + " copies, " + std::to_string(rt.launches) + " launches").c_str(), what);
+        rt.copies = rt.launches = 0;
+    };
+    const size_t n = (size_t)s.L->n;
+    rt.copies = rt.launches = 0;
+    done(drp_set_force(s.L, s.force[0].data(), s.force[1].data(), s.force[2].data(), n), where(s.L));
+    asked(3, 1, "force");
+    done(drp_set_populations(s.L, 0, s.pop[0].data(), 15 * n), where(s.L));
+    asked(1, 2, "populations and their moments");
+    // rows without padding, arrays apart
+    State d(config(64, 64, 50, DRP_FP64));
+    rt.copies = rt.launches = 0;
+    done(drp_set_populations(d.L, 0, d.pop[0].data(), 15 * (size_t)d.L->n), where(d.L));
+    asked(1, 2, "populations apart");
+    d.write(10);
+    // more than one buffer's worth: 4 of 131 x 70 x 97 at a time
+    State t(config(131, 70, 97, DRP_FP64));
+    t.write(11);
+    rt.device_limit = rt.device_bytes - 3 * (size_t)t.L->n * sizeof(double);  // and room for one
+    (void)hipFree(t.L->pack);
+    t.L->pack = nullptr;
+    t.L->pack_cap = 0;
+    t.write(12);
+    rt.device_limit = SIZE_MAX;
+}
+
 const struct {
     const char* name;
     void (*run)();
@@ -350,7 +382,7 @@ const struct {
               {"no device memory", no_device_memory}, {"earlier error", earlier_error},
               {"independence", independence}, {"plane memory", plane_memory},
               {"tight lattice", tight_lattice}, {"range parts", range_parts},
-              {"forced tiles", forced_tiles}};
+              {"forced tiles", forced_tiles}, {"few copies", few_copies}};
 
 }  // namespace
 
