@@ -445,14 +445,6 @@ __global__ __launch_bounds__(256) void pack_rows(int nx, int64_t rows, int64_t s
     if (row < rows) packed[i] = nodes[(i - row * nx) + stride * row];
 }
 
-// contiguous arrays of nx ny nz doubles each to `count` node arrays; one thread per value
-__global__ __launch_bounds__(256) void unpack_nodes(Grid G, int count, const double* __restrict__ packed,
-                                                    double* __restrict__ nodes) {
-    const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    const int64_t row = i / G.nx, rows = (int64_t)G.ny * G.nz, a = row / rows;
-    if (a < count) nodes[a * G.ns + G.px * (row - a * rows) + (i - row * G.nx)] = packed[i];
-}
-
 __global__ void range_set(uint64_t* range, int slot, double vmax, double vmin) {
     range_set_part(range, slot, threadIdx.x, ordered_bits(vmax), ordered_bits(vmin));
 }
@@ -506,12 +498,6 @@ hipError_t launch_reduce_fp64(const Grid& G, const Phys& ph, const double* mac, 
 
 hipError_t launch_pack_rows(int nx, int64_t rows, int64_t stride, const double* nodes, double* packed, hipStream_t st) {
     hipLaunchKernelGGL(pack_rows, dim3(nblk(nx * rows, 256)), dim3(256), 0, st, nx, rows, stride, nodes, packed);
-    return hipGetLastError();
-}
-
-hipError_t launch_unpack_nodes(const Grid& G, int count, const double* packed, double* nodes, hipStream_t st) {
-    hipLaunchKernelGGL(unpack_nodes, dim3(nblk((int64_t)G.nx * G.ny * G.nz * count, 256)), dim3(256), 0, st, G, count,
-                       packed, nodes);
     return hipGetLastError();
 }
 

@@ -1,4 +1,4 @@
-// host_io.hip — node arrays to the caller's host memory.
+// host_io.hip — node arrays to the caller's host memory, and from there.
 //
 // The caller's arrays are pageable, and usually fresh: the runtime's own copy moves
 // them through one staging buffer with one host thread, which also takes the page
@@ -6,7 +6,8 @@
 // its steps).  Here a kernel drops the row padding (and widens FP32 deviations)
 // straight into pinned host memory, chunk by chunk, and several host threads copy the
 // chunks out (one thread, for short arrays), so that the link, the copies and the page
-// faults overlap: 19 ms.
+// faults overlap: 19 ms.  Arrays from the host go the same way back, except where the
+// runtime's copies are the faster ones.
 //
 // The pinned chunks belong to the process: at most POOL_SLOTS of CHUNK_BYTES (64 MiB),
 // made on demand, shared by all lattices and threads, and freed with the last lattice.  A
@@ -40,6 +41,12 @@ constexpr int POOL_SLOTS = 2 * MAX_SLOTS;  // chunks of the process
 // FP32 members of 48..128^3, one thread 18 ms; the fields of 256^3 take 86 ms with
 // one and 35 ms with eight threads there, 63 and 17 ms on idle cores.
 constexpr int64_t PER_THREAD = (int64_t)1 << 21;
+// Host arrays of DIRECT_MIN doubles (512 KiB) or more go in by the runtime's copies as long as
+// they are DIRECT_TOTAL (16 MiB) together, which it reads where they lie faster than one
+// thread fills chunks: three force fields of 64^3 190 us, by chunks 234.  Shorter ones it may
+// write through the bus at 3 GB/s (24^3 44 or 150 us, by chunks 35), longer ones it moves
+// one after the other (populations of 128^3 8.4 ms, by chunks 5.2; of 64^3 880 us and 790).
+constexpr int64_t DIRECT_MIN = (int64_t)1 << 16, DIRECT_TOTAL = (int64_t)1 << 21;
 constexpr int64_t SHORT_CHUNK = (int64_t)1 << 17;  // doubles (1 MiB): smallest chunk of a transfer in parts
 
 // values [first, first + len) of the contiguous sequence of node arrays (nx ny nz
@@ -153,10 +160,11 @@ int to_host_unpinned(drp_lattice* L, const Grid& G, const T* nodes, int count, c
     return DRP_OK;
 }
 
-template <typename T>
-int to_host(drp_lattice* L, const Grid& G, const T* nodes, int count, const HostRef& ref, double* host) {
-    const OnDevice on(L->dev);
-    const int64_t total = (int64_t)G.nx * G.ny * G.nz * count;
+// Moves `total` values in chunks, each by launch(first, len, chunk), a kernel between the
+// node arrays and the pinned chunk, and copy(first, len, chunk), the host's part: after the
+// kernel to the host (OUT), before it from there.  `found` is false where there is no chunk.
+template <bool OUT, typename Launch, typename Copy>
+int transfer(drp_lattice* L, int64_t total, Launch&& launch, Copy&& copy, bool* found) {
     const int cores = std::max(1, (int)std::thread::hardware_concurrency());
     const int want = (int)std::max<int64_t>(1, std::min<int64_t>({MAX_SLOTS, cores, total / PER_THREAD}));
     std::vector<void*> slot;
@@ -165,32 +173,34 @@ int to_host(drp_lattice* L, const Grid& G, const T* nodes, int count, const Host
     } catch (...) {
         return drp_fail(DRP_ERR_ALLOC, "host allocation failed");
     }
-    if (slot.empty()) return to_host_unpinned(L, G, nodes, count, ref, host);
+    *found = !slot.empty();
+    if (slot.empty()) return DRP_OK;
     const int nt = std::min<int>(want, (int)slot.size()), deep = want == 1 ? (int)slot.size() : 1;
     const int64_t chunk = std::min(CHUNK, nt > 1 ? (total + nt - 1) / nt : std::max(SHORT_CHUNK, (total + 3) / 4));
     const int64_t chunks = (total + chunk - 1) / chunk;
     std::atomic<int64_t> next{0};
     std::atomic<int> failed{(int)hipSuccess};
-    // each thread takes the next chunk, has its slot filled (with two slots the other one
-    // meanwhile), waits for it and empties it
+    // each thread takes the next chunk and moves it through its slot (with two slots the other
+    // one meanwhile)
     auto work = [&](int t, bool own_thread) {
         hipError_t e = own_thread ? hipSetDevice(L->dev) : hipSuccess;
         hipEvent_t ev[2] = {nullptr, nullptr};
         int64_t chunk_of[2] = {chunks, chunks};
         for (int k = 0; k < deep && e == hipSuccess && chunks > 1; k++)
             e = hipEventCreateWithFlags(&ev[k], hipEventDisableTiming);
+        auto len_of = [&](int k) { return std::min(chunk, total - chunk_of[k] * chunk); };
         auto fill = [&](int k) {
-            const int64_t c = chunk_of[k] = next.fetch_add(1);
-            if (c >= chunks || e != hipSuccess) return;
-            e = launch_pack(G, nodes, ref, c * chunk, std::min(chunk, total - c * chunk), (double*)slot[t + k], L->stream);
+            chunk_of[k] = next.fetch_add(1);
+            if (chunk_of[k] >= chunks || e != hipSuccess) return;
+            if (!OUT) copy(chunk_of[k] * chunk, len_of(k), (double*)slot[t + k]);
+            e = launch(chunk_of[k] * chunk, len_of(k), (double*)slot[t + k]);
             if (e == hipSuccess && ev[k]) e = hipEventRecord(ev[k], L->stream);
         };
         for (int k = 0; k < deep; k++) fill(k);
         for (int k = 0; e == hipSuccess && chunk_of[k] < chunks && failed.load() == (int)hipSuccess; k = (k + 1) % deep) {
             e = ev[k] ? hipEventSynchronize(ev[k]) : hipStreamSynchronize(L->stream);
             if (e != hipSuccess) break;
-            const int64_t first = chunk_of[k] * chunk;
-            std::memcpy(host + first, slot[t + k], (size_t)std::min(chunk, total - first) * sizeof(double));
+            if (OUT) copy(chunk_of[k] * chunk, len_of(k), (double*)slot[t + k]);
             fill(k);
         }
         for (int k = 0; k < 2; k++)
@@ -206,11 +216,73 @@ int to_host(drp_lattice* L, const Grid& G, const T* nodes, int count, const Host
     }
     work(0, false);
     for (int t = 1; t < started; t++) threads[t].join();
-    // (a failed transfer may still have a kernel writing to a slot)
+    // (a failed transfer may still have a kernel at work on a slot)
     if (failed.load() != (int)hipSuccess) (void)hipStreamSynchronize(L->stream);
     slots().give(slot);
     const hipError_t e = (hipError_t)failed.load();
-    if (e != hipSuccess) return drp_fail(DRP_ERR_HIP, "copy to the host failed: %s", hipGetErrorString(e));
+    if (e != hipSuccess)
+        return drp_fail(DRP_ERR_HIP, "copy %s the host failed: %s", OUT ? "to" : "from", hipGetErrorString(e));
+    return DRP_OK;
+}
+
+template <typename T>
+int to_host(drp_lattice* L, const Grid& G, const T* nodes, int count, const HostRef& ref, double* host) {
+    const OnDevice on(L->dev);
+    bool found = false;
+    const int rc = transfer<true>(
+        L, (int64_t)G.nx * G.ny * G.nz * count,
+        [&](int64_t first, int64_t len, double* slot) { return launch_pack(G, nodes, ref, first, len, slot, L->stream); },
+        [&](int64_t first, int64_t len, double* slot) { std::memcpy(host + first, slot, len * sizeof(double)); }, &found);
+    return rc || found ? rc : to_host_unpinned(L, G, nodes, count, ref, host);
+}
+
+// values [first, first + len) of the arrays that follow each other, from a chunk to the
+// node arrays
+__global__ __launch_bounds__(256) void unpack_in(Grid G, const double* __restrict__ in, int64_t first, int64_t len,
+                                                 double* __restrict__ nodes) {
+    const int64_t n = (int64_t)G.nx * G.ny * G.nz;
+    for (int64_t j = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; j < len; j += (int64_t)gridDim.x * blockDim.x) {
+        const int64_t i = first + j, a = i / n, s = i - a * n, row = s / G.nx;
+        nodes[a * G.ns + G.px * row + (s - row * G.nx)] = in[j];
+    }
+}
+
+hipError_t launch_unpack(const Grid& G, const double* in, int64_t first, int64_t len, double* nodes, hipStream_t st) {
+    const unsigned nb = (unsigned)std::min<int64_t>((len + 255) / 256, 1024);
+    hipLaunchKernelGGL(unpack_in, dim3(nb), dim3(256), 0, st, G, in, first, len, nodes);
+    return hipGetLastError();
+}
+
+// Host arrays by the runtime's own copies: padded rows through a buffer without gaps, as
+// many arrays at a time as DIRECT_TOTAL holds, or row by row where there is no memory for
+// one; one copy for arrays that lie behind each other on both sides.
+int from_host_direct(drp_lattice* L, const double* const* host, int count, double* nodes) {
+    const Grid& G = L->G;
+    const int64_t n = L->n;
+    const size_t row = G.nx * sizeof(double);
+    const bool padded = G.px != G.nx;
+    int group = padded ? (int)std::max<int64_t>(1, std::min<int64_t>(count, DIRECT_TOTAL / n)) : count;
+    double* pack = nullptr;
+    while (padded && !(pack = pack_buffer(L, (size_t)group * n)) && group > 1) group /= 2;
+    hipError_t e = hipSuccess;
+    for (int k0 = 0; k0 < count && e == hipSuccess; k0 += group) {
+        const int k1 = std::min(count, k0 + group);
+        for (int k = k0, next; k < k1 && e == hipSuccess; k = next) {
+            double* const dst = pack ? pack + (k - k0) * n : nodes + k * G.ns;
+            next = k + 1;
+            if (pack || (!padded && G.ns == n))
+                while (next < k1 && host[next] == host[next - 1] + n) next++;
+            if (pack || !padded)
+                e = hipMemcpyAsync(dst, host[k], (next - k) * n * sizeof(double), hipMemcpyHostToDevice, L->stream);
+            else
+                e = hipMemcpy2DAsync(dst, G.px * sizeof(double), host[k], row, row, (size_t)G.ny * G.nz,
+                                     hipMemcpyHostToDevice, L->stream);
+        }
+        if (pack && e == hipSuccess) e = launch_unpack(G, pack, 0, (k1 - k0) * n, nodes + k0 * G.ns, L->stream);
+    }
+    const hipError_t s = hipStreamSynchronize(L->stream);
+    if (e == hipSuccess) e = s;
+    if (e != hipSuccess) return drp_fail(DRP_ERR_HIP, "copy from the host failed: %s", hipGetErrorString(e));
     return DRP_OK;
 }
 
@@ -225,4 +297,33 @@ int nodes_to_host(drp_lattice* L, const double* nodes, int count, double* host) 
 
 int nodes_to_host(drp_lattice* L, const float* nodes, int count, const HostRef& ref, double* host) {
     return to_host(L, L->G, nodes, count, ref, host);
+}
+
+int nodes_from_host(drp_lattice* L, const double* const* host, int count, double* nodes) {
+    const OnDevice on(L->dev);
+    const int64_t n = L->n, total = n * count;
+    bool found = false;
+    if (n < DIRECT_MIN || total > DIRECT_TOTAL) {
+        const int rc = transfer<false>(
+            L, total,
+            [&](int64_t first, int64_t len, double* slot) { return launch_unpack(L->G, slot, first, len, nodes, L->stream); },
+            [&](int64_t first, int64_t len, double* slot) {
+                while (len > 0) {
+                    const int64_t a = first / n, at = first - a * n, m = std::min(len, n - at);
+                    std::memcpy(slot, host[a] + at, m * sizeof(double));
+                    first += m;
+                    slot += m;
+                    len -= m;
+                }
+            },
+            &found);
+        if (rc || found) return rc;
+    }
+    return from_host_direct(L, host, count, nodes);
+}
+
+int nodes_from_host(drp_lattice* L, const double* host, int count, double* nodes) {
+    const double* h[15];
+    for (int k = 0; k < count; k++) h[k] = host + k * L->n;
+    return nodes_from_host(L, h, count, nodes);
 }

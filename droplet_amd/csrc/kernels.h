@@ -255,8 +255,6 @@ hipError_t launch_reduce_fp64(const Grid& G, const Phys& ph, const double* mac, 
                               double* work, hipStream_t st);
 // rows of nx doubles, `stride` apart, to contiguous rows
 hipError_t launch_pack_rows(int nx, int64_t rows, int64_t stride, const double* nodes, double* packed, hipStream_t st);
-// contiguous arrays of nx ny nz doubles to `count` node arrays
-hipError_t launch_unpack_nodes(const Grid& G, int count, const double* packed, double* nodes, hipStream_t st);
 // fill a range slot with (max, min) = (vmax, vmin)
 hipError_t launch_range_set(uint64_t* range, int slot, double vmax, double vmin, hipStream_t st);
 

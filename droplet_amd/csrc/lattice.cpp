@@ -6,7 +6,6 @@
 // launch per time step on the handle's stream.
 #include <hip/hip_runtime.h>
 
-#include <algorithm>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -140,49 +139,6 @@ double* pack_buffer(drp_lattice* L, size_t doubles) {
         }
     }
     return L->pack;
-}
-
-// Arrays with padded rows go through a buffer without gaps, as many at a time as 32 MiB hold:
-// one copy for those that lie behind each other on the host, and one launch for all.  So do
-// arrays that lie apart here only, if they lie behind each other on the host and the buffer
-// holds them all.  With a copy (and a launch) per array the populations of 100 x 50 x 30
-// took 763 us and those of 56^3 692; this way 529 and 611 (518 and 595 where arrays have no
-// gaps).  Others go straight (96^3 in four buffers 3.95 ms, straight 3.9), in one copy where
-// they are back to back on both sides.  Without memory for the buffer the runtime copies
-// padded rows one by one.
-constexpr size_t PACK_DOUBLES = (size_t)4 << 20;
-int nodes_from_host(drp_lattice* L, const double* const* host, int count, double* nodes) {
-    const OnDevice on(L->dev);
-    const Grid& G = L->G;
-    const size_t n = (size_t)L->n, row = G.nx * sizeof(double);
-    const bool padded = G.px != G.nx;
-    int group = (int)std::max<size_t>(1, std::min<size_t>(count, PACK_DOUBLES / n));
-    const bool gather = padded || (G.ns != L->n && count > 1 && group == count && host[1] == host[0] + n);
-    double* pack = nullptr;
-    while (gather && !(pack = pack_buffer(L, group * n)) && group > 1) group /= 2;
-    if (!gather) group = count;
-    for (int k0 = 0; k0 < count; k0 += group) {
-        const int k1 = std::min(count, k0 + group);
-        for (int k = k0, e; k < k1; k = e) {
-            double* const dst = pack ? pack + (k - k0) * n : nodes + k * G.ns;
-            e = k + 1;
-            if (pack || (!padded && G.ns == L->n))
-                while (e < k1 && host[e] == host[e - 1] + n) e++;
-            if (pack || !padded)
-                HIP_TRY(hipMemcpyAsync(dst, host[k], (e - k) * n * sizeof(double), hipMemcpyHostToDevice, L->stream));
-            else
-                HIP_TRY(hipMemcpy2DAsync(dst, G.px * sizeof(double), host[k], row, row, (size_t)G.ny * G.nz,
-                                         hipMemcpyHostToDevice, L->stream));
-        }
-        if (pack) HIP_TRY(launch_unpack_nodes(G, k1 - k0, pack, nodes + k0 * G.ns, L->stream));
-    }
-    return DRP_OK;
-}
-
-int nodes_from_host(drp_lattice* L, const double* host, int count, double* nodes) {
-    const double* h[15];
-    for (int k = 0; k < count; k++) h[k] = host + k * L->n;
-    return nodes_from_host(L, h, count, nodes);
 }
 
 static int validate(const drp_config* c) {

@@ -91,14 +91,13 @@ struct HostRef {
 };
 int nodes_to_host(drp_lattice* L, const double* nodes, int count, double* host);
 int nodes_to_host(drp_lattice* L, const float* nodes, int count, const HostRef& ref, double* host);
+// and `count` contiguous host arrays to node arrays, each where it lies or one behind the other
+int nodes_from_host(drp_lattice* L, const double* const* host, int count, double* nodes);
+int nodes_from_host(drp_lattice* L, const double* host, int count, double* nodes);
 // a lattice that uses it exists, or no longer does
 void host_io_retain();
 void host_io_release();
-// lattice.cpp: `count` contiguous host arrays to node arrays; host memory may be let go on
-// return, the arrays are there in stream order
-int nodes_from_host(drp_lattice* L, const double* const* host, int count, double* nodes);
-int nodes_from_host(drp_lattice* L, const double* host, int count, double* nodes);  // one behind the other
-// L->pack with room for that many doubles; null where there is no memory for it
+// lattice.cpp: L->pack with room for that many doubles; null where there is no memory for it
 double* pack_buffer(drp_lattice* L, size_t doubles);
 
 // spectral_diag.hip

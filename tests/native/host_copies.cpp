@@ -192,11 +192,13 @@ void no_pinned_memory() {
         for (int precision : {DRP_FP64, DRP_FP32_SHIFTED}) {
             State s(config(g[0], g[1], g[2], precision, DRP_FORCE_FIELD));
             s.read("values differ");
+            if (precision == DRP_FP64) s.write(13);
             // FP64 values need no memory of the device on their way either
             if (precision == DRP_FP64) {
                 State t(config(g[0], g[1], g[2], precision, DRP_FORCE_NONE));
                 rt.device_limit = rt.device_bytes;
                 t.read("values differ without device memory");
+                t.write(14);
                 rt.device_limit = SIZE_MAX;
             }
         }
@@ -343,36 +345,40 @@ void forced_tiles() {
         }
 }
 
-// Arrays with padded rows: one copy where they lie behind each other on the host, and one
-// launch for all.
-void few_copies() {
-    State s(config(45, 22, 26, DRP_FP64, DRP_FORCE_FIELD));
-    auto asked = [&](int copies, int launches, const char* what) {
-        check(rt.copies == copies && rt.launches == launches,
-              (std::to_string(rt.copies) + " copies, " + std::to_string(rt.launches) + " launches").c_str(), what);
+// Host arrays of a call go in together: through chunks (one launch where they fit one), or,
+// where the arrays are long and few, by the runtime's copies and one launch that unpacks
+// padded rows.
+void together() {
+    const struct {
+        int nx, ny, nz, force_copies, force_launches, pop_copies, pop_launches;
+    } cases[] = {{16, 7, 5, 0, 1, 0, 1}, {45, 22, 26, 0, 1, 0, 3}, {100, 50, 30, 3, 1, 0, 5}, {44, 40, 40, 3, 1, 1, 1},
+                 {48, 40, 40, 3, 0, 1, 0}};
+    for (const auto& k : cases) {
+        State s(config(k.nx, k.ny, k.nz, DRP_FP64, DRP_FORCE_FIELD));
+        const size_t n = (size_t)s.L->n;
+        auto asked = [&](int copies, int launches, const char* what) {
+            check(rt.copies == copies && rt.launches == launches,
+                  (std::to_string(rt.copies) + " copies, " + std::to_string(rt.launches) + " launches").c_str(),
+                  where(s.L) + " " + what);
+            rt.copies = rt.launches = 0;
+        };
         rt.copies = rt.launches = 0;
-    };
-    const size_t n = (size_t)s.L->n;
-    rt.copies = rt.launches = 0;
-    done(drp_set_force(s.L, s.force[0].data(), s.force[1].data(), s.force[2].data(), n), where(s.L));
-    asked(3, 1, "force");
-    done(drp_set_populations(s.L, 0, s.pop[0].data(), 15 * n), where(s.L));
-    asked(1, 2, "populations and their moments");
-    // rows without padding, arrays apart
-    State d(config(64, 64, 50, DRP_FP64));
-    rt.copies = rt.launches = 0;
-    done(drp_set_populations(d.L, 0, d.pop[0].data(), 15 * (size_t)d.L->n), where(d.L));
-    asked(1, 2, "populations apart");
-    d.write(10);
-    // more than one buffer's worth: 4 of 131 x 70 x 97 at a time
-    State t(config(131, 70, 97, DRP_FP64));
-    t.write(11);
-    rt.device_limit = rt.device_bytes - 3 * (size_t)t.L->n * sizeof(double);  // and room for one
-    (void)hipFree(t.L->pack);
-    t.L->pack = nullptr;
-    t.L->pack_cap = 0;
-    t.write(12);
-    rt.device_limit = SIZE_MAX;
+        done(drp_set_force(s.L, s.force[0].data(), s.force[1].data(), s.force[2].data(), n), where(s.L));
+        asked(k.force_copies, k.force_launches, "force");
+        done(drp_set_populations(s.L, 0, s.pop[0].data(), 15 * n), where(s.L));
+        asked(k.pop_copies, k.pop_launches + 1, "populations");  // (and their moments)
+        s.write(15);
+    }
+    // less memory than the runtime's copies ask for: an array at a time, then row by row
+    State t(config(44, 40, 40, DRP_FP64, DRP_FORCE_FIELD));
+    for (size_t room : {(size_t)8, (size_t)1, (size_t)0}) {
+        if (t.L->pack) (void)hipFree(t.L->pack);
+        t.L->pack = nullptr;
+        t.L->pack_cap = 0;
+        rt.device_limit = rt.device_bytes + room * (size_t)t.L->n * sizeof(double);
+        t.write(16 + (unsigned)room);
+        rt.device_limit = SIZE_MAX;
+    }
 }
 
 const struct {
@@ -382,7 +388,7 @@ const struct {
               {"no device memory", no_device_memory}, {"earlier error", earlier_error},
               {"independence", independence}, {"plane memory", plane_memory},
               {"tight lattice", tight_lattice}, {"range parts", range_parts},
-              {"forced tiles", forced_tiles}, {"few copies", few_copies}};
+              {"forced tiles", forced_tiles}, {"together", together}};
 
 }  // namespace
 

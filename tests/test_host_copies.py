@@ -21,7 +21,7 @@ CHECKS = {
     "tight lattice": "a lattice that fits the device without padding is made without it",
     "range parts": "the parts of a phi-range slot follow the default shape's tiles and stay with the lattice",
     "forced tiles": "default tiles of lattices with a force field",
-    "few copies": "host arrays go into padded node arrays in few copies and launches",
+    "together": "the host arrays of a call go in together",
 }
 
 
