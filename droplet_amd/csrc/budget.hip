@@ -468,12 +468,11 @@ extern "C" int drp_get_derived(drp_lattice* L, int kind, double* host, size_t n_
     double* out = nullptr;
     HIP_TRYB(hipMalloc((void**)&out, (size_t)L->n * sizeof(double)));
     hipError_t e = launch_derived_fp64(L->G, L->phys, mac, kind, out, L->cfg.nx, L->stream);
-    if (e == hipSuccess) e = hipMemcpyAsync(host, out, (size_t)L->n * sizeof(double), hipMemcpyDeviceToHost, L->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(L->stream);
+    const int rc = e == hipSuccess ? dense_to_host(L, out, host) : DRP_OK;
     const hipError_t f = hipFree(out);
     if (e == hipSuccess) e = f;
     if (e != hipSuccess) return drp_fail(DRP_ERR_HIP, "drp_get_derived: %s", hipGetErrorString(e));
-    return DRP_OK;
+    return rc;
 }
 
 extern "C" int drp_step_energy_budget(drp_lattice* L, double* terms) {

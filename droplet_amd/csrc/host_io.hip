@@ -299,6 +299,10 @@ int nodes_to_host(drp_lattice* L, const float* nodes, int count, const HostRef& 
     return to_host(L, L->G, nodes, count, ref, host);
 }
 
+int dense_to_host(drp_lattice* L, const double* values, double* host) {
+    return to_host(L, Grid{L->G.nx, L->G.ny, L->G.nz, L->G.nx, L->n}, values, 1, HostRef{}, host);
+}
+
 int nodes_from_host(drp_lattice* L, const double* const* host, int count, double* nodes) {
     const OnDevice on(L->dev);
     const int64_t n = L->n, total = n * count;

@@ -91,6 +91,7 @@ struct HostRef {
 };
 int nodes_to_host(drp_lattice* L, const double* nodes, int count, double* host);
 int nodes_to_host(drp_lattice* L, const float* nodes, int count, const HostRef& ref, double* host);
+int dense_to_host(drp_lattice* L, const double* values, double* host);  // n values without gaps
 // and `count` contiguous host arrays to node arrays, each where it lies or one behind the other
 int nodes_from_host(drp_lattice* L, const double* const* host, int count, double* nodes);
 int nodes_from_host(drp_lattice* L, const double* host, int count, double* nodes);

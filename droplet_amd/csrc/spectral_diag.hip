@@ -773,8 +773,8 @@ extern "C" int drp_filter_velocity(drp_lattice* L, int kind, int k, double* u1, 
         hipLaunchKernelGGL(real_part_scaled, dim3(nb), dim3(256), 0, L->stream, n, (const double2*)ca, 1.0 / (double)n,
                            (double*)out.p);
         HIP_TRYS(hipGetLastError());
-        HIP_TRYS(hipMemcpyAsync(dst[a], out.p, (size_t)n * sizeof(double), hipMemcpyDeviceToHost, L->stream));
-        HIP_TRYS(hipStreamSynchronize(L->stream));
+        rc = dense_to_host(L, (const double*)out.p, dst[a]);
+        if (rc) return rc;
     }
     return DRP_OK;
 }
