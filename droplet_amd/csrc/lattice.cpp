@@ -217,18 +217,21 @@ static int64_t tile_count(const drp_config& c, int shape) {
     const int* d = SHAPE_DIMS[shape];
     return (int64_t)((c.nx + d[0] - 1) / d[0]) * ((c.ny + d[1] - 1) / d[1]) * ((c.nz + d[2] - 1) / d[2]);
 }
+// Rows of up to 16 nodes leave half of a 32-wide tile's threads without a node.  Step
+// on the default and on 16x4x4 tiles, FP64 and FP32: 16^3 11.0 and 10.5 us, 9.8 and 8.2;
+// 16x64x64 17.3 and 12.7, 11.4 and 9.4; 16x200x200 136 and 88, 74 and 74; 8x100x100 35
+// and 24, 22 and 14; with forces, LES and nu(phi) alike.  Longer rows have no such line
+// (48^3 23.7 and 20.0, 40^3 15.8 and 22.4, 64^3 39.9 and 41.3)
+bool short_rows(const drp_config& c) {
+    return !std::getenv("DROPLET_SHAPE") && c.nx <= SHAPE_DIMS[SHAPE_16x4x4][0];
+}
 constexpr int CUS = 256;  // of an MI355X
 // per-variant default measured at 256^3 on MI355X (drp_autotune): the Allen-Cahn
 // step on 16x4x4 tiles (1.65 against 1.76 ms)
 static int pick_shape(const drp_config& c) {
     if (std::getenv("DROPLET_SHAPE")) return default_shape(c.precision);
     if (c.model == DRP_MODEL_ALLEN_CAHN) return SHAPE_16x4x4;
-    // rows of up to 16 nodes leave half of a 32-wide tile's threads without a node.  Step
-    // on the default and on 16x4x4 tiles, FP64 and FP32: 16^3 11.0 and 10.5 us, 9.8 and 8.2;
-    // 16x64x64 17.3 and 12.7, 11.4 and 9.4; 16x200x200 136 and 88, 74 and 75; 8x100x100 35
-    // and 24, 22 and 14; with forces, LES and nu(phi) alike.  Longer rows have no such line
-    // (48^3 23.7 and 20.0, 40^3 15.8 and 22.4, 64^3 39.9 and 41.3)
-    if (c.nx <= SHAPE_DIMS[SHAPE_16x4x4][0]) return SHAPE_16x4x4;
+    if (short_rows(c)) return SHAPE_16x4x4;
     const int usual = default_shape(c.precision);
     // A force field takes two barriers and a pass through LDS more in each workgroup: where
     // few of them run, a smaller one is done sooner.  FP64 where 16x4x4 tiles leave one

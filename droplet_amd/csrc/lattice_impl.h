@@ -73,6 +73,7 @@ int lattice_create(const drp_config* cfg, hipStream_t stream, drp_lattice** out)
 void lattice_free(drp_lattice* L);
 drp::StepArgs make_step_args(drp_lattice* L, int64_t nstep);
 int default_shape(int precision);
+bool short_rows(const drp_config& c);  // 16x4x4 tiles suit the lattice better, by its rows
 // SPECTRAL: recompute the force field from the current velocity (FP64 or FP32 fields)
 int spectral_update(drp_lattice* L, int64_t nstep);
 // scale-separated advection: the band-passed velocity the step's phi equilibria carry

@@ -65,3 +65,30 @@ def test_batch_tile_shapes_and_errors():
         b.step(1)
     with pytest.raises(DropletError):
         Batch([make_config(16), make_config(16, precision=DRP_FP32_SHIFTED)])
+
+
+@pytest.mark.parametrize("precision", [DRP_FP64, DRP_FP32_SHIFTED])
+@pytest.mark.parametrize("sizes", [[32] * 7, [32] * 8, [16, 12, 9], [16, 12, 17]], ids=["7", "8", "short", "not_short"])
+def test_batch_defaults(precision, sizes):
+    """On both sides of the numbers of members from which each folds its phi range in one
+    part, and of the row length up to which the tiles are narrow: steps of the batch, of its
+    members by themselves and of the batch again give what each gives alone."""
+    from droplet_amd.lattice import Batch, Lattice
+    cfgs = [make_config(n, n + i % 3, 20, precision=precision, nu1=0.05, nu2=0.2, kappa_g=0.004) for i, n in enumerate(sizes)]
+    drops = [[(0.5 * n, 0.4 * n, 8.0, 0.6 * n)] for n in sizes]
+    b = Batch(cfgs)
+    for m, d in zip(b.members, drops):
+        m.init_droplets(d)
+    b.step(8)
+    b.sync()
+    for m in b.members:
+        m.step(2)
+    b.step(7)
+    b.sync()
+    for m, cfg, d in zip(b.members, cfgs, drops):
+        solo = Lattice(cfg)
+        solo.init_droplets(d)
+        solo.step(17)
+        a, s = m.fields(), solo.fields()
+        for k in a:
+            np.testing.assert_array_equal(a[k], s[k])
