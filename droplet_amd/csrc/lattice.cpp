@@ -106,17 +106,20 @@ static int row_pitch(int nx, int ny, size_t esz) {
 // Elements from one population (or field) array to the next.  A step reads and
 // writes 70 arrays at the same offset in each; where their length is a large power
 // of two they meet in the same memory channels.  Arrays of 1 MiB and more therefore
-// start on 256-byte boundaries and 8 KiB + 256 B further apart than their length.
-// MLUPS of the shear droplet, arrays back to back -> apart: FP64 128^3 5040..6080 ->
-// 8070, 192^3 7860 -> 8240, 256^3 8130 -> 8350; FP32 128^3 14030 -> 15050, 256^3
-// 14730 -> 15850; 240^3 unchanged.  Of 0, 256, 512 .. 4096, 4352, 8448, 16640, 64 KiB,
-// 1 MiB and 2 MiB + 4352 B this is the best or within 2 % of it at all of these.
+// start on 256-byte boundaries and 20 KiB + 256 B further apart than their length.
+// Step of the shear droplet, arrays back to back -> apart, us: FP64 128^3 366..430 -> 267,
+// 192^3 880 -> 840, 256^3 2090 -> 1980; FP32 128^3 153..162 -> 144, 256^3 1130 -> 1047; 8
+// batched members of 64^3 281 -> 265, 3 of 128^3 1093 -> 787; 96^3 and 240^3 unchanged (FP32
+// batches of 96^3 339 -> 345).  Of 256, 4352, 8448, 12544, 20736, 28928, 37120, 65792 and
+// 69888 B this is within 4 % of the best at 30 sizes and batches, on three cards.  8 KiB +
+// 256 B, as good for one lattice, depends on where the allocations of several lie: 265 or
+// 331 us for the members of 64^3.
 // Shorter arrays stay back to back: they live in the caches, and one copy moves a
 // whole population set to the host.
 static int64_t stream_stride(int64_t slots, size_t esz) {
     const int64_t bytes = slots * (int64_t)esz;
     if (bytes < ((int64_t)1 << 20)) return slots;
-    return ((bytes + 255) / 256 * 256 + 8192 + 256) / (int64_t)esz;
+    return ((bytes + 255) / 256 * 256 + 20480 + 256) / (int64_t)esz;
 }
 
 static Grid choose_layout(const drp_config& c, bool apart) {
