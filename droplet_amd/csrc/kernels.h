@@ -10,7 +10,9 @@ enum { FORCE_NONE = 0, FORCE_TAYLOR_GREEN = 1, FORCE_FIELD = 2 };
 
 // Map the linear workgroup id to a tile so that each XCD (workgroups are dealt
 // round-robin to the 8 XCDs) gets a contiguous block of tiles: neighbouring
-// tiles, which share halo lines, then share one L2.
+// tiles, which share halo lines, then share one L2.  Where the number of workgroups is no
+// multiple of 8 the id is the tile, and neighbours lie on different XCDs (a launch may
+// round its number up: adjoint.hip).
 __device__ __forceinline__ int xcd_tile(int b, int nb) {
     if ((nb & 7) != 0) return b;
     return (b & 7) * (nb >> 3) + (b >> 3);

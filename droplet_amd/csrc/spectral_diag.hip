@@ -601,7 +601,11 @@ void diag_free(drp_lattice* L) {
 
 namespace {
 
-constexpr int SHELL_WGS = 1280;  // five workgroups of the z pass per CU
+// Workgroups of the z pass.  The lines and the bins of one take 33 KiB of LDS at 256^3, so
+// four fit a CU: of 1280 the last 256 start when others end.  1024 are no better: energy
+// spectrum 807 us with 1280, 834 with 1024, interaction 2081 and 2044 (768: 771 and 2154;
+// 128^3 212 and 209, 415 and 416).
+constexpr int SHELL_WGS = 1280;
 
 // L->diag with room for `spectra` half spectra
 int diag_get(drp_lattice* L, int spectra, drp_diag** out) {

@@ -18,6 +18,9 @@
  *  - The library owns all device memory; callers own host buffers.
  *  - One lattice handle is bound to one HIP stream; calls on one handle must be
  *    serialised by the caller.  Separate handles are independent.
+ *  - Calls that take or return host arrays work from any thread, whatever device is
+ *    current in it, and share up to 64 MiB of pinned host memory in the process while
+ *    lattices exist.
  *  - Naming: "phi populations" are the order-parameter populations (reference `f`),
  *    "momentum populations" carry pressure and momentum (reference `g`).
  *  - Host field layout is x fastest, then y, then z: index = x + nx*(y + ny*z).
@@ -379,8 +382,10 @@ int drp_droplet_census(drp_lattice* lat, double threshold, int64_t* count, int64
  * (the Nyquist plane k3 = nz/2 included, as the reference counts it), for
  * s = 0 .. nshells-1 (the reference's enesupe(s+1), an array of nx/2 + 1;
  * modes of higher shells, which it writes past that array, are dropped here).
- * The transforms' work space stays with the lattice from the first of these calls
- * on and is freed by drp_destroy. */
+ * The work space of drp_energy_spectrum, drp_scale_interaction and
+ * drp_phi_contribution (one, four and two half spectra of 8.5 B per node, and the shell
+ * sums) stays with the lattice, grows with the first call that needs more of it, and is
+ * freed by drp_destroy.  drp_filter_velocity allocates 56 B per node for each call. */
 int drp_energy_spectrum(drp_lattice* lat, double* E, int nshells);
 
 /* Spectral filters of the velocity (results to host, x fastest):
